@@ -271,6 +271,239 @@ __global__ __launch_bounds__(SC_NT) void k_qk_scores(qk_params P) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// Many query vectors per KV head (a question pass: G x Lq of them) on the matrix cores.
+//
+// The kernel above streams K once per four query vectors: at 192 vectors (48 queries, 4 heads a group) K passes 48 times
+// and the vector unit does the dot products (1536 rows x 32768 keys, head_dim 128: 520 us). Here K passes once: a wave
+// keeps 64 keys as matrix operands in registers for the whole kernel, the query vectors come by in chunks of 64 through
+// LDS (two buffers, one barrier per chunk), S^T = K Q^T in 32x32x16 steps: 44 us, 49 with the causal mask. What bounds it
+// is memory: 67 MB of K in and 100 MB of keys out take 35 us at the rate of a large copy; chunks of 32 vectors and three
+// or four waves per SIMD change nothing. The accumulator has four consecutive keys of one vector in a lane; rounded to the storage type they cross the
+// wave's own LDS tile so that every store is 16 bytes and every row gets whole 128-byte lines.
+// ---------------------------------------------------------------------------
+#define QM_NT 256
+#define QM_NW (QM_NT / SAH_WAVE)
+#define QM_KEYS 64                  // keys per wave
+#define QM_TILE (QM_KEYS * QM_NW)   // keys per workgroup
+#define QM_VECS 64                  // query vectors per LDS chunk
+#define QM_MIN_WGS 1024             // the vectors are dealt to several workgroups until there are this many
+
+// two rounded scores (storage type, packed) -> their two sort keys; -0 ranks as +0
+__device__ __forceinline__ uint32_t qm_sort_key2(uint32_t x) {
+  const uint32_t neg = ((x >> 15) & 0x00010001u) * 0xffffu;               // all ones in the negative halves
+  const uint32_t zero = (sah_pk_ne01_u16(x, 0x80008000u) ^ 0x00010001u) * 0xffffu;  // ... in the halves that hold -0
+  return (x ^ (neg | 0x80008000u)) ^ zero;
+}
+
+// (a native vector: an array of HIP's uint4, a structure, that is filled in one place and stored in another stays in memory)
+typedef uint32_t qm_u4 __attribute__((ext_vector_type(4)));
+typedef qm_u4 qm_u4_any __attribute__((aligned(2)));  // 16 bytes at an address that is only element aligned
+
+// a score's rounding remainder in DT's own bits, as k_qk_scores leaves it
+template <int DT>
+__device__ __forceinline__ uint32_t qm_remainder(float d) {
+  const float s = sah_round<DT>(d);
+  if (DT == SAH_BF16) return sah_float_to_bits(d - s) >> 16;
+  return fabsf(s) < INFINITY ? (uint32_t)sah_float_to_f16(d - s) : 0u;
+}
+
+template <int DT, int D, bool AM, bool RES>
+__global__ __launch_bounds__(QM_NT, 2) void k_qk_scores_mfma(qk_params P, int chunks_per_wg) {
+  static_assert(DT != SAH_F32 && (D == 64 || D == 128), "16-bit types, whole 16-dimension steps");
+  sah_touch_kernargs<sizeof(qk_params) + 8>();
+  constexpr int KS = D / 16;          // matrix steps per 32x32 tile
+  constexpr int QP = D + 8;           // elements per query row in LDS: 16 bytes of padding against bank conflicts
+  constexpr int OP = QM_KEYS + 8;     // elements per row of the output tile
+  constexpr int UPT = QM_VECS * (D / 8) / QM_NT;  // 16-byte units of a chunk per thread
+  __shared__ uint16_t s_q[2][QM_VECS * QP];
+  __shared__ uint16_t s_o[QM_NW][32 * OP];
+  __shared__ int s_row[2][QM_VECS];        // mask row of a vector, -1 beyond the last
+  __shared__ int64_t s_moff[2][AM ? QM_VECS : 1];
+  const int tid = threadIdx.x;
+  const int lane = tid & (SAH_WAVE - 1);
+  const int wave = sah_wave_id();
+  const int i32 = lane & 31, g = lane >> 5;
+  const int G = P.Hq / P.Hkv;
+  const int nvec = G * P.Lq;
+  const int bhk = blockIdx.y;
+  const int hk = bhk % P.Hkv;
+  const int b = bhk / P.Hkv;
+  const int n_chunks = (nvec + QM_VECS - 1) / QM_VECS;
+  const int c0 = blockIdx.z * chunks_per_wg;
+  const int c1 = c0 + chunks_per_wg < n_chunks ? c0 + chunks_per_wg : n_chunks;
+  if (c0 >= c1) return;
+
+  // a chunk's query vectors on their way to LDS; vectors beyond the last repeat it and are never stored
+  qm_u4 qr[UPT];
+  auto fetch = [&](int c) {
+#pragma unroll
+    for (int u = 0; u < UPT; ++u) {
+      const int idx = tid + u * QM_NT;
+      int v = c * QM_VECS + idx / (D / 8);
+      if (v >= nvec) v = nvec - 1;
+      const int h = hk * G + v / P.Lq, qi = v % P.Lq;
+      qr[u] = *(const qm_u4*)((const uint16_t*)P.q + (int64_t)b * P.qs_b + (int64_t)h * P.qs_h + (int64_t)qi * P.qs_l +
+                              (idx % (D / 8)) * 8);
+    }
+  };
+  auto park = [&](int c, int buf) {
+#pragma unroll
+    for (int u = 0; u < UPT; ++u) {
+      const int idx = tid + u * QM_NT;
+      *(qm_u4*)&s_q[buf][(idx / (D / 8)) * QP + (idx % (D / 8)) * 8] = qr[u];
+    }
+    if (tid < QM_VECS) {
+      const int v = c * QM_VECS + tid;
+      const int h = hk * G + v / P.Lq, qi = v % P.Lq;
+      s_row[buf][tid] = v < nvec ? (b * P.Hq + h) * P.Lq + qi : -1;
+      if (AM) s_moff[buf][tid] = (int64_t)b * P.ms_b + (int64_t)h * P.ms_h + (int64_t)qi * P.ms_l;
+    }
+  };
+
+  // this wave's keys as A operands: 2 tiles of 32 rows, lane (row i32, half g) holds dims 16 s + 8 g .. + 7
+  const int j0 = blockIdx.x * QM_TILE + wave * QM_KEYS;
+  uint4 kf[2][KS];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    int j = j0 + 32 * t + i32;
+    if (j > P.Lk - 1) j = P.Lk - 1;  // keys past the end repeat the last one; their scores are not stored
+    const uint16_t* kp = (const uint16_t*)P.k + (int64_t)b * P.ks_b + (int64_t)hk * P.ks_h + (int64_t)j * P.ks_l + 8 * g;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) kf[t][s] = *(const uint4*)(kp + 16 * s);
+  }
+  fetch(c0);
+  park(c0, 0);
+  __syncthreads();
+
+  for (int c = c0; c < c1; ++c) {
+    const int buf = (c - c0) & 1;
+    const bool more = c + 1 < c1;  // uniform across the workgroup
+    if (more) fetch(c + 1);
+    const int n_vt = nvec - c * QM_VECS > 32 ? 2 : 1;
+    for (int vt = 0; vt < n_vt; ++vt) {
+      sah_f32x16 acc0, acc1;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc0[v] = acc1[v] = 0.f;
+      const uint16_t* qrow = &s_q[buf][(vt * 32 + i32) * QP + 8 * g];
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        const uint4 bq = *(const uint4*)(qrow + 16 * s);
+        acc0 = sah_mfma_32x32x16<DT>(kf[0][s], bq, acc0);
+        acc1 = sah_mfma_32x32x16<DT>(kf[1][s], bq, acc1);
+      }
+      // lane (vector i32, g): element v is key 8 (v / 4) + 4 g + v % 4 of its tile
+      uint16_t* orow = &s_o[wave][i32 * OP + 4 * g];
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        *(uint2*)(orow + 8 * q4) = make_uint2(sah_pack2_hw<DT>(acc0[4 * q4], acc0[4 * q4 + 1]), sah_pack2_hw<DT>(acc0[4 * q4 + 2], acc0[4 * q4 + 3]));
+        *(uint2*)(orow + 32 + 8 * q4) = make_uint2(sah_pack2_hw<DT>(acc1[4 * q4], acc1[4 * q4 + 1]), sah_pack2_hw<DT>(acc1[4 * q4 + 2], acc1[4 * q4 + 3]));
+      }
+      sah_wave_lds_sync();
+      // eight keys of a row per lane, eight rows per store
+      const int k8 = (lane & 7) * 8;
+      const int j = j0 + k8;
+#pragma unroll
+      for (int it = 0; it < 4; ++it) {
+        const int rl = it * 8 + (lane >> 3);
+        const uint4 sc = *(const uint4*)&s_o[wave][rl * OP + k8];
+        const int row = s_row[buf][vt * 32 + rl];
+        uint32_t w[4] = {sc.x, sc.y, sc.z, sc.w};
+        const bool whole = row >= 0 && j + 8 <= P.Lk;
+        if (AM) {
+          const uint16_t* mp = (const uint16_t*)P.amask + s_moff[buf][vt * 32 + rl] + j;
+          uint32_t m[4] = {0u, 0u, 0u, 0u};
+          if (whole) {
+            const qm_u4 mv = *(const qm_u4_any*)mp;
+            m[0] = mv.x; m[1] = mv.y; m[2] = mv.z; m[3] = mv.w;
+          } else if (row >= 0) {
+#pragma unroll
+            for (int t = 0; t < 8; ++t)
+              if (j + t < P.Lk) m[t >> 1] |= (uint32_t)mp[t] << (16 * (t & 1));
+          }
+          if (__ballot((m[0] | m[1] | m[2] | m[3]) != 0)) {  // most of a mask is zeros: nothing to add, nothing to round
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+              float lo, hi, mlo, mhi;
+              if (DT == SAH_BF16) {
+                lo = sah_bits_to_float(w[t] << 16); hi = sah_bits_to_float(w[t] & 0xffff0000u);
+                mlo = sah_bits_to_float(m[t] << 16); mhi = sah_bits_to_float(m[t] & 0xffff0000u);
+              } else {
+                lo = sah_f16_to_float((uint16_t)w[t]); hi = sah_f16_to_float((uint16_t)(w[t] >> 16));
+                mlo = sah_f16_to_float((uint16_t)m[t]); mhi = sah_f16_to_float((uint16_t)(m[t] >> 16));
+              }
+              w[t] = sah_pack2_hw<DT>(lo + mlo, hi + mhi);
+            }
+          }
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) w[t] = qm_sort_key2(w[t]);
+        uint16_t* kout = (uint16_t*)P.keys_out + (int64_t)row * P.key_pitch + j;
+        if (whole) {
+          *(uint4*)kout = make_uint4(w[0], w[1], w[2], w[3]);
+        } else if (row >= 0) {
+#pragma unroll
+          for (int t = 0; t < 8; ++t)
+            if (j + t < P.Lk) kout[t] = (uint16_t)(w[t >> 1] >> (16 * (t & 1)));
+        }
+      }
+      sah_wave_lds_sync();  // the tile is free again
+      if constexpr (RES) {
+        // the remainders the same way, through the same tile
+        auto rem2 = [](float lo, float hi) { return qm_remainder<DT>(lo) | (qm_remainder<DT>(hi) << 16); };
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4) {
+          *(uint2*)(orow + 8 * q4) = make_uint2(rem2(acc0[4 * q4], acc0[4 * q4 + 1]), rem2(acc0[4 * q4 + 2], acc0[4 * q4 + 3]));
+          *(uint2*)(orow + 32 + 8 * q4) = make_uint2(rem2(acc1[4 * q4], acc1[4 * q4 + 1]), rem2(acc1[4 * q4 + 2], acc1[4 * q4 + 3]));
+        }
+        sah_wave_lds_sync();
+#pragma unroll
+        for (int it = 0; it < 4; ++it) {
+          const int rl = it * 8 + (lane >> 3);
+          const uint4 rm = *(const uint4*)&s_o[wave][rl * OP + k8];
+          const int row = s_row[buf][vt * 32 + rl];
+          uint16_t* rout = (uint16_t*)P.resid_out + (int64_t)row * P.key_pitch + j;
+          if (row >= 0 && j + 8 <= P.Lk) {
+            *(uint4*)rout = rm;
+          } else if (row >= 0) {
+            const uint32_t w[4] = {rm.x, rm.y, rm.z, rm.w};
+#pragma unroll
+            for (int t = 0; t < 8; ++t)
+              if (j + t < P.Lk) rout[t] = (uint16_t)(w[t >> 1] >> (16 * (t & 1)));
+          }
+        }
+        sah_wave_lds_sync();
+      }
+    }
+    if (more) park(c + 1, buf ^ 1);  // last read before the previous barrier
+    __syncthreads();
+  }
+}
+
+// May this call run on the matrix cores, and does it pay? More query vectors per KV head than one pass of the streaming
+// kernel serves (4): from there on that kernel reads K twice, this one once.
+static bool qm_ok(const sah_qk_scores_args* a) {
+  return a->dtype != SAH_F32 && (a->D == 64 || a->D == 128) && (a->Hq / a->Hkv) * a->Lq > SC_NQ &&
+         a->key_pitch % 8 == 0 && ((uintptr_t)a->keys_out | (uintptr_t)a->resid_out) % 16 == 0;
+}
+
+template <int DT, int D>
+static int qm_launch(const sah_qk_scores_args* a, const qk_params& P) {
+  const int nvec = (a->Hq / a->Hkv) * a->Lq;
+  const int tiles = (a->Lk + QM_TILE - 1) / QM_TILE;
+  const int n_chunks = (nvec + QM_VECS - 1) / QM_VECS;
+  const int64_t wgs = (int64_t)tiles * a->B * a->Hkv;
+  int z = (int)((QM_MIN_WGS + wgs - 1) / wgs);
+  if (z > n_chunks) z = n_chunks;
+  const int per = (n_chunks + z - 1) / z;
+  dim3 g(tiles, a->B * a->Hkv, (n_chunks + per - 1) / per);
+  sah_timed timed("k_qk_scores_mfma", a->stream);
+  if (a->amask) hipLaunchKernelGGL((k_qk_scores_mfma<DT, D, true, false>), g, dim3(QM_NT), 0, (hipStream_t)a->stream, P, per);
+  else if (a->resid_out) hipLaunchKernelGGL((k_qk_scores_mfma<DT, D, false, true>), g, dim3(QM_NT), 0, (hipStream_t)a->stream, P, per);
+  else hipLaunchKernelGGL((k_qk_scores_mfma<DT, D, false, false>), g, dim3(QM_NT), 0, (hipStream_t)a->stream, P, per);
+  return sah_launch_status("sah_qk_scores");
+}
+
 template <int DT, int D, bool FULL>
 static int qk_launch(const sah_qk_scores_args* a, const qk_params& P) {
   const int G = a->Hq / a->Hkv;
@@ -331,6 +564,10 @@ extern "C" int sah_qk_scores(const sah_qk_scores_args* a) {
   P.resid_out = a->resid_out;
   if (a->resid_out && (a->amask || a->dtype == SAH_F32 || (a->D != 64 && a->D != 128)))
     return sah_fail(SAH_EINVAL, "sah_qk_scores: resid_out needs a 16-bit dtype, head_dim 64 or 128 and no additive mask");
+  if (qm_ok(a)) {
+    if (a->dtype == SAH_BF16) return a->D == 128 ? qm_launch<SAH_BF16, 128>(a, P) : qm_launch<SAH_BF16, 64>(a, P);
+    return a->D == 128 ? qm_launch<SAH_F16, 128>(a, P) : qm_launch<SAH_F16, 64>(a, P);
+  }
   switch (a->dtype) {
     case SAH_F32: return qk_dispatch_d<SAH_F32>(a, P);
     case SAH_BF16: return qk_dispatch_d<SAH_BF16>(a, P);
