@@ -147,6 +147,23 @@ static int att_launch(const sah_attention_args* a, const att_params& P, bool tim
 }
 
 template <int DT>
+static int att_combine_d(const sah_attention_args* a, int n_split) {
+  sah_timed timed("k_attn_combine", a->stream);
+  if (a->D == 64)
+    hipLaunchKernelGGL((k_attn_combine<DT, 64>), dim3(a->rows.n_rows), dim3(64), 0, (hipStream_t)a->stream, (const float*)a->work,
+                       n_split, a->Hq, a->Lq, a->D, a->sinks, a->out, a->stats_out);
+  else
+    hipLaunchKernelGGL((k_attn_combine<DT, 128>), dim3(a->rows.n_rows), dim3(128), 0, (hipStream_t)a->stream, (const float*)a->work,
+                       n_split, a->Hq, a->Lq, a->D, a->sinks, a->out, a->stats_out);
+  return sah_launch_status("sah_members_attention(combine)");
+}
+
+// merges n_split partial results per row (16-bit types, head_dim 64 / 128): for the matrix-core form
+int att_launch_combine(const sah_attention_args* a, int n_split) {
+  return a->dtype == SAH_BF16 ? att_combine_d<SAH_BF16>(a, n_split) : att_combine_d<SAH_F16>(a, n_split);
+}
+
+template <int DT>
 static int att_dispatch_d(const sah_attention_args* a, const att_params& P, bool timing) {
   switch (a->D) {
     case 16: return att_launch<DT, 16, true>(a, P, timing);
@@ -347,6 +364,7 @@ extern "C" int sah_run_chain(const sah_chain_args* a) {
   if (a->pq_adc && (rc = sah_pq_adc_scores(a->pq_adc))) return rc;
   if (a->select && a->attention) return sah_select_topk_attention(a->select, a->attention, a->tickets);  // one kernel when shapes allow
   if (a->select && (rc = sah_select_topk(a->select))) return rc;
+  if (a->attention && a->attention->Lq > 1 && !a->hash_decode) return sah_members_attention(a->attention);  // bitmaps are complete
   if (a->attention && (rc = sah_sparse_attention(a->attention))) return rc;
   return SAH_OK;
 }

@@ -583,3 +583,5 @@ static inline bool att_use_row_form(int n_rows, int max_cnt) {
 
 // defined with the attention kernels: validation of a sah_sparse_attention call and its parameter block
 int att_prepare(const sah_attention_args* a, att_params& P);
+// ... and of the matrix-core form for many query vectors per KV head: is it the better one for this (prepared) call?
+bool members_attention_pays(const sah_attention_args* a, const att_params& P);

@@ -173,9 +173,11 @@ extern "C" int sah_select_topk_attention(const sah_select_topk_args* s, const sa
       // one workgroup per row pays when the rows are short enough for the whole-row form; several per row always
       // several workgroups per row read the row's count while one of them rewrites it: fresh rows only
       (parts > 1 ? (tickets && t->work && t->work_floats >= need && s->fresh) : worst <= 8192);
-  if (!one_kernel) {
+  // several queries per row: the rows' bitmaps, once complete, let the attention run dense on the matrix cores
+  const bool members = t->Lq > 1 && !s->skip_bitmap && members_attention_pays(t, A);
+  if (!one_kernel || members) {
     if ((rc = sah_select_topk(s))) return rc;
-    return sah_sparse_attention(t);
+    return members ? sah_members_attention(t) : sah_sparse_attention(t);
   }
   selattn_params P;
   P.R = s->rows;

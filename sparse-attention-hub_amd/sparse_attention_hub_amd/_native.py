@@ -53,6 +53,8 @@ EXPECTED_SYMBOLS = (
     "sah_sparse_attention_work_floats",
     "sah_sparse_attention",
     "sah_sparse_attention_static",
+    "sah_members_attention_work_floats",
+    "sah_members_attention",
     "sah_attention_weights",
     "sah_run_chain",
     "sah_amask_classify",
@@ -419,10 +421,13 @@ def lib() -> C.CDLL:
     handle.sah_last_error.restype = C.c_char_p
     handle.sah_sparse_attention_work_floats.restype = C.c_int64
     handle.sah_sparse_attention_work_floats.argtypes = [C.c_int32, C.c_int32, C.c_int32]
+    handle.sah_members_attention_work_floats.restype = C.c_int64
+    handle.sah_members_attention_work_floats.argtypes = [C.c_int32] * 6
     handle.sah_pq_adc_lut_bytes.restype = C.c_int64
     handle.sah_pq_adc_lut_bytes.argtypes = [C.c_int32] * 7
     for name in EXPECTED_SYMBOLS:
         if name in ("sah_version", "sah_last_error", "sah_sparse_attention_work_floats", "sah_pq_adc_lut_bytes",
+                    "sah_members_attention_work_floats",
                     "sah_timing_enable", "sah_timing_collect"):
             continue
         if name == "sah_hash_signatures_pair":
@@ -480,6 +485,10 @@ def timing_collect(max_names: int = 64):
 
 def work_floats(n_rows: int, max_cnt: int, head_dim: int) -> int:
     return int(lib().sah_sparse_attention_work_floats(n_rows, max_cnt, head_dim))
+
+
+def members_work_floats(B: int, Hq: int, Hkv: int, Lq: int, Lk: int, head_dim: int) -> int:
+    return int(lib().sah_members_attention_work_floats(B, Hq, Hkv, Lq, Lk, head_dim))
 
 
 def require_device(t: torch.Tensor, what: str) -> None:

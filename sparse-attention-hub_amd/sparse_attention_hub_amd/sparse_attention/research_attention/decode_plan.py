@@ -252,7 +252,8 @@ class DecodePlan:
             se = self.select
             se.rows, se.keys, se.key_pitch, se.key_bits = rows, self.keybuf.data_ptr(), self.keybuf_pitch, self.key_bits
             se.n_cand, se.col_offset, se.k, se.excluded_key, se.stream = Lk, 0, k_eff, self._excluded_min, stream
-            se.skip_bitmap = 1  # only the attention reads these rows, and it reads the column lists
+            # only the attention reads these rows: one query per row by the column lists, several by the bitmaps
+            se.skip_bitmap = 1 if Lq == 1 else 0
             chain.select = C.addressof(se)
             if Lq == 1:
                 # one query per row: the selection kernel writes the sink + local rows itself
@@ -307,7 +308,8 @@ class DecodePlan:
             se = self.select
             se.rows, se.keys, se.key_pitch, se.key_bits = rows, self.keybuf.data_ptr(), self.keybuf_pitch, self.key_bits
             se.n_cand, se.col_offset, se.k, se.excluded_key, se.stream = current, off, k_eff, self._excluded_min, stream
-            se.skip_bitmap = 1  # only the attention reads these rows, and it reads the column lists
+            # only the attention reads these rows: one query per row by the column lists, several by the bitmaps
+            se.skip_bitmap = 1 if Lq == 1 else 0
             chain.select = C.addressof(se)
             if Lq == 1:
                 # one query per row: the selection kernel writes the sink + local rows itself
@@ -317,7 +319,10 @@ class DecodePlan:
                 se.fresh = 0
 
         out = torch.empty((self.B, Lq, self.Hq, self.D), dtype=self.dtype, device=self.device)
-        work = _workspace(self.device, N.work_floats(self.n_rows, cap, self.D))
+        floats = N.work_floats(self.n_rows, cap, self.D)
+        if Lq > 1:
+            floats = max(floats, N.members_work_floats(self.B, self.Hq, self.Hkv, Lq, Lk, self.D))
+        work = _workspace(self.device, floats)
         at = self.att
         at.rows = rows
         at.q, at.qs_b, at.qs_h, at.qs_l = q.data_ptr(), q.stride(0), q.stride(1), q.stride(2)

@@ -152,6 +152,8 @@ def _run_attention(
     if out is None:
         out = torch.empty((B, Lq, Hq, D), dtype=q.dtype, device=dev)
     floats = N.work_floats(n_rows, max_cnt, D)
+    if Lq > 1:  # many query vectors per KV head: the matrix-core form keeps partial results of its own
+        floats = max(floats, N.members_work_floats(B, Hq, Hkv, Lq, Lk, D))
     work = _workspace(dev, floats)
     logits = stats = None
     if return_attention_weights:
@@ -182,7 +184,8 @@ def _run_attention(
             and sk.ndim == 2 and sk.shape[0] == n_rows and sk.stride(1) == 1 and sk.stride(0) >= Lk
             and sr.dtype == sk.dtype and sr.shape == sk.shape and sr.stride() == sk.stride()):
         args.score_keys, args.score_resid, args.score_pitch = sk.data_ptr(), sr.data_ptr(), sk.stride(0)
-    N.call("sah_sparse_attention", args)
+    # the rows' bitmap is coherent with their lists here (or the call is dense)
+    N.call("sah_members_attention" if Lq > 1 else "sah_sparse_attention", args)
     if return_stats:
         return out, stats
     weights = None

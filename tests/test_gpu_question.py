@@ -73,3 +73,64 @@ def test_scores_of_many_query_vectors(cuda, dtype, kind, shape):
         assert bool(((s.double() + rem.double() - exact).abs() <= 2.0 ** -15 * exact.abs() + D * 2.0 ** -24 * mass + 2.0 ** -24).all())
         s2, _, keys2 = score_keys(N, q, k, None)
         assert torch.equal(keys, keys2)  # the remainders change nothing about the keys
+
+
+def launched(N):
+    names = set(N.timing_collect())
+    N.timing_enable(False)
+    return names
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("kind", [None, "causal", "general"])
+@pytest.mark.parametrize("shape,density", [  # rows per KV head around 32, 64 and 128; keys around a 32-key tile and a 64-key
+    # stage; batches that make these small calls rows enough for the matrix-core form
+    ((12, 8, 2, 8, 257, 128), 0.3), ((14, 14, 2, 5, 300, 64), 0.5), ((8, 4, 1, 40, 130, 128), 0.2), ((1, 8, 2, 33, 1000, 64), 0.3),
+    ((1, 8, 2, 32, 1025, 128), 0.1), ((160, 2, 2, 2, 31, 128), 1.0), ((64, 4, 2, 3, 96, 64), None)])
+def test_attention_of_many_query_vectors(cuda, dtype, kind, shape, density):
+    """Against fp64. Bound per element: half a unit of the output type, the two-term weights (2^-16 of sum p |v|), and the
+    logit's error (fp32 products and the mask's addition: D 2^-23 of the largest |q||k|) in the weights.
+    density None: no mask at all (dense attention)."""
+    import sparse_attention_hub_amd.sparse_attention as sa
+    from sparse_attention_hub_amd import _native as N
+    from sparse_attention_hub_amd.sparse_attention.utils.mask_attention_utils import get_masked_attention_output
+
+    B, Hq, Hkv, Lq, Lk, D = shape
+    q, k, v = make_qkv(B, Hq, Hkv, Lq, Lk, D, dtype, seed=3, device=cuda)
+    am = question_mask(B, Lq, Lk, dtype, cuda, kind)
+    sinks = torch.linspace(-1.0, 2.0, Hq) if kind == "causal" else None
+    if density is None:
+        member = torch.ones(B, Hq, Lq, Lk, dtype=torch.bool)
+        mask = sa.Mask.create_full_mask((B, Hq, Lq, Lk), dtype=dtype, device=cuda)
+    else:
+        g = torch.Generator().manual_seed(1)
+        member = torch.rand(B, Hq, Lq, Lk, generator=g) < density
+        member[..., 0] = True           # no empty row
+        member[0, 0, 0, 1:] = False     # a row of one entry
+        member[0, -1, -1, :] = True     # and one of all
+        mask = sa.Mask.create_mask_from_dense_mask((B, Hq, Lq, Lk), member.to(dtype).to(cuda), dtype)
+    N.timing_enable(True)
+    out = get_masked_attention_output(None, q, k, v, am, None if sinks is None else sinks.to(cuda), D ** -0.5, 0.0, mask)
+    torch.cuda.synchronize()
+    assert "k_members_attn_mfma" in launched(N)
+
+    G = Hq // Hkv
+    qq, kk, vv = q.double().cpu(), k.double().cpu().repeat_interleave(G, 1), v.double().cpu().repeat_interleave(G, 1)
+    z = qq @ kk.transpose(-1, -2) * D ** -0.5
+    if am is not None:
+        z = z + am.double().cpu()
+    z = z.masked_fill(~member, -float("inf"))
+    top = z.amax(-1, keepdim=True)
+    e = torch.exp(z - top)
+    den = e.sum(-1, keepdim=True)
+    if sinks is not None:
+        den = den + torch.exp(sinks.double().view(1, Hq, 1, 1) - top)
+    p = e / den
+    ref = (p @ vv).transpose(1, 2)
+    mass = (p @ vv.abs()).transpose(1, 2)
+    half = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)  # 8 / 11 significant bits: half a unit is 2^-8 / 2^-11 of the value at most
+    logit = D * 2.0 ** -23 * float((qq.abs() @ kk.abs().transpose(-1, -2)).max()) * D ** -0.5
+    tiny = 2.0 ** -24 if dtype == torch.float16 else 0.0  # fp16: weights below its normal range lose their second term
+    bound = half * ref.abs() * 1.01 + (2.0 ** -16 + 2 * logit) * mass + 1e-6 + tiny * vv.abs().sum(2).amax()
+    worst = float(((out.double().cpu() - ref).abs() / bound).max())
+    assert worst <= 1.0, worst
