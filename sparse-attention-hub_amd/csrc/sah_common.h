@@ -8,7 +8,7 @@
 #include <stdarg.h>
 #include <type_traits>
 
-#include "../../include/sah.h"
+#include "../../include/sah_ext.h"
 
 #define SAH_WAVE 64
 

@@ -53,13 +53,15 @@ EXPECTED_SYMBOLS = (
     "sah_sparse_attention_work_floats",
     "sah_sparse_attention",
     "sah_sparse_attention_static",
-    "sah_members_attention_work_floats",
-    "sah_members_attention",
     "sah_attention_weights",
     "sah_run_chain",
     "sah_amask_classify",
     "sah_select_topk_attention",
 )
+# include/sah_ext.h: name -> number of argument blocks
+EXTENSION_SYMBOLS = {
+    "sah_members_attention": 1,
+}
 
 
 class NativeLibraryError(RuntimeError):
@@ -427,7 +429,6 @@ def lib() -> C.CDLL:
     handle.sah_pq_adc_lut_bytes.argtypes = [C.c_int32] * 7
     for name in EXPECTED_SYMBOLS:
         if name in ("sah_version", "sah_last_error", "sah_sparse_attention_work_floats", "sah_pq_adc_lut_bytes",
-                    "sah_members_attention_work_floats",
                     "sah_timing_enable", "sah_timing_collect"):
             continue
         if name == "sah_hash_signatures_pair":
@@ -441,6 +442,9 @@ def lib() -> C.CDLL:
         fn = getattr(handle, name)
         fn.restype = C.c_int
         fn.argtypes = [C.c_void_p]
+    for name, n_blocks in EXTENSION_SYMBOLS.items():
+        getattr(handle, name).restype = C.c_int
+        getattr(handle, name).argtypes = [C.c_void_p] * n_blocks
     _lib = handle
     return handle
 
