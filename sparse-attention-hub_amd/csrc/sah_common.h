@@ -330,6 +330,17 @@ __device__ __forceinline__ uint32_t sah_pk_ne01_u16(uint32_t a, uint32_t b) {
 #endif
 }
 
+// two rounded scores (storage type, packed) -> their two sort keys; -0 ranks as +0
+__device__ __forceinline__ uint32_t sah_sort_key2(uint32_t x) {
+  const uint32_t neg = ((x >> 15) & 0x00010001u) * 0xffffu;               // all ones in the negative halves
+  const uint32_t zero = (sah_pk_ne01_u16(x, 0x80008000u) ^ 0x00010001u) * 0xffffu;  // ... in the halves that hold -0
+  return (x ^ (neg | 0x80008000u)) ^ zero;
+}
+
+// (a native vector: an array of HIP's uint4, a structure, that is filled in one place and stored in another stays in memory)
+typedef uint32_t sah_u4 __attribute__((ext_vector_type(4)));
+typedef sah_u4 sah_u4_any __attribute__((aligned(2)));  // 16 bytes at an address that is only element aligned
+
 // ---------------------------------------------------------------------------
 // Hand-over between workgroups of one kernel, without a cache write-back.
 // An MI355X has eight L2 caches (one per die). A device-scope release fence makes a workgroup's ordinary stores

@@ -289,17 +289,6 @@ __global__ __launch_bounds__(SC_NT) void k_qk_scores(qk_params P) {
 #define QM_VECS 64                  // query vectors per LDS chunk
 #define QM_MIN_WGS 1024             // the vectors are dealt to several workgroups until there are this many
 
-// two rounded scores (storage type, packed) -> their two sort keys; -0 ranks as +0
-__device__ __forceinline__ uint32_t qm_sort_key2(uint32_t x) {
-  const uint32_t neg = ((x >> 15) & 0x00010001u) * 0xffffu;               // all ones in the negative halves
-  const uint32_t zero = (sah_pk_ne01_u16(x, 0x80008000u) ^ 0x00010001u) * 0xffffu;  // ... in the halves that hold -0
-  return (x ^ (neg | 0x80008000u)) ^ zero;
-}
-
-// (a native vector: an array of HIP's uint4, a structure, that is filled in one place and stored in another stays in memory)
-typedef uint32_t qm_u4 __attribute__((ext_vector_type(4)));
-typedef qm_u4 qm_u4_any __attribute__((aligned(2)));  // 16 bytes at an address that is only element aligned
-
 // a score's rounding remainder in DT's own bits, as k_qk_scores leaves it
 template <int DT>
 __device__ __forceinline__ uint32_t qm_remainder(float d) {
@@ -335,7 +324,7 @@ __global__ __launch_bounds__(QM_NT, 2) void k_qk_scores_mfma(qk_params P, int ch
   if (c0 >= c1) return;
 
   // a chunk's query vectors on their way to LDS; vectors beyond the last repeat it and are never stored
-  qm_u4 qr[UPT];
+  sah_u4 qr[UPT];
   auto fetch = [&](int c) {
 #pragma unroll
     for (int u = 0; u < UPT; ++u) {
@@ -343,7 +332,7 @@ __global__ __launch_bounds__(QM_NT, 2) void k_qk_scores_mfma(qk_params P, int ch
       int v = c * QM_VECS + idx / (D / 8);
       if (v >= nvec) v = nvec - 1;
       const int h = hk * G + v / P.Lq, qi = v % P.Lq;
-      qr[u] = *(const qm_u4*)((const uint16_t*)P.q + (int64_t)b * P.qs_b + (int64_t)h * P.qs_h + (int64_t)qi * P.qs_l +
+      qr[u] = *(const sah_u4*)((const uint16_t*)P.q + (int64_t)b * P.qs_b + (int64_t)h * P.qs_h + (int64_t)qi * P.qs_l +
                               (idx % (D / 8)) * 8);
     }
   };
@@ -351,7 +340,7 @@ __global__ __launch_bounds__(QM_NT, 2) void k_qk_scores_mfma(qk_params P, int ch
 #pragma unroll
     for (int u = 0; u < UPT; ++u) {
       const int idx = tid + u * QM_NT;
-      *(qm_u4*)&s_q[buf][(idx / (D / 8)) * QP + (idx % (D / 8)) * 8] = qr[u];
+      *(sah_u4*)&s_q[buf][(idx / (D / 8)) * QP + (idx % (D / 8)) * 8] = qr[u];
     }
     if (tid < QM_VECS) {
       const int v = c * QM_VECS + tid;
@@ -414,7 +403,7 @@ __global__ __launch_bounds__(QM_NT, 2) void k_qk_scores_mfma(qk_params P, int ch
           const uint16_t* mp = (const uint16_t*)P.amask + s_moff[buf][vt * 32 + rl] + j;
           uint32_t m[4] = {0u, 0u, 0u, 0u};
           if (whole) {
-            const qm_u4 mv = *(const qm_u4_any*)mp;
+            const sah_u4 mv = *(const sah_u4_any*)mp;
             m[0] = mv.x; m[1] = mv.y; m[2] = mv.z; m[3] = mv.w;
           } else if (row >= 0) {
 #pragma unroll
@@ -437,7 +426,7 @@ __global__ __launch_bounds__(QM_NT, 2) void k_qk_scores_mfma(qk_params P, int ch
           }
         }
 #pragma unroll
-        for (int t = 0; t < 4; ++t) w[t] = qm_sort_key2(w[t]);
+        for (int t = 0; t < 4; ++t) w[t] = sah_sort_key2(w[t]);
         uint16_t* kout = (uint16_t*)P.keys_out + (int64_t)row * P.key_pitch + j;
         if (whole) {
           *(uint4*)kout = make_uint4(w[0], w[1], w[2], w[3]);

@@ -425,6 +425,98 @@ __global__ __launch_bounds__(256) void k_hamming_scores(const uint2* kcodes, int
   ((key_t*)keys_out)[(int64_t)r * key_pitch + j] = (key_t)sah_sort_key<DT>(s);
 }
 
+// The same for 16-bit types, one head's queries together. A thread owns eight consecutive keys: their codes stay in
+// registers while the head's queries come by (uniform: scalar loads), and every row's scores leave as one 16-byte store.
+// One thread per score read the codes and wrote two bytes per query: 33 queries x 32 heads x 32801 keys, bf16 with the
+// causal mask: 123 us, against 29 us here. Bound: the keys written (69 MB, 14 us at copy rate) and ten vector
+// instructions a score (10 us). The queries are dealt to several workgroups until there are HS_MIN_WGS of them.
+#define HS_NT 256
+#define HS_TILE (HS_NT * 8)  // keys per workgroup
+#define HS_MIN_WGS 2048
+template <int DT, bool AM>
+__global__ __launch_bounds__(HS_NT) void k_hamming_scores16(const uint2* __restrict__ kcodes, int64_t code_pitch,
+                                                            const uint2* __restrict__ qcodes, int Hq, int Lq, int q_per_wg,
+                                                            int n_keys, const uint16_t* __restrict__ amask, int64_t ms_b,
+                                                            int64_t ms_h, int64_t ms_l, uint16_t* __restrict__ keys_out,
+                                                            int64_t key_pitch) {
+  const int bh = blockIdx.y;
+  const int q0 = blockIdx.z * q_per_wg;
+  const int q1 = q0 + q_per_wg < Lq ? q0 + q_per_wg : Lq;
+  const int j = blockIdx.x * HS_TILE + threadIdx.x * 8;
+  if (j >= n_keys) return;
+  const bool whole = j + 8 <= n_keys;
+  const uint2* kc = kcodes + (int64_t)bh * code_pitch + j;
+  uint2 code[8];
+  if (whole) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const uint4 c = ((const uint4*)kc)[t];
+      code[2 * t] = make_uint2(c.x, c.y);
+      code[2 * t + 1] = make_uint2(c.z, c.w);
+    }
+  } else {
+#pragma unroll
+    for (int t = 0; t < 8; ++t) code[t] = j + t < n_keys ? kc[t] : make_uint2(0u, 0u);
+  }
+  const uint16_t* mrow = AM ? amask + (int64_t)(bh / Hq) * ms_b + (int64_t)(bh % Hq) * ms_h + j : nullptr;
+#pragma unroll 2
+  for (int qi = q0; qi < q1; ++qi) {
+    const uint2 qc = qcodes[(int64_t)bh * Lq + qi];
+    sah_u4 m = {0u, 0u, 0u, 0u};
+    if (AM) {
+      const uint16_t* mp = mrow + (int64_t)qi * ms_l;  // rows of a mask of odd length are only element aligned
+      if (whole) {
+        m = *(const sah_u4_any*)mp;
+      } else {
+#pragma unroll
+        for (int t = 0; t < 8; ++t)
+          if (j + t < n_keys) m[t >> 1] |= (uint32_t)mp[t] << (16 * (t & 1));
+      }
+    }
+    sah_u4 w;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      float lo = (float)sig_score(qc, code[2 * t]), hi = (float)sig_score(qc, code[2 * t + 1]);
+      if (AM) {
+        if (DT == SAH_BF16) {
+          lo += sah_bits_to_float(m[t] << 16);
+          hi += sah_bits_to_float(m[t] & 0xffff0000u);
+        } else {
+          lo += sah_f16_to_float((uint16_t)m[t]);
+          hi += sah_f16_to_float((uint16_t)(m[t] >> 16));
+        }
+      }
+      w[t] = sah_sort_key2(sah_pack2_hw<DT>(lo, hi));
+    }
+    uint16_t* out = keys_out + ((int64_t)bh * Lq + qi) * key_pitch + j;
+    if (whole) {
+      *(sah_u4*)out = w;
+    } else {
+#pragma unroll
+      for (int t = 0; t < 8; ++t)
+        if (j + t < n_keys) out[t] = (uint16_t)(w[t >> 1] >> (16 * (t & 1)));
+    }
+  }
+}
+
+template <int DT>
+static int hs16_launch(const sah_hamming_scores_args* a) {
+  const int tiles = (a->n_keys + HS_TILE - 1) / HS_TILE, heads = a->B * a->Hq;
+  int split = (HS_MIN_WGS + tiles * heads - 1) / (tiles * heads);
+  if (split > a->Lq) split = a->Lq;
+  const int q_per_wg = (a->Lq + split - 1) / split;
+  dim3 g(tiles, heads, (a->Lq + q_per_wg - 1) / q_per_wg), blk(HS_NT);
+  sah_timed timed("k_hamming_scores16", a->stream);
+#define SAH_HS16_LAUNCH(AMC)                                                                                          \
+  hipLaunchKernelGGL((k_hamming_scores16<DT, AMC>), g, blk, 0, (hipStream_t)a->stream, (const uint2*)a->kcodes,       \
+                     a->code_pitch, (const uint2*)a->qcodes, a->Hq, a->Lq, q_per_wg, a->n_keys,                       \
+                     (const uint16_t*)a->amask, a->ms_b, a->ms_h, a->ms_l, (uint16_t*)a->keys_out, a->key_pitch)
+  if (a->amask) SAH_HS16_LAUNCH(true);
+  else SAH_HS16_LAUNCH(false);
+#undef SAH_HS16_LAUNCH
+  return sah_launch_status("sah_hamming_scores");
+}
+
 extern "C" int sah_hamming_scores(const sah_hamming_scores_args* a) {
   if (!a) return sah_fail(SAH_ENULL, "sah_hamming_scores: args is NULL");
   if (!a->kcodes || !a->qcodes || !a->keys_out) return sah_fail(SAH_ENULL, "sah_hamming_scores: NULL tensor");
@@ -433,6 +525,10 @@ extern "C" int sah_hamming_scores(const sah_hamming_scores_args* a) {
   if (a->code_pitch < a->n_keys || a->key_pitch < a->n_keys) return sah_fail(SAH_ECAPACITY, "sah_hamming_scores: pitch < n_keys");
   const int n_rows = a->B * a->Hq * a->Lq;
   if (n_rows > 65535) return sah_fail(SAH_ESHAPE, "sah_hamming_scores: more than 65535 rows");
+  // 16-byte loads of two codes and stores of eight keys: rows of codes and of keys that start 16-byte aligned
+  if ((a->dtype == SAH_BF16 || a->dtype == SAH_F16) && a->code_pitch % 2 == 0 && (uintptr_t)a->kcodes % 16 == 0 &&
+      a->key_pitch % 8 == 0 && (uintptr_t)a->keys_out % 16 == 0)
+    return a->dtype == SAH_BF16 ? hs16_launch<SAH_BF16>(a) : hs16_launch<SAH_F16>(a);
   dim3 g((a->n_keys + 255) / 256, n_rows), blk(256);
   hipStream_t st = (hipStream_t)a->stream;
   sah_timed timed("k_hamming_scores", a->stream);

@@ -134,3 +134,47 @@ def test_attention_of_many_query_vectors(cuda, dtype, kind, shape, density):
     bound = half * ref.abs() * 1.01 + (2.0 ** -16 + 2 * logit) * mass + 1e-6 + tiny * vv.abs().sum(2).amax()
     worst = float(((out.double().cpu() - ref).abs() / bound).max())
     assert worst <= 1.0, worst
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("kind", [None, "causal", "general"])
+@pytest.mark.parametrize("shape,pitch", [  # keys on either side of a lane's 8 and a workgroup's 2048; an odd code pitch: the
+    # form of one thread per score
+    ((1, 2, 3, 5), 16), ((2, 3, 4, 2049), 2050), ((1, 4, 33, 2055), 2064), ((1, 2, 1, 4096), 4096), ((1, 2, 5, 40), 41)])
+def test_signature_scores_of_many_queries(cuda, dtype, kind, shape, pitch):
+    """Whole numbers plus the mask, rounded once to the tensor type: exactly torch's values."""
+    from sparse_attention_hub_amd import _native as N
+
+    B, Hq, Lq, Lk = shape
+    g = torch.Generator().manual_seed(Lk)
+
+    def planes(*n):  # per component -1, 0 or 1, zeros rare
+        v = torch.randint(0, 2, (*n, 32), generator=g) * 2 - 1
+        return v * (torch.rand(*n, 32, generator=g) > 0.05)
+
+    def pack(v):
+        w = 2 ** torch.arange(32, dtype=torch.int64)
+        p = torch.stack([((v > 0) * w).sum(-1), ((v != 0) * w).sum(-1)], -1)
+        return torch.where(p >= 2 ** 31, p - 2 ** 32, p).to(torch.int32)
+
+    kv, qv = planes(B, Hq, Lk), planes(B, Hq, Lq)
+    codes = torch.zeros((B, Hq, pitch, 2), dtype=torch.int32)
+    codes[:, :, :Lk] = pack(kv)
+    codes, qcodes = codes.to(cuda), pack(qv).reshape(-1, 2).contiguous().to(cuda)
+    am = question_mask(B, Lq, Lk, dtype, cuda, kind)
+    ms = (0, 0, 0) if am is None else (am.stride(0), 0, am.stride(2))
+    kp = (Lk + 63) // 64 * 64
+    keys = torch.zeros((B * Hq * Lq, kp), dtype=torch.int16, device=cuda)
+    N.timing_enable(True)
+    N.call("sah_hamming_scores", N.HammingScoresArgs(codes.data_ptr(), pitch, qcodes.data_ptr(), B, Hq, Lq, Lk,
+                                                     None if am is None else am.data_ptr(), *ms, N.dtype_code(dtype),
+                                                     keys.data_ptr(), kp, N.stream_ptr(cuda)))
+    torch.cuda.synchronize()
+    assert ("k_hamming_scores16" if pitch % 2 == 0 else "k_hamming_scores") in launched(N)
+    u = keys.cpu().to(torch.int32) & 0xFFFF
+    assert bool((u[:, Lk:] == 0).all())  # nothing is written beyond the row's keys
+    bits = torch.where((u & 0x8000) != 0, u & 0x7FFF, (~u) & 0xFFFF).to(torch.int16)
+    ref = (qv.float() @ kv.float().transpose(-1, -2)).to(dtype)
+    if am is not None:
+        ref = ref + am.cpu()
+    assert torch.equal(bits.view(dtype)[:, :Lk], ref.reshape(-1, Lk))
