@@ -17,6 +17,34 @@ extern "C" {
 int64_t sah_members_attention_work_floats(int32_t B, int32_t Hq, int32_t Hkv, int32_t Lq, int32_t Lk, int32_t D);
 int sah_members_attention(const sah_attention_args* a);
 
+/* A whole Lloyd run: sah_pq_keys_absmax, then max_iter times sah_pq_kmeans_assign and sah_pq_kmeans_update, in one call
+ * and without host-made random numbers. given_start != 0: centres hold the start. Otherwise the start is vector
+ * start_idx[g][c] (written here, scratch of the caller) of every group: one vector of each of n_cent equal strata of
+ * [0, n_keys), chosen by number g * n_cent + c of torch.rand(float64) with a CPU generator seeded with start_seed. In
+ * iteration i an empty centre takes vector number (i * n_groups + g) * n_cent + c of torch.randint(0, n_keys) with a CPU
+ * generator seeded with reseed_seed (below 2^28 keys; beyond, where torch draws 64 bits, still the 32-bit number modulo
+ * n_keys). The seeds' low 32 bits count, as in torch. sums, counts, state and absmax_bits must
+ * be zero before the call (sums and counts are zero again after it); the codes are the assignment to the centres that
+ * entered the last iteration carried out. */
+typedef struct sah_pq_kmeans_args {
+  const void* k; int64_t ks_b, ks_h, ks_l;
+  int32_t dtype;
+  int32_t B, Hkv, n_sub, d_sub, n_cent;
+  int32_t key_offset, n_keys;
+  float* centres;                 /* [n_groups, n_cent, d_sub] */
+  uint8_t* codes; int64_t code_pitch; int64_t code_offset;
+  int64_t* sums; int32_t* counts; /* [n_groups, n_cent, d_sub], [n_groups, n_cent] */
+  float* shift2;                  /* [n_groups] */
+  int32_t* state;                 /* [4] */
+  uint32_t* absmax_bits;          /* [1] */
+  int32_t* start_idx;             /* [n_groups, n_cent]; may be NULL with given_start */
+  uint64_t start_seed, reseed_seed;
+  float tol;
+  int32_t max_iter, given_start;
+  void* stream;
+} sah_pq_kmeans_args;
+int sah_pq_kmeans(const sah_pq_kmeans_args* a);
+
 #ifdef __cplusplus
 }
 #endif

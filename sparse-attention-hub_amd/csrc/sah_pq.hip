@@ -10,6 +10,7 @@
 // different 16 B slices of the same key rows run next to each other and share
 // the rows in L2.
 #include "sah_common.h"
+#include "sah_mt.h"
 
 #define PQ_NT 256
 #define PQ_MAX_D 17  // widest sub-vector of the kernels that keep a key in registers: 16 plus the extra coordinate of
@@ -553,18 +554,25 @@ struct pq_update_params {
   const void* k; int64_t ks_b, ks_h, ks_l;
   int Hkv, n_sub, d_sub, n_cent, key_offset;
   float* centres;
-  const long long* sums; const int* counts;
+  long long* sums; int* counts;
   const uint32_t* absmax_bits;
-  const int* reseed_idx;
+  const int* reseed_idx;   // NULL: vector i of an empty centre is number reseed_first + g * n_cent + c of the generator
+  uint32_t reseed_seed;    // seeded with reseed_seed, modulo n_keys (torch.randint of the whole run, drawn where needed)
+  int64_t reseed_first;
+  int n_keys;
+  int clear;               // sums and counts are left zero for the next assignment
   float* shift2;
   float tol;
   int* state;
   int n_groups;
 };
 
+// One workgroup per group, a thread per centre. What bounds it is latency (a group's 18 KB): the sums of eight
+// dimensions are requested together.
 template <int DT>
 __global__ __launch_bounds__(PQ_NT) void k_pq_update(pq_update_params P) {
   __shared__ float s_red[PQ_NT / SAH_WAVE];
+  __shared__ mt_lds s_mt;
   if (P.state[2]) return;
   const int tid = threadIdx.x;
   const int g = blockIdx.x;
@@ -574,24 +582,50 @@ __global__ __launch_bounds__(PQ_NT) void k_pq_update(pq_update_params P) {
   const int b = bh / P.Hkv;
   const int d_sub = P.d_sub, n_cent = P.n_cent;
   float move = 0.f;
+  int cn = 1, ridx = 0;
+  if (tid < n_cent) {
+    cn = P.counts[(int64_t)g * n_cent + tid];
+    if (cn == 0 && P.reseed_idx) ridx = P.reseed_idx[(int64_t)g * n_cent + tid];
+  }
+  if (!P.reseed_idx && __syncthreads_or(cn == 0)) {  // rare: the generator runs only where a centre is empty
+    const int64_t first = P.reseed_first + (int64_t)g * n_cent;
+    const int64_t mine = first + (tid < n_cent ? tid : 0);
+    const int last = (int)((first + n_cent - 1) / MT_N);
+    mt_seed(s_mt, P.reseed_seed);
+    for (int blk = 0; blk <= last; ++blk) {
+      mt_next(s_mt, blk & 1);
+      if (mine / MT_N == blk) ridx = (int)(mt_temper(s_mt.st[(blk & 1) ^ 1][mine % MT_N]) % (uint32_t)P.n_keys);
+    }
+  }
   if (tid < n_cent) {
     const int c = tid;
-    const int cn = P.counts[(int64_t)g * n_cent + c];
     float* cc = P.centres + ((int64_t)g * n_cent + c) * d_sub;
-    const long long* ss = P.sums + ((int64_t)g * n_cent + c) * d_sub;
+    long long* ss = P.sums + ((int64_t)g * n_cent + c) * d_sub;
     const double unscale = 1.0 / ((double)pq_sum_scale(*P.absmax_bits) * (double)(cn > 0 ? cn : 1));
     float acc = 0.f;
-    int64_t roff = 0;
-    if (cn == 0) {
-      const int ridx = P.reseed_idx[(int64_t)g * n_cent + c];
-      roff = (int64_t)b * P.ks_b + (int64_t)hk * P.ks_h + (int64_t)(P.key_offset + ridx) * P.ks_l + (int64_t)s * d_sub;
+    const int64_t roff =
+        (int64_t)b * P.ks_b + (int64_t)hk * P.ks_h + (int64_t)(P.key_offset + ridx) * P.ks_l + (int64_t)s * d_sub;
+    for (int d0 = 0; d0 < d_sub; d0 += 8) {
+      long long sv[8];
+      float ov[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int d = d0 + u < d_sub ? d0 + u : d_sub - 1;
+        sv[u] = ss[d];
+        ov[u] = cc[d];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int d = d0 + u;
+        if (d >= d_sub) break;
+        const float nv = (cn > 0) ? (float)((double)sv[u] * unscale) : sah_load<DT>(P.k, roff + d);
+        const float df = nv - ov[u];
+        acc = fmaf(df, df, acc);
+        cc[d] = nv;
+        if (P.clear) ss[d] = 0;
+      }
     }
-    for (int d = 0; d < d_sub; ++d) {
-      const float nv = (cn > 0) ? (float)((double)ss[d] * unscale) : sah_load<DT>(P.k, roff + d);
-      const float df = nv - cc[d];
-      acc = fmaf(df, df, acc);
-      cc[d] = nv;
-    }
+    if (P.clear) P.counts[(int64_t)g * n_cent + c] = 0;
     move = sqrtf(acc);
   }
   move = sah_wave_sum(move);
@@ -602,23 +636,58 @@ __global__ __launch_bounds__(PQ_NT) void k_pq_update(pq_update_params P) {
     for (int i = 0; i < PQ_NT / SAH_WAVE; ++i) tot += s_red[i];
     const float sh2 = tot * tot;
     P.shift2[g] = sh2;
+    // the verdict's two counters only: the converged count is in before the ticket is taken, nothing else is handed over
     if (sh2 < P.tol) atomicAdd(&P.state[0], 1);
-    __threadfence();
+    sah_stores_done();
     const int ticket = atomicAdd(&P.state[1], 1);
     if (ticket == P.n_groups - 1) {
-      // last group of this iteration: publish the verdict and reset the counters
+      // last group of this iteration, every other has read the done flag: publish the verdict, reset the counters
       const int conv = atomicAdd(&P.state[0], 0);
-      P.state[3] = (conv == P.n_groups) ? 1 : 0;
+      if (conv == P.n_groups) P.state[2] = 1;
       P.state[0] = 0;
       P.state[1] = 0;
     }
   }
 }
 
-// state[3] -> state[2] is promoted by a separate one-thread kernel so that every
-// group of the iteration in flight still sees the old flag.
-__global__ void k_pq_promote(int* state) {
-  if (threadIdx.x == 0 && blockIdx.x == 0 && state[3]) state[2] = 1;
+// Start vectors of every group: number (g, c) of a seeded torch.rand in float64 picks one vector of stratum c of
+// [0, n_keys) (n_cent equal strata). One workgroup draws the whole sequence (0.4 us per 312 numbers; on the host, copy
+// included, 128 groups x 256 centres took 0.5 ms and more).
+#define PQI_NT 320
+__global__ __launch_bounds__(PQI_NT) void k_pq_start(uint32_t seed, int n_groups, int n_cent, int n_keys, double stratum, int* idx) {
+  __shared__ mt_lds S;
+  mt_seed(S, seed);
+  const int64_t total = (int64_t)n_groups * n_cent;
+  int from = 0;
+  for (int64_t first = 0; first < total; first += MT_N / 2, from ^= 1) {
+    mt_next(S, from);
+    const int64_t i = first + threadIdx.x;
+    if (threadIdx.x < MT_N / 2 && i < total) {
+      const uint32_t hi = mt_temper(S.st[from ^ 1][2 * threadIdx.x]), lo = mt_temper(S.st[from ^ 1][2 * threadIdx.x + 1]);
+      const double u = (double)((((uint64_t)hi << 32) | lo) & ((1ull << 53) - 1)) * 0x1p-53;
+      const int c = (int)(i % n_cent);
+      const long long b = (long long)floor((double)c * stratum);
+      long long e = (long long)floor((double)(c + 1) * stratum);
+      if (e > n_keys) e = n_keys;
+      const long long width = e - b > 1 ? e - b : 1;
+      const long long v = b + (long long)floor(u * (double)width);
+      idx[i] = (int)(v < n_keys - 1 ? v : n_keys - 1);
+    }
+  }
+}
+
+// centres[g][c][:] = vector idx[g][c] of the group, as fp32
+template <int DT>
+__global__ __launch_bounds__(PQ_NT) void k_pq_gather(const void* k, int64_t ks_b, int64_t ks_h, int64_t ks_l, int Hkv, int n_sub,
+                                                     int d_sub, int n_cent, int key_offset, int64_t total, const int* idx,
+                                                     float* centres) {
+  const int64_t i = (int64_t)blockIdx.x * PQ_NT + threadIdx.x;
+  if (i >= total) return;
+  const int64_t gc = i / d_sub;
+  const int d = (int)(i - gc * d_sub);
+  const int g = (int)(gc / n_cent), s = g % n_sub, bh = g / n_sub;
+  centres[i] = sah_load<DT>(k, (int64_t)(bh / Hkv) * ks_b + (int64_t)(bh % Hkv) * ks_h + (int64_t)(key_offset + idx[gc]) * ks_l +
+                                   (int64_t)s * d_sub + d);
 }
 
 struct pq_adc_params {
@@ -966,17 +1035,53 @@ static int pq_check_common(const char* what, int B, int Hkv, int n_sub, int d_su
 
 // Largest |element| of the keys [key_offset, key_offset + n_keys) of every (b, kv head), as float bits (non-negative
 // floats order like their bit patterns, so an integer atomic max does it). *out must be zero before the launch.
-template <int DT>
+// VEC elements a load: 16 bytes where the rows allow it (an element at a time, with a 64-bit division each, a 33 MB
+// cache took 72 us; its bytes take 7).
+template <int DT, int VEC>
 __global__ __launch_bounds__(PQ_NT) void k_pq_absmax(const void* k, int64_t ks_b, int64_t ks_h, int64_t ks_l, int Hkv, int D,
                                                      int key_offset, int n_keys, uint32_t* out) {
   const int bh = blockIdx.y;
-  const int64_t base = (int64_t)(bh / Hkv) * ks_b + (int64_t)(bh % Hkv) * ks_h;
-  const int64_t total = (int64_t)n_keys * D;
+  const int64_t base = (int64_t)(bh / Hkv) * ks_b + (int64_t)(bh % Hkv) * ks_h + (int64_t)key_offset * ks_l;
+  const int upr = D / VEC;  // loads per row
+  const int64_t total = (int64_t)n_keys * upr;
+  const int64_t step = (int64_t)gridDim.x * PQ_NT;
   uint32_t best = 0u;
-  for (int64_t i = (int64_t)blockIdx.x * PQ_NT + threadIdx.x; i < total; i += (int64_t)gridDim.x * PQ_NT) {
-    const int n = (int)(i / D), d = (int)(i % D);
-    const uint32_t bits = sah_float_to_bits(sah_load<DT>(k, base + (int64_t)(key_offset + n) * ks_l + d)) & 0x7fffffffu;
+  auto take = [&](uint32_t bits) {
+    bits &= 0x7fffffffu;
     if (bits <= 0x7f800000u) best = bits > best ? bits : best;  // NaN is skipped
+  };
+  int64_t i = (int64_t)blockIdx.x * PQ_NT + threadIdx.x;
+  int64_t n = i / upr;
+  int c = (int)(i - n * upr);
+  const int64_t dn = step / upr;
+  const int dc = (int)(step - dn * upr);
+#pragma unroll 4
+  for (; i < total; i += step) {
+    const int64_t off = base + n * ks_l + (int64_t)c * VEC;
+    if constexpr (VEC == 1) {
+      take(sah_float_to_bits(sah_load<DT>(k, off)));
+    } else {
+      const uint4 q = *(const uint4*)((const char*)k + off * (DT == SAH_F32 ? 4 : 2));
+      const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        if (DT == SAH_F32) {
+          take(w[t]);
+        } else if (DT == SAH_BF16) {
+          take(w[t] << 16);
+          take(w[t] & 0xffff0000u);
+        } else {
+          take(sah_float_to_bits(sah_f16_to_float((uint16_t)w[t])));
+          take(sah_float_to_bits(sah_f16_to_float((uint16_t)(w[t] >> 16))));
+        }
+      }
+    }
+    n += dn;
+    c += dc;
+    if (c >= upr) {
+      c -= upr;
+      ++n;
+    }
   }
 #pragma unroll
   for (int o = 1; o < SAH_WAVE; o <<= 1) {
@@ -986,22 +1091,33 @@ __global__ __launch_bounds__(PQ_NT) void k_pq_absmax(const void* k, int64_t ks_b
   if ((threadIdx.x & (SAH_WAVE - 1)) == 0 && best) atomicMax(out, best);
 }
 
+template <int DT>
+static void pq_absmax_launch(const sah_pq_absmax_args* a) {
+  constexpr int VEC = DT == SAH_F32 ? 4 : 8;
+  const bool vec = a->D % VEC == 0 && a->ks_b % VEC == 0 && a->ks_h % VEC == 0 && a->ks_l % VEC == 0 && (uintptr_t)a->k % 16 == 0;
+  const int64_t total = (int64_t)a->n_keys * (vec ? a->D / VEC : a->D);
+  int64_t gx = (total + PQ_NT * 8 - 1) / (PQ_NT * 8);
+  const int64_t most = (2048 + (int64_t)a->B * a->Hkv - 1) / ((int64_t)a->B * a->Hkv);
+  gx = gx < 1 ? 1 : (gx > most ? most : gx);
+  dim3 g((unsigned)gx, a->B * a->Hkv), blk(PQ_NT);
+  hipStream_t st = (hipStream_t)a->stream;
+  if (vec)
+    hipLaunchKernelGGL((k_pq_absmax<DT, VEC>), g, blk, 0, st, a->k, a->ks_b, a->ks_h, a->ks_l, a->Hkv, a->D, a->key_offset, a->n_keys, a->absmax_bits);
+  else
+    hipLaunchKernelGGL((k_pq_absmax<DT, 1>), g, blk, 0, st, a->k, a->ks_b, a->ks_h, a->ks_l, a->Hkv, a->D, a->key_offset, a->n_keys, a->absmax_bits);
+}
+
 extern "C" int sah_pq_keys_absmax(const sah_pq_absmax_args* a) {
   if (!a) return sah_fail(SAH_ENULL, "sah_pq_keys_absmax: args is NULL");
   if (!a->k || !a->absmax_bits) return sah_fail(SAH_ENULL, "sah_pq_keys_absmax: NULL tensor");
   if (a->B <= 0 || a->Hkv <= 0 || a->D <= 0 || a->key_offset < 0 || a->n_keys < 0 || (int64_t)a->B * a->Hkv > 65535)
     return sah_fail(SAH_EINVAL, "sah_pq_keys_absmax: bad B/Hkv/D/key range");
   if (a->n_keys == 0) return SAH_OK;
-  const int64_t total = (int64_t)a->n_keys * a->D;
-  int gx = (int)((total + PQ_NT * 16 - 1) / (PQ_NT * 16));
-  gx = gx < 1 ? 1 : (gx > 64 ? 64 : gx);
-  dim3 g(gx, a->B * a->Hkv), blk(PQ_NT);
-  hipStream_t st = (hipStream_t)a->stream;
   sah_timed timed("k_pq_absmax", a->stream);
   switch (a->dtype) {
-    case SAH_F32: hipLaunchKernelGGL(k_pq_absmax<SAH_F32>, g, blk, 0, st, a->k, a->ks_b, a->ks_h, a->ks_l, a->Hkv, a->D, a->key_offset, a->n_keys, a->absmax_bits); break;
-    case SAH_BF16: hipLaunchKernelGGL(k_pq_absmax<SAH_BF16>, g, blk, 0, st, a->k, a->ks_b, a->ks_h, a->ks_l, a->Hkv, a->D, a->key_offset, a->n_keys, a->absmax_bits); break;
-    case SAH_F16: hipLaunchKernelGGL(k_pq_absmax<SAH_F16>, g, blk, 0, st, a->k, a->ks_b, a->ks_h, a->ks_l, a->Hkv, a->D, a->key_offset, a->n_keys, a->absmax_bits); break;
+    case SAH_F32: pq_absmax_launch<SAH_F32>(a); break;
+    case SAH_BF16: pq_absmax_launch<SAH_BF16>(a); break;
+    case SAH_F16: pq_absmax_launch<SAH_F16>(a); break;
     default: return sah_fail(SAH_EDTYPE, "sah_pq_keys_absmax: dtype %d", a->dtype);
   }
   return sah_launch_status("sah_pq_keys_absmax");
@@ -1082,34 +1198,91 @@ extern "C" int sah_pq_kmeans_assign(const sah_pq_assign_args* a) {
   return sah_launch_status("sah_pq_kmeans_assign");
 }
 
+static int pq_update_launch(const pq_update_params& P, int dtype, void* stream, const char* what) {
+  dim3 g(P.n_groups), blk(PQ_NT);
+  hipStream_t st = (hipStream_t)stream;
+  sah_timed timed("k_pq_update", stream);
+  switch (dtype) {
+    case SAH_F32: hipLaunchKernelGGL(k_pq_update<SAH_F32>, g, blk, 0, st, P); break;
+    case SAH_BF16: hipLaunchKernelGGL(k_pq_update<SAH_BF16>, g, blk, 0, st, P); break;
+    case SAH_F16: hipLaunchKernelGGL(k_pq_update<SAH_F16>, g, blk, 0, st, P); break;
+    default: return sah_fail(SAH_EDTYPE, "%s: dtype %d", what, dtype);
+  }
+  return sah_launch_status(what);
+}
+
 extern "C" int sah_pq_kmeans_update(const sah_pq_update_args* a) {
   if (!a) return sah_fail(SAH_ENULL, "sah_pq_kmeans_update: args is NULL");
   int rc = pq_check_common("sah_pq_kmeans_update", a->B, a->Hkv, a->n_sub, a->d_sub, a->n_cent);
   if (rc) return rc;
   if (!a->k || !a->centres || !a->sums || !a->counts || !a->reseed_idx || !a->shift2 || !a->state || !a->absmax_bits)
     return sah_fail(SAH_ENULL, "sah_pq_kmeans_update: NULL tensor");
-  pq_update_params P;
+  pq_update_params P = {};
   P.k = a->k; P.ks_b = a->ks_b; P.ks_h = a->ks_h; P.ks_l = a->ks_l;
   P.Hkv = a->Hkv; P.n_sub = a->n_sub; P.d_sub = a->d_sub; P.n_cent = a->n_cent; P.key_offset = a->key_offset;
-  P.centres = a->centres; P.sums = (const long long*)a->sums; P.counts = a->counts; P.reseed_idx = a->reseed_idx;
+  P.centres = a->centres; P.sums = (long long*)a->sums; P.counts = (int*)a->counts;  // read only: P.clear is 0
+  P.reseed_idx = a->reseed_idx; P.n_keys = 1;
   P.absmax_bits = a->absmax_bits;
   P.shift2 = a->shift2; P.tol = a->tol; P.state = a->state;
   P.n_groups = a->B * a->Hkv * a->n_sub;
-  dim3 g(P.n_groups), blk(PQ_NT);
-  hipStream_t st = (hipStream_t)a->stream;
-  {
-    sah_timed timed("k_pq_update", a->stream);
-    switch (a->dtype) {
-      case SAH_F32: hipLaunchKernelGGL(k_pq_update<SAH_F32>, g, blk, 0, st, P); break;
-      case SAH_BF16: hipLaunchKernelGGL(k_pq_update<SAH_BF16>, g, blk, 0, st, P); break;
-      case SAH_F16: hipLaunchKernelGGL(k_pq_update<SAH_F16>, g, blk, 0, st, P); break;
-      default: return sah_fail(SAH_EDTYPE, "sah_pq_kmeans_update: dtype %d", a->dtype);
-    }
-  }
-  rc = sah_launch_status("sah_pq_kmeans_update");
+  return pq_update_launch(P, a->dtype, a->stream, "sah_pq_kmeans_update");
+}
+
+extern "C" int sah_pq_kmeans(const sah_pq_kmeans_args* a) {
+  if (!a) return sah_fail(SAH_ENULL, "sah_pq_kmeans: args is NULL");
+  int rc = pq_check_common("sah_pq_kmeans", a->B, a->Hkv, a->n_sub, a->d_sub, a->n_cent);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_pq_promote, dim3(1), dim3(SAH_WAVE), 0, st, a->state);
-  return sah_launch_status("sah_pq_kmeans_update(promote)");
+  if (!a->k || !a->centres || !a->codes || !a->sums || !a->counts || !a->shift2 || !a->state || !a->absmax_bits ||
+      (!a->given_start && !a->start_idx))
+    return sah_fail(SAH_ENULL, "sah_pq_kmeans: NULL tensor");
+  if (a->n_keys <= 0 || a->key_offset < 0 || a->max_iter < 0)
+    return sah_fail(SAH_EINVAL, "sah_pq_kmeans: n_keys must be > 0, key_offset and max_iter >= 0");
+  if (a->code_offset < 0 || a->code_pitch < a->code_offset + a->n_keys)
+    return sah_fail(SAH_ECAPACITY, "sah_pq_kmeans: code_pitch %lld < code_offset %lld + n_keys %d", (long long)a->code_pitch,
+                    (long long)a->code_offset, a->n_keys);
+  const int n_groups = a->B * a->Hkv * a->n_sub;
+  hipStream_t st = (hipStream_t)a->stream;
+  if (!a->given_start) {
+    if (a->n_keys < a->n_cent) return sah_fail(SAH_EINVAL, "sah_pq_kmeans: fewer keys than centres");
+    const int64_t total = (int64_t)n_groups * a->n_cent * a->d_sub;
+    sah_timed timed("k_pq_start", a->stream);
+    hipLaunchKernelGGL(k_pq_start, dim3(1), dim3(PQI_NT), 0, st, (uint32_t)a->start_seed, n_groups, a->n_cent, a->n_keys,
+                       (double)a->n_keys / (double)a->n_cent, a->start_idx);
+    dim3 g((unsigned)((total + PQ_NT - 1) / PQ_NT)), blk(PQ_NT);
+#define SAH_PQG(DTC)                                                                                                          \
+  hipLaunchKernelGGL(k_pq_gather<DTC>, g, blk, 0, st, a->k, a->ks_b, a->ks_h, a->ks_l, a->Hkv, a->n_sub, a->d_sub, a->n_cent, \
+                     a->key_offset, total, a->start_idx, a->centres)
+    switch (a->dtype) {
+      case SAH_F32: SAH_PQG(SAH_F32); break;
+      case SAH_BF16: SAH_PQG(SAH_BF16); break;
+      case SAH_F16: SAH_PQG(SAH_F16); break;
+      default: return sah_fail(SAH_EDTYPE, "sah_pq_kmeans: dtype %d", a->dtype);
+    }
+#undef SAH_PQG
+    if ((rc = sah_launch_status("sah_pq_kmeans(start)"))) return rc;
+  }
+  sah_pq_absmax_args m = {a->k, a->ks_b, a->ks_h, a->ks_l, a->dtype, a->B, a->Hkv, a->n_sub * a->d_sub, a->key_offset, a->n_keys,
+                          a->absmax_bits, a->stream};
+  if ((rc = sah_pq_keys_absmax(&m))) return rc;
+  sah_pq_assign_args as = {};
+  as.k = a->k; as.ks_b = a->ks_b; as.ks_h = a->ks_h; as.ks_l = a->ks_l;
+  as.dtype = a->dtype; as.B = a->B; as.Hkv = a->Hkv; as.n_sub = a->n_sub; as.d_sub = a->d_sub; as.n_cent = a->n_cent;
+  as.key_offset = a->key_offset; as.n_keys = a->n_keys; as.centres = a->centres;
+  as.codes = a->codes; as.code_pitch = a->code_pitch; as.code_offset = a->code_offset;
+  as.sums = a->sums; as.counts = a->counts; as.skip_flag = a->state + 2; as.stream = a->stream; as.absmax_bits = a->absmax_bits;
+  pq_update_params P = {};
+  P.k = a->k; P.ks_b = a->ks_b; P.ks_h = a->ks_h; P.ks_l = a->ks_l;
+  P.Hkv = a->Hkv; P.n_sub = a->n_sub; P.d_sub = a->d_sub; P.n_cent = a->n_cent; P.key_offset = a->key_offset;
+  P.centres = a->centres; P.sums = (long long*)a->sums; P.counts = a->counts;
+  P.reseed_seed = (uint32_t)a->reseed_seed; P.n_keys = a->n_keys; P.clear = 1;
+  P.absmax_bits = a->absmax_bits;
+  P.shift2 = a->shift2; P.tol = a->tol; P.state = a->state; P.n_groups = n_groups;
+  for (int it = 0; it < a->max_iter; ++it) {
+    if ((rc = sah_pq_kmeans_assign(&as))) return rc;
+    P.reseed_first = (int64_t)it * n_groups * a->n_cent;
+    if ((rc = pq_update_launch(P, a->dtype, a->stream, "sah_pq_kmeans"))) return rc;
+  }
+  return SAH_OK;
 }
 
 extern "C" int64_t sah_pq_adc_lut_bytes(int32_t B, int32_t Hq, int32_t Hkv, int32_t Lq, int32_t n_sub, int32_t n_cent,

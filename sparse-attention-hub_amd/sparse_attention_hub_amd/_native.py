@@ -61,6 +61,7 @@ EXPECTED_SYMBOLS = (
 # include/sah_ext.h: name -> number of argument blocks
 EXTENSION_SYMBOLS = {
     "sah_members_attention": 1,
+    "sah_pq_kmeans": 1,
 }
 
 
@@ -194,6 +195,26 @@ class PqAssignArgs(C.Structure):
         ("skip_flag", C.c_void_p),
         ("stream", C.c_void_p),
         ("absmax_bits", C.c_void_p),
+    ]
+
+
+class PqKmeansArgs(C.Structure):
+    _fields_ = [
+        ("k", C.c_void_p), ("ks_b", C.c_int64), ("ks_h", C.c_int64), ("ks_l", C.c_int64),
+        ("dtype", C.c_int32),
+        ("B", C.c_int32), ("Hkv", C.c_int32), ("n_sub", C.c_int32), ("d_sub", C.c_int32), ("n_cent", C.c_int32),
+        ("key_offset", C.c_int32), ("n_keys", C.c_int32),
+        ("centres", C.c_void_p),
+        ("codes", C.c_void_p), ("code_pitch", C.c_int64), ("code_offset", C.c_int64),
+        ("sums", C.c_void_p), ("counts", C.c_void_p),
+        ("shift2", C.c_void_p),
+        ("state", C.c_void_p),
+        ("absmax_bits", C.c_void_p),
+        ("start_idx", C.c_void_p),
+        ("start_seed", C.c_uint64), ("reseed_seed", C.c_uint64),
+        ("tol", C.c_float),
+        ("max_iter", C.c_int32), ("given_start", C.c_int32),
+        ("stream", C.c_void_p),
     ]
 
 

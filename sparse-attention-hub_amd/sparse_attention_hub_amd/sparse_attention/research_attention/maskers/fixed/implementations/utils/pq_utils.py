@@ -78,44 +78,32 @@ def kmeans_keys_batched(
     dev = keys.device
     if keys.stride(-1) != 1:
         keys = keys.contiguous()
-    if cluster_centers is None:
-        start = seeded_initial_centres(n_groups, n_keys, n_cent, seed, dev)
-        centres = gather_sub_vectors(keys, key_offset, n_sub, start)
-    else:
-        if tuple(cluster_centers.shape) != (n_groups, n_cent, d_sub):
-            raise ValueError(
-                f"cluster_centers shape mismatch. Expected ({n_groups}, {n_cent}, {d_sub}), got {tuple(cluster_centers.shape)}"
-            )
-        centres = cluster_centers.to(device=dev, dtype=torch.float32).contiguous().clone()
-    sums = torch.empty((n_groups, n_cent, d_sub), dtype=torch.int64, device=dev)  # fixed point: order-independent
-    counts = torch.empty((n_groups, n_cent), dtype=torch.int32, device=dev)
-    shift2 = torch.zeros((n_groups,), dtype=torch.float32, device=dev)
-    state = torch.zeros((4,), dtype=torch.int32, device=dev)
-    gen = torch.Generator(device="cpu").manual_seed(int(seed) + 1)
-    reseed = torch.randint(0, n_keys, (max(max_iter, 1), n_groups, n_cent), generator=gen, dtype=torch.int32).to(dev)
+    if cluster_centers is not None and tuple(cluster_centers.shape) != (n_groups, n_cent, d_sub):
+        raise ValueError(
+            f"cluster_centers shape mismatch. Expected ({n_groups}, {n_cent}, {d_sub}), got {tuple(cluster_centers.shape)}"
+        )
+    if cluster_centers is None and n_keys < n_cent:
+        raise ValueError(f"k-means needs at least {n_cent} vectors, got {n_keys}")
     dt = N.dtype_code(keys.dtype)
     stream = N.stream_ptr(dev)
-    absmax = torch.zeros((1,), dtype=torch.int32, device=dev)
-    N.call("sah_pq_keys_absmax", N.PqAbsmaxArgs(
-        keys.data_ptr(), keys.stride(0), keys.stride(1), keys.stride(2), dt, B, Hkv, n_sub * d_sub, key_offset, n_keys,
-        absmax.data_ptr(), stream))
-    for it in range(max_iter):
-        sums.zero_()
-        counts.zero_()
-        a = N.PqAssignArgs(
-            keys.data_ptr(), keys.stride(0), keys.stride(1), keys.stride(2), dt,
-            B, Hkv, n_sub, d_sub, n_cent, key_offset, n_keys,
-            centres.data_ptr(), codes.data_ptr(), code_pitch, code_offset,
-            sums.data_ptr(), counts.data_ptr(), 0, state[2:].data_ptr(), stream, absmax.data_ptr(),
-        )
-        N.call("sah_pq_kmeans_assign", a)
-        u = N.PqUpdateArgs(
-            keys.data_ptr(), keys.stride(0), keys.stride(1), keys.stride(2), dt,
-            B, Hkv, n_sub, d_sub, n_cent, key_offset,
-            centres.data_ptr(), sums.data_ptr(), counts.data_ptr(), reseed[it].data_ptr(),
-            shift2.data_ptr(), float(tol), state.data_ptr(), stream, absmax.data_ptr(),
-        )
-        N.call("sah_pq_kmeans_update", u)
+    n_all = n_groups * n_cent
+    # one cleared buffer: fixed-point sums (order-independent), counts, squared shifts, state and the largest |element|
+    work = torch.zeros((n_all * d_sub * 2 + n_all + n_groups + 5,), dtype=torch.int32, device=dev)
+    counts = work[n_all * d_sub * 2:]
+    shift2 = counts[n_all:n_all + n_groups].view(torch.float32)
+    state = counts[n_all + n_groups:]
+    if cluster_centers is None:
+        centres = torch.empty((n_groups, n_cent, d_sub), dtype=torch.float32, device=dev)
+        start = torch.empty((n_groups, n_cent), dtype=torch.int32, device=dev)
+    else:
+        centres = cluster_centers.to(device=dev, dtype=torch.float32).contiguous().clone()
+        start = None
+    low64 = (1 << 64) - 1
+    N.call("sah_pq_kmeans", N.PqKmeansArgs(
+        keys.data_ptr(), keys.stride(0), keys.stride(1), keys.stride(2), dt, B, Hkv, n_sub, d_sub, n_cent, key_offset, n_keys,
+        centres.data_ptr(), codes.data_ptr(), code_pitch, code_offset, work.data_ptr(), counts.data_ptr(), shift2.data_ptr(),
+        state.data_ptr(), state[4:].data_ptr(), None if start is None else start.data_ptr(), int(seed) & low64,
+        (int(seed) + 1) & low64, float(tol), max_iter, 0 if start is not None else 1, stream))
     return centres, shift2
 
 

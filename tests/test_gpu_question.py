@@ -178,3 +178,29 @@ def test_signature_scores_of_many_queries(cuda, dtype, kind, shape, pitch):
     if am is not None:
         ref = ref + am.cpu()
     assert torch.equal(bits.view(dtype)[:, :Lk], ref.reshape(-1, Lk))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("shape", [  # (batch, KV heads, keys, head_dim, sub-spaces, centres): a few draws, and more than a block of
+    (1, 1, 40, 16, 2, 8), (2, 3, 300, 64, 8, 256), (1, 2, 1500, 32, 4, 128)])  # 624 words of the generator; vector and matrix forms
+def test_clustering_draws_its_start_and_its_reseeds_as_torch_does(cuda, dtype, shape):
+    """Keys of three distinct, well separated vectors: most centres are empty in every iteration and are reseeded, a mean of
+    equal vectors is that vector, and equal distances go to the lowest centre. Codes and centres are then exact."""
+    from oracle import reference_path as O
+    from sparse_attention_hub_amd.sparse_attention.research_attention.maskers.fixed.implementations.utils.pq_utils import (
+        gather_sub_vectors, kmeans_keys_batched, seeded_initial_centres,
+    )
+
+    B, Hkv, n, D, n_sub, n_cent = shape
+    off, iters, seed = 3, 3, 7919 * 2
+    g = torch.Generator().manual_seed(n)
+    vecs = torch.tensor([-4.0, 0.5, 8.0]).view(3, 1).expand(3, D) * torch.tensor([1.0, -1.0]).repeat(D // 2)
+    k = vecs[torch.randint(0, 3, (B, Hkv, n + off), generator=g)].to(dtype)
+    groups = B * Hkv * n_sub
+    codes = torch.zeros((B, Hkv, n, n_sub), dtype=torch.uint8, device=cuda)
+    centres, _ = kmeans_keys_batched(k.to(cuda), off, n_sub, n_cent, iters, codes, n, tol=-1.0, seed=seed)
+    start = gather_sub_vectors(k, off, n_sub, seeded_initial_centres(groups, n, n_cent, seed, torch.device("cpu")))
+    reseed = torch.randint(0, n, (iters, groups, n_cent), generator=torch.Generator().manual_seed(seed + 1), dtype=torch.int32)
+    codes_o, cent_o = O.kmeans_lloyd(O.pq_split(k, off, n_sub), start, iters, reseed_idx=reseed, tol=-1.0)
+    assert torch.equal(centres.cpu().reshape(-1), cent_o.float().reshape(-1))
+    assert torch.equal(codes.cpu().permute(0, 1, 3, 2).reshape(groups, n).long(), codes_o.reshape(groups, n).long())
