@@ -224,9 +224,9 @@ struct att_lane {
       }
     }
   }
-  // the batch's logits (scaled, plus the additive mask; -inf for a lane without a key), and their maximum over the wave
+  // the batch's logits (scaled, plus the additive mask's am[u]; -inf for a lane without a key), and their maximum over the wave
   template <int UB, bool PLAIN = false>
-  __device__ __forceinline__ float logits(const att_params& P, int64_t moff, const float (&qv)[8], const att_batch<DT, UB>& B,
+  __device__ __forceinline__ float logits(const att_params& P, const float (&am)[UB], const float (&qv)[8], const att_batch<DT, UB>& B,
                                           float (&z)[UB]) const {
     float mb = -INFINITY;
 #pragma unroll
@@ -238,7 +238,7 @@ struct att_lane {
       for (int e = 0; e < 8; ++e) d = fmaf(qv[e], kf[e], d);
       d = att_group_sum<LPK>(d) * P.scaling;
       if (B.id[u] >= 0) {
-        if (!PLAIN && P.amask) d += sah_load<DT>(P.amask, moff + B.id[u]);
+        if (!PLAIN && P.amask) d += am[u];
       } else {
         d = -INFINITY;
       }
@@ -252,7 +252,7 @@ struct att_lane {
   }
   // the same from score keys: key[u] holds q.k of the lane's key in iteration u as (key, remainder)
   template <int UB, bool PLAIN = false>
-  __device__ __forceinline__ float logits_of_keys(const att_params& P, int64_t moff, const uint32_t (&key)[UB],
+  __device__ __forceinline__ float logits_of_keys(const att_params& P, const float (&am)[UB], const uint32_t (&key)[UB],
                                                   const att_batch<DT, UB>& B, float (&z)[UB]) const {
     float mb = -INFINITY;
     if constexpr (DT != SAH_F32) {
@@ -260,7 +260,7 @@ struct att_lane {
       for (int u = 0; u < UB; ++u) {
         float d = att_key_score<DT>(key[u]) * P.scaling;
         if (B.id[u] >= 0) {
-          if (!PLAIN && P.amask) d += sah_load<DT>(P.amask, moff + B.id[u]);
+          if (!PLAIN && P.amask) d += am[u];
         } else {
           d = -INFINITY;
         }
@@ -333,12 +333,14 @@ __device__ __forceinline__ void att_walk(const att_params& P, int r, int b, int 
     const int my = cbase + lane;
     int idx_l = -1;
     uint32_t key_l = 0;
+    float am_l = 0.f;  // the additive mask of the lane's key: with the columns, not behind the wait for the batch's rows
     float invw_l = P.unit_inv_w, invw_den_l = P.unit_inv_w;
     if (my < bound) {
       idx_l = col_of(my);
       invw_l = inv_w_of(my);
       if (idx_l < 0 || idx_l >= P.Lk) idx_l = -1;
       if (KEYED && idx_l >= 0) key_l = key_of(my, idx_l);
+      if (!PLAIN && P.amask && idx_l >= 0) am_l = sah_load<DT>(P.amask, moff + idx_l);
       invw_den_l = invw_l;
       if (DROP && idx_l >= 0) {
         invw_l *= P.drop.factor(r, idx_l);
@@ -352,15 +354,17 @@ __device__ __forceinline__ void att_walk(const att_params& P, int r, int b, int 
 #pragma unroll
       for (int u = 0; u < UB; ++u) B.id[u] = __shfl(idx_l, (ib + u) * KPI + L.grp);
       L.template request<UB, KEYED>(B);
-      float z[UB];
+      float z[UB], am[UB];
+#pragma unroll
+      for (int u = 0; u < UB; ++u) am[u] = (!PLAIN && P.amask) ? __shfl(am_l, (ib + u) * KPI + L.grp) : 0.f;
       float mb;
       if constexpr (KEYED) {
         uint32_t kz[UB];
 #pragma unroll
         for (int u = 0; u < UB; ++u) kz[u] = (uint32_t)__shfl((int)key_l, (ib + u) * KPI + L.grp);
-        mb = L.template logits_of_keys<UB, PLAIN>(P, moff, kz, B, z);
+        mb = L.template logits_of_keys<UB, PLAIN>(P, am, kz, B, z);
       } else {
-        mb = L.template logits<UB, PLAIN>(P, moff, qv, B, z);
+        mb = L.template logits<UB, PLAIN>(P, am, qv, B, z);
       }
       if (!PLAIN && P.logits_out && L.sub == 0) {
 #pragma unroll

@@ -34,7 +34,8 @@ struct selattn_params {
 // KEYED: the score keys are q.k itself, rounded as torch's matmul rounds it, and come with the remainders of that
 // rounding (the exact scoring pass of OracleTopK): the walk takes its logits from there (two 2-byte reads per entry,
 // of lines the selection has just pulled through the L2) and reads V rows only.
-template <int DT, int D, int CPW, bool KEYED>
+// MASKED: the attention adds an additive mask (fresh rows, not KEYED): a form of its own, the others carry no trace of it.
+template <int DT, int D, int CPW, bool KEYED, bool MASKED>
 __global__ __launch_bounds__(SF_NT) void k_select16_attn(selattn_params P, att_params A) {
   sah_touch_kernargs<sizeof(selattn_params) + sizeof(att_params)>();
   constexpr int NW = SF_NT / SAH_WAVE;
@@ -89,7 +90,11 @@ __global__ __launch_bounds__(SF_NT) void k_select16_attn(selattn_params P, att_p
   const uint16_t* krow = P.keys + (int64_t)r * P.pitch;
   const uint16_t* rrow = KEYED ? P.resid + (int64_t)r * P.pitch : nullptr;
   auto key_of = [&](int, int col) { return (uint32_t)krow[col] | ((uint32_t)rrow[col] << 16); };  // col_offset is 0
-  if (KEYED && P.fresh)
+  if (MASKED)
+    att_walk<DT, D, false, false>(
+        A, r, b, h, hk, qi, first, bound, SAH_WAVE,
+        [&](int i) { return i >= earlier ? s_cols[i] : (i < s_hi ? i : lo2 + (i - s_hi)); }, [&](int) { return unit; }, st);
+  else if (KEYED && P.fresh)
     att_walk<DT, D, false, true>(
         A, r, b, h, hk, qi, first, bound, SAH_WAVE,
         [&](int i) { return i >= earlier ? s_cols[i] : (i < s_hi ? i : lo2 + (i - s_hi)); }, [&](int) { return unit; }, st, key_of);
@@ -129,22 +134,25 @@ int64_t selattn_work_floats(int n_rows, int D) {
   return (int64_t)n_rows * parts * (D + 2);
 }
 
-template <int DT, int D, int CPW, bool KEYED>
+template <int DT, int D, int CPW, bool KEYED, bool MASKED>
 static int selattn_launch(const sah_select_topk_args* s, const selattn_params& P, const att_params& A, size_t lds) {
-  if (int rc = sah_allow_lds((const void*)k_select16_attn<DT, D, CPW, KEYED>, 150 * 1024, "sah_select_topk_attention")) return rc;
+  if (int rc = sah_allow_lds((const void*)k_select16_attn<DT, D, CPW, KEYED, MASKED>, 150 * 1024, "sah_select_topk_attention")) return rc;
   const int G = A.Hq / A.Hkv;
   const int n_tiles = P.R.n_rows / G;
   const int n_wg = (n_tiles + ATT_XCDS - 1) / ATT_XCDS * ATT_XCDS * G * P.parts;
   sah_timed timed("k_select16_attn", s->stream);
-  hipLaunchKernelGGL((k_select16_attn<DT, D, CPW, KEYED>), dim3(n_wg), dim3(SF_NT), lds, (hipStream_t)s->stream, P, A);
+  hipLaunchKernelGGL((k_select16_attn<DT, D, CPW, KEYED, MASKED>), dim3(n_wg), dim3(SF_NT), lds, (hipStream_t)s->stream, P, A);
   return sah_launch_status("sah_select_topk_attention");
 }
 
 template <int DT, int D>
 static int selattn_launch_c(const sah_select_topk_args* s, const selattn_params& P, const att_params& A, size_t lds, int cpw,
                             bool keyed) {
-  if (keyed) return cpw <= 4 ? selattn_launch<DT, D, 4, true>(s, P, A, lds) : selattn_launch<DT, D, 8, true>(s, P, A, lds);
-  return cpw <= 4 ? selattn_launch<DT, D, 4, false>(s, P, A, lds) : selattn_launch<DT, D, 8, false>(s, P, A, lds);
+  if (A.amask)
+    return cpw <= 4 ? selattn_launch<DT, D, 4, false, true>(s, P, A, lds) : selattn_launch<DT, D, 8, false, true>(s, P, A, lds);
+  if (keyed)
+    return cpw <= 4 ? selattn_launch<DT, D, 4, true, false>(s, P, A, lds) : selattn_launch<DT, D, 8, true, false>(s, P, A, lds);
+  return cpw <= 4 ? selattn_launch<DT, D, 4, false, false>(s, P, A, lds) : selattn_launch<DT, D, 8, false, false>(s, P, A, lds);
 }
 
 extern "C" int sah_select_topk_attention(const sah_select_topk_args* s, const sah_attention_args* t, uint32_t* tickets) {
@@ -167,7 +175,7 @@ extern "C" int sah_select_topk_attention(const sah_select_topk_args* s, const sa
   if (worst > s->rows.cap) worst = s->rows.cap;
   const bool one_kernel =
       sel16_ok(s) && cpw <= 8 && (size_t)s->rows.cap * 4 <= sf_hist_bytes() && lds + 10 * 1024 <= 150 * 1024 && !s->rows.w &&
-      !t->dense && !t->closed_form && !t->amask && !t->logits_out && !t->rows.w && t->dropout_p == 0.f &&
+      !t->dense && !t->closed_form && (!t->amask || (s->fresh && !keyed)) && !t->logits_out && !t->rows.w && t->dropout_p == 0.f &&
       t->rows.cols == s->rows.cols && t->rows.cnt == s->rows.cnt && t->rows.cap == s->rows.cap && t->rows.n_rows == n_rows &&
       t->stream == s->stream && (t->dtype == SAH_BF16 || t->dtype == SAH_F16) && (t->D == 128 || t->D == 64) &&
       // one workgroup per row pays when the rows are short enough for the whole-row form; several per row always

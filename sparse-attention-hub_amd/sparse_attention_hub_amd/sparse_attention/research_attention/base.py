@@ -94,7 +94,7 @@ class ResearchAttention(SparseAttention):
         want_error = metrics.is_metric_enabled("research_attention_output_error")
 
         if (not (want_density or want_error)  # the metrics read the finished mask: masker-by-masker path
-                and not self.return_attention_weights and attention_mask is None and self._plan_kind is not None
+                and not self.return_attention_weights and (attention_mask is None or queries.shape[2] == 1) and self._plan_kind is not None
                 and not isinstance(kwargs.get("s_aux"), torch.Tensor) and queries.dim() == 4
                 and not (dropout > 0.0 and module is not None and getattr(module, "training", False))):
             # decode fast path: the whole chain as one native call over cached argument blocks
@@ -103,7 +103,7 @@ class ResearchAttention(SparseAttention):
             plan = self._plans.get(key)
             if plan is None:
                 plan = self._plans[key] = DecodePlan(self.maskers, self._plan_kind, queries, keys)
-            out = plan.run(queries, keys, values, scaling, sparse_meta_data, kwargs.get("layer_idx"))
+            out = plan.run(queries, keys, values, scaling, sparse_meta_data, kwargs.get("layer_idx"), attention_mask)
             if out is not None:
                 return out, None
 

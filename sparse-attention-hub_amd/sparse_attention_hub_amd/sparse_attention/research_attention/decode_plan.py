@@ -4,8 +4,8 @@
 its maskers in Python and then calls the masked attention. For the chains every decode
 benchmark of this path uses —
 
-    Sink, Local [, HashAttentionTopK | OracleTopK | PQCache]      (no additive mask, no sink
-                                                                    logits, weights not requested)
+    Sink, Local [, HashAttentionTopK | OracleTopK | PQCache]      (no sink logits, weights not requested; an
+                                                                    additive mask with one query per row)
 
 — the same kernels can be driven from argument blocks that are built once and patched per
 step (tensor pointers, key count), then handed to `sah_run_chain` in ONE native call. The
@@ -13,7 +13,7 @@ results are those of the masker-by-masker path (same kernels, same order); what 
 is the per-step Python: Mask objects, row-buffer allocation, five ctypes dispatches.
 
 Anything the plan does not cover (first call of a layer that has to hash every key or run
-k-means, a full-mask short-circuit, an additive attention mask, ...) returns None and the
+k-means, a full-mask short-circuit, an additive mask over several queries, ...) returns None and the
 caller takes the general path.
 """
 from __future__ import annotations
@@ -24,7 +24,7 @@ from typing import Any, Dict, Optional, Tuple
 import torch
 
 from ... import _native as N
-from ..utils.mask_attention_utils import _workspace, unit_inverse_weight
+from ..utils.mask_attention_utils import _workspace, additive_mask_args, unit_inverse_weight
 from .maskers.fixed.base import sortable_key_of
 from .maskers.fixed.implementations.basic_fixed import LocalMasker, SinkMasker
 from .maskers.fixed.implementations.hashattention_top_k import HashAttentionTopKMasker, PackedSignatureCache
@@ -88,6 +88,7 @@ class DecodePlan:
         self.sink_local = N.SinkLocalArgs()
         self.hamming = N.HammingTopkArgs()
         self.hash_decode = N.HashDecodeArgs()
+        self.scores = N.HammingScoresArgs()
         self.compact = N.HashCompactArgs()
         self.qk = N.QkScoresArgs()
         self.pq_assign = N.PqAssignArgs()
@@ -100,6 +101,7 @@ class DecodePlan:
         # arrival counters of the one-kernel selection + attention (zero between calls: the kernel puts them back)
         self.tickets = torch.zeros((self.n_rows,), dtype=torch.int32, device=self.device)
         self._excluded_min = sortable_key_of(torch.finfo(q.dtype).min, q.dtype)
+        self._excluded_inf = sortable_key_of(float("-inf"), q.dtype)
 
     def signature(self, q: torch.Tensor, k: torch.Tensor) -> Tuple:
         return (q.device, q.dtype, tuple(q.shape), k.shape[1])
@@ -131,8 +133,11 @@ class DecodePlan:
 
     # --------------------------------------------------------------------- run
     def run(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scaling: float,
-            sparse_meta_data: Dict[Any, Any], layer_idx: Optional[int]) -> Optional[torch.Tensor]:
+            sparse_meta_data: Dict[Any, Any], layer_idx: Optional[int],
+            attention_mask: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
         """One layer-step; returns the attention output (B, Lq, Hq, D) or None if not applicable."""
+        if attention_mask is not None and (self.Lq != 1 or attention_mask.dim() != 4):
+            return None
         Lk = k.shape[2]
         Lq = self.Lq
         sink = self.sink_masker._calculate_effective_sink_size(Lk)
@@ -149,6 +154,8 @@ class DecodePlan:
                 return None
         if q.stride(3) != 1 or k.stride(3) != 1 or v.stride(3) != 1 or v.shape[2] != Lk:
             return None
+        masked = attention_mask is not None
+        am_keep, am_ptr, am_b, am_h, am_l = additive_mask_args(attention_mask, q, Lk)
         stream = N.stream_ptr(self.device)
         cap = sink + window + k_eff
         self._ensure_rows(cap, Lk)
@@ -200,7 +207,22 @@ class DecodePlan:
             bq.x = q.data_ptr()
             bq.xs_b, bq.xs_h, bq.xs_l, bq.stream = q.stride(0), q.stride(1), q.stride(2), stream
             chain.sig_b = C.addressof(bq)
-            if Lq == 1:
+            if masked:
+                # an additive mask takes part in the scores: they go through memory as sortable keys, and the
+                # selection writes the sink + local rows itself (the codes of keys that are still inside the window,
+                # perhaps not hashed yet, belong to columns it leaves out)
+                self._ensure_keybuf(Lk)
+                sc = self.scores
+                sc.kcodes, sc.code_pitch, sc.qcodes = cache.codes.data_ptr(), cache.capacity, self.qcodes.data_ptr()
+                sc.B, sc.Hq, sc.Lq, sc.n_keys = self.B, self.Hq, Lq, Lk
+                sc.amask, sc.ms_b, sc.ms_h, sc.ms_l = am_ptr, am_b, am_h, am_l
+                sc.dtype, sc.keys_out, sc.key_pitch, sc.stream = self.dt, self.keybuf.data_ptr(), self.keybuf_pitch, stream
+                se = self.select
+                se.rows, se.keys, se.key_pitch, se.key_bits = rows, self.keybuf.data_ptr(), self.keybuf_pitch, self.key_bits
+                se.n_cand, se.col_offset, se.k, se.excluded_key, se.stream = Lk, 0, k_eff, self._excluded_inf, stream
+                se.skip_bitmap, se.fresh, se.fresh_sink, se.fresh_window = 1, 1, sink, window
+                chain.sink_local = None
+            elif Lq == 1:
                 # the whole mask-building half of the step as one entry point (one kernel when shapes allow);
                 # a single new key is hashed inside it, a block of them by one launch in front of it
                 hd = self.hash_decode
@@ -244,10 +266,10 @@ class DecodePlan:
             qa = self.qk
             qa.q, qa.qs_b, qa.qs_h, qa.qs_l = q.data_ptr(), q.stride(0), q.stride(1), q.stride(2)
             qa.k, qa.ks_b, qa.ks_h, qa.ks_l = k.data_ptr(), k.stride(0), k.stride(1), k.stride(2)
-            qa.amask = None
+            qa.amask, qa.ms_b, qa.ms_h, qa.ms_l = am_ptr, am_b, am_h, am_l
             qa.dtype, qa.B, qa.Hq, qa.Hkv, qa.Lq, qa.Lk, qa.D = self.dt, self.B, self.Hq, self.Hkv, Lq, Lk, self.D
             qa.keys_out, qa.key_pitch, qa.stream = self.keybuf.data_ptr(), self.keybuf_pitch, stream
-            qa.resid_out = None if self.residbuf is None else self.residbuf.data_ptr()
+            qa.resid_out = None if masked or self.residbuf is None else self.residbuf.data_ptr()
             chain.qk = C.addressof(qa)
             se = self.select
             se.rows, se.keys, se.key_pitch, se.key_bits = rows, self.keybuf.data_ptr(), self.keybuf_pitch, self.key_bits
@@ -328,7 +350,7 @@ class DecodePlan:
         at.q, at.qs_b, at.qs_h, at.qs_l = q.data_ptr(), q.stride(0), q.stride(1), q.stride(2)
         at.k, at.ks_b, at.ks_h, at.ks_l = k.data_ptr(), k.stride(0), k.stride(1), k.stride(2)
         at.v, at.vs_b, at.vs_h, at.vs_l = v.data_ptr(), v.stride(0), v.stride(1), v.stride(2)
-        at.amask = None
+        at.amask, at.ms_b, at.ms_h, at.ms_l = am_ptr, am_b, am_h, am_l
         at.sinks = None
         at.dtype, at.B, at.Hq, at.Hkv, at.Lq, at.Lk, at.D = self.dt, self.B, self.Hq, self.Hkv, Lq, Lk, self.D
         at.scaling, at.unit_inv_w, at.dense, at.max_cnt = float(scaling), self.unit, 0, cap
@@ -337,15 +359,22 @@ class DecodePlan:
         at.closed_form = 0
         # an exact scoring pass came before: its 16-bit keys are the attention's logits, K is not read again
         at.score_keys, at.score_resid, at.score_pitch = None, None, 0
-        if self.kind == "oracle" and self.residbuf is not None:
+        if self.kind == "oracle" and self.residbuf is not None and not masked:
             at.score_keys, at.score_resid, at.score_pitch = self.keybuf.data_ptr(), self.residbuf.data_ptr(), self.keybuf_pitch
-        if self.kind == "fixed" and Lq == 1:
+        if self.kind == "fixed" and Lq == 1 and not masked:
             # Sink + Local alone: the attention kernel takes the columns in closed form, no row is ever written
             at.closed_form, at.closed_sink, at.closed_window = 1, sink, window
             chain.sink_local = None
         at.stream = stream
         chain.attention = C.addressof(at)
         chain.tickets = self.tickets.data_ptr()
+        if masked and self.kind == "hash":
+            # signatures, then the masked scores, then selection and attention
+            chain.attention = None
+            N.call("sah_run_chain", chain)
+            N.call("sah_hamming_scores", self.scores)
+            chain.sig_a = chain.sig_b = None
+            chain.select, chain.attention = C.addressof(self.select), C.addressof(at)
         N.call("sah_run_chain", chain)
         for obj, name, value in commit:
             setattr(obj, name, value)

@@ -204,3 +204,54 @@ def test_clustering_draws_its_start_and_its_reseeds_as_torch_does(cuda, dtype, s
     codes_o, cent_o = O.kmeans_lloyd(O.pq_split(k, off, n_sub), start, iters, reseed_idx=reseed, tol=-1.0)
     assert torch.equal(centres.cpu().reshape(-1), cent_o.float().reshape(-1))
     assert torch.equal(codes.cpu().permute(0, 1, 3, 2).reshape(groups, n).long(), codes_o.reshape(groups, n).long())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("chain", ["fixed", "hash", "oracle", "pq"])
+@pytest.mark.parametrize("kind", ["padded", "hidden", "general"])
+@pytest.mark.parametrize("shape", [(3, 8, 2, 1201, 128), (1, 14, 2, 700, 64), (24, 8, 8, 333, 64)])  # 24, 14 and 192 rows:
+def test_masked_decode_plan_against_masker_by_masker(cuda, dtype, chain, kind, shape):  # several workgroups a row, and one
+    """Decode steps under an additive mask, the cache growing by single keys and by a block: the planned steps against the
+    masker-by-masker path. Same scores and selection; the softmax's sums are taken in another order, which moves a 16-bit
+    result by its last bit here and there (2^-8 / 2^-11 of single elements) and an fp32 one by a few 2^-24 of its sums."""
+    import sparse_attention_hub_amd.sparse_attention as sa
+    from sparse_attention_hub_amd.sparse_attention.utils.hashattention_utils import random_hat_weights
+
+    B, Hq, Hkv, Lk, D = shape
+    cfgs = [sa.SinkMaskerConfig(sink_size=9), sa.LocalMaskerConfig(window_size=70)]
+    if chain == "hash":
+        cfgs.append(sa.HashAttentionTopKMaskerConfig(
+            heavy_size=50, hat_bits=32, hat_mlp_layers=3, hat_mlp_hidden_size=128, hat_mlp_activation="silu",
+            hat_weights=random_hat_weights(1, Hq, D, 32, 3, 128, dtype=dtype, seed=1)))
+    elif chain == "oracle":
+        cfgs.append(sa.OracleTopKConfig(heavy_size=50))
+    elif chain == "pq":
+        cfgs.append(sa.PQCacheConfig(heavy_size=50, pq_group_factor=8, pq_bits=4, kmeans_iter=3, init_offset=9, metric="euclidean"))
+    steps = [Lk - 69, Lk - 68, Lk - 67, Lk - 1, Lk]
+    _, k, v = make_qkv(B, Hq, Hkv, 1, Lk, D, dtype, seed=5, device=cuda)
+    outs = []
+    for planned in (True, False):
+        ra = sa.ResearchAttention.create_from_config(sa.ResearchAttentionConfig(masker_configs=cfgs))
+        ra.return_attention_weights = False
+        assert ra._plan_kind == chain
+        if not planned:
+            ra._plan_kind = None
+        meta, got = {}, []
+        for i, n in enumerate([steps[0]] + steps):  # the first call fills the layer's cache
+            q = make_qkv(B, Hq, Hkv, 1, 1, D, dtype, seed=100 + i, device=cuda)[0]
+            m = torch.zeros((B, 1, 1, n + 3))  # wider than the keys
+            hidden = -float("inf") if kind == "hidden" else float(torch.finfo(dtype).min)
+            for b in range(B):
+                m[b, ..., : (b + 1) * n // (2 * B + 2)] = hidden
+            if kind == "general":
+                m[..., ::3] -= 1.5
+                m.clamp_(min=float(torch.finfo(dtype).min))
+            out, _ = ra.custom_attention(None, q, k[:, :, :n], v[:, :, :n], m.to(dtype).to(cuda), D ** -0.5, 0.0,
+                                         sparse_meta_data=meta, layer_idx=0)
+            got.append(out.double().cpu())
+        assert bool(ra._plans) == planned
+        outs.append(torch.stack(got))
+    a, b = outs
+    assert bool(torch.isfinite(b).all())
+    unit = {torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10, torch.float32: 2.0 ** -18}[dtype]
+    assert bool(((a - b).abs() <= unit * b.abs() + (1e-6 if dtype == torch.float32 else 2.0 ** -18)).all())
