@@ -285,35 +285,64 @@ __global__ __launch_bounds__(PQB_NT) void k_pq_assign_block(pq_assign_params P) 
 
 // ---------------------------------------------------------------------------
 // Lloyd assignment on the matrix cores. argmin_c ||x - c||^2 = argmin_c (||c||^2 - 2 x.c): the key x centre
-// contraction is an fp32 MFMA (32 centres x 32 keys x 2 dims per instruction) whose accumulator starts at
-// ||c||^2 and whose A operand is -2 c, so the accumulator IS the quantity to minimise. A lane owns one key
-// (column) and, per centre tile, 16 centres (rows) in ascending order: the running argmin needs no cross-lane
-// work until the two lanes of a key are merged at the end. Centres (pre-scaled, in operand order) and their
-// norms sit in LDS; per-centre sums for the update step are accumulated in LDS and flushed once.
+// contraction is a 32 x 32 matrix product whose accumulator starts at ||c||^2 and whose A operand is -2 c, so the
+// accumulator IS the quantity to minimise. A lane owns one key (column) and, per centre tile, 16 centres (rows) in
+// ascending order: the running argmin needs no cross-lane work until the two lanes of a key are merged at the end.
+// Centres (pre-scaled, in operand order) and their norms sit in LDS; per-centre sums for the update step are
+// accumulated in LDS and flushed once.
+// SPLIT (bf16 keys): -2 c is cut into three bf16 terms of 8 bits each, which together ARE the fp32 number, and the
+// product runs on the bf16 instructions (32 cycles for 16 dimensions x 1 term; in fp32 64 cycles for 2 dimensions):
+// every x * term is exact in fp32, the accumulation is fp32 as before.
+// Measured (bf16, 8 heads x 16405 keys, 16 sub-vectors of 8, 256 centres, sums included): 205 -> 80 us, of which the
+// search takes 64 (what bounds it: 27 vector and 2 matrix instructions a tile); fp16 (no split: terms of small centres
+// would leave its range) 206 -> 132. 32768 keys, 2 sub-vectors of 64, 64 centres: 214 -> 47. Sums in [centre][d] order
+// and a flush of one centre a lane took 40 (8 dims) to 100 us (64 dims) of these.
 // The expansion rounds differently from the difference form of the reference ((A - B)^2 summed,
 // pq_utils.py:220-257): a key whose two nearest centres tie to the last bits may take the other one.
 // ---------------------------------------------------------------------------
-#define PQM_NT 256
+#define PQM_NT 512
 #define PQM_NW (PQM_NT / SAH_WAVE)
-#define PQM_KEY_TILES 16  // 32-key tiles per wave and workgroup: 2048 keys per workgroup
-#define PQM_MAX_D 128     // widest sub-vector of the matrix-core assignment (64 k-steps)
+#define PQM_MIN_TILES 64   // 32-key tiles a workgroup takes at least: 2048 keys
+#define PQM_WGS 512        // and no more workgroups than this where the keys allow it (two per CU): every workgroup
+                           // loads the centres and flushes n_cent * d_sub 64-bit sums with atomics
+#define PQM_MAX_D 128      // widest sub-vector of the matrix-core assignment (64 k-steps)
 #define PQM_FUSED_LDS (80 * 1024)  // operands + sums up to this much LDS: sums in the same kernel, two workgroups a CU
+#define PQM_MAX_LDS (144 * 1024)
+#define PQM_MIN(a, b) __builtin_elementwise_minimum(a, b)  // three-way minimum instruction, no quieting of its operands
+
+// 16-byte operands per lane and centre tile of the split form: terms x dimensions in slots of 16 (sub-vectors of 8: two
+// instructions; beyond: three per 16 dimensions)
+__host__ __device__ constexpr int pqm_split_ops(int ks) { return ks <= 4 ? 2 : 3 * (ks / 8); }
 
 // LDS of the assignment kernel: A operands, centre norms and, when the sums are fused, the fixed-point sums and counts
-static size_t pqm_lds_bytes(int n_cent, int d_sub, int ks, bool sums) {
+static size_t pqm_lds_bytes(int n_cent, int d_sub, int ks, bool sums, bool split) {
   const size_t n_tiles = (size_t)(n_cent + 31) / 32;
-  size_t bytes = n_tiles * 64 * ks * 4 + n_tiles * 32 * 4;
+  size_t bytes = n_tiles * 64 * (split ? 16 * (size_t)pqm_split_ops(ks) : 4 * (size_t)ks) + n_tiles * 32 * 4;
   if (sums) bytes += (size_t)n_cent * d_sub * 8 + (size_t)n_cent * 4;
   return bytes;
 }
 
+// term 0, 1, 2 of a float as bf16 bits: eight significant bits each, their sum is the float (a float that is not finite
+// stays in term 0)
+__device__ __forceinline__ uint32_t pqm_term(float c, int term) {
+  uint32_t hi = sah_float_to_bits(c) & 0xffff0000u;
+  if ((hi & 0x7f800000u) == 0x7f800000u) return term ? 0u : (hi >> 16) | ((sah_float_to_bits(c) & 0xffffu) ? 1u : 0u);
+  for (int i = 0; i < term; ++i) {
+    c -= sah_bits_to_float(hi);
+    hi = sah_float_to_bits(c) & 0xffff0000u;
+  }
+  return hi >> 16;
+}
+
 // (two waves per SIMD at least: with at most 256 registers a wave the compiler keeps the accumulators in ordinary
 // vector registers, which the minimum search reads directly)
-// KS k-steps of two dimensions each: sub-vectors of up to 2 KS dimensions (the operands beyond d_sub are zero).
-// SUMS: the per-centre sums of the update step are accumulated here (P.sums given and the LDS holds them).
-template <int DT, int KS, bool SUMS>
-__global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P) {
+// KS k-steps of two dimensions each: sub-vectors of up to 2 KS dimensions (the operands beyond d_sub are zero), of
+// exactly 2 KS in the split form. SUMS: the per-centre sums of the update step are accumulated here (P.sums given and
+// the LDS holds them). A workgroup takes wg_tiles tiles of 32 keys of one group.
+template <int DT, int KS, bool SUMS, bool SPLIT>
+__global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P, int wg_tiles) {
   HIP_DYNAMIC_SHARED(unsigned char, pqm_dyn)
+  static_assert(!SPLIT || (DT == SAH_BF16 && KS >= 4), "the split form multiplies bf16 keys in sub-vectors of 8 and more");
   if (P.skip_flag && *P.skip_flag) return;
   const int tid = threadIdx.x;
   const int lane = tid & (SAH_WAVE - 1);
@@ -325,33 +354,66 @@ __global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P
   const int hk = bh % P.Hkv;
   const int b = bh / P.Hkv;
   const int grp = bh * P.n_sub + s_idx;
-  const int n_cent = P.n_cent, d_sub = P.d_sub;
+  const int n_cent = P.n_cent, d_sub = SPLIT ? 2 * KS : P.d_sub;
   const int n_tiles = (n_cent + 31) >> 5;
   const float* cbase = P.centres + (int64_t)grp * n_cent * d_sub;
-  // -2 c as the A operand: element (k-step s, half g, centre row i of tile t). Four k-steps of a row sit together
+  constexpr int SQ = KS >= 4 ? 4 : KS;          // k-steps per 16-byte (8-byte) group of the fp32 form
+  constexpr int OPS = pqm_split_ops(KS);        // 16-byte operands of the split form
+  constexpr int TILE_A = SPLIT ? 64 * 4 * OPS : 64 * KS;  // 32-bit words of a tile's A operands
+  // Sub-vectors of 8 leave slots of their first operand free: the norm's three terms stand there, against ones in the key
+  // operand, instead of four 16-byte LDS reads per tile (16 x 8 dims x 256 centres, 8 heads x 16405 keys: 67 -> 64 us).
+  constexpr bool NORM_IN_A = SPLIT && KS == 4;
+  // -2 c as the A operand. fp32: element (k-step s, half g, centre row i of tile t); four k-steps of a row sit together
   // and consecutive rows follow each other, so that a wave's 16-byte reads are conflict-free whatever KS is.
   float* s_a = (float*)pqm_dyn;                                    // [tile][g][s / 4][i][s % 4]   (KS = 2: [tile][g][i][s])
-  float* s_cn = s_a + (size_t)n_tiles * 64 * KS;                   // ||c||^2, [tile][g][v]
-  long long* s_sum = (long long*)(s_cn + (size_t)n_tiles * 32);    // [centre][d]      (SUMS only; 8-byte aligned: both
-  int* s_cnt = (int*)(s_sum + (size_t)n_cent * d_sub);             // [centre]          sizes above are multiples of 8)
+                                                                   // SPLIT: [tile][op][g][i] of eight bf16
+  float* s_cn = s_a + (size_t)n_tiles * TILE_A;                    // ||c||^2, [tile][g][v]
+  long long* s_sum = (long long*)(s_cn + (size_t)n_tiles * 32);    // [d][centre] (SUMS only; 8-byte aligned: both sizes
+  int* s_cnt = (int*)(s_sum + (size_t)n_cent * d_sub);             // [centre]     above are multiples of 8). A wave adds
+                                                                   // one dimension at a time: the centres of its keys
+                                                                   // spread over the banks
   const float sum_scale = SUMS ? pq_sum_scale(*P.absmax_bits) : 1.f;
-  constexpr int SQ = KS >= 4 ? 4 : KS;  // k-steps per 16-byte (8-byte) group
 
-  for (int idx = tid; idx < n_tiles * 64 * KS; idx += PQM_NT) {
-    const int s4 = idx % SQ, i = (idx / SQ) & 31, q = (idx / (SQ * 32)) % (KS / SQ), gg = (idx / (SQ * 32 * (KS / SQ))) & 1,
-              t = idx / (64 * KS);
-    const int c = t * 32 + i, d = 2 * (q * SQ + s4) + gg;
-    s_a[idx] = (c < n_cent && d < d_sub) ? -2.0f * cbase[c * d_sub + d] : 0.f;
-  }
-  for (int idx = tid; idx < n_tiles * 32; idx += PQM_NT) {
-    const int v = idx & 15, gg = (idx >> 4) & 1, t = idx >> 5;
-    const int c = t * 32 + 8 * (v >> 2) + 4 * gg + (v & 3);
-    float nn = INFINITY;  // centres beyond n_cent never win
-    if (c < n_cent) {
-      nn = 0.f;
-      for (int d = 0; d < d_sub; ++d) nn = fmaf(cbase[c * d_sub + d], cbase[c * d_sub + d], nn);
+  auto norm2 = [&](int c) {
+    if (c >= n_cent) return INFINITY;  // centres beyond n_cent never win
+    float nn = 0.f;
+    for (int d = 0; d < d_sub; ++d) nn = fmaf(cbase[c * d_sub + d], cbase[c * d_sub + d], nn);
+    return nn;
+  };
+  if constexpr (SPLIT) {
+    for (int idx = tid; idx < n_tiles * TILE_A; idx += PQM_NT) {  // one pair of slots each
+      const int e2 = (idx & 3) * 2, i = (idx >> 2) & 31, gg = (idx >> 7) & 1, op = (idx >> 8) % OPS, t = (idx >> 8) / OPS;
+      const int c = t * 32 + i;
+      uint32_t w = 0;
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        int d, term;  // smallest terms first: they meet the accumulator while it holds the norm alone
+        if constexpr (KS == 4) {
+          d = e2 + u;
+          term = op ? gg : (gg ? 3 : 2);
+        } else {
+          d = (op % (KS / 8)) * 16 + 8 * gg + e2 + u;
+          term = 2 - op / (KS / 8);
+        }
+        if (NORM_IN_A && term == 3) {
+          if (e2 + u < 3) w |= pqm_term(norm2(c), e2 + u) << (16 * u);
+        } else if (c < n_cent) w |= pqm_term(-2.0f * cbase[c * d_sub + d], term) << (16 * u);
+      }
+      ((uint32_t*)s_a)[idx] = w;
     }
-    s_cn[idx] = nn;
+  } else {
+    for (int idx = tid; idx < n_tiles * TILE_A; idx += PQM_NT) {
+      const int s4 = idx % SQ, i = (idx / SQ) & 31, q = (idx / (SQ * 32)) % (KS / SQ), gg = (idx / (SQ * 32 * (KS / SQ))) & 1,
+                t = idx / (64 * KS);
+      const int c = t * 32 + i, d = 2 * (q * SQ + s4) + gg;
+      s_a[idx] = (c < n_cent && d < d_sub) ? -2.0f * cbase[c * d_sub + d] : 0.f;
+    }
+  }
+  if (!NORM_IN_A) {
+    for (int idx = tid; idx < n_tiles * 32; idx += PQM_NT) {
+      const int v = idx & 15, gg = (idx >> 4) & 1, t = idx >> 5;
+      s_cn[idx] = norm2(t * 32 + 8 * (v >> 2) + 4 * gg + (v & 3));
+    }
   }
   if (SUMS) {
     for (int i = tid; i < n_cent * d_sub; i += PQM_NT) s_sum[i] = 0;
@@ -360,26 +422,46 @@ __global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P
   __syncthreads();
 
   const int64_t kbase = (int64_t)b * P.ks_b + (int64_t)hk * P.ks_h + (int64_t)s_idx * d_sub;
-  for (int kt = 0; kt < PQM_KEY_TILES; ++kt) {
-    const int n0 = ((tg * PQM_KEY_TILES + kt) * PQM_NW + wave) * 32;
+  constexpr int NB = SPLIT ? (KS >= 8 ? KS / 8 : 1) : 1;  // key operands of 16 dimensions
+  for (int kt = wave; kt < wg_tiles; kt += PQM_NW) {
+    const int n0 = (tg * wg_tiles + kt) * 32;
     if (n0 >= P.n_keys) break;  // uniform across the wave
     const int n = n0 + j;
     const bool valid = n < P.n_keys;
     const int64_t off = kbase + (int64_t)(P.key_offset + (valid ? n : P.n_keys - 1)) * P.ks_l;
-    float xs[KS];  // this lane's dims 2 s + g of its key
+    float xs[SPLIT ? 1 : KS];  // this lane's dims 2 s + g of its key
+    uint4 xb[NB];              // SPLIT: dims 16 q + 8 g .. + 7 (sub-vectors of 8: both halves hold all)
+    uint4 x0;                  // key operand of the first instruction: with the norm in A, ones against its terms
+    if constexpr (SPLIT) {
+      const uint16_t* kp = (const uint16_t*)P.k + off;
+      if constexpr (KS == 4) {
+        xb[0] = *(const uint4*)kp;
+      } else {
 #pragma unroll
-    for (int s = 0; s < KS; ++s) xs[s] = (2 * s + g < d_sub) ? sah_load<DT>(P.k, off + 2 * s + g) : 0.f;
-    float best = INFINITY;
-    int bidx = 0;
-    // accumulator of centre tile t: seeded with the norms, then the KS matrix instructions
-    auto product = [&](sah_f32x16& acc, int t) {
-      const float4* cn4 = (const float4*)(s_cn + (t * 2 + g) * 16);
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        const float4 c4 = cn4[q4];
-        acc[4 * q4] = c4.x; acc[4 * q4 + 1] = c4.y; acc[4 * q4 + 2] = c4.z; acc[4 * q4 + 3] = c4.w;
+        for (int q = 0; q < NB; ++q) xb[q] = *(const uint4*)(kp + 16 * q + 8 * g);
       }
-      if constexpr (KS >= 4) {
+      x0 = KS == 4 && g ? make_uint4(0x3f803f80u, 0x3f80u, 0u, 0u) : xb[0];
+    } else {
+#pragma unroll
+      for (int s = 0; s < KS; ++s) xs[s] = (2 * s + g < d_sub) ? sah_load<DT>(P.k, off + 2 * s + g) : 0.f;
+    }
+    // accumulator of centre tile t: seeded with the norms, then the matrix instructions
+    auto product = [&](sah_f32x16& acc, int t) {
+      if constexpr (NORM_IN_A) {
+        acc = sah_f32x16{};
+      } else {
+        const float4* cn4 = (const float4*)(s_cn + (t * 2 + g) * 16);
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4) {
+          const float4 c4 = cn4[q4];
+          acc[4 * q4] = c4.x; acc[4 * q4 + 1] = c4.y; acc[4 * q4 + 2] = c4.z; acc[4 * q4 + 3] = c4.w;
+        }
+      }
+      if constexpr (SPLIT) {
+        const uint4* ap = (const uint4*)s_a + (size_t)t * 64 * OPS + g * 32 + j;
+#pragma unroll
+        for (int op = 0; op < OPS; ++op) acc = sah_mfma_32x32x16<SAH_BF16>(ap[op * 64], op ? xb[op % NB] : x0, acc);
+      } else if constexpr (KS >= 4) {
         const float4* ap = (const float4*)(s_a + (size_t)(t * 2 + g) * 32 * KS) + j;
 #pragma unroll
         for (int q = 0; q < KS / 4; ++q) {
@@ -395,25 +477,23 @@ __global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P
         for (int s = 0; s < KS; ++s) acc = sah_mfma_32x32x2_f32(ap[s], xs[s], acc);
       }
     };
-    // the tile's first minimum and its accumulator slot (constants), then one comparison with the best so far:
-    // bidx holds 16 t + slot until the end
+    // The smallest value, its tile, and that tile's 16 values, from which the slot is found once at the end: 27 vector
+    // instructions a tile (eight three-way minima, one comparison, 18 selects) where a search for the slot takes 48.
+    // Strictly smaller in ascending tiles, lowest slot: the first minimum is kept.
+    float best = INFINITY;
+    int bt = 0;
+    sah_f32x16 kept = {};
     auto take_min = [&](const sah_f32x16& acc, int t) {
       float m = acc[0];
-      int mv = 0;
 #pragma unroll
-      for (int v = 1; v < 16; ++v) {  // ascending centre index: the first minimum is kept
-        if (acc[v] < m) {
-          m = acc[v];
-          mv = v;
-        }
-      }
-      if (m < best) {
-        best = m;
-        bidx = t * 16 + mv;
-      }
+      for (int v = 1; v < 16; ++v) m = PQM_MIN(m, acc[v]);
+      const bool less = m < best;
+      best = less ? m : best;
+      bt = less ? t : bt;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) kept[v] = less ? acc[v] : kept[v];
     };
-    // Two accumulators: while the matrix unit works on one tile, the vector unit takes the minimum of the tile
-    // before (48 vector instructions against 4 matrix instructions of 16 passes: about the same time).
+    // two accumulators: while the matrix unit works on one tile, the vector unit takes the minimum of the tile before
     sah_f32x16 acc0, acc1;
     product(acc0, 0);
     int t = 0;
@@ -430,33 +510,56 @@ __global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P
     } else {
       take_min(acc0, t);
     }
-    bidx = (bidx >> 4) * 32 + 8 * ((bidx >> 2) & 3) + 4 * g + (bidx & 3);  // tile, slot -> centre
+    int slot = 0;
+#pragma unroll
+    for (int v = 15; v >= 0; --v) slot = kept[v] == best ? v : slot;
+    int bidx = bt * 32 + 8 * (slot >> 2) + 4 * g + (slot & 3);  // tile, slot -> centre
     const float ob = __shfl_xor(best, 32);
     const int oi = __shfl_xor(bidx, 32);
     if (ob < best || (ob == best && oi < bidx)) {
       best = ob;
       bidx = oi;
     }
+    bidx = bidx < n_cent ? bidx : 0;  // (a key that is not finite compares with nothing)
     if (valid) {
       if (g == 0) P.codes[(((int64_t)bh * P.code_pitch) + P.code_offset + n) * P.n_sub + s_idx] = (uint8_t)bidx;
       if (SUMS) {
+        if constexpr (SPLIT) {
+          auto add2 = [&](uint32_t w, int d) {  // two dimensions of a packed word
+            pq_sum_add(&s_sum[d * n_cent + bidx], sah_bits_to_float(w << 16), sum_scale);
+            pq_sum_add(&s_sum[(d + 1) * n_cent + bidx], sah_bits_to_float(w & 0xffff0000u), sum_scale);
+          };
+          if constexpr (KS == 4) {
+            add2(g ? xb[0].z : xb[0].x, 4 * g);
+            add2(g ? xb[0].w : xb[0].y, 4 * g + 2);
+          } else {
 #pragma unroll
-        for (int s = 0; s < KS; ++s)
-          if (2 * s + g < d_sub) pq_sum_add(&s_sum[bidx * d_sub + 2 * s + g], xs[s], sum_scale);
+            for (int q = 0; q < NB; ++q) {
+              add2(xb[q].x, 16 * q + 8 * g);
+              add2(xb[q].y, 16 * q + 8 * g + 2);
+              add2(xb[q].z, 16 * q + 8 * g + 4);
+              add2(xb[q].w, 16 * q + 8 * g + 6);
+            }
+          }
+        } else {
+#pragma unroll
+          for (int s = 0; s < KS; ++s)
+            if (2 * s + g < d_sub) pq_sum_add(&s_sum[(2 * s + g) * n_cent + bidx], xs[s], sum_scale);
+        }
         if (g == 0) atomicAdd(&s_cnt[bidx], 1);
       }
     }
   }
   if (!SUMS) return;
   __syncthreads();
-  for (int c = tid; c < n_cent; c += PQM_NT) {
-    const int cn = s_cnt[c];
-    if (cn) {
-      atomicAdd(&P.counts[(int64_t)grp * n_cent + c], cn);
-      for (int d = 0; d < d_sub; ++d)
-        atomicAdd((unsigned long long*)&P.sums[(int64_t)grp * n_cent * d_sub + c * d_sub + d], (unsigned long long)s_sum[c * d_sub + d]);
-    }
+  // the workgroup's sums, consecutive lanes at consecutive addresses
+  for (int i = tid; i < n_cent * d_sub; i += PQM_NT) {
+    const int c = i / d_sub, d = i - c * d_sub;
+    if (s_cnt[c])
+      atomicAdd((unsigned long long*)&P.sums[(int64_t)grp * n_cent * d_sub + i], (unsigned long long)s_sum[d * n_cent + c]);
   }
+  for (int c = tid; c < n_cent; c += PQM_NT)
+    if (s_cnt[c]) atomicAdd(&P.counts[(int64_t)grp * n_cent + c], s_cnt[c]);
 }
 
 // Per-centre sums and counts from the codes an assignment wrote, for shapes whose sums do not fit beside the
@@ -506,20 +609,33 @@ __global__ __launch_bounds__(PQS_NT) void k_pq_sums(pq_assign_params P, int d_ch
       if (s_cnt[c]) atomicAdd(&P.counts[(int64_t)grp * n_cent + c], s_cnt[c]);
 }
 
-template <int DT, int KS>
+template <int DT, int KS, bool SPLIT>
 static int pq_launch_mfma_ks(const sah_pq_assign_args* a, const pq_assign_params& P, bool fused, size_t lds) {
-  const int per_wg = PQM_NW * 32 * PQM_KEY_TILES;
-  dim3 g(((a->n_keys + per_wg - 1) / per_wg) * a->n_sub, a->B * a->Hkv), blk(PQM_NT);
+  const int tiles = (a->n_keys + 31) / 32;
+  const int64_t all = (int64_t)tiles * a->n_sub * a->B * a->Hkv;
+  int64_t wg_tiles = (all + PQM_WGS - 1) / PQM_WGS;
+  if (wg_tiles < PQM_MIN_TILES) wg_tiles = PQM_MIN_TILES;
+  const int wgs = (int)((tiles + wg_tiles - 1) / wg_tiles);  // per group, of about the same size
+  const int per = (tiles + wgs - 1) / wgs;
+  dim3 g((unsigned)((tiles + per - 1) / per) * a->n_sub, a->B * a->Hkv), blk(PQM_NT);
   hipStream_t st = (hipStream_t)a->stream;
   sah_timed timed("k_pq_assign_mfma", a->stream);
   if (fused) {
-    if (int rc = sah_allow_lds((const void*)k_pq_assign_mfma<DT, KS, true>, 160 * 1024, "sah_pq_kmeans_assign")) return rc;
-    hipLaunchKernelGGL((k_pq_assign_mfma<DT, KS, true>), g, blk, lds, st, P);
+    if (int rc = sah_allow_lds((const void*)k_pq_assign_mfma<DT, KS, true, SPLIT>, 160 * 1024, "sah_pq_kmeans_assign")) return rc;
+    hipLaunchKernelGGL((k_pq_assign_mfma<DT, KS, true, SPLIT>), g, blk, lds, st, P, per);
   } else {
-    if (int rc = sah_allow_lds((const void*)k_pq_assign_mfma<DT, KS, false>, 160 * 1024, "sah_pq_kmeans_assign")) return rc;
-    hipLaunchKernelGGL((k_pq_assign_mfma<DT, KS, false>), g, blk, lds, st, P);
+    if (int rc = sah_allow_lds((const void*)k_pq_assign_mfma<DT, KS, false, SPLIT>, 160 * 1024, "sah_pq_kmeans_assign")) return rc;
+    hipLaunchKernelGGL((k_pq_assign_mfma<DT, KS, false, SPLIT>), g, blk, lds, st, P, per);
   }
   return sah_launch_status("sah_pq_kmeans_assign");
+}
+
+template <int DT, int KS>
+static int pq_launch_mfma_form(const sah_pq_assign_args* a, const pq_assign_params& P, bool split, bool fused, size_t lds) {
+  if constexpr (DT == SAH_BF16 && KS >= 4) {
+    if (split) return pq_launch_mfma_ks<DT, KS, true>(a, P, fused, lds);
+  }
+  return pq_launch_mfma_ks<DT, KS, false>(a, P, fused, lds);
 }
 
 template <int DT>
@@ -527,16 +643,22 @@ static int pq_launch_mfma(const sah_pq_assign_args* a, const pq_assign_params& P
   int ks = 2;
   while (2 * ks < a->d_sub) ks *= 2;  // 2, 4, 8, 16, 32, 64 k-steps: sub-vectors of up to 4 ... 128 dimensions
   const bool want_sums = a->sums != nullptr;
-  const bool fused = want_sums && pqm_lds_bytes(a->n_cent, a->d_sub, ks, true) <= PQM_FUSED_LDS;
-  const size_t lds = pqm_lds_bytes(a->n_cent, a->d_sub, ks, fused);
+  // The split form: bf16 keys, sub-vectors that fill its operands, key rows whose slices can be read 16 bytes at a time,
+  // and centres whose three terms fit LDS. Sub-vectors of 4 stay in fp32: their two matrix instructions take about the
+  // time of the minimum search anyway.
+  const uint64_t align = (uint64_t)(uintptr_t)a->k | 2 * (uint64_t)a->ks_b | 2 * (uint64_t)a->ks_h | 2 * (uint64_t)a->ks_l;
+  const bool split = DT == SAH_BF16 && ks >= 4 && a->d_sub == 2 * ks && align % 16 == 0 &&
+                     pqm_lds_bytes(a->n_cent, a->d_sub, ks, false, true) <= PQM_MAX_LDS;
+  const bool fused = want_sums && pqm_lds_bytes(a->n_cent, a->d_sub, ks, true, split) <= PQM_FUSED_LDS;
+  const size_t lds = pqm_lds_bytes(a->n_cent, a->d_sub, ks, fused, split);
   int rc;
   switch (ks) {
-    case 2: rc = pq_launch_mfma_ks<DT, 2>(a, P, fused, lds); break;
-    case 4: rc = pq_launch_mfma_ks<DT, 4>(a, P, fused, lds); break;
-    case 8: rc = pq_launch_mfma_ks<DT, 8>(a, P, fused, lds); break;
-    case 16: rc = pq_launch_mfma_ks<DT, 16>(a, P, fused, lds); break;
-    case 32: rc = pq_launch_mfma_ks<DT, 32>(a, P, fused, lds); break;
-    default: rc = pq_launch_mfma_ks<DT, 64>(a, P, fused, lds); break;
+    case 2: rc = pq_launch_mfma_form<DT, 2>(a, P, split, fused, lds); break;
+    case 4: rc = pq_launch_mfma_form<DT, 4>(a, P, split, fused, lds); break;
+    case 8: rc = pq_launch_mfma_form<DT, 8>(a, P, split, fused, lds); break;
+    case 16: rc = pq_launch_mfma_form<DT, 16>(a, P, split, fused, lds); break;
+    case 32: rc = pq_launch_mfma_form<DT, 32>(a, P, split, fused, lds); break;
+    default: rc = pq_launch_mfma_form<DT, 64>(a, P, split, fused, lds); break;
   }
   if (rc || !want_sums || fused) return rc;
   // the sums from the codes just written, in a launch of their own

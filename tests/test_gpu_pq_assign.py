@@ -1,0 +1,61 @@
+"""Lloyd assignment on the matrix cores (`sah_pq_kmeans_assign`): the split form (bf16 keys in sub-vectors of 8 and more) and
+the fp32 form at the edges of their tiles, against fp64; sums and counts against the codes, bit for bit."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("sums", [True, False])
+@pytest.mark.parametrize("shape", [  # (B, Hkv, keys, sub-vectors, dims, centres, row stride beyond the sub-vectors)
+    (1, 2, 1024, 16, 8, 256, 0), (1, 1, 1057, 3, 8, 33, 0), (2, 1, 2081, 2, 16, 31, 8), (1, 1, 1, 2, 32, 5, 0),
+    (1, 1, 95, 2, 64, 64, 0), (1, 1, 700, 1, 128, 65, 0), (1, 1, 700, 1, 128, 256, 0),  # the last: three terms outgrow LDS
+    (1, 2, 1030, 4, 8, 40, 4), (1, 2, 1030, 4, 4, 100, 0)])  # rows of 72 bytes, sub-vectors of 4: the fp32 form
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_assignment(cuda, dtype, shape, sums):
+    """The chosen centre's ||c||^2 - 2 x.c in fp64 is within the evaluation's error of the smallest: two values, each with at
+    most 3 d + 4 roundings (the fp32 norm's d, the product's, a few for the alignment inside an instruction) of
+    2^-23 (||c||^2 + 2 sum |x c|)."""
+    from sparse_attention_hub_amd import _native as N
+
+    B, H, n, n_sub, d, n_cent, pad = shape
+    g = torch.Generator().manual_seed(n + d)
+    k = torch.randn(B, H, n, n_sub * d + pad, generator=g).to(dtype)
+    k[..., 1] *= 8.0
+    c = torch.randn(B * H * n_sub, n_cent, d, generator=g) * torch.linspace(0.01, 3.0, n_cent).view(1, -1, 1)
+    kd, cd = k.to(cuda), c.to(cuda)
+    codes = torch.full((B * H, n + 3, n_sub), 255, dtype=torch.uint8, device=cuda)
+    S = torch.zeros(B * H * n_sub, n_cent, d, dtype=torch.int64, device=cuda)
+    C = torch.zeros(B * H * n_sub, n_cent, dtype=torch.int32, device=cuda)
+    top = kd.float().abs().max().view(1)
+    flag = torch.zeros(1, dtype=torch.int32, device=cuda)  # given as in the Lloyd loop: few keys go the same way as many
+    a = N.PqAssignArgs()
+    a.k = kd.data_ptr(); a.ks_b, a.ks_h, a.ks_l = kd.stride()[:3]; a.dtype = N.dtype_code(dtype)
+    a.B, a.Hkv, a.n_sub, a.d_sub, a.n_cent, a.key_offset, a.n_keys = B, H, n_sub, d, n_cent, 0, n
+    a.centres = cd.data_ptr(); a.codes = codes.data_ptr(); a.code_pitch = n + 3; a.code_offset = 3
+    a.skip_flag = flag.data_ptr(); a.stream = N.stream_ptr(cuda)
+    if sums:
+        a.sums = S.data_ptr(); a.counts = C.data_ptr(); a.absmax_bits = top.data_ptr()
+    N.timing_enable(True)
+    N.call("sah_pq_kmeans_assign", a)
+    torch.cuda.synchronize()
+    names = set(N.timing_collect())
+    N.timing_enable(False)
+    if d > 17 or n >= 1024:
+        assert "k_pq_assign_mfma" in names
+    assert bool((codes[:, :3] == 255).all())
+    got = codes[:, 3:].cpu().permute(0, 2, 1).reshape(-1, n).long()
+    x = k[..., : n_sub * d].reshape(B * H, n, n_sub, d).permute(0, 2, 1, 3).reshape(-1, n, d).double()
+    y = c.double()
+    norm = (y * y).sum(-1).unsqueeze(1)
+    dist = norm - 2 * x @ y.transpose(-1, -2)
+    mass = (norm + 2 * x.abs() @ y.abs().transpose(-1, -2)).amax(-1)
+    chosen = dist.gather(2, got.unsqueeze(-1)).squeeze(-1)
+    assert bool((chosen - dist.amin(-1) <= 2 * (3 * d + 4) * 2.0 ** -23 * mass).all())
+    if sums:
+        scale = 2.0 ** (40 - math.frexp(float(top))[1])
+        fixed = torch.round(x * scale).to(torch.int64)  # exact: a power of two and 24 bits
+        assert torch.equal(S.cpu(), torch.zeros_like(S.cpu()).scatter_add_(1, got.unsqueeze(-1).expand(-1, -1, d), fixed))
+        assert torch.equal(C.cpu(), torch.zeros_like(C.cpu()).scatter_add_(1, got, torch.ones_like(got, dtype=torch.int32)))
