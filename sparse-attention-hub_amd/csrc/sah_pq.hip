@@ -293,9 +293,9 @@ __global__ __launch_bounds__(PQB_NT) void k_pq_assign_block(pq_assign_params P) 
 // SPLIT (bf16 keys): -2 c is cut into three bf16 terms of 8 bits each, which together ARE the fp32 number, and the
 // product runs on the bf16 instructions (32 cycles for 16 dimensions x 1 term; in fp32 64 cycles for 2 dimensions):
 // every x * term is exact in fp32, the accumulation is fp32 as before.
-// Measured (bf16, 8 heads x 16405 keys, 16 sub-vectors of 8, 256 centres, sums included): 205 -> 80 us, of which the
-// search takes 64 (what bounds it: 27 vector and 2 matrix instructions a tile); fp16 (no split: terms of small centres
-// would leave its range) 206 -> 132. 32768 keys, 2 sub-vectors of 64, 64 centres: 214 -> 47. Sums in [centre][d] order
+// Measured (bf16, 8 heads x 16405 keys, 16 sub-vectors of 8, 256 centres, sums included): 205 -> 71 us, of which the
+// search takes 62 (what bounds it: 27 vector and 2 matrix instructions a tile); fp16 (no split: terms of small centres
+// would leave its range) 206 -> 127. 32768 keys, 2 sub-vectors of 64, 64 centres: 214 -> 45. Sums in [centre][d] order
 // and a flush of one centre a lane took 40 (8 dims) to 100 us (64 dims) of these.
 // The expansion rounds differently from the difference form of the reference ((A - B)^2 summed,
 // pq_utils.py:220-257): a key whose two nearest centres tie to the last bits may take the other one.
@@ -340,7 +340,7 @@ __device__ __forceinline__ uint32_t pqm_term(float c, int term) {
 // exactly 2 KS in the split form. SUMS: the per-centre sums of the update step are accumulated here (P.sums given and
 // the LDS holds them). A workgroup takes wg_tiles tiles of 32 keys of one group.
 template <int DT, int KS, bool SUMS, bool SPLIT>
-__global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P, int wg_tiles) {
+__global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P, int wg_tiles, int ranges, int n_heads) {
   HIP_DYNAMIC_SHARED(unsigned char, pqm_dyn)
   static_assert(!SPLIT || (DT == SAH_BF16 && KS >= 4), "the split form multiplies bf16 keys in sub-vectors of 8 and more");
   if (P.skip_flag && *P.skip_flag) return;
@@ -348,9 +348,14 @@ __global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P
   const int lane = tid & (SAH_WAVE - 1);
   const int wave = sah_wave_id();
   const int j = lane & 31, g = lane >> 5;
-  const int s_idx = blockIdx.x % P.n_sub;
-  const int tg = blockIdx.x / P.n_sub;
-  const int bh = blockIdx.y;
+  // The workgroups of all sub-vectors of a range of keys read slices of the same rows and write bytes of the same code
+  // words: they follow each other on one XCD (workgroups are dealt to the eight XCDs in turn) and meet in its L2
+  // (with the next tile's keys requested ahead: 80 -> 71 us, 16 sub-vectors of 8, 8 heads x 16405 keys).
+  const int s_idx = (blockIdx.x >> 3) % P.n_sub;
+  const int unit = (int)((blockIdx.x >> 3) / P.n_sub) * 8 + (blockIdx.x & 7);  // (key range, head)
+  const int bh = unit / ranges;
+  const int tg = unit - bh * ranges;
+  if (bh >= n_heads) return;
   const int hk = bh % P.Hkv;
   const int b = bh / P.Hkv;
   const int grp = bh * P.n_sub + s_idx;
@@ -423,25 +428,33 @@ __global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P
 
   const int64_t kbase = (int64_t)b * P.ks_b + (int64_t)hk * P.ks_h + (int64_t)s_idx * d_sub;
   constexpr int NB = SPLIT ? (KS >= 8 ? KS / 8 : 1) : 1;  // key operands of 16 dimensions
+  auto key_offset = [&](int n) { return kbase + (int64_t)(P.key_offset + (n < P.n_keys ? n : P.n_keys - 1)) * P.ks_l; };
+  uint4 nb[NB];  // SPLIT: the next tile's keys, requested while this one is searched
+  auto request = [&](int n) {
+    const uint16_t* kp = (const uint16_t*)P.k + key_offset(n);
+    if constexpr (KS == 4) {
+      nb[0] = *(const uint4*)kp;
+    } else {
+#pragma unroll
+      for (int q = 0; q < NB; ++q) nb[q] = *(const uint4*)(kp + 16 * q + 8 * g);
+    }
+  };
+  if constexpr (SPLIT) request((tg * wg_tiles + wave) * 32 + j);
   for (int kt = wave; kt < wg_tiles; kt += PQM_NW) {
     const int n0 = (tg * wg_tiles + kt) * 32;
     if (n0 >= P.n_keys) break;  // uniform across the wave
     const int n = n0 + j;
     const bool valid = n < P.n_keys;
-    const int64_t off = kbase + (int64_t)(P.key_offset + (valid ? n : P.n_keys - 1)) * P.ks_l;
     float xs[SPLIT ? 1 : KS];  // this lane's dims 2 s + g of its key
     uint4 xb[NB];              // SPLIT: dims 16 q + 8 g .. + 7 (sub-vectors of 8: both halves hold all)
     uint4 x0;                  // key operand of the first instruction: with the norm in A, ones against its terms
     if constexpr (SPLIT) {
-      const uint16_t* kp = (const uint16_t*)P.k + off;
-      if constexpr (KS == 4) {
-        xb[0] = *(const uint4*)kp;
-      } else {
 #pragma unroll
-        for (int q = 0; q < NB; ++q) xb[q] = *(const uint4*)(kp + 16 * q + 8 * g);
-      }
+      for (int q = 0; q < NB; ++q) xb[q] = nb[q];
+      request(n + 32 * PQM_NW);
       x0 = KS == 4 && g ? make_uint4(0x3f803f80u, 0x3f80u, 0u, 0u) : xb[0];
     } else {
+      const int64_t off = key_offset(n);
 #pragma unroll
       for (int s = 0; s < KS; ++s) xs[s] = (2 * s + g < d_sub) ? sah_load<DT>(P.k, off + 2 * s + g) : 0.f;
     }
@@ -617,15 +630,18 @@ static int pq_launch_mfma_ks(const sah_pq_assign_args* a, const pq_assign_params
   if (wg_tiles < PQM_MIN_TILES) wg_tiles = PQM_MIN_TILES;
   const int wgs = (int)((tiles + wg_tiles - 1) / wg_tiles);  // per group, of about the same size
   const int per = (tiles + wgs - 1) / wgs;
-  dim3 g((unsigned)((tiles + per - 1) / per) * a->n_sub, a->B * a->Hkv), blk(PQM_NT);
+  const int ranges = (tiles + per - 1) / per, heads = a->B * a->Hkv;
+  const int64_t n_wg = (((int64_t)ranges * heads + 7) / 8) * 8 * a->n_sub;
+  if (n_wg > 0x7fffffff) return sah_fail(SAH_ESHAPE, "sah_pq_kmeans_assign: too many workgroups");
+  dim3 g((unsigned)n_wg), blk(PQM_NT);
   hipStream_t st = (hipStream_t)a->stream;
   sah_timed timed("k_pq_assign_mfma", a->stream);
   if (fused) {
     if (int rc = sah_allow_lds((const void*)k_pq_assign_mfma<DT, KS, true, SPLIT>, 160 * 1024, "sah_pq_kmeans_assign")) return rc;
-    hipLaunchKernelGGL((k_pq_assign_mfma<DT, KS, true, SPLIT>), g, blk, lds, st, P, per);
+    hipLaunchKernelGGL((k_pq_assign_mfma<DT, KS, true, SPLIT>), g, blk, lds, st, P, per, ranges, heads);
   } else {
     if (int rc = sah_allow_lds((const void*)k_pq_assign_mfma<DT, KS, false, SPLIT>, 160 * 1024, "sah_pq_kmeans_assign")) return rc;
-    hipLaunchKernelGGL((k_pq_assign_mfma<DT, KS, false, SPLIT>), g, blk, lds, st, P, per);
+    hipLaunchKernelGGL((k_pq_assign_mfma<DT, KS, false, SPLIT>), g, blk, lds, st, P, per, ranges, heads);
   }
   return sah_launch_status("sah_pq_kmeans_assign");
 }
@@ -1158,7 +1174,7 @@ static int pq_check_common(const char* what, int B, int Hkv, int n_sub, int d_su
 // Largest |element| of the keys [key_offset, key_offset + n_keys) of every (b, kv head), as float bits (non-negative
 // floats order like their bit patterns, so an integer atomic max does it). *out must be zero before the launch.
 // VEC elements a load: 16 bytes where the rows allow it (an element at a time, with a 64-bit division each, a 33 MB
-// cache took 72 us; its bytes take 7).
+// cache took 72 us; its bytes take 7; with one atomic per wave 51, as here 17).
 template <int DT, int VEC>
 __global__ __launch_bounds__(PQ_NT) void k_pq_absmax(const void* k, int64_t ks_b, int64_t ks_h, int64_t ks_l, int Hkv, int D,
                                                      int key_offset, int n_keys, uint32_t* out) {
@@ -1210,7 +1226,15 @@ __global__ __launch_bounds__(PQ_NT) void k_pq_absmax(const void* k, int64_t ks_b
     const uint32_t other = (uint32_t)__shfl_xor((int)best, o);
     best = other > best ? other : best;
   }
-  if ((threadIdx.x & (SAH_WAVE - 1)) == 0 && best) atomicMax(out, best);
+  // one atomic per workgroup: all go to one address, 5 ns each (8192 of them, one per wave, took 41 us)
+  __shared__ uint32_t s_best[PQ_NT / SAH_WAVE];
+  if ((threadIdx.x & (SAH_WAVE - 1)) == 0) s_best[threadIdx.x / SAH_WAVE] = best;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int w = 1; w < PQ_NT / SAH_WAVE; ++w) best = s_best[w] > best ? s_best[w] : best;
+    if (best) atomicMax(out, best);
+  }
 }
 
 template <int DT>
@@ -1219,7 +1243,7 @@ static void pq_absmax_launch(const sah_pq_absmax_args* a) {
   const bool vec = a->D % VEC == 0 && a->ks_b % VEC == 0 && a->ks_h % VEC == 0 && a->ks_l % VEC == 0 && (uintptr_t)a->k % 16 == 0;
   const int64_t total = (int64_t)a->n_keys * (vec ? a->D / VEC : a->D);
   int64_t gx = (total + PQ_NT * 8 - 1) / (PQ_NT * 8);
-  const int64_t most = (2048 + (int64_t)a->B * a->Hkv - 1) / ((int64_t)a->B * a->Hkv);
+  const int64_t most = (1024 + (int64_t)a->B * a->Hkv - 1) / ((int64_t)a->B * a->Hkv);
   gx = gx < 1 ? 1 : (gx > most ? most : gx);
   dim3 g((unsigned)gx, a->B * a->Hkv), blk(PQ_NT);
   hipStream_t st = (hipStream_t)a->stream;
