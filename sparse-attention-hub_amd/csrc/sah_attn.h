@@ -224,9 +224,9 @@ struct att_lane {
       }
     }
   }
-  // the batch's logits (scaled, plus the additive mask's am[u]; -inf for a lane without a key), and their maximum over the wave
-  template <int UB, bool PLAIN = false>
-  __device__ __forceinline__ float logits(const att_params& P, const float (&am)[UB], const float (&qv)[8], const att_batch<DT, UB>& B,
+  // the batch's logits (scaled, plus the additive mask's mask_of(u); -inf for a lane without a key), and their maximum over the wave
+  template <int UB, bool PLAIN = false, typename MaskOf>
+  __device__ __forceinline__ float logits(const att_params& P, MaskOf mask_of, const float (&qv)[8], const att_batch<DT, UB>& B,
                                           float (&z)[UB]) const {
     float mb = -INFINITY;
 #pragma unroll
@@ -238,7 +238,7 @@ struct att_lane {
       for (int e = 0; e < 8; ++e) d = fmaf(qv[e], kf[e], d);
       d = att_group_sum<LPK>(d) * P.scaling;
       if (B.id[u] >= 0) {
-        if (!PLAIN && P.amask) d += am[u];
+        if (!PLAIN && P.amask) d += mask_of(u);
       } else {
         d = -INFINITY;
       }
@@ -251,8 +251,8 @@ struct att_lane {
     return mb;
   }
   // the same from score keys: key[u] holds q.k of the lane's key in iteration u as (key, remainder)
-  template <int UB, bool PLAIN = false>
-  __device__ __forceinline__ float logits_of_keys(const att_params& P, const float (&am)[UB], const uint32_t (&key)[UB],
+  template <int UB, bool PLAIN = false, typename MaskOf>
+  __device__ __forceinline__ float logits_of_keys(const att_params& P, MaskOf mask_of, const uint32_t (&key)[UB],
                                                   const att_batch<DT, UB>& B, float (&z)[UB]) const {
     float mb = -INFINITY;
     if constexpr (DT != SAH_F32) {
@@ -260,7 +260,7 @@ struct att_lane {
       for (int u = 0; u < UB; ++u) {
         float d = att_key_score<DT>(key[u]) * P.scaling;
         if (B.id[u] >= 0) {
-          if (!PLAIN && P.amask) d += am[u];
+          if (!PLAIN && P.amask) d += mask_of(u);
         } else {
           d = -INFINITY;
         }
@@ -313,7 +313,11 @@ struct att_lane {
 // key_of (anything but att_no_key): key_of(i, column) is q.k for entry i as score key (low half) and remainder (high
 // half) - the caller has scored every column already (an exact-score top-k came before); K is then not read at all,
 // and a batch holds twice as many V rows.
-template <int DT, int D, bool DROP = false, bool PLAIN = false, bool FULL = true, typename ColOf, typename InvWOf,
+// MASKED: the caller knows that there is an additive mask. A key's element is then read with its column and not behind the
+// wait for the batch's rows (four layers of a padded batch of 4 at 12K keys: 416 -> 198 us with the planned step). Where the
+// mask is a runtime question the lane's element and its shuffles cost registers and time even without one: 512 rows of
+// 128K keys, no mask, 335 us against 381.
+template <int DT, int D, bool DROP = false, bool PLAIN = false, bool FULL = true, bool MASKED = false, typename ColOf, typename InvWOf,
           typename KeyOf = att_no_key>
 __device__ __forceinline__ void att_walk(const att_params& P, int r, int b, int h, int hk, int qi, int first, int bound,
                                          int stride, ColOf col_of, InvWOf inv_w_of, att_wave_state& st, KeyOf key_of = KeyOf()) {
@@ -333,14 +337,14 @@ __device__ __forceinline__ void att_walk(const att_params& P, int r, int b, int 
     const int my = cbase + lane;
     int idx_l = -1;
     uint32_t key_l = 0;
-    float am_l = 0.f;  // the additive mask of the lane's key: with the columns, not behind the wait for the batch's rows
+    float am_l = 0.f;  // MASKED: the additive mask of the lane's key
     float invw_l = P.unit_inv_w, invw_den_l = P.unit_inv_w;
     if (my < bound) {
       idx_l = col_of(my);
       invw_l = inv_w_of(my);
       if (idx_l < 0 || idx_l >= P.Lk) idx_l = -1;
       if (KEYED && idx_l >= 0) key_l = key_of(my, idx_l);
-      if (!PLAIN && P.amask && idx_l >= 0) am_l = sah_load<DT>(P.amask, moff + idx_l);
+      if (MASKED && idx_l >= 0) am_l = sah_load<DT>(P.amask, moff + idx_l);
       invw_den_l = invw_l;
       if (DROP && idx_l >= 0) {
         invw_l *= P.drop.factor(r, idx_l);
@@ -354,17 +358,24 @@ __device__ __forceinline__ void att_walk(const att_params& P, int r, int b, int 
 #pragma unroll
       for (int u = 0; u < UB; ++u) B.id[u] = __shfl(idx_l, (ib + u) * KPI + L.grp);
       L.template request<UB, KEYED>(B);
-      float z[UB], am[UB];
+      float z[UB];
+      float am[MASKED ? UB : 1];
+      if constexpr (MASKED) {
 #pragma unroll
-      for (int u = 0; u < UB; ++u) am[u] = (!PLAIN && P.amask) ? __shfl(am_l, (ib + u) * KPI + L.grp) : 0.f;
+        for (int u = 0; u < UB; ++u) am[u] = __shfl(am_l, (ib + u) * KPI + L.grp);
+      }
+      auto mask_of = [&](int u) -> float {
+        if constexpr (MASKED) return am[u];
+        return sah_load<DT>(P.amask, moff + B.id[u]);
+      };
       float mb;
       if constexpr (KEYED) {
         uint32_t kz[UB];
 #pragma unroll
         for (int u = 0; u < UB; ++u) kz[u] = (uint32_t)__shfl((int)key_l, (ib + u) * KPI + L.grp);
-        mb = L.template logits_of_keys<UB, PLAIN>(P, am, kz, B, z);
+        mb = L.template logits_of_keys<UB, PLAIN>(P, mask_of, kz, B, z);
       } else {
-        mb = L.template logits<UB, PLAIN>(P, am, qv, B, z);
+        mb = L.template logits<UB, PLAIN>(P, mask_of, qv, B, z);
       }
       if (!PLAIN && P.logits_out && L.sub == 0) {
 #pragma unroll

@@ -91,7 +91,7 @@ __global__ __launch_bounds__(SF_NT) void k_select16_attn(selattn_params P, att_p
   const uint16_t* rrow = KEYED ? P.resid + (int64_t)r * P.pitch : nullptr;
   auto key_of = [&](int, int col) { return (uint32_t)krow[col] | ((uint32_t)rrow[col] << 16); };  // col_offset is 0
   if (MASKED)
-    att_walk<DT, D, false, false>(
+    att_walk<DT, D, false, false, true, true>(
         A, r, b, h, hk, qi, first, bound, SAH_WAVE,
         [&](int i) { return i >= earlier ? s_cols[i] : (i < s_hi ? i : lo2 + (i - s_hi)); }, [&](int) { return unit; }, st);
   else if (KEYED && P.fresh)
