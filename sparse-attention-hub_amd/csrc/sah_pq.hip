@@ -506,7 +506,8 @@ __global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P
 #pragma unroll
       for (int v = 0; v < 16; ++v) kept[v] = less ? acc[v] : kept[v];
     };
-    // two accumulators: while the matrix unit works on one tile, the vector unit takes the minimum of the tile before
+    // two accumulators: a tile's products are issued before the minimum of the tile before is taken, which so never waits
+    // for a product just started
     sah_f32x16 acc0, acc1;
     product(acc0, 0);
     int t = 0;
