@@ -293,10 +293,14 @@ __global__ __launch_bounds__(PQB_NT) void k_pq_assign_block(pq_assign_params P) 
 // SPLIT (bf16 keys): -2 c is cut into three bf16 terms of 8 bits each, which together ARE the fp32 number, and the
 // product runs on the bf16 instructions (32 cycles for 16 dimensions x 1 term; in fp32 64 cycles for 2 dimensions):
 // every x * term is exact in fp32, the accumulation is fp32 as before.
-// Measured (bf16, 8 heads x 16405 keys, 16 sub-vectors of 8, 256 centres, sums included): 205 -> 71 us, of which the
-// search takes 62 (what bounds it: 27 vector and 2 matrix instructions a tile); fp16 (no split: terms of small centres
-// would leave its range) 206 -> 127. 32768 keys, 2 sub-vectors of 64, 64 centres: 214 -> 45. Sums in [centre][d] order
-// and a flush of one centre a lane took 40 (8 dims) to 100 us (64 dims) of these.
+// The split form's rounding is another one (and smaller), so where two centres come within both forms' rounding of each
+// other the key tile is evaluated a second time in fp32: the codes are those of the fp32 form, bit for bit, whichever
+// form the alignment and shape of the keys allow (without: 1e-6 of the codes of an iteration, 5e-4 after ten).
+// Measured (bf16, 8 heads x 16405 keys, 16 sub-vectors of 8, 256 centres, sums included): 204 -> 78 us, 64 of them without
+// the second evaluation (what bounds it: 28 vector and 2 matrix instructions a tile); keys moved by five times their spread,
+// where more centres are near: 94. fp16 (no split: terms of small centres would leave its range) 202 -> 121. 32768 keys,
+// 2 sub-vectors of 64, 64 centres: 218 -> 62. Sums in [centre][d] order and a flush of one centre a lane took 40 (8 dims)
+// to 100 us (64 dims) of these.
 // The expansion rounds differently from the difference form of the reference ((A - B)^2 summed,
 // pq_utils.py:220-257): a key whose two nearest centres tie to the last bits may take the other one.
 // ---------------------------------------------------------------------------
@@ -307,7 +311,7 @@ __global__ __launch_bounds__(PQB_NT) void k_pq_assign_block(pq_assign_params P) 
                            // loads the centres and flushes n_cent * d_sub 64-bit sums with atomics
 #define PQM_MAX_D 128      // widest sub-vector of the matrix-core assignment (64 k-steps)
 #define PQM_FUSED_LDS (80 * 1024)  // operands + sums up to this much LDS: sums in the same kernel, two workgroups a CU
-#define PQM_MAX_LDS (144 * 1024)
+#define PQM_MAX_LDS (144 * 1024)  // operands at most (128 dimensions x 256 centres in fp32: 129 KB); the rest of a CU is static LDS
 #define PQM_MIN(a, b) __builtin_elementwise_minimum(a, b)  // three-way minimum instruction, no quieting of its operands
 
 // 16-byte operands per lane and centre tile of the split form: terms x dimensions in slots of 16 (sub-vectors of 8: two
@@ -414,11 +418,10 @@ __global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P
       s_a[idx] = (c < n_cent && d < d_sub) ? -2.0f * cbase[c * d_sub + d] : 0.f;
     }
   }
-  if (!NORM_IN_A) {
-    for (int idx = tid; idx < n_tiles * 32; idx += PQM_NT) {
-      const int v = idx & 15, gg = (idx >> 4) & 1, t = idx >> 5;
-      s_cn[idx] = norm2(t * 32 + 8 * (v >> 2) + 4 * gg + (v & 3));
-    }
+  for (int idx = tid; idx < n_tiles * 32; idx += PQM_NT) {
+    const int v = idx & 15, gg = (idx >> 4) & 1, t = idx >> 5;
+    const int c = t * 32 + 8 * (v >> 2) + 4 * gg + (v & 3);
+    s_cn[idx] = norm2(c);
   }
   if (SUMS) {
     for (int i = tid; i < n_cent * d_sub; i += PQM_NT) s_sum[i] = 0;
@@ -491,15 +494,17 @@ __global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P
       }
     };
     // The smallest value, its tile, and that tile's 16 values, from which the slot is found once at the end: 27 vector
-    // instructions a tile (eight three-way minima, one comparison, 18 selects) where a search for the slot takes 48.
-    // Strictly smaller in ascending tiles, lowest slot: the first minimum is kept.
-    float best = INFINITY;
+    // instructions a tile (eight three-way minima, one comparison, 18 selects; SPLIT: 28, with the second smallest of the
+    // tiles' minima) where a search for the slot takes 48. Strictly smaller in ascending tiles, lowest slot: the first
+    // minimum is kept.
+    float best = INFINITY, second = INFINITY;
     int bt = 0;
     sah_f32x16 kept = {};
     auto take_min = [&](const sah_f32x16& acc, int t) {
       float m = acc[0];
 #pragma unroll
       for (int v = 1; v < 16; ++v) m = PQM_MIN(m, acc[v]);
+      if (SPLIT) second = __builtin_amdgcn_fmed3f(best, second, m);
       const bool less = m < best;
       best = less ? m : best;
       bt = less ? t : bt;
@@ -524,17 +529,100 @@ __global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P
     } else {
       take_min(acc0, t);
     }
-    int slot = 0;
+    int slot = 0, bidx;
+    bool again;  // uniform: the key tile is evaluated in fp32
+    if constexpr (SPLIT) {
+      // The split form's values round differently from the fp32 form's, and the codes are the fp32 form's whichever form
+      // ran. They agree where no other centre comes within twice the two forms' difference of the smallest value. With
+      // u = 2^-24, fp32's value is off by at most d u of the mass ||c||^2 + 2 sum |x c| (one rounding per product), and the
+      // two by up to 2.8 sqrt(d) u of it from each other (measured over 4e6 pairs each of 8 to 128 dimensions; the split
+      // form is the closer one to fp64): min(2 d, 6 sqrt(d)) u is allowed. A centre that can win is no farther from 0
+      // than |x| + r, r the distance to the nearest, so its mass is at most 3 (|x| + r)^2; 3.5 leaves room for those beyond.
+      float x2 = 0.f;
 #pragma unroll
-    for (int v = 15; v >= 0; --v) slot = kept[v] == best ? v : slot;
-    int bidx = bt * 32 + 8 * (slot >> 2) + 4 * g + (slot & 3);  // tile, slot -> centre
-    const float ob = __shfl_xor(best, 32);
-    const int oi = __shfl_xor(bidx, 32);
-    if (ob < best || (ob == best && oi < bidx)) {
-      best = ob;
-      bidx = oi;
+      for (int q = 0; q < NB; ++q) {
+        const uint32_t w[4] = {xb[q].x, xb[q].y, xb[q].z, xb[q].w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float lo = sah_bits_to_float(w[e] << 16), hi = sah_bits_to_float(w[e] & 0xffff0000u);
+          x2 = fmaf(lo, lo, fmaf(hi, hi, x2));
+        }
+      }
+      if (KS != 4) x2 += __shfl_xor(x2, 32);
+      const float ob = __shfl_xor(best, 32);
+      best = ob < best ? ob : best;
+      float r2 = best + x2;
+      r2 = r2 < 0.f ? 0.f : r2;
+      const float reach = sqrtf(x2) + sqrtf(r2);
+      constexpr float FORMS = KS == 4 ? 16.f : KS == 8 ? 24.f : KS == 16 ? 34.f : KS == 32 ? 48.f : 68.f;
+      const float lim = best + 7.0f * 0x1p-24f * FORMS * reach * reach;  // (not finite where the key is not)
+      // the centres within it, of this lane's 16 of the winning tile and of the other tiles' minima: exactly one wins
+      uint64_t one = 0, two = 0;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const bool near = kept[v] <= lim;
+        slot = near ? v : slot;
+        const uint64_t m = __ballot(near);
+        two |= one & m;
+        one |= m;
+      }
+      const uint64_t m = __ballot(second <= lim);
+      two |= one & m;
+      one |= m;
+      const uint32_t lo1 = (uint32_t)one, hi1 = (uint32_t)(one >> 32);
+      again = ((uint32_t)two | (uint32_t)(two >> 32) | ~(lo1 ^ hi1)) != 0;
+      bidx = bt * 32 + 8 * (slot >> 2) + 4 * g + (slot & 3);  // tile, slot -> centre
+      const int oi = __shfl_xor(bidx, 32);
+      bidx = ((one >> lane) & 1) ? bidx : oi;
+    } else {
+#pragma unroll
+      for (int v = 15; v >= 0; --v) slot = kept[v] == best ? v : slot;
+      bidx = bt * 32 + 8 * (slot >> 2) + 4 * g + (slot & 3);
+      const float ob = __shfl_xor(best, 32);
+      const int oi = __shfl_xor(bidx, 32);
+      if (ob < best || (ob == best && oi < bidx)) bidx = oi;
+      again = false;
     }
-    bidx = bidx < n_cent ? bidx : 0;  // (a key that is not finite compares with nothing)
+    if (again) {  // in fp32, operands straight from memory
+      best = INFINITY;
+      bidx = 0;
+      const int64_t off = key_offset(n);
+      for (int t2 = 0; t2 < n_tiles; ++t2) {
+        sah_f32x16 acc;
+        const float4* cn4 = (const float4*)(s_cn + (t2 * 2 + g) * 16);
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4) {
+          const float4 c4 = cn4[q4];
+          acc[4 * q4] = c4.x; acc[4 * q4 + 1] = c4.y; acc[4 * q4 + 2] = c4.z; acc[4 * q4 + 3] = c4.w;
+        }
+        const bool there = t2 * 32 + j < n_cent;
+        const float* cp = cbase + (there ? t2 * 32 + j : 0) * d_sub;
+#pragma unroll 8
+        for (int s = 0; s < KS; ++s) {
+          const int d = 2 * s + g;
+          const bool in = d < d_sub;
+          const float a = in ? -2.0f * cp[d] : 0.f;
+          acc = sah_mfma_32x32x2_f32(there ? a : 0.f, in ? sah_load<DT>(P.k, off + d) : 0.f, acc);
+        }
+        float m = INFINITY;
+        int mv = 0;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          if (acc[v] < m) {
+            m = acc[v];
+            mv = v;
+          }
+        }
+        if (m < best) {
+          best = m;
+          bidx = t2 * 16 + mv;
+        }
+      }
+      bidx = (bidx >> 4) * 32 + 8 * ((bidx >> 2) & 3) + 4 * g + (bidx & 3);
+      const float ob = __shfl_xor(best, 32);
+      const int oi = __shfl_xor(bidx, 32);
+      if (ob < best || (ob == best && oi < bidx)) bidx = oi;
+    }
     if (valid) {
       if (g == 0) P.codes[(((int64_t)bh * P.code_pitch) + P.code_offset + n) * P.n_sub + s_idx] = (uint8_t)bidx;
       if (SUMS) {
@@ -638,10 +726,10 @@ static int pq_launch_mfma_ks(const sah_pq_assign_args* a, const pq_assign_params
   hipStream_t st = (hipStream_t)a->stream;
   sah_timed timed("k_pq_assign_mfma", a->stream);
   if (fused) {
-    if (int rc = sah_allow_lds((const void*)k_pq_assign_mfma<DT, KS, true, SPLIT>, 160 * 1024, "sah_pq_kmeans_assign")) return rc;
+    if (int rc = sah_allow_lds((const void*)k_pq_assign_mfma<DT, KS, true, SPLIT>, PQM_MAX_LDS, "sah_pq_kmeans_assign")) return rc;
     hipLaunchKernelGGL((k_pq_assign_mfma<DT, KS, true, SPLIT>), g, blk, lds, st, P, per, ranges, heads);
   } else {
-    if (int rc = sah_allow_lds((const void*)k_pq_assign_mfma<DT, KS, false, SPLIT>, 160 * 1024, "sah_pq_kmeans_assign")) return rc;
+    if (int rc = sah_allow_lds((const void*)k_pq_assign_mfma<DT, KS, false, SPLIT>, PQM_MAX_LDS, "sah_pq_kmeans_assign")) return rc;
     hipLaunchKernelGGL((k_pq_assign_mfma<DT, KS, false, SPLIT>), g, blk, lds, st, P, per, ranges, heads);
   }
   return sah_launch_status("sah_pq_kmeans_assign");

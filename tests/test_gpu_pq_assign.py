@@ -59,3 +59,39 @@ def test_assignment(cuda, dtype, shape, sums):
         fixed = torch.round(x * scale).to(torch.int64)  # exact: a power of two and 24 bits
         assert torch.equal(S.cpu(), torch.zeros_like(S.cpu()).scatter_add_(1, got.unsqueeze(-1).expand(-1, -1, d), fixed))
         assert torch.equal(C.cpu(), torch.zeros_like(C.cpu()).scatter_add_(1, got, torch.ones_like(got, dtype=torch.int32)))
+
+
+def _assign(N, dev, k, n_sub, d, c):
+    """Codes (heads, keys, sub-vectors) of keys (1, H, n, .) against centres (H n_sub, n_cent, d)."""
+    H, n = k.shape[1], k.shape[2]
+    codes = torch.full((H, n, n_sub), 255, dtype=torch.uint8, device=dev)
+    flag = torch.zeros(1, dtype=torch.int32, device=dev)
+    a = N.PqAssignArgs()
+    a.k = k.data_ptr(); a.ks_b, a.ks_h, a.ks_l = k.stride()[:3]; a.dtype = N.dtype_code(k.dtype)
+    a.B, a.Hkv, a.n_sub, a.d_sub, a.n_cent, a.key_offset, a.n_keys = 1, H, n_sub, d, c.shape[1], 0, n
+    a.centres = c.data_ptr(); a.codes = codes.data_ptr(); a.code_pitch = n; a.code_offset = 0
+    a.skip_flag = flag.data_ptr(); a.stream = N.stream_ptr(dev)
+    N.call("sah_pq_kmeans_assign", a)
+    torch.cuda.synchronize()
+    return codes.cpu()
+
+
+@pytest.mark.parametrize("d,n_sub,n_cent", [(8, 16, 256), (8, 2, 33), (16, 4, 128), (32, 2, 64), (64, 2, 64), (128, 1, 65)])
+def test_the_split_form_gives_the_codes_of_the_fp32_form(cuda, d, n_sub, n_cent):
+    """bf16 keys in rows of whole 16 bytes (split form) and the same keys in rows that are not (fp32 form): equal codes, also
+    where centres come in pairs a few units of the last place apart, and in equal pairs."""
+    from sparse_attention_hub_amd import _native as N
+
+    n, H = 1500, 2
+    g = torch.Generator().manual_seed(d)
+    k = torch.randn(1, H, n, n_sub * d, generator=g)
+    k[..., 1] *= 8.0
+    k[:, :, :200] += 20.0
+    k = k.bfloat16().to(cuda)
+    c = torch.randn(H * n_sub, n_cent, d, generator=g)
+    half = n_cent // 2
+    c[:, half:2 * half] = c[:, :half] * (1 + torch.randint(-3, 4, (H * n_sub, half, 1), generator=g) * 2.0 ** -23)
+    c = c.to(cuda)
+    wide = torch.zeros(1, H, n, n_sub * d + 4, dtype=torch.bfloat16, device=cuda)
+    wide[..., : n_sub * d] = k
+    assert torch.equal(_assign(N, cuda, k, n_sub, d, c), _assign(N, cuda, wide[..., : n_sub * d], n_sub, d, c))
