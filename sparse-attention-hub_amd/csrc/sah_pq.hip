@@ -418,16 +418,18 @@ __global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P
       s_a[idx] = (c < n_cent && d < d_sub) ? -2.0f * cbase[c * d_sub + d] : 0.f;
     }
   }
+  int odd = 0;  // a centre that is not finite
   for (int idx = tid; idx < n_tiles * 32; idx += PQM_NT) {
     const int v = idx & 15, gg = (idx >> 4) & 1, t = idx >> 5;
     const int c = t * 32 + 8 * (v >> 2) + 4 * gg + (v & 3);
     s_cn[idx] = norm2(c);
+    if (c < n_cent && !(s_cn[idx] < INFINITY)) odd = 1;
   }
   if (SUMS) {
     for (int i = tid; i < n_cent * d_sub; i += PQM_NT) s_sum[i] = 0;
     for (int i = tid; i < n_cent; i += PQM_NT) s_cnt[i] = 0;
   }
-  __syncthreads();
+  odd = __syncthreads_or(odd);
 
   const int64_t kbase = (int64_t)b * P.ks_b + (int64_t)hk * P.ks_h + (int64_t)s_idx * d_sub;
   constexpr int NB = SPLIT ? (KS >= 8 ? KS / 8 : 1) : 1;  // key operands of 16 dimensions
@@ -496,15 +498,17 @@ __global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P
     // The smallest value, its tile, and that tile's 16 values, from which the slot is found once at the end: 27 vector
     // instructions a tile (eight three-way minima, one comparison, 18 selects; SPLIT: 28, with the second smallest of the
     // tiles' minima) where a search for the slot takes 48. Strictly smaller in ascending tiles, lowest slot: the first
-    // minimum is kept.
+    // minimum is kept. A value that is not a number makes the tile's minimum one: such key tiles are evaluated again below.
     float best = INFINITY, second = INFINITY;
     int bt = 0;
+    bool nan = false;
     sah_f32x16 kept = {};
     auto take_min = [&](const sah_f32x16& acc, int t) {
       float m = acc[0];
 #pragma unroll
       for (int v = 1; v < 16; ++v) m = PQM_MIN(m, acc[v]);
       if (SPLIT) second = __builtin_amdgcn_fmed3f(best, second, m);
+      else nan |= m != m;
       const bool less = m < best;
       best = less ? m : best;
       bt = less ? t : bt;
@@ -570,7 +574,7 @@ __global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P
       two |= one & m;
       one |= m;
       const uint32_t lo1 = (uint32_t)one, hi1 = (uint32_t)(one >> 32);
-      again = ((uint32_t)two | (uint32_t)(two >> 32) | ~(lo1 ^ hi1)) != 0;
+      again = odd || ((uint32_t)two | (uint32_t)(two >> 32) | ~(lo1 ^ hi1)) != 0;
       bidx = bt * 32 + 8 * (slot >> 2) + 4 * g + (slot & 3);  // tile, slot -> centre
       const int oi = __shfl_xor(bidx, 32);
       bidx = ((one >> lane) & 1) ? bidx : oi;
@@ -581,9 +585,9 @@ __global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P
       const float ob = __shfl_xor(best, 32);
       const int oi = __shfl_xor(bidx, 32);
       if (ob < best || (ob == best && oi < bidx)) bidx = oi;
-      again = false;
+      again = odd || __ballot(nan) != 0;
     }
-    if (again) {  // in fp32, operands straight from memory
+    if (again) {  // in fp32, operands straight from memory; a value that is not a number loses to any other
       best = INFINITY;
       bidx = 0;
       const int64_t off = key_offset(n);

@@ -79,7 +79,7 @@ def _assign(N, dev, k, n_sub, d, c):
 @pytest.mark.parametrize("d,n_sub,n_cent", [(8, 16, 256), (8, 2, 33), (16, 4, 128), (32, 2, 64), (64, 2, 64), (128, 1, 65)])
 def test_the_split_form_gives_the_codes_of_the_fp32_form(cuda, d, n_sub, n_cent):
     """bf16 keys in rows of whole 16 bytes (split form) and the same keys in rows that are not (fp32 form): equal codes, also
-    where centres come in pairs a few units of the last place apart, and in equal pairs."""
+    where centres come in pairs a few units of the last place apart, in equal pairs, and for keys that are not finite."""
     from sparse_attention_hub_amd import _native as N
 
     n, H = 1500, 2
@@ -87,6 +87,7 @@ def test_the_split_form_gives_the_codes_of_the_fp32_form(cuda, d, n_sub, n_cent)
     k = torch.randn(1, H, n, n_sub * d, generator=g)
     k[..., 1] *= 8.0
     k[:, :, :200] += 20.0
+    k[0, 0, 300, 3], k[0, 1, 301, 0], k[0, 0, 302, 5] = float("inf"), float("-inf"), float("nan")
     k = k.bfloat16().to(cuda)
     c = torch.randn(H * n_sub, n_cent, d, generator=g)
     half = n_cent // 2
@@ -95,3 +96,19 @@ def test_the_split_form_gives_the_codes_of_the_fp32_form(cuda, d, n_sub, n_cent)
     wide = torch.zeros(1, H, n, n_sub * d + 4, dtype=torch.bfloat16, device=cuda)
     wide[..., : n_sub * d] = k
     assert torch.equal(_assign(N, cuda, k, n_sub, d, c), _assign(N, cuda, wide[..., : n_sub * d], n_sub, d, c))
+
+
+@pytest.mark.parametrize("d", [4, 8, 16, 64])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_a_centre_that_is_not_a_number_loses_alone(cuda, dtype, d):
+    """Such a centre takes no key, and the others of its tile take theirs: as if it were far away."""
+    from sparse_attention_hub_amd import _native as N
+
+    g = torch.Generator().manual_seed(d)
+    k = torch.randn(1, 2, 1200, 2 * d, generator=g).to(dtype).to(cuda)
+    c = torch.randn(4, 70, d, generator=g).to(cuda)
+    far = c.clone()
+    for at in (0, 37, 68):  # slot 0 of a tile, and others
+        c[:, at, d - 1] = float("nan")
+        far[:, at] = 1e6
+    assert torch.equal(_assign(N, cuda, k, 2, d, c), _assign(N, cuda, k, 2, d, far))
