@@ -394,7 +394,8 @@ extern "C" int64_t sah_members_attention_work_floats(int32_t B, int32_t Hq, int3
 // entries. At 32 heads x 48 queries x 32768 keys the two meet at 1.5 % (67 us); with 4 queries at 10 % (37 us).
 bool members_attention_pays(const sah_attention_args* a, const att_params& P) {
   if (a->dtype == SAH_F32 || (a->D != 64 && a->D != 128) || a->Lq < 2) return false;
-  if (P.drop.thresh || a->logits_out || a->rows.w || P.dense == 2 || !(a->scaling > 0.f)) return false;
+  // (a row's running maximum lags behind its largest logit, see QA_SLACK: statistics come from the gather)
+  if (P.drop.thresh || a->logits_out || a->stats_out || a->rows.w || P.dense == 2 || !(a->scaling > 0.f)) return false;
   if (a->ks_l * QA_STAGE >= (1 << 30) || a->vs_l * QA_STAGE >= (1 << 30)) return false;  // 32-bit offsets inside a stage
   const int64_t need = sah_members_attention_work_floats(a->B, a->Hq, a->Hkv, a->Lq, a->Lk, a->D);
   if (!a->work || a->work_floats < need) return false;

@@ -137,6 +137,48 @@ def test_attention_of_many_query_vectors(cuda, dtype, kind, shape, density):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("kind", [None, "causal"])
+@pytest.mark.parametrize("density", [None, 0.2])
+def test_statistics_of_many_query_vectors(cuda, dtype, kind, density):
+    """The row's largest logit and the denominator relative to it, at a shape whose plain call takes the matrix-core form,
+    against fp64, and what is built on them. Bounds: a logit's fp32 error, D 2^-23 of sum |q k|, and for the numerator the
+    output's rounding."""
+    import sparse_attention_hub_amd.sparse_attention as sa
+    from sparse_attention_hub_amd.sparse_attention.utils import mask_attention_utils as U
+
+    B, Hq, Hkv, Lq, Lk, D = 1, 8, 2, 48, 2048, 128
+    q, k, v = make_qkv(B, Hq, Hkv, Lq, Lk, D, dtype, seed=11, device=cuda)
+    am = question_mask(B, Lq, Lk, dtype, cuda, kind)
+    member = torch.ones(B, Hq, Lq, Lk, dtype=torch.bool)
+    if density is not None:
+        member = torch.rand(B, Hq, Lq, Lk, generator=torch.Generator().manual_seed(2)) < density
+        member[..., 0] = True
+    mask = (sa.Mask.create_full_mask(member.shape, dtype=dtype, device=cuda) if density is None
+            else sa.Mask.create_mask_from_dense_mask(member.shape, member.to(dtype).to(cuda), dtype))
+    z = q.double().cpu() @ k.double().cpu().repeat_interleave(Hq // Hkv, 1).transpose(-1, -2) * D ** -0.5
+    if am is not None:
+        z = z + am.double().cpu()
+    vv = v.double().cpu().repeat_interleave(Hq // Hkv, 1)
+    sel = z.masked_fill(~member, -float("inf"))
+    top, top_all = sel.amax(-1, keepdim=True), z.amax(-1, keepdim=True)
+    _, stats = U._run_attention(q, k, v, am, None, D ** -0.5, None if density is None else mask.to_rows(0), False, return_stats=True)
+    assert float((stats[:, 0].double().cpu().view_as(top) - top).abs().max()) < 1e-4
+    want = torch.exp(sel - top).sum(-1, keepdim=True)
+    assert float(((stats[:, 1].double().cpu().view_as(top) - want) / want).abs().max()) < 1e-4
+    e = torch.exp(sel - top_all)
+    den = U.get_attention_denominator(None, q, k, am, D ** -0.5, 0.0, mask)
+    num = U.get_attention_numerator(None, q, k, v, am, D ** -0.5, 0.0, mask)
+    assert float(((den.double().cpu() - e.sum(-1, keepdim=True)) / e.sum(-1, keepdim=True)).abs().max()) < 2e-4
+    half = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    assert bool(((num.double().cpu() - e @ vv).abs() <= 1.01 * half * (e @ vv).abs() + 3e-4 * (e @ vv.abs())).all())
+    sinks = torch.linspace(-2.0, 6.0, Hq)
+    _, den2, _ = U.apply_sink_bias(num, den, None, q, k, am, sinks.to(cuda), D ** -0.5)
+    new = torch.maximum(top_all, sinks.double().view(1, Hq, 1, 1))
+    want2 = e.sum(-1, keepdim=True) * torch.exp(top_all - new) + torch.exp(sinks.double().view(1, Hq, 1, 1) - new)
+    assert float(((den2.double().cpu() - want2) / want2).abs().max()) < 2e-4
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("kind", [None, "causal", "general"])
 @pytest.mark.parametrize("shape,pitch", [  # keys on either side of a lane's 8 and a workgroup's 2048; an odd code pitch: the
     # form of one thread per score
