@@ -147,23 +147,6 @@ static int att_launch(const sah_attention_args* a, const att_params& P, bool tim
 }
 
 template <int DT>
-static int att_combine_d(const sah_attention_args* a, int n_split) {
-  sah_timed timed("k_attn_combine", a->stream);
-  if (a->D == 64)
-    hipLaunchKernelGGL((k_attn_combine<DT, 64>), dim3(a->rows.n_rows), dim3(64), 0, (hipStream_t)a->stream, (const float*)a->work,
-                       n_split, a->Hq, a->Lq, a->D, a->sinks, a->out, a->stats_out);
-  else
-    hipLaunchKernelGGL((k_attn_combine<DT, 128>), dim3(a->rows.n_rows), dim3(128), 0, (hipStream_t)a->stream, (const float*)a->work,
-                       n_split, a->Hq, a->Lq, a->D, a->sinks, a->out, a->stats_out);
-  return sah_launch_status("sah_members_attention(combine)");
-}
-
-// merges n_split partial results per row (16-bit types, head_dim 64 / 128): for the matrix-core form
-int att_launch_combine(const sah_attention_args* a, int n_split) {
-  return a->dtype == SAH_BF16 ? att_combine_d<SAH_BF16>(a, n_split) : att_combine_d<SAH_F16>(a, n_split);
-}
-
-template <int DT>
 static int att_dispatch_d(const sah_attention_args* a, const att_params& P, bool timing) {
   switch (a->D) {
     case 16: return att_launch<DT, 16, true>(a, P, timing);

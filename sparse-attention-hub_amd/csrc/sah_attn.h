@@ -108,10 +108,10 @@ __device__ __forceinline__ void att_unpack(const att_raw<DT>& r, float (&o)[8]) 
 // merge the splits of one row: out = sum_s acc_s e^(m_s-M) / sum_s l_s e^(m_s-M).
 // The (m, l) pairs go through LDS and each thread's partial values are requested together,
 // so the merge costs about two memory round trips whatever the number of splits. Every thread of the
-// workgroup calls it (one barrier inside); thread d < D produces output element d.
+// workgroup calls it (one barrier inside); thread d < D produces numerator element d.
 template <int DT, int D>
-__device__ __forceinline__ void att_combine_row(const float* work, int n_split, int r, int Hq, int Lq, int d_real, const float* sinks,
-                                                void* out, float* stats, float* s_m, float* s_l) {
+__device__ __forceinline__ void att_merge_splits(const float* work, int n_split, int r, float* s_m, float* s_l, float& a, float& M,
+                                                 float& L) {
   const int d = threadIdx.x;
   const float* w = work + (int64_t)r * n_split * (D + 2);
   if (d < n_split) {
@@ -119,8 +119,9 @@ __device__ __forceinline__ void att_combine_row(const float* work, int n_split, 
     s_l[d] = w[(int64_t)d * (D + 2) + 1];
   }
   float part[ATT_MAX_SPLIT / 4];
-  float a = 0.f;
-  float M = -INFINITY, L = 0.f;
+  a = 0.f;
+  M = -INFINITY;
+  L = 0.f;
   for (int s0 = 0; s0 < n_split; s0 += ATT_MAX_SPLIT / 4) {
 #pragma unroll
     for (int u = 0; u < ATT_MAX_SPLIT / 4; ++u) {
@@ -139,6 +140,15 @@ __device__ __forceinline__ void att_combine_row(const float* work, int n_split, 
       if (sidx < n_split && s_m[sidx] != -INFINITY) a = fmaf(part[u], att_exp<DT>(s_m[sidx] - M), a);
     }
   }
+}
+
+// ... and writes the row
+template <int DT, int D>
+__device__ __forceinline__ void att_combine_row(const float* work, int n_split, int r, int Hq, int Lq, int d_real, const float* sinks,
+                                                void* out, float* stats, float* s_m, float* s_l) {
+  const int d = threadIdx.x;
+  float a, M, L;
+  att_merge_splits<DT, D>(work, n_split, r, s_m, s_l, a, M, L);
   const int qi = r % Lq;
   const int h = (r / Lq) % Hq;
   const int b = r / (Lq * Hq);

@@ -15,7 +15,7 @@
 // (2^-17 relative for bf16), so that nothing but the output is rounded to the storage type.
 // What bounds it: per wave and 32-key tile 24 matrix instructions (768 cycles) and about 150 vector ones with 17
 // exponentials (800 cycles), which do not overlap on a SIMD.
-// Keys are split over workgroups; the partial results (m, l, acc) are merged by the kernel of the split form.
+// Keys are split over workgroups; the partial results (m, l, acc) are merged by a second kernel.
 #include "sah_common.h"
 #include "sah_attn.h"
 
@@ -362,6 +362,39 @@ __global__ __launch_bounds__(QA_NT, 2) void k_members_attn_mfma(att_params P, qa
   }
 }
 
+// Merges a row's partial results. The products above meet every key of a stage, so a key that is not finite reaches rows
+// that do not hold it (-inf plus a NaN product in the logits, 0 times it in the second product); what reaches a row is not
+// finite either. Such a row, and one whose sums left the range of fp32, is done again entry by entry: its result is the
+// gather's, from the keys it holds alone.
+template <int DT, int D>
+__global__ __launch_bounds__(D) void k_members_merge(att_params P, int n_split) {
+  constexpr int NW = D / SAH_WAVE;
+  __shared__ float s_sm[ATT_MAX_SPLIT];
+  __shared__ float s_sl[ATT_MAX_SPLIT];
+  __shared__ float s_m[NW];
+  __shared__ float s_l[NW];
+  __shared__ float s_acc[NW][D];
+  const int r = blockIdx.x;
+  const int qi = r % P.Lq;
+  const int h = (r / P.Lq) % P.Hq;
+  const int b = r / (P.Lq * P.Hq);
+  float a, M, L;
+  att_merge_splits<DT, D>(P.work, n_split, r, s_sm, s_sl, a, M, L);
+  if (__syncthreads_or(!(fabsf(a) < INFINITY) || !(fabsf(L) < INFINITY))) {
+    int cnt = P.dense ? P.Lk : P.rows.cnt[r];
+    if (!P.dense && cnt > P.rows.cap) cnt = P.rows.cap;
+    const int* cols = P.dense ? nullptr : P.rows.cols + (int64_t)r * P.rows.cap;
+    att_wave_state st;
+    st.clear();
+    att_walk<DT, D>(P, r, b, h, h / (P.Hq / P.Hkv), qi, sah_wave_id() * SAH_WAVE, cnt, D, [&](int i) { return cols ? cols[i] : i; },
+                    [&](int) { return P.unit_inv_w; }, st);
+    att_park<D, NW>(st, sah_wave_id(), s_m, s_l, s_acc);
+    __syncthreads();
+    att_gather<DT, D, NW>(s_m, s_l, s_acc, a, M, L);
+  }
+  att_store_row<DT, D>(P, r, b, h, qi, a, M, L);
+}
+
 // ---------------------------------------------------------------------------
 // host
 // ---------------------------------------------------------------------------
@@ -418,8 +451,6 @@ static void qa_launch_rw(const att_params& P, const qa_params& Q, unsigned n_wg,
   }
 }
 
-int att_launch_combine(const sah_attention_args* a, int n_split);  // the merge kernel of the split form
-
 template <int DT, int D>
 static int qa_launch(const sah_attention_args* a, const att_params& P) {
   int rw;
@@ -434,7 +465,9 @@ static int qa_launch(const sah_attention_args* a, const att_params& P) {
     else qa_launch_rw<DT, D, 2>(P, Q, (unsigned)n_wg, (hipStream_t)a->stream);
     if (int rc = sah_launch_status("sah_members_attention")) return rc;
   }
-  return att_launch_combine(a, Q.n_split);
+  sah_timed timed("k_members_merge", a->stream);
+  hipLaunchKernelGGL((k_members_merge<DT, D>), dim3(a->rows.n_rows), dim3(D), 0, (hipStream_t)a->stream, P, Q.n_split);
+  return sah_launch_status("sah_members_attention(merge)");
 }
 
 extern "C" int sah_members_attention(const sah_attention_args* a) {

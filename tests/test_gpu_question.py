@@ -138,6 +138,42 @@ def test_attention_of_many_query_vectors(cuda, dtype, kind, shape, density):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("kind", [None, "causal"])
+@pytest.mark.parametrize("shape", [(1, 8, 2, 48, 2048, 128), (2, 8, 2, 66, 2100, 64), (2, 4, 4, 40, 1030, 128)])
+def test_keys_that_are_not_finite_stay_with_the_rows_that_hold_them(cuda, dtype, kind, shape):
+    """A few keys whose K or V row is not finite: rows without them have the result they have without such keys (two
+    summation orders: the last bit of the type, and 2^-12 of its largest value where a sum cancels), rows with them are not finite."""
+    import sparse_attention_hub_amd.sparse_attention as sa
+    from sparse_attention_hub_amd import _native as N
+    from sparse_attention_hub_amd.sparse_attention.utils.mask_attention_utils import get_masked_attention_output
+
+    B, Hq, Hkv, Lq, Lk, D = shape
+    q, k, v = make_qkv(B, Hq, Hkv, Lq, Lk, D, dtype, seed=13, device=cuda)
+    am = question_mask(B, Lq, Lk, dtype, cuda, kind)
+    member = torch.rand(B, Hq, Lq, Lk, generator=torch.Generator().manual_seed(4)) < 0.5
+    member[..., 0] = True
+    bad = {5: ("k", float("nan")), 70: ("k", float("inf")), 333: ("v", float("nan")), 900: ("v", float("-inf")), 1000: ("k", float("-inf"))}
+    member[:, :, : Lq // 2][..., list(bad)] = False
+    holds = member[..., list(bad)].any(-1).transpose(1, 2)
+    mask = sa.Mask.create_mask_from_dense_mask(member.shape, member.to(dtype).to(cuda), dtype)
+    clean = get_masked_attention_output(None, q, k, v, am, None, D ** -0.5, 0.0, mask).double().cpu()
+    for at, (which, value) in bad.items():
+        (k if which == "k" else v)[:, 0, at, 3] = value
+    N.timing_enable(True)
+    out = get_masked_attention_output(None, q, k, v, am, None, D ** -0.5, 0.0, mask).double().cpu()
+    assert "k_members_attn_mfma" in launched(N)
+    first = torch.arange(Hq) < Hq // Hkv  # the KV head with such keys
+    held = holds & first
+    unit = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)
+    near = (out - clean).abs() <= unit * clean.abs() + 2.0 ** -12 * float(clean.abs().max())
+    assert bool(near[~held].all())
+    bad_v = member[..., [333, 900]].any(-1).transpose(1, 2) & first
+    assert bool(bad_v.any()) and not bool(torch.isfinite(out[..., 3][bad_v]).any())
+    nan_k = member[..., 5].transpose(1, 2) & first
+    assert bool(nan_k.any()) and not bool(torch.isfinite(out[nan_k]).any())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("kind", [None, "causal"])
 @pytest.mark.parametrize("density", [None, 0.2])
 def test_statistics_of_many_query_vectors(cuda, dtype, kind, density):
     """The row's largest logit and the denominator relative to it, at a shape whose plain call takes the matrix-core form,
