@@ -11,10 +11,13 @@
 // wave owns 32 mask rows: S^T = K Q^T puts row j in lane j (16 of a tile's 32 keys in lane j, 16 in lane j + 32), so
 // maximum, weights and sums of a row need one exchange between two lanes, and the weights are where the second product,
 // O^T = V^T P^T, wants its B operand, with the key slots of a 16-key step taken in the order [0-3][8-11] / [4-7][12-15]:
-// the transposing LDS reads of V follow that order. The weights enter the second product as two 16-bit terms, p = hi + lo
-// (2^-17 relative for bf16), so that nothing but the output is rounded to the storage type.
-// What bounds it: per wave and 32-key tile 24 matrix instructions (768 cycles) and about 150 vector ones with 17
-// exponentials (800 cycles), which do not overlap on a SIMD.
+// the transposing LDS reads of V follow that order. The weights enter the second product as 16-bit terms that
+// together are the fp32 weight (qa_weights), so that nothing but the output is rounded to the storage type. Before that
+// rounding the result is off by 2.4e-7 (2-norm, 4096 keys, bf16; fp16 3.5e-7) where the gather's is by 1.6e-7 (1.8e-7): the
+// order of the fp32 sums. With two terms for bf16 2.3e-6.
+// What bounds it: per wave and 32-key tile 32 matrix instructions (fp16: 24; 1024 and 768 cycles) and about 190 vector ones
+// with 17 exponentials (150; 960 and 800 cycles), which do not overlap on a SIMD. The third term costs 4 of the 66 us with
+// the causal mask.
 // Keys are split over workgroups; the partial results (m, l, acc) are merged by a second kernel.
 #include "sah_common.h"
 #include "sah_attn.h"
@@ -55,10 +58,18 @@ __device__ __forceinline__ qa_u2 qa_read_tr(const uint16_t* lds) {
 #endif
 }
 
-// How far a row's maximum may rise, in powers of two, before the row is rescaled: the weights are then at most 2^8
+// How far a row's maximum may rise, in powers of two, before the row is rescaled: the weights are then at most 2^SLACK
 // relative to the maximum in use, which costs a floating-point sum nothing. A row's maximum rises in most of the few
-// tiles a workgroup sees; it rises by this much in one or two of them.
-#define QA_SLACK 8.0f
+// tiles a workgroup sees; it rises by 2^8 in one or two of them.
+// The weights enter the second product in 16-bit terms that together are the fp32 weight: three for bf16 (8 bits each),
+// two for fp16 (11 bits and a sign each), whose range is used to its upper end, the weights scaled by 2^SCALE: what its
+// smallest number, 2^-24, then cuts off is 2^-39 of the row's largest weight or less.
+template <int DT> struct qa_weights {
+  static constexpr int TERMS = DT == SAH_BF16 ? 3 : 2;
+  static constexpr float SLACK = DT == SAH_BF16 ? 8.0f : 1.0f;
+  static constexpr float SCALE = DT == SAH_BF16 ? 0.0f : 14.0f;     // SLACK + SCALE <= 15
+  static constexpr float UNSCALE = DT == SAH_BF16 ? 1.0f : 0x1p-14f;
+};
 
 // RW: waves along the rows (4: 128 rows a workgroup; 2: 64 rows, and the two 32-key tiles of a stage go to two waves)
 // AM: additive mask. DENSE: every key counts (no bitmap).
@@ -227,7 +238,7 @@ __global__ __launch_bounds__(QA_NT, 2) void k_members_attn_mfma(att_params P, qa
     mx = fmaxf(mx, __shfl_xor(mx, 32));
     if (!biased) mx *= P.scaling;
     // (-inf - -inf is NaN: no rise)
-    if (__ballot((mx - m_run) * LOG2E > QA_SLACK) != 0) {  // uniform: some row's maximum has risen too far
+    if (__ballot((mx - m_run) * LOG2E > qa_weights<DT>::SLACK) != 0) {  // uniform: some row's maximum has risen too far
       const float m_new = fmaxf(m_run, mx);
       const float up = m_run == -INFINITY ? 0.f : exp2f((m_run - m_new) * LOG2E);
       m_run = m_new;
@@ -241,11 +252,11 @@ __global__ __launch_bounds__(QA_NT, 2) void k_members_attn_mfma(att_params P, qa
     if (biased) {
       const float m_use = m_run == -INFINITY ? 0.f : m_run;
 #pragma unroll
-      for (int e = 0; e < 16; ++e) z[e] = __builtin_amdgcn_exp2f((s[e] - m_use) * LOG2E);
+      for (int e = 0; e < 16; ++e) z[e] = __builtin_amdgcn_exp2f(fmaf(s[e] - m_use, LOG2E, qa_weights<DT>::SCALE));
     } else {
       // a row whose every key so far is hidden has a maximum near the type's lowest value, and none here if it holds no
       // key of this tile: kept in range, so that -inf products come to 0
-      const float mc = fmaxf(m_run, -1e37f) * LOG2E;
+      const float mc = fmaxf(m_run, -1e37f) * LOG2E - qa_weights<DT>::SCALE;
       const float c_exp = P.scaling * LOG2E;
 #pragma unroll
       for (int e = 0; e < 16; ++e) z[e] = __builtin_amdgcn_exp2f(fmaf(s[e], c_exp, -mc));
@@ -261,27 +272,31 @@ __global__ __launch_bounds__(QA_NT, 2) void k_members_attn_mfma(att_params P, qa
         const qa_u2 a0 = qa_read_tr(vp), a1 = qa_read_tr(vp + 8 * D);
         va[t] = make_uint4(a0.x, a0.y, a1.x, a1.y);
       }
-      uint32_t hi[4], lo[4];
+      constexpr int TERMS = qa_weights<DT>::TERMS;
+      uint32_t term[TERMS][4];
 #pragma unroll
       for (int p = 0; p < 4; ++p) {
-        const float p0 = z[8 * st + 2 * p], p1 = z[8 * st + 2 * p + 1];
-        hi[p] = sah_pack2_hw<DT>(p0, p1);
-        sah_keep(hi[p]);  // taken apart as it is, instead of converted a second time
-        float h0, h1;
-        if (DT == SAH_BF16) {
-          h0 = sah_bits_to_float(hi[p] << 16);
-          h1 = sah_bits_to_float(hi[p] & 0xffff0000u);
-        } else {
-          h0 = sah_f16_to_float((uint16_t)hi[p]);
-          h1 = sah_f16_to_float((uint16_t)(hi[p] >> 16));
+        float p0 = z[8 * st + 2 * p], p1 = z[8 * st + 2 * p + 1];
+#pragma unroll
+        for (int i = 0; i < TERMS; ++i) {
+          term[i][p] = sah_pack2_hw<DT>(p0, p1);
+          if (i + 1 == TERMS) break;
+          sah_keep(term[i][p]);  // taken apart as it is, instead of converted a second time
+          if (DT == SAH_BF16) {
+            p0 -= sah_bits_to_float(term[i][p] << 16);
+            p1 -= sah_bits_to_float(term[i][p] & 0xffff0000u);
+          } else {
+            p0 -= sah_f16_to_float((uint16_t)term[i][p]);
+            p1 -= sah_f16_to_float((uint16_t)(term[i][p] >> 16));
+          }
         }
-        lo[p] = sah_pack2_hw<DT>(p0 - h0, p1 - h1);
       }
-      const uint4 ph = make_uint4(hi[0], hi[1], hi[2], hi[3]), pl = make_uint4(lo[0], lo[1], lo[2], lo[3]);
 #pragma unroll
-      for (int t = 0; t < DTL; ++t) acc[t] = sah_mfma_32x32x16<DT>(va[t], ph, acc[t]);
+      for (int i = 0; i < TERMS; ++i) {
+        const uint4 pt = make_uint4(term[i][0], term[i][1], term[i][2], term[i][3]);
 #pragma unroll
-      for (int t = 0; t < DTL; ++t) acc[t] = sah_mfma_32x32x16<DT>(va[t], pl, acc[t]);
+        for (int t = 0; t < DTL; ++t) acc[t] = sah_mfma_32x32x16<DT>(va[t], pt, acc[t]);
+      }
     }
   };
   auto stage = [&](int buf, int st) __attribute__((always_inline)) {  // buf: a constant in the loop below, LDS offsets are immediates
@@ -346,18 +361,19 @@ __global__ __launch_bounds__(QA_NT, 2) void k_members_attn_mfma(att_params P, qa
   }
   if (!live) return;
   // every entry of unit weight carries the factor unit_inv_w, in numerator and denominator
+  const float unit = P.unit_inv_w * qa_weights<DT>::UNSCALE;
   float* w = P.work + ((int64_t)r * Q.n_split + split) * (D + 2);
   if (g == 0) {
     w[0] = m_run;
-    w[1] = l_run * P.unit_inv_w;
+    w[1] = l_run * unit;
   }
 #pragma unroll
   for (int t = 0; t < DTL; ++t) {
 #pragma unroll
     for (int q4 = 0; q4 < 4; ++q4) {
       float2* o = (float2*)(w + 2 + 32 * t + 8 * q4 + 4 * g);
-      o[0] = make_float2(acc[t][4 * q4] * P.unit_inv_w, acc[t][4 * q4 + 1] * P.unit_inv_w);
-      o[1] = make_float2(acc[t][4 * q4 + 2] * P.unit_inv_w, acc[t][4 * q4 + 3] * P.unit_inv_w);
+      o[0] = make_float2(acc[t][4 * q4] * unit, acc[t][4 * q4 + 1] * unit);
+      o[1] = make_float2(acc[t][4 * q4 + 2] * unit, acc[t][4 * q4 + 3] * unit);
     }
   }
 }
@@ -427,7 +443,7 @@ extern "C" int64_t sah_members_attention_work_floats(int32_t B, int32_t Hq, int3
 // entries. At 32 heads x 48 queries x 32768 keys the two meet at 1.5 % (67 us); with 4 queries at 10 % (37 us).
 bool members_attention_pays(const sah_attention_args* a, const att_params& P) {
   if (a->dtype == SAH_F32 || (a->D != 64 && a->D != 128) || a->Lq < 2) return false;
-  // (a row's running maximum lags behind its largest logit, see QA_SLACK: statistics come from the gather)
+  // (a row's running maximum lags behind its largest logit, see SLACK: statistics come from the gather)
   if (P.drop.thresh || a->logits_out || a->stats_out || a->rows.w || P.dense == 2 || !(a->scaling > 0.f)) return false;
   if (a->ks_l * QA_STAGE >= (1 << 30) || a->vs_l * QA_STAGE >= (1 << 30)) return false;  // 32-bit offsets inside a stage
   const int64_t need = sah_members_attention_work_floats(a->B, a->Hq, a->Hkv, a->Lq, a->Lk, a->D);

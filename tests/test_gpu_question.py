@@ -173,6 +173,45 @@ def test_keys_that_are_not_finite_stay_with_the_rows_that_hold_them(cuda, dtype,
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_weights_keep_their_fp32_precision(cuda, dtype):
+    """Rows of two entries whose values nearly cancel: what is left shows the weights' error, 2^-20 of the values here
+    (exp2 of a logit up to 4 in size and a few fp32 operations), beside the output's own rounding. One in eight rows holds
+    the other keys: one of value 0 whose weight is 2^20 to 2^30 times the others', of value 1, whose sum is all that is left
+    (logits up to 21: 2^-19)."""
+    import sparse_attention_hub_amd.sparse_attention as sa
+    from sparse_attention_hub_amd import _native as N
+    from sparse_attention_hub_amd.sparse_attention.utils.mask_attention_utils import get_masked_attention_output
+
+    B, H, Lq, Lk, D = 1, 8, 64, 4096, 128
+    g = torch.Generator().manual_seed(8)
+    q, k, v = torch.zeros(B, H, Lq, D), torch.zeros(B, H, Lk, D), torch.ones(B, H, Lk, D)
+    q[..., 0] = torch.randint(-256, 257, (B, H, Lq), generator=g) / 64.0   # key 0: this logit; key 1: 0
+    k[:, :, 0, 0] = 1.0
+    v[:, :, :2] = 1 + torch.rand(B, H, 2, D, generator=g)
+    v[:, :, 1] *= -1
+    q[:, :, ::8] = 0.0
+    q[:, :, ::8, 1] = torch.arange(H).view(1, H, 1) + 14.0 - 0.25
+    k[:, :, 2, 1] = 1.0
+    v[:, :, 2] = 0.0
+    q, k, v = q.to(dtype), k.to(dtype), v.to(dtype)
+    member = torch.zeros(B, H, Lq, Lk, dtype=torch.bool)
+    member[..., :2] = True
+    member[:, :, ::8, :2] = False
+    member[:, :, ::8, 2:] = True
+    mask = sa.Mask.create_mask_from_dense_mask(member.shape, member.to(dtype).to(cuda), dtype)
+    N.timing_enable(True)
+    out = get_masked_attention_output(None, q.to(cuda), k.to(cuda), v.to(cuda), None, None, 1.0, 0.0, mask).double().cpu()
+    assert "k_members_attn_mfma" in launched(N)
+    z = (q.double() @ k.double().transpose(-1, -2)).masked_fill(~member, -float("inf"))
+    p = torch.softmax(z, -1)
+    ref, mass = (p @ v.double()).transpose(1, 2), (p @ v.double().abs()).transpose(1, 2)
+    half = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    exps = torch.where(torch.arange(Lq) % 8 == 0, 2.0 ** -19, 2.0 ** -20).view(1, Lq, 1, 1)
+    worst = (out - ref).abs() / (1.01 * half * ref.abs() + exps * mass + (2.0 ** -25 if dtype == torch.float16 else 0.0))
+    assert float(worst.max()) <= 1.0
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("kind", [None, "causal"])
 @pytest.mark.parametrize("density", [None, 0.2])
 def test_statistics_of_many_query_vectors(cuda, dtype, kind, density):
