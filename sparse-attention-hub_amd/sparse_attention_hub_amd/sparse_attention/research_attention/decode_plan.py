@@ -344,7 +344,7 @@ class DecodePlan:
         floats = N.work_floats(self.n_rows, cap, self.D)
         if Lq > 1:
             floats = max(floats, N.members_work_floats(self.B, self.Hq, self.Hkv, Lq, Lk, self.D))
-        work = _workspace(self.device, floats)
+        work = _workspace(self.device, floats, stream)
         at = self.att
         at.rows = rows
         at.q, at.qs_b, at.qs_h, at.qs_l = q.data_ptr(), q.stride(0), q.stride(1), q.stride(2)

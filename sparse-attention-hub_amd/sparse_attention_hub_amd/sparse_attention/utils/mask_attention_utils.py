@@ -10,6 +10,7 @@ reference, utils/mask.py:733-735).
 """
 from __future__ import annotations
 
+import threading
 from typing import Any, Dict, Optional, Tuple, Union
 
 
@@ -22,16 +23,30 @@ from .kv_utils import _get_num_key_value_groups
 from .mask import Mask
 from .native_rows import NativeRows
 
-_WORK: Dict[Tuple[str, int], torch.Tensor] = {}
+_WORK_STREAMS = 8  # scratch buffers a thread keeps
 
 
-def _workspace(device: torch.device, floats: int) -> torch.Tensor:
-    """Grow-only fp32 scratch per device; reused across calls on the same stream."""
-    key = (device.type, device.index if device.index is not None else -1)
-    buf = _WORK.get(key)
+class _Scratch(threading.local):
+    def __init__(self) -> None:
+        self.buffers: Dict[Tuple[Optional[int], int], torch.Tensor] = {}
+
+
+_WORK = _Scratch()
+
+
+def _workspace(device: torch.device, floats: int, stream: int) -> torch.Tensor:
+    """Grow-only fp32 scratch of the calling thread for the current stream of `device` (whose handle is `stream`): calls on
+    other streams are not ordered with this one's, and another thread's may come between the two kernels of a call. The
+    latest few streams' buffers are kept until the thread ends; one that goes was allocated on its stream, so torch's
+    allocator hands its memory to later work of that stream."""
+    key = (device.index, stream)
+    buffers = _WORK.buffers
+    buf = buffers.get(key)
     if buf is None or buf.numel() < floats:
-        buf = torch.empty(max(floats, 1 << 16), dtype=torch.float32, device=device)
-        _WORK[key] = buf
+        buffers.pop(key, None)
+        if len(buffers) >= _WORK_STREAMS:
+            del buffers[next(iter(buffers))]
+        buf = buffers[key] = torch.empty(max(floats, 1 << 16), dtype=torch.float32, device=device)
     return buf
 
 
@@ -154,7 +169,8 @@ def _run_attention(
     floats = N.work_floats(n_rows, max_cnt, D)
     if Lq > 1:  # many query vectors per KV head: the matrix-core form keeps partial results of its own
         floats = max(floats, N.members_work_floats(B, Hq, Hkv, Lq, Lk, D))
-    work = _workspace(dev, floats)
+    stream = N.stream_ptr(dev)
+    work = _workspace(dev, floats, stream)
     logits = stats = None
     if return_attention_weights:
         logits = torch.empty((n_rows, Lk if dense else rows.cap), dtype=torch.float32, device=dev)
@@ -176,7 +192,7 @@ def _run_attention(
         work.data_ptr(), work.numel(),
         None if logits is None else logits.data_ptr(),
         None if stats is None else stats.data_ptr(),
-        N.stream_ptr(dev),
+        stream,
         dropout[0], dropout[1], dropout[2], int(dropout_numerator_only),
     )
     sk, sr = score_keys if score_keys is not None else (None, None)

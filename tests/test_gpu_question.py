@@ -372,3 +372,34 @@ def test_masked_decode_plan_against_masker_by_masker(cuda, dtype, chain, kind, s
     assert bool(torch.isfinite(b).all())
     unit = {torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10, torch.float32: 2.0 ** -18}[dtype]
     assert bool(((a - b).abs() <= unit * b.abs() + (1e-6 if dtype == torch.float32 else 2.0 ** -18)).all())
+
+
+def test_scratch_belongs_to_one_stream_and_one_thread(cuda):
+    """Partial results of calls that nothing orders do not share memory; what a thread keeps is bounded."""
+    import threading
+
+    from sparse_attention_hub_amd import _native as N
+    from sparse_attention_hub_amd.sparse_attention.utils.mask_attention_utils import _workspace
+
+    def own():
+        return _workspace(cuda, 1000, N.stream_ptr(cuda))
+
+    mine = own()
+    assert own() is mine and _workspace(cuda, mine.numel() + 1, N.stream_ptr(cuda)).numel() > mine.numel()
+    mine = own()
+    other, held = torch.cuda.Stream(), {mine.data_ptr()}
+    with torch.cuda.stream(other):
+        there = own()
+        assert own() is there and there.data_ptr() not in held
+    assert own() is mine
+    got = []
+    t = threading.Thread(target=lambda: got.append(own()))
+    t.start()
+    t.join()
+    assert got[0].data_ptr() not in {mine.data_ptr(), there.data_ptr()}
+    streams = [torch.cuda.Stream() for _ in range(12)]  # as many handles at once
+    for st in streams:
+        with torch.cuda.stream(st):
+            own()
+    with torch.cuda.stream(other):
+        assert own() is not there  # given back
