@@ -8,6 +8,7 @@ dense (B, Hq, Lq, Lk) tensor unless the caller asks for the attention weights.
 """
 from __future__ import annotations
 
+import threading
 from dataclasses import dataclass
 from typing import Any, Dict, List, Optional, Tuple
 
@@ -99,10 +100,14 @@ class ResearchAttention(SparseAttention):
                 and not (dropout > 0.0 and module is not None and getattr(module, "training", False))):
             # decode fast path: the whole chain as one native call over cached argument blocks
             _native.require_device(queries, "queries")
-            key = (queries.device, queries.dtype, tuple(queries.shape), keys.shape[1])
+            masked = attention_mask is not None
+            key = (queries.device, queries.dtype, tuple(queries.shape), keys.shape[1], masked)
+            # A masked step's buffers belong to the stream and thread of their plan, as those of the masker-by-masker path
+            # belong to the call: a step on another stream is not ordered with the ones that use them.
+            owner = (_native.stream_ptr(queries.device), threading.get_ident()) if masked else None
             plan = self._plans.get(key)
-            if plan is None:
-                plan = self._plans[key] = DecodePlan(self.maskers, self._plan_kind, queries, keys)
+            if plan is None or plan.owner != owner:
+                plan = self._plans[key] = DecodePlan(self.maskers, self._plan_kind, queries, keys, owner)
             out = plan.run(queries, keys, values, scaling, sparse_meta_data, kwargs.get("layer_idx"), attention_mask)
             if out is not None:
                 return out, None

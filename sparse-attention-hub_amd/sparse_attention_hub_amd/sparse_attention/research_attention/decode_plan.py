@@ -65,8 +65,9 @@ class _LayerBlocks:
 
 
 class DecodePlan:
-    def __init__(self, maskers, kind: str, q: torch.Tensor, k: torch.Tensor):
+    def __init__(self, maskers, kind: str, q: torch.Tensor, k: torch.Tensor, owner: Optional[Tuple[int, int]] = None):
         self.kind = kind
+        self.owner = owner  # (stream, thread) the plan's buffers are for; None: the caller's own order
         self.sink_masker, self.local_masker = maskers[0], maskers[1]
         self.top = maskers[2] if len(maskers) == 3 else None
         self.device = q.device

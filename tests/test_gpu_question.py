@@ -403,3 +403,35 @@ def test_scratch_belongs_to_one_stream_and_one_thread(cuda):
             own()
     with torch.cuda.stream(other):
         assert own() is not there  # given back
+
+
+def test_a_masked_step_on_another_stream_has_buffers_of_its_own(cuda):
+    """Planned steps under a mask on two streams, nothing between them: neither waits for the other, so they share no row
+    buffers, keys or counters; results are those of steps one after the other."""
+    import sparse_attention_hub_amd.sparse_attention as sa
+
+    B, Hq, Hkv, Lk, D = 2, 8, 2, 900, 64
+    _, k, v = make_qkv(B, Hq, Hkv, 1, Lk, D, torch.bfloat16, seed=5, device=cuda)
+    qs = [make_qkv(B, Hq, Hkv, 1, 1, D, torch.bfloat16, seed=s, device=cuda)[0] for s in (1, 2)]
+    m = torch.zeros((B, 1, 1, Lk), dtype=torch.bfloat16, device=cuda)
+    m[0, ..., :100] = torch.finfo(torch.bfloat16).min
+    ra = sa.ResearchAttention.create_from_config(sa.ResearchAttentionConfig(masker_configs=[
+        sa.SinkMaskerConfig(sink_size=9), sa.LocalMaskerConfig(window_size=70), sa.OracleTopKConfig(heavy_size=50)]))
+    ra.return_attention_weights = False
+
+    def step(q):
+        return ra.custom_attention(None, q, k, v, m, D ** -0.5, 0.0, sparse_meta_data={}, layer_idx=0)[0]
+
+    want = [step(q) for q in qs]
+    torch.cuda.synchronize()
+    first = next(iter(ra._plans.values()))
+    side = torch.cuda.Stream()
+    a = step(qs[0])
+    with torch.cuda.stream(side):
+        b = step(qs[1])
+    second = next(iter(ra._plans.values()))
+    assert len(ra._plans) == 1 and second is not first
+    assert {t.data_ptr() for t in (first.cols, first.keybuf, first.tickets)}.isdisjoint(
+        {t.data_ptr() for t in (second.cols, second.keybuf, second.tickets)})
+    torch.cuda.synchronize()
+    assert torch.equal(a, want[0]) and torch.equal(b, want[1])
