@@ -469,11 +469,19 @@ __global__ __launch_bounds__(QM_NT, 2) void k_qk_scores_mfma(qk_params P, int ch
   }
 }
 
-// May this call run on the matrix cores, and does it pay? More query vectors per KV head than one pass of the streaming
-// kernel serves (4): from there on that kernel reads K twice, this one once.
+// May this call run on the matrix cores, and does it pay? It needs more query vectors per KV head than one pass of the
+// streaming kernel serves (from there on that kernel reads K twice, this one once) and key rows enough to fill the chip: a
+// workgroup here owns 256 keys for up to 64 vectors at a time, the streaming kernel deals the vectors out as well. The two
+// meet at about 20K key rows of 128 dims, at 96K while the streaming kernel gets by with two passes (up to 8 vectors): of 500
+// measured pairs (head_dim 64 and 128, 1 to 128 heads, 5 to 160 vectors each, 300 to 128K keys, with and without mask and
+// remainders) 3 are then more than 3 % slower here than there. 487 keys x 2 heads x 88 vectors, masked: 11.9 us here,
+// 4.9 there; 20008 keys x 128 heads x 44 vectors, masked: 194 and 1246.
 static bool qm_ok(const sah_qk_scores_args* a) {
-  return a->dtype != SAH_F32 && (a->D == 64 || a->D == 128) && (a->Hq / a->Hkv) * a->Lq > SC_NQ &&
-         a->key_pitch % 8 == 0 && ((uintptr_t)a->keys_out | (uintptr_t)a->resid_out) % 16 == 0;
+  const int64_t nvec = (int64_t)(a->Hq / a->Hkv) * a->Lq;
+  if (a->dtype == SAH_F32 || (a->D != 64 && a->D != 128) || nvec <= SC_NQ || a->key_pitch % 8 ||
+      ((uintptr_t)a->keys_out | (uintptr_t)a->resid_out) % 16)
+    return false;
+  return (int64_t)a->B * a->Hkv * a->Lk * a->D >= (nvec > 2 * SC_NQ ? 20480 : 98304) * 128;
 }
 
 template <int DT, int D>

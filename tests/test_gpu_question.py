@@ -43,9 +43,14 @@ def score_keys(N, q, k, amask, resid=False):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("kind", [None, "causal", "general"])
-@pytest.mark.parametrize("shape", [  # vectors per KV head on either side of 32 and 64, keys on either side of 64 and 256
-    (1, 14, 2, 1, 255, 128), (1, 8, 2, 8, 257, 128), (2, 4, 4, 33, 64, 64), (1, 8, 2, 17, 1000, 64), (1, 2, 1, 66, 129, 128)])
-def test_scores_of_many_query_vectors(cuda, dtype, kind, shape):
+@pytest.mark.parametrize("shape,form", [  # vectors per KV head on either side of 32 and 64, keys on either side of 64 and 256
+    ((1, 14, 2, 1, 255, 128), "k_qk_scores"), ((1, 8, 2, 8, 257, 128), "k_qk_scores"), ((2, 4, 4, 33, 64, 64), "k_qk_scores"),
+    ((1, 8, 2, 17, 1000, 64), "k_qk_scores"), ((1, 2, 1, 66, 129, 128), "k_qk_scores"),
+    # ... and batches that make them key rows enough for the matrix cores
+    ((40, 14, 2, 1, 1255, 128), "k_qk_scores_mfma"), ((25, 8, 2, 8, 511, 128), "k_qk_scores_mfma"),
+    ((26, 4, 4, 33, 513, 64), "k_qk_scores_mfma"), ((40, 8, 2, 17, 641, 64), "k_qk_scores_mfma"),
+    ((96, 2, 1, 66, 257, 128), "k_qk_scores_mfma")])
+def test_scores_of_many_query_vectors(cuda, dtype, kind, shape, form):
     """Keys are the scores rounded to the tensor type where torch rounds them: after the product, and again after the mask
     is added. Bound: half a unit of the type per rounding, plus fp32 accumulation of D products (D 2^-24 of sum |q k|)."""
     from sparse_attention_hub_amd import _native as N
@@ -54,7 +59,9 @@ def test_scores_of_many_query_vectors(cuda, dtype, kind, shape):
     q, k, _ = make_qkv(B, Hq, Hkv, Lq, Lk, D, dtype, seed=7, outliers=True, device=cuda)
     q = q.transpose(1, 2).contiguous().transpose(1, 2)  # the layout HuggingFace hands over
     am = question_mask(B, Lq, Lk, dtype, cuda, kind)
+    N.timing_enable(True)
     s, rem, keys = score_keys(N, q, k, am, resid=kind is None)
+    assert launched(N) == {form}
     kk = k.double().cpu().repeat_interleave(Hq // Hkv, dim=1)
     exact = (q.double().cpu() @ kk.transpose(-1, -2)).reshape(-1, Lk)
     mass = (q.double().cpu().abs() @ kk.abs().transpose(-1, -2)).reshape(-1, Lk)
