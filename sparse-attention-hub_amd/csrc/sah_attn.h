@@ -608,5 +608,7 @@ static inline bool att_use_row_form(int n_rows, int max_cnt) {
 
 // defined with the attention kernels: validation of a sah_sparse_attention call and its parameter block
 int att_prepare(const sah_attention_args* a, att_params& P);
-// ... and of the matrix-core form for many query vectors per KV head: is it the better one for this (prepared) call?
-bool members_attention_pays(const sah_attention_args* a, const att_params& P);
+// ... and of the matrix-core form for many query vectors per KV head: is it the better one for this (prepared) call, whose
+// other choice is the gather or (one_kernel) the kernel that selects and gathers; and the form itself
+bool members_attention_pays(const sah_attention_args* a, const att_params& P, bool one_kernel);
+int members_attention(const sah_attention_args* a, const att_params& P);

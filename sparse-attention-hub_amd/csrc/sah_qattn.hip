@@ -437,23 +437,42 @@ extern "C" int64_t sah_members_attention_work_floats(int32_t B, int32_t Hq, int3
   return (int64_t)B * Hq * Lq * Q.n_split * (D + 2);
 }
 
-// May the call run here, and does it pay? Both forms' times in microseconds, fitted to 200 measured pairs (head_dim 64 and
-// 128, 8 to 128 KV heads, 2 to 192 query vectors each, 2048 to 32768 keys, 1 to 10 % of them in a row; bf16; within 20 %
-// from 20 us on). This form: two launches, K and V once, rows (padded to 32) x keys. The gather: a launch, the rows, their
-// entries. At 32 heads x 48 queries x 32768 keys the two meet at 1.5 % (67 us); with 4 queries at 10 % (37 us).
-bool members_attention_pays(const sah_attention_args* a, const att_params& P) {
+// May the call run here, and does it pay? one_kernel: the other choice is not sah_sparse_attention's gather but the kernel
+// that selects the rows' columns and gathers them (sah_select_topk_attention). The two sides' times in microseconds, up to
+// what both have in common, fitted to 1800 measured pairs of layer-steps (head_dim 64 and 128, 1 to 128 KV heads, 2 to 270
+// query vectors each, 1024 to 65536 keys, 1 to 20 % of them in a row or all, with and without a mask; bf16 and fp16). This form:
+// its workgroups' stages one after the other (two workgroups a CU share its matrix units), the partial results merged.
+// The gather: a workgroup per row in the whole-row and one-kernel forms, so rounds of 256 rows; half the bytes where score
+// keys stand for K. Of 900 pairs of other shapes 12 are more than 4 % slower here than there where this says they pay (30 % at
+// most), and the sum of the times is within 1 % of the best choice. 128 vectors x 2 heads x 32768 keys of which 1175 count:
+// 48 us of a step there, 66 here; 48 queries x 32 heads x 32768 keys, 2278 of them, causal mask: 825 there, 245 here.
+bool members_attention_pays(const sah_attention_args* a, const att_params& P, bool one_kernel) {
   if (a->dtype == SAH_F32 || (a->D != 64 && a->D != 128) || a->Lq < 2) return false;
   // (a row's running maximum lags behind its largest logit, see SLACK: statistics come from the gather)
   if (P.drop.thresh || a->logits_out || a->stats_out || a->rows.w || P.dense == 2 || !(a->scaling > 0.f)) return false;
   if (a->ks_l * QA_STAGE >= (1 << 30) || a->vs_l * QA_STAGE >= (1 << 30)) return false;  // 32-bit offsets inside a stage
   const int64_t need = sah_members_attention_work_floats(a->B, a->Hq, a->Hkv, a->Lq, a->Lk, a->D);
   if (!a->work || a->work_floats < need) return false;
-  const int nvec = a->Hq / a->Hkv * a->Lq;
-  const double heads = (double)a->B * a->Hkv, D = a->D, Lk = a->Lk;
-  const double rows = heads * nvec, padded = heads * ((nvec + 31) / 32 * 32);
-  const double here = 16.0 + heads * Lk * D * 4.0 / 6.7e6 + padded * Lk * D * 4.7e-9;
-  const double gather = 8.0 + 0.014 * rows + rows * (a->dense ? Lk : (double)a->max_cnt) * D * 4.5e-7;
-  return here < gather;
+  int rw;
+  qa_params Q;
+  qa_plan(a->B, a->Hkv, a->Hq / a->Hkv * a->Lq, a->Lk, &rw, &Q);
+  const double d = a->D / 128.0, rows = a->rows.n_rows;
+  const double wgs = (double)a->B * a->Hkv * Q.row_tiles * Q.n_split;
+  double stage = (wgs <= 256 ? 1.3 * d : 2.8 * d) + 0.45 + (P.amask ? 0.6 : 0.0) + (a->dtype == SAH_BF16 ? 0.2 * d : 0.0);
+  if (rw == 2) stage *= 0.5;         // one tile of a stage per wave
+  if (wgs > 512) stage *= wgs / 512;
+  const double here = Q.stages_per_split * stage + 0.1 * Q.n_split + rows * (5e-4 + 4.2e-5 * d * Q.n_split);
+  const double cnt = 1e-3 * (a->dense ? a->Lk : a->max_cnt < a->rows.cap ? a->max_cnt : a->rows.cap), work = cnt * d;
+  const double rounds = ceil(rows / 256);
+  const bool keyed = P.score_keys != nullptr;
+  double there;
+  if (one_kernel)
+    there = keyed ? rounds * (1.7 + 3.0 * work + 1.3e-4 * a->Lk) - 1.6 : rounds * (2.2 + 3.9 * work + 6e-5 * a->Lk) - 0.3;
+  else if (P.n_split == 0)
+    there = keyed ? rounds * (1.2 + 2.0 * work) - 1.0 : rounds * (3.6 + 6.5 * work + (P.amask ? 2.0 * cnt : 0.0)) - 5.5;
+  else
+    there = keyed ? rows / 256 * 6.6 * work + rounds * 0.3 + 0.3 : rows / 256 * 7.1 * work + rounds * (P.amask ? 0.8 * cnt : 0.0) + 3.3;
+  return 1.03 * here + 1.0 < there;
 }
 
 template <int DT, int D, int RW>
@@ -486,11 +505,14 @@ static int qa_launch(const sah_attention_args* a, const att_params& P) {
   return sah_launch_status("sah_members_attention(merge)");
 }
 
+int members_attention(const sah_attention_args* a, const att_params& P) {
+  if (a->dtype == SAH_BF16) return a->D == 128 ? qa_launch<SAH_BF16, 128>(a, P) : qa_launch<SAH_BF16, 64>(a, P);
+  return a->D == 128 ? qa_launch<SAH_F16, 128>(a, P) : qa_launch<SAH_F16, 64>(a, P);
+}
+
 extern "C" int sah_members_attention(const sah_attention_args* a) {
   att_params P;
   const int rc = att_prepare(a, P);
   if (rc) return rc;
-  if (!members_attention_pays(a, P)) return sah_sparse_attention(a);
-  if (a->dtype == SAH_BF16) return a->D == 128 ? qa_launch<SAH_BF16, 128>(a, P) : qa_launch<SAH_BF16, 64>(a, P);
-  return a->D == 128 ? qa_launch<SAH_F16, 128>(a, P) : qa_launch<SAH_F16, 64>(a, P);
+  return members_attention_pays(a, P, false) ? members_attention(a, P) : sah_sparse_attention(a);
 }

@@ -91,9 +91,9 @@ def launched(N):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("kind", [None, "causal", "general"])
 @pytest.mark.parametrize("shape,density", [  # rows per KV head around 32, 64 and 128; keys around a 32-key tile and a 64-key
-    # stage; batches that make these small calls rows enough for the matrix-core form
+    # stage; batches that make these small calls rows enough for the matrix-core form (256 rows are one round of the gather)
     ((12, 8, 2, 8, 257, 128), 0.3), ((14, 14, 2, 5, 300, 64), 0.5), ((8, 4, 1, 40, 130, 128), 0.2), ((1, 8, 2, 33, 1000, 64), 0.3),
-    ((1, 8, 2, 32, 1025, 128), 0.1), ((160, 2, 2, 2, 31, 128), 1.0), ((64, 4, 2, 3, 96, 64), None)])
+    ((4, 8, 2, 32, 1025, 128), 0.1), ((160, 2, 2, 2, 31, 128), 1.0), ((64, 4, 2, 3, 96, 64), None)])
 def test_attention_of_many_query_vectors(cuda, dtype, kind, shape, density):
     """Against fp64. Bound per element: half a unit of the output type, the two-term weights (2^-16 of sum p |v|), and the
     logit's error (fp32 products and the mask's addition: D 2^-23 of the largest |q||k|) in the weights.
@@ -143,9 +143,42 @@ def test_attention_of_many_query_vectors(cuda, dtype, kind, shape, density):
     assert worst <= 1.0, worst
 
 
+@pytest.mark.parametrize("chain", ["oracle", "hash"])
+@pytest.mark.parametrize("shape,heavy,dense", [  # one round of rows, and a share of a round too many; rows and entries enough
+    ((1, 8, 2, 32, 8192, 128), 250, False), ((1, 8, 2, 48, 2048, 128), 60, False), ((2, 32, 8, 40, 4096, 128), 400, True)])
+def test_rows_go_dense_where_that_pays(cuda, chain, shape, heavy, dense):
+    """Planned steps of several queries: which form the attention takes, and that the result is the masker-by-masker path's
+    (another order of the sums: the last bit of bf16, and 2^-12 of the largest value where a sum cancels)."""
+    import sparse_attention_hub_amd.sparse_attention as sa
+    from sparse_attention_hub_amd import _native as N
+    from sparse_attention_hub_amd.sparse_attention.utils.hashattention_utils import random_hat_weights
+
+    B, Hq, Hkv, Lq, Lk, D = shape
+    q, k, v = make_qkv(B, Hq, Hkv, Lq, Lk, D, torch.bfloat16, seed=9, device=cuda)
+    top = sa.OracleTopKConfig(heavy_size=heavy) if chain == "oracle" else sa.HashAttentionTopKMaskerConfig(
+        heavy_size=heavy, hat_bits=32, hat_mlp_layers=3, hat_mlp_hidden_size=128, hat_mlp_activation="silu",
+        hat_weights=random_hat_weights(1, Hq, D, 32, 3, 128, dtype=torch.bfloat16, seed=1))
+    outs = []
+    for planned in (True, False):
+        ra = sa.ResearchAttention.create_from_config(sa.ResearchAttentionConfig(masker_configs=[
+            sa.SinkMaskerConfig(sink_size=16), sa.LocalMaskerConfig(window_size=64), top]))
+        ra.return_attention_weights = False
+        if not planned:
+            ra._plan_kind = None
+        meta = {}
+        for _ in range(2):  # the first call fills the layer's cache
+            N.timing_enable(True)
+            out = ra.custom_attention(None, q, k, v, None, D ** -0.5, 0.0, sparse_meta_data=meta, layer_idx=0)[0]
+            torch.cuda.synchronize()
+            names = launched(N)
+        assert ("k_members_attn_mfma" in names) == dense
+        outs.append(out.double().cpu())
+    assert bool(((outs[0] - outs[1]).abs() <= 2.0 ** -7 * outs[1].abs() + 2.0 ** -12 * float(outs[1].abs().max())).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("kind", [None, "causal"])
-@pytest.mark.parametrize("shape", [(1, 8, 2, 48, 2048, 128), (2, 8, 2, 66, 2100, 64), (2, 4, 4, 40, 1030, 128)])
+@pytest.mark.parametrize("shape", [(1, 8, 2, 48, 2048, 128), (2, 8, 2, 66, 2100, 64), (4, 4, 4, 40, 1030, 128)])
 def test_keys_that_are_not_finite_stay_with_the_rows_that_hold_them(cuda, dtype, kind, shape):
     """A few keys whose K or V row is not finite: rows without them have the result they have without such keys (two
     summation orders: the last bit of the type, and 2^-12 of its largest value where a sum cancels), rows with them are not finite."""
