@@ -666,7 +666,10 @@ int sah_amask_classify(const sah_amask_classify_args* a);
  * ResearchAttention.custom_attention (research_attention/base.py:108-148) on the
  * decode path; stops at the first stage that fails and returns its code.
  * hash_decode directly followed by attention runs as sah_hash_decode_attention,
- * select directly followed by attention as sah_select_topk_attention.
+ * select directly followed by attention as sah_select_topk_attention. Attention with several queries per row goes as
+ * sah_members_attention (sah_ext.h) where a stage of the chain has just written the rows' bitmaps (sink_local or
+ * hamming, nothing that may leave them stale after it) or it is dense; rows that come from elsewhere are read by their
+ * column lists alone, their bitmaps may be stale.
  * ------------------------------------------------------------------------- */
 typedef struct sah_chain_args {
   const sah_sink_local_args* sink_local;

@@ -347,7 +347,11 @@ extern "C" int sah_run_chain(const sah_chain_args* a) {
   if (a->pq_adc && (rc = sah_pq_adc_scores(a->pq_adc))) return rc;
   if (a->select && a->attention) return sah_select_topk_attention(a->select, a->attention, a->tickets);  // one kernel when shapes allow
   if (a->select && (rc = sah_select_topk(a->select))) return rc;
-  if (a->attention && a->attention->Lq > 1 && !a->hash_decode) return sah_members_attention(a->attention);  // bitmaps are complete
-  if (a->attention && (rc = sah_sparse_attention(a->attention))) return rc;
-  return SAH_OK;
+  if (!a->attention) return SAH_OK;
+  // The dense form for several queries reads the rows' bitmaps. They are complete where a builder of this chain has just
+  // written them; rows that the caller brings may come from a call that was asked to skip them.
+  const uint32_t* bm = a->attention->rows.bitmap;
+  const bool built = (a->hamming && a->hamming->rows.bitmap == bm) ||
+                     (a->sink_local && a->sink_local->rows.bitmap == bm && !a->hash_decode && !a->select);
+  return built || a->attention->dense ? sah_members_attention(a->attention) : sah_sparse_attention(a->attention);
 }

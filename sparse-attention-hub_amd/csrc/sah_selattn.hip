@@ -182,7 +182,8 @@ extern "C" int sah_select_topk_attention(const sah_select_topk_args* s, const sa
       // several workgroups per row read the row's count while one of them rewrites it: fresh rows only
       (parts > 1 ? (tickets && t->work && t->work_floats >= need && s->fresh) : worst <= 8192);
   // several queries per row: the rows' bitmaps, once complete, let the attention run dense on the matrix cores
-  const bool members = t->Lq > 1 && !s->skip_bitmap && members_attention_pays(t, A, one_kernel);
+  const bool members =
+      t->Lq > 1 && !s->skip_bitmap && t->rows.bitmap == s->rows.bitmap && members_attention_pays(t, A, one_kernel);
   if (!one_kernel || members) {
     if ((rc = sah_select_topk(s))) return rc;
     return members ? members_attention(t, A) : sah_sparse_attention(t);

@@ -176,6 +176,49 @@ def test_rows_go_dense_where_that_pays(cuda, chain, shape, heavy, dense):
     assert bool(((outs[0] - outs[1]).abs() <= 2.0 ** -7 * outs[1].abs() + 2.0 ** -12 * float(outs[1].abs().max())).all())
 
 
+def test_a_chain_reads_the_bitmaps_it_has_built_and_no_others(cuda):
+    """Rows that the caller brings need no bitmap (their builder may have been asked to skip it); rows that a builder of the
+    chain writes have one. A shape that goes dense where it may."""
+    import ctypes as C
+
+    import sparse_attention_hub_amd.sparse_attention as sa
+    from sparse_attention_hub_amd import _native as N
+
+    B, Hq, Hkv, Lq, Lk, D = 1, 8, 2, 48, 2048, 128
+    q, k, v = make_qkv(B, Hq, Hkv, Lq, Lk, D, torch.bfloat16, seed=3, device=cuda)
+    member = torch.rand(B, Hq, Lq, Lk, generator=torch.Generator().manual_seed(1)) < 0.6
+    member[0, 0, 0] = True  # rows have room for every key
+    rows = sa.Mask.create_mask_from_dense_mask(member.shape, member.to(q.dtype).to(cuda), q.dtype).to_rows(0)
+    work = torch.empty(N.members_work_floats(B, Hq, Hkv, Lq, Lk, D), device=cuda)
+
+    def attend(call, **fields):
+        out = torch.empty(B, Lq, Hq, D, dtype=q.dtype, device=cuda)
+        a = N.AttentionArgs()
+        a.rows, a.q, a.k, a.v, a.out = rows.as_struct(), q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr()
+        (a.qs_b, a.qs_h, a.qs_l), (a.ks_b, a.ks_h, a.ks_l), (a.vs_b, a.vs_h, a.vs_l) = q.stride()[:3], k.stride()[:3], v.stride()[:3]
+        a.dtype, a.B, a.Hq, a.Hkv, a.Lq, a.Lk, a.D = N.dtype_code(q.dtype), B, Hq, Hkv, Lq, Lk, D
+        a.scaling, a.unit_inv_w, a.max_cnt, a.work, a.work_floats = D ** -0.5, 1.0, rows.cap, work.data_ptr(), work.numel()
+        a.stream = N.stream_ptr(cuda)
+        chain = N.ChainArgs()
+        chain.attention = C.addressof(a)
+        for name, block in fields.items():
+            setattr(chain, name, C.addressof(block))
+        N.timing_enable(True)
+        N.call(call, chain if call == "sah_run_chain" else a)
+        torch.cuda.synchronize()
+        return out, "k_members_attn_mfma" in launched(N)
+
+    want, _ = attend("sah_sparse_attention")
+    assert attend("sah_members_attention")[1]
+    stale = rows.bitmap.clone()
+    rows.bitmap.zero_()
+    got, went_dense = attend("sah_run_chain")
+    assert torch.equal(got, want) and not went_dense
+    rows.bitmap.copy_(stale)
+    sl = N.SinkLocalArgs(rows.as_struct(), Lq, 1024, 600, 1, 1, N.stream_ptr(cuda))
+    assert attend("sah_run_chain", sink_local=sl)[1]
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("kind", [None, "causal"])
 @pytest.mark.parametrize("shape", [(1, 8, 2, 48, 2048, 128), (2, 8, 2, 66, 2100, 64), (4, 4, 4, 40, 1030, 128)])
