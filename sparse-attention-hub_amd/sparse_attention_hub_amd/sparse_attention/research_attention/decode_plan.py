@@ -24,7 +24,7 @@ from typing import Any, Dict, Optional, Tuple
 import torch
 
 from ... import _native as N
-from ..utils.mask_attention_utils import _workspace, additive_mask_args, unit_inverse_weight
+from ..utils.mask_attention_utils import _workspace, additive_mask_args, dense_rows_possible, unit_inverse_weight
 from .maskers.fixed.base import sortable_key_of
 from .maskers.fixed.implementations.basic_fixed import LocalMasker, SinkMasker
 from .maskers.fixed.implementations.hashattention_top_k import HashAttentionTopKMasker, PackedSignatureCache
@@ -76,6 +76,7 @@ class DecodePlan:
         self.B, self.Hq, self.Lq, self.D = q.shape
         self.Hkv = k.shape[1]
         self.n_rows = self.B * self.Hq * self.Lq
+        self.by_bitmap = dense_rows_possible(self.Lq, q.dtype, self.D)  # the attention may read the rows' bitmaps
         self.es = q.element_size()
         self.key_bits = 32 if q.dtype == torch.float32 else 16
         self.cap = 0
@@ -275,8 +276,8 @@ class DecodePlan:
             se = self.select
             se.rows, se.keys, se.key_pitch, se.key_bits = rows, self.keybuf.data_ptr(), self.keybuf_pitch, self.key_bits
             se.n_cand, se.col_offset, se.k, se.excluded_key, se.stream = Lk, 0, k_eff, self._excluded_min, stream
-            # only the attention reads these rows: one query per row by the column lists, several by the bitmaps
-            se.skip_bitmap = 1 if Lq == 1 else 0
+            # only the attention reads these rows: by the column lists, or by the bitmaps where they may go dense
+            se.skip_bitmap = 0 if self.by_bitmap else 1
             chain.select = C.addressof(se)
             if Lq == 1:
                 # one query per row: the selection kernel writes the sink + local rows itself
@@ -331,8 +332,8 @@ class DecodePlan:
             se = self.select
             se.rows, se.keys, se.key_pitch, se.key_bits = rows, self.keybuf.data_ptr(), self.keybuf_pitch, self.key_bits
             se.n_cand, se.col_offset, se.k, se.excluded_key, se.stream = current, off, k_eff, self._excluded_min, stream
-            # only the attention reads these rows: one query per row by the column lists, several by the bitmaps
-            se.skip_bitmap = 1 if Lq == 1 else 0
+            # only the attention reads these rows: by the column lists, or by the bitmaps where they may go dense
+            se.skip_bitmap = 0 if self.by_bitmap else 1
             chain.select = C.addressof(se)
             if Lq == 1:
                 # one query per row: the selection kernel writes the sink + local rows itself
@@ -343,7 +344,7 @@ class DecodePlan:
 
         out = torch.empty((self.B, Lq, self.Hq, self.D), dtype=self.dtype, device=self.device)
         floats = N.work_floats(self.n_rows, cap, self.D)
-        if Lq > 1:
+        if self.by_bitmap:
             floats = max(floats, N.members_work_floats(self.B, self.Hq, self.Hkv, Lq, Lk, self.D))
         work = _workspace(self.device, floats, stream)
         at = self.att

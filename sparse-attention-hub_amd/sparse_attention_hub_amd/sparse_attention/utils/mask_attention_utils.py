@@ -50,6 +50,12 @@ def _workspace(device: torch.device, floats: int, stream: int) -> torch.Tensor:
     return buf
 
 
+def dense_rows_possible(n_queries: int, dtype: torch.dtype, head_dim: int) -> bool:
+    """May attention over unit-weight rows of this geometry take the matrix-core form (`sah_members_attention`), which needs
+    the rows' bitmaps and scratch of its own?"""
+    return n_queries > 1 and dtype != torch.float32 and head_dim in (64, 128)
+
+
 def _inner_contiguous(t: torch.Tensor) -> torch.Tensor:
     return t if t.stride(-1) == 1 else t.contiguous()
 
@@ -167,7 +173,9 @@ def _run_attention(
     if out is None:
         out = torch.empty((B, Lq, Hq, D), dtype=q.dtype, device=dev)
     floats = N.work_floats(n_rows, max_cnt, D)
-    if Lq > 1:  # many query vectors per KV head: the matrix-core form keeps partial results of its own
+    members = (dense_rows_possible(Lq, q.dtype, D) and not return_attention_weights and not return_stats
+               and dropout[0] == 0.0 and (dense or rows.w is None))
+    if members:  # many query vectors per KV head: the matrix-core form keeps partial results of its own
         floats = max(floats, N.members_work_floats(B, Hq, Hkv, Lq, Lk, D))
     stream = N.stream_ptr(dev)
     work = _workspace(dev, floats, stream)
@@ -201,7 +209,7 @@ def _run_attention(
             and sr.dtype == sk.dtype and sr.shape == sk.shape and sr.stride() == sk.stride()):
         args.score_keys, args.score_resid, args.score_pitch = sk.data_ptr(), sr.data_ptr(), sk.stride(0)
     # the rows' bitmap is coherent with their lists here (or the call is dense)
-    N.call("sah_members_attention" if Lq > 1 else "sah_sparse_attention", args)
+    N.call("sah_members_attention" if members else "sah_sparse_attention", args)
     if return_stats:
         return out, stats
     weights = None

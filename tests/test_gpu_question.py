@@ -457,6 +457,28 @@ def test_masked_decode_plan_against_masker_by_masker(cuda, dtype, chain, kind, s
     assert bool(((a - b).abs() <= unit * b.abs() + (1e-6 if dtype == torch.float32 else 2.0 ** -18)).all())
 
 
+@pytest.mark.parametrize("dtype,D,weights", [(torch.float32, 128, False), (torch.bfloat16, 32, False), (torch.bfloat16, 128, True)])
+def test_calls_that_cannot_go_dense_ask_for_no_scratch_or_bitmaps_for_it(cuda, monkeypatch, dtype, D, weights):
+    import sparse_attention_hub_amd.sparse_attention as sa
+    from sparse_attention_hub_amd import _native as N
+
+    asked = []
+    monkeypatch.setattr(N, "members_work_floats", lambda *a: asked.append(a) or 0)
+    q, k, v = make_qkv(1, 4, 2, 6, 700, D, dtype, seed=3, device=cuda)
+    for planned in (True, False):
+        ra = sa.ResearchAttention.create_from_config(sa.ResearchAttentionConfig(masker_configs=[
+            sa.SinkMaskerConfig(sink_size=9), sa.LocalMaskerConfig(window_size=70), sa.OracleTopKConfig(heavy_size=50)]))
+        ra.return_attention_weights = weights
+        if not planned:
+            ra._plan_kind = None
+        ra.custom_attention(None, q, k, v, None, D ** -0.5, 0.0, sparse_meta_data={}, layer_idx=0)
+        for plan in ra._plans.values():
+            assert plan.select.skip_bitmap == 1
+        assert bool(ra._plans) == (planned and not weights)
+    torch.cuda.synchronize()
+    assert not asked
+
+
 def test_scratch_belongs_to_one_stream_and_one_thread(cuda):
     """Partial results of calls that nothing orders do not share memory; what a thread keeps is bounded."""
     import threading
