@@ -510,6 +510,39 @@ def test_scratch_belongs_to_one_stream_and_one_thread(cuda):
         assert own() is not there  # given back
 
 
+def test_a_captured_call_keeps_its_scratch(cuda):
+    """Replays write to memory of their graph, also when the buffer of the capturing stream has gone to other tensors."""
+    import sparse_attention_hub_amd.sparse_attention as sa
+    from sparse_attention_hub_amd import _native as N
+    from sparse_attention_hub_amd.sparse_attention.utils import mask_attention_utils as U
+
+    B, Hq, Hkv, Lk, D = 1, 8, 2, 3000, 128
+    q, k, v = make_qkv(B, Hq, Hkv, 1, Lk, D, torch.bfloat16, seed=5, device=cuda)
+    floats = N.work_floats(B * Hq, Lk, D)
+    assert floats > 0
+    mask = sa.Mask.create_full_mask((B, Hq, 1, Lk), dtype=q.dtype, device=cuda)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        def step():
+            return U.get_masked_attention_output(None, q, k, v, None, None, D ** -0.5, 0.0, mask)
+
+        want = step()
+        kept = dict(U._WORK.buffers)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            out = step()
+        assert {key: t.data_ptr() for key, t in U._WORK.buffers.items()} == {key: t.data_ptr() for key, t in kept.items()}
+        n = max(t.numel() for t in kept.values())
+        U._WORK.buffers.clear()
+        kept.clear()
+        others = [torch.full((n,), 7.0, device=cuda) for _ in range(12)]
+        for _ in range(3):
+            out.zero_()
+            graph.replay()
+            side.synchronize()
+            assert torch.equal(out, want) and all(bool((t == 7.0).all()) for t in others)
+
+
 def test_a_masked_step_on_another_stream_has_buffers_of_its_own(cuda):
     """Planned steps under a mask on two streams, nothing between them: neither waits for the other, so they share no row
     buffers, keys or counters; results are those of steps one after the other."""
