@@ -103,11 +103,15 @@ class ResearchAttention(SparseAttention):
             masked = attention_mask is not None
             key = (queries.device, queries.dtype, tuple(queries.shape), keys.shape[1], masked)
             # A masked step's buffers belong to the stream and thread of their plan, as those of the masker-by-masker path
-            # belong to the call: a step on another stream is not ordered with the ones that use them.
+            # belong to the call: a step on another stream is not ordered with the ones that use them. A captured one's
+            # belong to its graph alone: what its plan clears is clear when the graph runs, not now.
             owner = (_native.stream_ptr(queries.device), threading.get_ident()) if masked else None
-            plan = self._plans.get(key)
-            if plan is None or plan.owner != owner:
-                plan = self._plans[key] = DecodePlan(self.maskers, self._plan_kind, queries, keys, owner)
+            if masked and torch.cuda.is_current_stream_capturing():
+                plan = DecodePlan(self.maskers, self._plan_kind, queries, keys)
+            else:
+                plan = self._plans.get(key)
+                if plan is None or plan.owner != owner:
+                    plan = self._plans[key] = DecodePlan(self.maskers, self._plan_kind, queries, keys, owner)
             out = plan.run(queries, keys, values, scaling, sparse_meta_data, kwargs.get("layer_idx"), attention_mask)
             if out is not None:
                 return out, None

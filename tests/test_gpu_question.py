@@ -573,3 +573,48 @@ def test_a_masked_step_on_another_stream_has_buffers_of_its_own(cuda):
         {t.data_ptr() for t in (second.cols, second.keybuf, second.tickets)})
     torch.cuda.synchronize()
     assert torch.equal(a, want[0]) and torch.equal(b, want[1])
+
+
+@pytest.mark.parametrize("chain", ["fixed", "hash", "oracle", "pq"])
+def test_captured_masked_steps_share_nothing(cuda, chain):
+    """Two graphs of a step under a mask, captured one after the other on one stream: each runs by itself, in any order,
+    with other work in between, and leaves no plan behind whose counters only a replay would clear."""
+    import sparse_attention_hub_amd.sparse_attention as sa
+    from sparse_attention_hub_amd.sparse_attention.utils.hashattention_utils import random_hat_weights
+
+    B, Hq, Hkv, Lk, D = 2, 8, 2, 900, 64
+    _, k, v = make_qkv(B, Hq, Hkv, 1, Lk, D, torch.bfloat16, seed=5, device=cuda)
+    q = make_qkv(B, Hq, Hkv, 1, 1, D, torch.bfloat16, seed=1, device=cuda)[0]
+    m = torch.zeros((B, 1, 1, Lk), dtype=torch.bfloat16, device=cuda)
+    m[0, ..., :100] = torch.finfo(torch.bfloat16).min
+    top = {"oracle": sa.OracleTopKConfig(heavy_size=50),
+           "pq": sa.PQCacheConfig(heavy_size=50, pq_group_factor=8, pq_bits=4, kmeans_iter=3, init_offset=9, metric="euclidean"),
+           "hash": sa.HashAttentionTopKMaskerConfig(
+               heavy_size=50, hat_bits=32, hat_mlp_layers=3, hat_mlp_hidden_size=128, hat_mlp_activation="silu",
+               hat_weights=random_hat_weights(1, Hq, D, 32, 3, 128, dtype=torch.bfloat16, seed=1))}
+    ra = sa.ResearchAttention.create_from_config(sa.ResearchAttentionConfig(
+        masker_configs=[sa.SinkMaskerConfig(sink_size=9), sa.LocalMaskerConfig(window_size=70)] + ([top[chain]] if chain in top else [])))
+    ra.return_attention_weights = False
+    meta = {}
+
+    def step():
+        return ra.custom_attention(None, q, k, v, m, D ** -0.5, 0.0, sparse_meta_data=meta, layer_idx=0)[0]
+
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        step()  # fills the layer's cache
+        want = step()
+        plans = dict(ra._plans)
+        pairs = []
+        for _ in range(2):
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=side):
+                out = step()
+            pairs.append((graph, out))
+        assert ra._plans == plans and plans
+        for graph, out in pairs[::-1] * 3:
+            out.zero_()
+            graph.replay()
+            side.synchronize()
+            assert torch.equal(out, want)
+            assert torch.equal(step(), want)
