@@ -80,6 +80,7 @@ class DecodePlan:
         self.es = q.element_size()
         self.key_bits = 32 if q.dtype == torch.float32 else 16
         self.cap = 0
+        self.work_cap, self.work_need = -1, 0
         self.words_alloc = 0
         self.cols = self.cnt = self.bitmap = None
         self.qcodes = None
@@ -157,7 +158,8 @@ class DecodePlan:
         if q.stride(3) != 1 or k.stride(3) != 1 or v.stride(3) != 1 or v.shape[2] != Lk:
             return None
         masked = attention_mask is not None
-        am_keep, am_ptr, am_b, am_h, am_l = additive_mask_args(attention_mask, q, Lk)
+        if masked:  # (a plan is for masked steps or for others: the blocks of the others keep their NULL masks)
+            am_keep, am_ptr, am_b, am_h, am_l = additive_mask_args(attention_mask, q, Lk)
         stream = N.stream_ptr(self.device)
         cap = sink + window + k_eff
         self._ensure_rows(cap, Lk)
@@ -268,7 +270,8 @@ class DecodePlan:
             qa = self.qk
             qa.q, qa.qs_b, qa.qs_h, qa.qs_l = q.data_ptr(), q.stride(0), q.stride(1), q.stride(2)
             qa.k, qa.ks_b, qa.ks_h, qa.ks_l = k.data_ptr(), k.stride(0), k.stride(1), k.stride(2)
-            qa.amask, qa.ms_b, qa.ms_h, qa.ms_l = am_ptr, am_b, am_h, am_l
+            if masked:
+                qa.amask, qa.ms_b, qa.ms_h, qa.ms_l = am_ptr, am_b, am_h, am_l
             qa.dtype, qa.B, qa.Hq, qa.Hkv, qa.Lq, qa.Lk, qa.D = self.dt, self.B, self.Hq, self.Hkv, Lq, Lk, self.D
             qa.keys_out, qa.key_pitch, qa.stream = self.keybuf.data_ptr(), self.keybuf_pitch, stream
             qa.resid_out = None if masked or self.residbuf is None else self.residbuf.data_ptr()
@@ -343,7 +346,10 @@ class DecodePlan:
                 se.fresh = 0
 
         out = torch.empty((self.B, Lq, self.Hq, self.D), dtype=self.dtype, device=self.device)
-        floats = N.work_floats(self.n_rows, cap, self.D)
+        if cap != self.work_cap:  # (a function of the geometry alone)
+            self.work_need = N.work_floats(self.n_rows, cap, self.D)
+            self.work_cap = cap
+        floats = self.work_need
         if self.by_bitmap:
             floats = max(floats, N.members_work_floats(self.B, self.Hq, self.Hkv, Lq, Lk, self.D))
         work = _workspace(self.device, floats, stream)
@@ -352,7 +358,8 @@ class DecodePlan:
         at.q, at.qs_b, at.qs_h, at.qs_l = q.data_ptr(), q.stride(0), q.stride(1), q.stride(2)
         at.k, at.ks_b, at.ks_h, at.ks_l = k.data_ptr(), k.stride(0), k.stride(1), k.stride(2)
         at.v, at.vs_b, at.vs_h, at.vs_l = v.data_ptr(), v.stride(0), v.stride(1), v.stride(2)
-        at.amask, at.ms_b, at.ms_h, at.ms_l = am_ptr, am_b, am_h, am_l
+        if masked:
+            at.amask, at.ms_b, at.ms_h, at.ms_l = am_ptr, am_b, am_h, am_l
         at.sinks = None
         at.dtype, at.B, at.Hq, at.Hkv, at.Lq, at.Lk, at.D = self.dt, self.B, self.Hq, self.Hkv, Lq, Lk, self.D
         at.scaling, at.unit_inv_w, at.dense, at.max_cnt = float(scaling), self.unit, 0, cap
