@@ -511,6 +511,7 @@ int members_attention(const sah_attention_args* a, const att_params& P) {
 }
 
 extern "C" int sah_members_attention(const sah_attention_args* a) {
+  if (!a) return sah_fail(SAH_ENULL, "sah_members_attention: args is NULL");
   att_params P;
   const int rc = att_prepare(a, P);
   if (rc) return rc;

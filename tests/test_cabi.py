@@ -11,7 +11,11 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 def _declared_functions():
-    text = open(os.path.join(ROOT, "include", "sah.h")).read()
+    return _functions_of("sah.h")
+
+
+def _functions_of(header):
+    text = open(os.path.join(ROOT, "include", header)).read()
     text = re.sub(r"/\*.*?\*/", "", text, flags=re.S)
     return sorted(set(re.findall(r"\b(?:int|int64_t|const char\*)\s+(sah_\w+)\s*\(", text)))
 
@@ -39,6 +43,35 @@ def test_every_declared_symbol_is_exported_and_bound():
     for name in declared:
         assert hasattr(handle, name), f"{name} declared in include/sah.h but not exported"
     assert sorted(N.EXPECTED_SYMBOLS) == declared
+
+
+def test_the_extension_header_is_exported_bound_and_checked():
+    """include/sah_ext.h: every function is exported and bound; NULL and bad argument blocks are refused by name, on the host."""
+    declared = _functions_of("sah_ext.h")
+    plain = {"sah_members_attention_work_floats"}
+    assert set(declared) == set(N.EXTENSION_SYMBOLS) | plain
+    lib = N.lib()
+    for fn in N.EXTENSION_SYMBOLS:
+        assert getattr(lib, fn)(None) == -2 and fn.encode() in lib.sah_last_error(), fn
+    assert N.members_work_floats(1, 8, 2, 0, 100, 128) == 0 and N.members_work_floats(1, 8, 3, 4, 100, 128) == 0
+    assert N.members_work_floats(1, 8, 2, 4, 100, 128) == 8 * 4 * 130
+    # 10 pointers and 7 numbers of 8 bytes, 11 of 4, padding
+    assert ctypes.sizeof(N.PqKmeansArgs) == 184
+    buf = ctypes.create_string_buffer(4096)  # stands for device memory: never dereferenced by the checks
+    ptr = ctypes.addressof(buf)
+
+    def kmeans(**changed):
+        a = N.PqKmeansArgs(ptr, 64, 64, 16, 1, 1, 1, 2, 8, 16, 0, 100, ptr, ptr, 100, 0, ptr, ptr, ptr, ptr, ptr, ptr, 1, 2, 0.0, 3, 0, None)
+        for name, value in changed.items():
+            setattr(a, name, value)
+        rc = lib.sah_pq_kmeans(ctypes.byref(a))
+        assert b"sah_pq_kmeans" in lib.sah_last_error()
+        return rc
+
+    assert kmeans(n_sub=0) == -1 and kmeans(n_keys=0) == -1 and kmeans(key_offset=-1) == -1 and kmeans(max_iter=-1) == -1
+    assert kmeans(centres=None) == -2 and kmeans(start_idx=None) == -2 and kmeans(absmax_bits=None) == -2
+    assert kmeans(code_pitch=99) == -4 and kmeans(code_offset=-1) == -4
+    assert kmeans(n_keys=15) == -1 and b"fewer keys" in lib.sah_last_error()
 
 
 def test_argument_errors_are_reported_without_a_gpu():
