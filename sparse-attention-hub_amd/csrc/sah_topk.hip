@@ -430,6 +430,9 @@ __global__ __launch_bounds__(256) void k_hamming_scores(const uint2* kcodes, int
 // One thread per score read the codes and wrote two bytes per query: 33 queries x 32 heads x 32801 keys, bf16 with the
 // causal mask: 123 us, against 29 us here. Bound: the keys written (69 MB, 14 us at copy rate) and ten vector
 // instructions a score (10 us). The queries are dealt to several workgroups until there are HS_MIN_WGS of them.
+// Few scores stay with one thread each, eight times the threads: below 200K scores (3.2 us both; 70K with a mask: 2.9 there,
+// 3.3 here; 550K: 4.4 and 3.8).
+#define HS_MIN_SCORES 200000
 #define HS_NT 256
 #define HS_TILE (HS_NT * 8)  // keys per workgroup
 #define HS_MIN_WGS 2048
@@ -526,8 +529,8 @@ extern "C" int sah_hamming_scores(const sah_hamming_scores_args* a) {
   const int n_rows = a->B * a->Hq * a->Lq;
   if (n_rows > 65535) return sah_fail(SAH_ESHAPE, "sah_hamming_scores: more than 65535 rows");
   // 16-byte loads of two codes and stores of eight keys: rows of codes and of keys that start 16-byte aligned
-  if ((a->dtype == SAH_BF16 || a->dtype == SAH_F16) && a->code_pitch % 2 == 0 && (uintptr_t)a->kcodes % 16 == 0 &&
-      a->key_pitch % 8 == 0 && (uintptr_t)a->keys_out % 16 == 0)
+  if ((a->dtype == SAH_BF16 || a->dtype == SAH_F16) && (int64_t)n_rows * a->n_keys >= HS_MIN_SCORES &&
+      a->code_pitch % 2 == 0 && (uintptr_t)a->kcodes % 16 == 0 && a->key_pitch % 8 == 0 && (uintptr_t)a->keys_out % 16 == 0)
     return a->dtype == SAH_BF16 ? hs16_launch<SAH_BF16>(a) : hs16_launch<SAH_F16>(a);
   dim3 g((a->n_keys + 255) / 256, n_rows), blk(256);
   hipStream_t st = (hipStream_t)a->stream;

@@ -338,10 +338,12 @@ def test_statistics_of_many_query_vectors(cuda, dtype, kind, density):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("kind", [None, "causal", "general"])
-@pytest.mark.parametrize("shape,pitch", [  # keys on either side of a lane's 8 and a workgroup's 2048; an odd code pitch: the
-    # form of one thread per score
-    ((1, 2, 3, 5), 16), ((2, 3, 4, 2049), 2050), ((1, 4, 33, 2055), 2064), ((1, 2, 1, 4096), 4096), ((1, 2, 5, 40), 41)])
-def test_signature_scores_of_many_queries(cuda, dtype, kind, shape, pitch):
+@pytest.mark.parametrize("shape,pitch,form", [  # keys on either side of a lane's 8 and a workgroup's 2048; an odd code pitch
+    # and few scores: the form of one thread per score
+    ((1, 2, 3, 5), 16, "k_hamming_scores"), ((2, 3, 4, 2049), 2050, "k_hamming_scores"), ((1, 4, 33, 2055), 2064, "k_hamming_scores16"),
+    ((1, 2, 1, 4096), 4096, "k_hamming_scores"), ((1, 2, 5, 40), 41, "k_hamming_scores"), ((64, 16, 33, 7), 16, "k_hamming_scores16"),
+    ((9, 3, 4, 2049), 2050, "k_hamming_scores16"), ((25, 2, 1, 4096), 4096, "k_hamming_scores16"), ((9, 3, 4, 2049), 2051, "k_hamming_scores")])
+def test_signature_scores_of_many_queries(cuda, dtype, kind, shape, pitch, form):
     """Whole numbers plus the mask, rounded once to the tensor type: exactly torch's values."""
     from sparse_attention_hub_amd import _native as N
 
@@ -370,7 +372,7 @@ def test_signature_scores_of_many_queries(cuda, dtype, kind, shape, pitch):
                                                      None if am is None else am.data_ptr(), *ms, N.dtype_code(dtype),
                                                      keys.data_ptr(), kp, N.stream_ptr(cuda)))
     torch.cuda.synchronize()
-    assert ("k_hamming_scores16" if pitch % 2 == 0 else "k_hamming_scores") in launched(N)
+    assert launched(N) == {form}
     u = keys.cpu().to(torch.int32) & 0xFFFF
     assert bool((u[:, Lk:] == 0).all())  # nothing is written beyond the row's keys
     bits = torch.where((u & 0x8000) != 0, u & 0x7FFF, (~u) & 0xFFFF).to(torch.int16)
