@@ -263,8 +263,9 @@ typedef struct sah_select_topk_args {
   int32_t fresh_window;   /* writes - in the same launch when the keys are 16-bit and 16-byte aligned      */
   void* stream;
   int32_t skip_bitmap;    /* != 0: rows.bitmap need not be brought up to date (a caller that hands the rows */
-                          /* to the attention only, which reads the column lists); honoured where it saves  */
-                          /* work: by sah_select_topk_attention's one-kernel form                           */
+                          /* to the attention only and has it read the column lists); honoured where it     */
+                          /* saves work: by sah_select_topk_attention's one-kernel form. With 0 that call   */
+                          /* may give rows of several queries to sah_members_attention (sah_ext.h)          */
 } sah_select_topk_args;
 int sah_select_topk(const sah_select_topk_args* a);
 
@@ -347,7 +348,7 @@ typedef struct sah_pq_update_args {
   const int32_t* reseed_idx;
   float* shift2;       /* [n_groups] */
   float tol;
-  int32_t* state;      /* int32[4]: converged count, ticket, done flag, pending verdict */
+  int32_t* state;      /* int32[4]: converged count, ticket, done flag, unused */
   void* stream;
   const uint32_t* absmax_bits;        /* the value the assignment used */
 } sah_pq_update_args;
@@ -625,8 +626,8 @@ int sah_hash_decode_attention(const sah_hash_decode_args* a, const sah_attention
  * the attention's sums. Replaces the tail of a chain with a scoring pass of its own - `topk; scatter_` and
  * get_masked_attention_output (oracle_top_k.py:73-79, pq_top_k.py:513-537, utils/mask_attention_utils.py:406-491).
  * When the selection is the 16-bit form with at most 65536 candidates and the attention is the plain decode case
- * (no additive mask, unit weights, no logits output, no dropout, head_dim 64 or 128, 2-byte dtype, same rows and
- * stream) both run in ONE kernel: every row is given several workgroups when there are fewer rows than compute
+ * (unit weights, no logits output, no dropout, head_dim 64 or 128, 2-byte dtype, same rows and stream; an additive mask
+ * only with fresh rows and without score keys of the attention's own) both run in ONE kernel: every row is given several workgroups when there are fewer rows than compute
  * units; each finds the row's columns by itself, attends to its share of them, and the one that finishes last
  * merges the partial results, which meet in t->work (sah_sparse_attention_work_floats covers them).
  * tickets: rows.n_rows 32-bit words in which the workgroups of a row count their arrivals; zero before the first

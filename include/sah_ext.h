@@ -10,10 +10,12 @@ extern "C" {
 
 /* sah_sparse_attention for a caller whose rows.bitmap holds exactly the rows' entries (what every row builder and
  * selection of this library leaves unless asked to skip it): same arguments, same results. With several queries per row
- * (16-bit tensors, head_dim 64 / 128, unit weights, no dropout, no logits or statistics output, scaling > 0) and rows that hold more
- * than a small share of the keys the products run dense on the matrix cores and the bitmap decides which entries count;
- * the weights of the softmax then enter the second product as 16-bit terms that together are the fp32 weight. It needs a->work to hold
- * sah_members_attention_work_floats(...) floats; with less, or in any other case, the call is sah_sparse_attention. */
+ * (16-bit tensors, head_dim 64 / 128, unit weights, no dropout, no logits or statistics output, scaling > 0) and rows
+ * that hold more than a small share of the keys the products run dense on the matrix cores and the bitmap decides which
+ * entries count; the weights of the softmax then enter the second product as 16-bit terms that together are the fp32
+ * weight, and rows that a key of another row could have reached (K or V not finite) are done again entry by entry. It
+ * needs a->work to hold sah_members_attention_work_floats(...) floats; with less, or in any other case, the call is
+ * sah_sparse_attention. */
 int64_t sah_members_attention_work_floats(int32_t B, int32_t Hq, int32_t Hkv, int32_t Lq, int32_t Lk, int32_t D);
 int sah_members_attention(const sah_attention_args* a);
 

@@ -3,8 +3,8 @@
 // In a question pass every KV head has G x Lq mask rows, each with its own columns. Gathering them row by row
 // (k_sparse_attn) reads K and V once per entry: 1536 rows of 2278 entries, head_dim 128, are 1.8 GB through the caches,
 // 195 us. Together the rows of a head touch nearly every key, so here the whole of K and V passes once per 128 (or 64)
-// rows, the products run dense on the matrix cores and the rows' bitmaps decide which entries count: 60 us (70 with the
-// causal mask) and 10 for the merge. Work grows with rows x keys instead of rows x entries: see members_attention_pays().
+// rows, the products run dense on the matrix cores and the rows' bitmaps decide which entries count: 63 us (74 with the
+// causal mask) and 9 for the merge. Work grows with rows x keys instead of rows x entries: see members_attention_pays().
 //
 // A workgroup: 4 waves over stages of 64 keys, K and V staged in LDS by loads that write there themselves (two buffers,
 // the next stage under way while the current one is worked on; through registers, with V transposed on the way, 87 us). A
@@ -16,8 +16,8 @@
 // rounding the result is off by 2.4e-7 (2-norm, 4096 keys, bf16; fp16 3.5e-7) where the gather's is by 1.6e-7 (1.8e-7): the
 // order of the fp32 sums. With two terms for bf16 2.3e-6.
 // What bounds it: per wave and 32-key tile 32 matrix instructions (fp16: 24; 1024 and 768 cycles) and about 190 vector ones
-// with 17 exponentials (150; 960 and 800 cycles), which do not overlap on a SIMD. The third term costs 4 of the 66 us with
-// the causal mask.
+// with 17 exponentials (150; 960 and 800 cycles), which do not overlap on a SIMD. The third term costs 3 us of a pass of 244
+// with the causal mask.
 // Keys are split over workgroups; the partial results (m, l, acc) are merged by a second kernel.
 #include "sah_common.h"
 #include "sah_attn.h"

@@ -277,7 +277,8 @@ __global__ __launch_bounds__(SC_NT) void k_qk_scores(qk_params P) {
 // The kernel above streams K once per four query vectors: at 192 vectors (48 queries, 4 heads a group) K passes 48 times
 // and the vector unit does the dot products (1536 rows x 32768 keys, head_dim 128: 520 us). Here K passes once: a wave
 // keeps 64 keys as matrix operands in registers for the whole kernel, the query vectors come by in chunks of 64 through
-// LDS (two buffers, one barrier per chunk), S^T = K Q^T in 32x32x16 steps: 44 us, 49 with the causal mask. What bounds it
+// LDS (two buffers, one barrier per chunk), S^T = K Q^T in 32x32x16 steps: 44 us, 47 with the causal mask, 57 with the
+// remainders of the scores beside the keys. What bounds it
 // is memory: 67 MB of K in and 100 MB of keys out take 35 us at the rate of a large copy; chunks of 32 vectors and three
 // or four waves per SIMD change nothing. The accumulator has four consecutive keys of one vector in a lane; rounded to the storage type they cross the
 // wave's own LDS tile so that every store is 16 bytes and every row gets whole 128-byte lines.

@@ -428,7 +428,7 @@ __global__ __launch_bounds__(256) void k_hamming_scores(const uint2* kcodes, int
 // The same for 16-bit types, one head's queries together. A thread owns eight consecutive keys: their codes stay in
 // registers while the head's queries come by (uniform: scalar loads), and every row's scores leave as one 16-byte store.
 // One thread per score read the codes and wrote two bytes per query: 33 queries x 32 heads x 32801 keys, bf16 with the
-// causal mask: 123 us, against 29 us here. Bound: the keys written (69 MB, 14 us at copy rate) and ten vector
+// causal mask: 123 us, against 23 us here. Bound: the keys written (69 MB, 14 us at copy rate) and ten vector
 // instructions a score (10 us). The queries are dealt to several workgroups until there are HS_MIN_WGS of them.
 // Few scores stay with one thread each, eight times the threads: below 200K scores (3.2 us both; 70K with a mask: 2.9 there,
 // 3.3 here; 550K: 4.4 and 3.8).
