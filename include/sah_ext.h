@@ -25,7 +25,8 @@ int sah_members_attention(const sah_attention_args* a);
  * [0, n_keys), chosen by number g * n_cent + c of torch.rand(float64) with a CPU generator seeded with start_seed. In
  * iteration i an empty centre takes vector number (i * n_groups + g) * n_cent + c of torch.randint(0, n_keys) with a CPU
  * generator seeded with reseed_seed (below 2^28 keys; beyond, where torch draws 64 bits, still the 32-bit number modulo
- * n_keys). The seeds' low 32 bits count, as in torch. sums, counts, state and absmax_bits must
+ * n_keys). reseed_idx, optional scratch: all these numbers are drawn into it first, in one pass; without it a group with an
+ * empty centre draws the sequence up to its own numbers by itself, which is the cheaper way up to some millions of them. The seeds' low 32 bits count, as in torch. sums, counts, state and absmax_bits must
  * be zero before the call (sums and counts are zero again after it); the codes are the assignment to the centres that
  * entered the last iteration carried out. */
 typedef struct sah_pq_kmeans_args {
@@ -40,6 +41,7 @@ typedef struct sah_pq_kmeans_args {
   int32_t* state;                 /* [4] */
   uint32_t* absmax_bits;          /* [1] */
   int32_t* start_idx;             /* [n_groups, n_cent]; may be NULL with given_start */
+  int32_t* reseed_idx;            /* [max_iter, n_groups, n_cent] or NULL */
   uint64_t start_seed, reseed_seed;
   float tol;
   int32_t max_iter, given_start;

@@ -211,6 +211,7 @@ class PqKmeansArgs(C.Structure):
         ("state", C.c_void_p),
         ("absmax_bits", C.c_void_p),
         ("start_idx", C.c_void_p),
+        ("reseed_idx", C.c_void_p),
         ("start_seed", C.c_uint64), ("reseed_seed", C.c_uint64),
         ("tol", C.c_float),
         ("max_iter", C.c_int32), ("given_start", C.c_int32),

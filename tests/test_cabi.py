@@ -55,13 +55,13 @@ def test_the_extension_header_is_exported_bound_and_checked():
         assert getattr(lib, fn)(None) == -2 and fn.encode() in lib.sah_last_error(), fn
     assert N.members_work_floats(1, 8, 2, 0, 100, 128) == 0 and N.members_work_floats(1, 8, 3, 4, 100, 128) == 0
     assert N.members_work_floats(1, 8, 2, 4, 100, 128) == 8 * 4 * 130
-    # 10 pointers and 7 numbers of 8 bytes, 11 of 4, padding
-    assert ctypes.sizeof(N.PqKmeansArgs) == 184
+    # 11 pointers and 7 numbers of 8 bytes, 11 of 4, padding
+    assert ctypes.sizeof(N.PqKmeansArgs) == 192
     buf = ctypes.create_string_buffer(4096)  # stands for device memory: never dereferenced by the checks
     ptr = ctypes.addressof(buf)
 
     def kmeans(**changed):
-        a = N.PqKmeansArgs(ptr, 64, 64, 16, 1, 1, 1, 2, 8, 16, 0, 100, ptr, ptr, 100, 0, ptr, ptr, ptr, ptr, ptr, ptr, 1, 2, 0.0, 3, 0, None)
+        a = N.PqKmeansArgs(ptr, 64, 64, 16, 1, 1, 1, 2, 8, 16, 0, 100, ptr, ptr, 100, 0, ptr, ptr, ptr, ptr, ptr, ptr, None, 1, 2, 0.0, 3, 0, None)
         for name, value in changed.items():
             setattr(a, name, value)
         rc = lib.sah_pq_kmeans(ctypes.byref(a))

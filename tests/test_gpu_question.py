@@ -382,17 +382,22 @@ def test_signature_scores_of_many_queries(cuda, dtype, kind, shape, pitch, form)
     assert torch.equal(bits.view(dtype)[:, :Lk], ref.reshape(-1, Lk))
 
 
+@pytest.mark.parametrize("table", [False, True])  # reseeds drawn where a centre is empty, and ahead of the run
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("shape", [  # (batch, KV heads, keys, head_dim, sub-spaces, centres): a few draws, and more than a block of
     (1, 1, 40, 16, 2, 8), (2, 3, 300, 64, 8, 256), (1, 2, 1500, 32, 4, 128)])  # 624 words of the generator; vector and matrix forms
-def test_clustering_draws_its_start_and_its_reseeds_as_torch_does(cuda, dtype, shape):
+def test_clustering_draws_its_start_and_its_reseeds_as_torch_does(cuda, monkeypatch, dtype, shape, table):
     """Keys of three distinct, well separated vectors: most centres are empty in every iteration and are reseeded, a mean of
     equal vectors is that vector, and equal distances go to the lowest centre. Codes and centres are then exact."""
     from oracle import reference_path as O
+    from sparse_attention_hub_amd import _native as N
+    from sparse_attention_hub_amd.sparse_attention.research_attention.maskers.fixed.implementations.utils import pq_utils
     from sparse_attention_hub_amd.sparse_attention.research_attention.maskers.fixed.implementations.utils.pq_utils import (
         gather_sub_vectors, kmeans_keys_batched, seeded_initial_centres,
     )
 
+    if table:
+        monkeypatch.setattr(pq_utils, "_RESEED_TABLE_FROM", 0)
     B, Hkv, n, D, n_sub, n_cent = shape
     off, iters, seed = 3, 3, 7919 * 2
     g = torch.Generator().manual_seed(n)
@@ -400,7 +405,10 @@ def test_clustering_draws_its_start_and_its_reseeds_as_torch_does(cuda, dtype, s
     k = vecs[torch.randint(0, 3, (B, Hkv, n + off), generator=g)].to(dtype)
     groups = B * Hkv * n_sub
     codes = torch.zeros((B, Hkv, n, n_sub), dtype=torch.uint8, device=cuda)
+    N.timing_enable(True)
     centres, _ = kmeans_keys_batched(k.to(cuda), off, n_sub, n_cent, iters, codes, n, tol=-1.0, seed=seed)
+    torch.cuda.synchronize()
+    assert ("k_pq_reseed" in launched(N)) == table
     start = gather_sub_vectors(k, off, n_sub, seeded_initial_centres(groups, n, n_cent, seed, torch.device("cpu")))
     reseed = torch.randint(0, n, (iters, groups, n_cent), generator=torch.Generator().manual_seed(seed + 1), dtype=torch.int32)
     codes_o, cent_o = O.kmeans_lloyd(O.pq_split(k, off, n_sub), start, iters, reseed_idx=reseed, tol=-1.0)
