@@ -512,6 +512,8 @@ def test_scratch_belongs_to_one_stream_and_one_thread(cuda):
     t.start()
     t.join()
     assert got[0].data_ptr() not in {mine.data_ptr(), there.data_ptr()}
+    large = _workspace(cuda, (1 << 24) + 1, N.stream_ptr(cuda))
+    assert large.numel() > 1 << 24 and own() is mine
     streams = [torch.cuda.Stream() for _ in range(12)]  # as many handles at once
     for st in streams:
         with torch.cuda.stream(st):
