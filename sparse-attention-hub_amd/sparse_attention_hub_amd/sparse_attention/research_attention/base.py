@@ -107,11 +107,11 @@ class ResearchAttention(SparseAttention):
             # belong to its graph alone: what its plan clears is clear when the graph runs, not now.
             owner = (_native.stream_ptr(queries.device), threading.get_ident()) if masked else None
             if masked and torch.cuda.is_current_stream_capturing():
-                plan = DecodePlan(self.maskers, self._plan_kind, queries, keys)
+                plan = DecodePlan(self.maskers, self._plan_kind, queries, keys, True)
             else:
                 plan = self._plans.get(key)
                 if plan is None or plan.owner != owner:
-                    plan = self._plans[key] = DecodePlan(self.maskers, self._plan_kind, queries, keys, owner)
+                    plan = self._plans[key] = DecodePlan(self.maskers, self._plan_kind, queries, keys, masked, owner)
             out = plan.run(queries, keys, values, scaling, sparse_meta_data, kwargs.get("layer_idx"), attention_mask)
             if out is not None:
                 return out, None

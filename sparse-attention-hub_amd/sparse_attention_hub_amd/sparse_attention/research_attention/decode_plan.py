@@ -65,8 +65,10 @@ class _LayerBlocks:
 
 
 class DecodePlan:
-    def __init__(self, maskers, kind: str, q: torch.Tensor, k: torch.Tensor, owner: Optional[Tuple[int, int]] = None):
+    def __init__(self, maskers, kind: str, q: torch.Tensor, k: torch.Tensor, masked: bool = False,
+                 owner: Optional[Tuple[int, int]] = None):
         self.kind = kind
+        self.masked = masked  # for steps under an additive mask, or for steps without
         self.owner = owner  # (stream, thread) the plan's buffers are for; None: the caller's own order
         self.sink_masker, self.local_masker = maskers[0], maskers[1]
         self.top = maskers[2] if len(maskers) == 3 else None
@@ -130,16 +132,17 @@ class DecodePlan:
             kdt = torch.int32 if self.dtype == torch.float32 else torch.int16
             self.keybuf = torch.empty((self.n_rows, self.keybuf_pitch), dtype=kdt, device=self.device)
             # exact scores (OracleTopK) of 16-bit tensors: what their rounding took away goes beside the keys, and the
-            # attention takes its logits from the two instead of reading K again
+            # attention takes its logits from the two instead of reading K again (a masked score's rounding is another)
             self.residbuf = (torch.empty_like(self.keybuf)
-                             if self.kind == "oracle" and kdt == torch.int16 and self.D in (64, 128) else None)
+                             if self.kind == "oracle" and not self.masked and kdt == torch.int16 and self.D in (64, 128) else None)
 
     # --------------------------------------------------------------------- run
     def run(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scaling: float,
             sparse_meta_data: Dict[Any, Any], layer_idx: Optional[int],
             attention_mask: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
         """One layer-step; returns the attention output (B, Lq, Hq, D) or None if not applicable."""
-        if attention_mask is not None and (self.Lq != 1 or attention_mask.dim() != 4):
+        masked = self.masked
+        if masked and (self.Lq != 1 or attention_mask.dim() != 4):
             return None
         Lk = k.shape[2]
         Lq = self.Lq
@@ -157,8 +160,7 @@ class DecodePlan:
                 return None
         if q.stride(3) != 1 or k.stride(3) != 1 or v.stride(3) != 1 or v.shape[2] != Lk:
             return None
-        masked = attention_mask is not None
-        if masked:  # (a plan is for masked steps or for others: the blocks of the others keep their NULL masks)
+        if masked:  # (the blocks of other plans keep their NULL masks)
             am_keep, am_ptr, am_b, am_h, am_l = additive_mask_args(attention_mask, q, Lk)
         stream = N.stream_ptr(self.device)
         cap = sink + window + k_eff
@@ -274,7 +276,7 @@ class DecodePlan:
                 qa.amask, qa.ms_b, qa.ms_h, qa.ms_l = am_ptr, am_b, am_h, am_l
             qa.dtype, qa.B, qa.Hq, qa.Hkv, qa.Lq, qa.Lk, qa.D = self.dt, self.B, self.Hq, self.Hkv, Lq, Lk, self.D
             qa.keys_out, qa.key_pitch, qa.stream = self.keybuf.data_ptr(), self.keybuf_pitch, stream
-            qa.resid_out = None if masked or self.residbuf is None else self.residbuf.data_ptr()
+            qa.resid_out = None if self.residbuf is None else self.residbuf.data_ptr()
             chain.qk = C.addressof(qa)
             se = self.select
             se.rows, se.keys, se.key_pitch, se.key_bits = rows, self.keybuf.data_ptr(), self.keybuf_pitch, self.key_bits
@@ -368,7 +370,7 @@ class DecodePlan:
         at.closed_form = 0
         # an exact scoring pass came before: its 16-bit keys are the attention's logits, K is not read again
         at.score_keys, at.score_resid, at.score_pitch = None, None, 0
-        if self.kind == "oracle" and self.residbuf is not None and not masked:
+        if self.kind == "oracle" and self.residbuf is not None:
             at.score_keys, at.score_resid, at.score_pitch = self.keybuf.data_ptr(), self.residbuf.data_ptr(), self.keybuf_pitch
         if self.kind == "fixed" and Lq == 1 and not masked:
             # Sink + Local alone: the attention kernel takes the columns in closed form, no row is ever written

@@ -581,6 +581,7 @@ def test_a_masked_step_on_another_stream_has_buffers_of_its_own(cuda):
         b = step(qs[1])
     second = next(iter(ra._plans.values()))
     assert len(ra._plans) == 1 and second is not first
+    assert second.keybuf is not None and second.residbuf is None  # no remainders of masked scores
     assert {t.data_ptr() for t in (first.cols, first.keybuf, first.tickets)}.isdisjoint(
         {t.data_ptr() for t in (second.cols, second.keybuf, second.tickets)})
     torch.cuda.synchronize()
