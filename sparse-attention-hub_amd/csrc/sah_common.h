@@ -307,6 +307,16 @@ __device__ __forceinline__ uint32_t sah_pk_gt01_u16(uint32_t a, uint32_t b) {
   return ((a & 0xffffu) > (b & 0xffffu) ? 1u : 0u) | ((a >> 16) > (b >> 16) ? 0x10000u : 0u);
 #endif
 }
+// a - b per 16-bit half, modulo 2^16
+__device__ __forceinline__ uint32_t sah_pk_sub_u16(uint32_t a, uint32_t b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  uint32_t d;
+  asm("v_pk_sub_u16 %0, %1, %2" : "=v"(d) : "v"(a), "v"(b));
+  return d;
+#else
+  return ((a - b) & 0xffffu) | (((a >> 16) - (b >> 16)) << 16);
+#endif
+}
 // larger of the two unsigned 16-bit halves, per half
 __device__ __forceinline__ uint32_t sah_pk_max_u16(uint32_t a, uint32_t b) {
 #if defined(__HIP_DEVICE_COMPILE__)

@@ -8,7 +8,9 @@
 // low byte from a small histogram that only the keys of that bin touch. Longer rows, or a threshold
 // further down: two 256-bin histogram levels (high byte with one counter per lane and bin, then the
 // low byte of the keys inside the chosen bin). Either way the pass count is fixed: threshold, count,
-// write; rows of up to 131072 candidates stay in registers from the first pass on.
+// write. This form serves the kernels that attend to a row as soon as it is selected (up to 65536 candidates, kept in
+// registers from the first pass on), few short rows, and rows of more than 131072 candidates (read again in every pass); the
+// others take the form of sah_selq.h.
 // Winners above the threshold are written by every wave independently; only the wave that
 // holds the last accepted tie walks its candidates in column order, which keeps the
 // canonical rule "equal keys: lowest column first" at the cost of one ordered wave.
@@ -202,14 +204,12 @@ __device__ __forceinline__ int sf_select_impl(sf_lds& S, unsigned char* dyn, con
   constexpr bool REG = CPW > 0;
   constexpr int NREG = REG ? CPW : 1;
   static_assert(!FUSED || (REG && CPW <= 8), "the fused form keeps a row's keys and its emission masks in registers");
-  // The short way to the threshold (below) costs four packed compares per key word and pays up to 64 keys per
-  // thread; longer rows amortise the histograms' fixed cost better (512 x 131072: 134 us against 107)
-  constexpr bool SHORT = REG && CPW <= 8;
+  static_assert(CPW <= 8, "longer rows of keys in registers: sah_selq.h");
+  constexpr bool SHORT = REG;  // the short way to the threshold (below)
   const int tid = threadIdx.x;
   const int lane = tid & (SAH_WAVE - 1);
-  // rows of more than 64 keys per thread: a scalar wave index keeps the chunk bases of all passes out of the vector
-  // registers (they were spilled); shorter rows are 0.2 us faster with the plain one
-  const int wave = (CPW == 0 || CPW > 8) ? sah_wave_id() : tid / SAH_WAVE;
+  // (rows held in registers are 0.2 us faster with the plain wave index than with the scalar one)
+  const int wave = REG ? tid / SAH_WAVE : sah_wave_id();
   const int n_chunks = (n_cand + SF_CHUNK - 1) / SF_CHUNK;
   const int cpw = (n_chunks + SF_NW - 1) / SF_NW;  // <= CPW when REG (the host picks CPW)
   const int c0 = wave * cpw;
@@ -465,8 +465,7 @@ __device__ __forceinline__ int sf_select_impl(sf_lds& S, unsigned char* dyn, con
   // ---- pass 3: winners and ties per lane and wave --------------------------------------------
   // Rows held in registers keep the two masks of every chunk (16 bits, two chunks to a register) for the passes
   // below, which then do not compare a key again; not when active candidates may rank (their flags come from LDS).
-  // (up to 64 keys per thread: beyond that the registers are full)
-  constexpr bool KEEP = REG && CPW <= 8;
+  constexpr bool KEEP = REG;
   constexpr int NPM = KEEP ? (NREG + 1) / 2 : 1;
   const bool stored = KEEP && !slow;  // uniform across the workgroup
   uint32_t pm[NPM];
@@ -662,6 +661,7 @@ static inline size_t sf_hist_bytes() { return (size_t)2 * 256 * SF_COPIES * 4; }
 // argument checks of sah_select_topk (defined with it), for entry points that run the same selection
 int sel_validate(const sah_select_topk_args* a, const char* who);
 // may this call take the eight-keys-per-lane kernel? (16-bit keys, aligned rows, the LDS fits)
-static inline bool sel16_ok(const sah_select_topk_args* a) {
-  return a->key_bits == 16 && a->key_pitch % 8 == 0 && ((uintptr_t)a->keys % 16) == 0 && sf_lds_bytes(a->rows.n_words) <= 150 * 1024;
+static inline bool sel16_aligned(const sah_select_topk_args* a) {
+  return a->key_bits == 16 && a->key_pitch % 8 == 0 && ((uintptr_t)a->keys % 16) == 0;
 }
+static inline bool sel16_ok(const sah_select_topk_args* a) { return sel16_aligned(a) && sf_lds_bytes(a->rows.n_words) <= 150 * 1024; }

@@ -11,7 +11,7 @@
 // touched by no other wave and need no atomics.
 #include "sah_common.h"
 #include "sah_hsw.h"
-#include "sah_sel16.h"
+#include "sah_selq.h"
 
 #define SEL_NT 1024
 #define SEL_NW (SEL_NT / SAH_WAVE)
@@ -387,16 +387,37 @@ __global__ __launch_bounds__(HSW_NT) void k_hamming_topk_swar(sah_rows R, const 
   hsw_select_row(R, r, kcodes + (int64_t)(r / lq) * pitch, qcodes[r], k, cnt0, s_bm, s_key, S, buf);
 }
 
+// Registers for four, three or two workgroups of eight waves a CU (16 waves: one or two): a row alone on a CU leaves the
+// vector unit idle at every barrier and while its keys arrive. 1536 rows x 32768 candidates, k 1638, bf16 scores: 41 us, 25 of
+// them the issue of 1270 vector instructions a wave, the rest 100 MB of keys; one workgroup of 16 waves a CU with the passes
+// of sah_sel16.h takes 65 us (fp16 scores, whose threshold lies in no top bin: 39 and 122). 512 x 131072, k 2621: 57 and 93;
+// 1536 x 4096: 20 and 37; 1056 x 32801 signature scores: 46 and 68; rows of one key throughout: 133 and 157. Nine chunks a
+// wave for rows a little longer than 32768, five for those beyond 16384: 16 and 8 leave registers for fewer workgroups
+// (1056 x 32801: 59 us).
+#define SQ_WAVES_PER_SIMD(NW, CPW) ((CPW) <= 5 ? 8 : (CPW) <= 9 && (NW) == 8 ? 6 : 4)
+template <int NW, int CPW>
+__global__ __launch_bounds__(NW * SAH_WAVE, SQ_WAVES_PER_SIMD(NW, CPW)) void k_select16(
+    sah_rows R, const uint16_t* keys, int64_t pitch, int n_cand, int col_offset, int k, uint32_t excluded_key, int fresh, int sink,
+    int window) {
+  sah_touch_kernargs<sizeof(sah_rows) + 56>();
+  __shared__ sq_lds S;
+  HIP_DYNAMIC_SHARED(unsigned char, sq_dyn)
+  const int r = blockIdx.x;
+  sq_select_row<NW, CPW>(S, sq_dyn, R, r, keys + (int64_t)r * pitch, n_cand, col_offset, k < n_cand ? k : n_cand, excluded_key,
+                         fresh, sink, window);
+}
+
+// CPW = 4: few short rows, which the latency of one row's passes bounds (128 rows x 12011: 9.0 us here, 10.3 in the form above;
+// 32 x 32678: 11.6 and 11.2). CPW = 0: rows too long for the registers of a workgroup; their keys are read in every pass.
 template <int CPW>
-__global__ __launch_bounds__(SF_NT) void k_select16(sah_rows R, const uint16_t* keys, int64_t pitch, int n_cand,
-                                                    int col_offset, int k, uint32_t excluded_key, int fresh, int sink,
-                                                    int window) {
+__global__ __launch_bounds__(SF_NT) void k_select16_row(sah_rows R, const uint16_t* keys, int64_t pitch, int n_cand, int col_offset,
+                                                        int k, uint32_t excluded_key, int fresh, int sink, int window) {
   sah_touch_kernargs<sizeof(sah_rows) + 56>();
   __shared__ sf_lds S;
   HIP_DYNAMIC_SHARED(unsigned char, sf_dyn)
   const int r = blockIdx.x;
-  sf_select_row<CPW>(S, sf_dyn, R, r, keys + (int64_t)r * pitch, n_cand, col_offset, k < n_cand ? k : n_cand,
-                     excluded_key, fresh, sink, window);
+  sf_select_row<CPW>(S, sf_dyn, R, r, keys + (int64_t)r * pitch, n_cand, col_offset, k < n_cand ? k : n_cand, excluded_key, fresh,
+                     sink, window);
 }
 
 // kernels may use up to 160 KB of LDS; HIP needs to be told once per kernel
@@ -575,23 +596,37 @@ extern "C" int sah_select_topk(const sah_select_topk_args* a) {
   int rc = sel_validate(a, "sah_select_topk");
   if (rc) return rc;
   hipStream_t st = (hipStream_t)a->stream;
-  if (sel16_ok(a)) {
+  const int n_chunks = (a->n_cand + SF_CHUNK - 1) / SF_CHUNK;
+  if (sel16_aligned(a) && (n_chunks <= SQ_MAX_CHUNKS ? sq_lds_bytes(a->rows.n_words, 16, 16) <= 150 * 1024 : sel16_ok(a))) {
     // eight keys per lane: needs 16-byte aligned key rows
-    const size_t lds = sf_lds_bytes(a->rows.n_words);
-    const int cpw = sf_chunks_per_wave(a->n_cand);
     sah_timed timed("k_select_topk", a->stream);
-#define SAH_SEL16(CPW)                                                                                      \
+#define SAH_SEL16(KERNEL, NT, LDS)                                                                          \
   do {                                                                                                      \
-    rc = sel_allow_lds(k_select16<CPW>, lds, "sah_select_topk");                                            \
+    const size_t lds = LDS;                                                                                 \
+    rc = sel_allow_lds(KERNEL, lds, "sah_select_topk");                                                     \
     if (rc) return rc;                                                                                      \
-    hipLaunchKernelGGL(k_select16<CPW>, dim3(a->rows.n_rows), dim3(SF_NT), lds, st, a->rows,                \
-                       (const uint16_t*)a->keys, a->key_pitch, a->n_cand, a->col_offset, a->k, a->excluded_key, \
-                       a->fresh ? 1 : 0, a->fresh_sink, a->fresh_window);                                   \
+    hipLaunchKernelGGL(KERNEL, dim3(a->rows.n_rows), dim3(NT), lds, st, a->rows, (const uint16_t*)a->keys,  \
+                       a->key_pitch, a->n_cand, a->col_offset, a->k, a->excluded_key, a->fresh ? 1 : 0,     \
+                       a->fresh_sink, a->fresh_window);                                                     \
   } while (0)
-    if (cpw <= 4) SAH_SEL16(4);
-    else if (cpw <= 8) SAH_SEL16(8);
-    else if (cpw <= 16) SAH_SEL16(16);
-    else SAH_SEL16(0);
+#define SAH_SELQ(NW, CPW) SAH_SEL16((k_select16<NW, CPW>), NW * SAH_WAVE, sq_lds_bytes(a->rows.n_words, NW, CPW))
+    const bool few = a->rows.n_rows <= 256;  // at most one row a CU
+    if (n_chunks > SQ_MAX_CHUNKS) SAH_SEL16(k_select16_row<0>, SF_NT, sf_lds_bytes(a->rows.n_words));
+    else if (few && n_chunks <= 32 && sel16_ok(a)) SAH_SEL16(k_select16_row<4>, SF_NT, sf_lds_bytes(a->rows.n_words));
+    else if (few || n_chunks > 128) {
+      if (n_chunks <= 64) SAH_SELQ(16, 4);
+      else if (n_chunks <= 128) SAH_SELQ(16, 8);
+      else SAH_SELQ(16, 16);
+    } else {
+      if (n_chunks <= 8) SAH_SELQ(8, 1);
+      else if (n_chunks <= 16) SAH_SELQ(8, 2);
+      else if (n_chunks <= 32) SAH_SELQ(8, 4);
+      else if (n_chunks <= 40) SAH_SELQ(8, 5);
+      else if (n_chunks <= 64) SAH_SELQ(8, 8);
+      else if (n_chunks <= 72) SAH_SELQ(8, 9);
+      else SAH_SELQ(8, 16);
+    }
+#undef SAH_SELQ
 #undef SAH_SEL16
     return sah_launch_status("sah_select_topk");
   }
