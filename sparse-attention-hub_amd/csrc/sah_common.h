@@ -442,6 +442,27 @@ __device__ __forceinline__ float sah_wave_max(float v) {
   return v;
 }
 
+// the values the lanes l % 32 and l % 32 + 32 hold, to both of them: one instruction, no LDS
+__device__ __forceinline__ void sah_half_both(uint32_t v, uint32_t& lo, uint32_t& hi) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  lo = r[0];
+  hi = r[1];
+#else
+  lo = hi = v;
+#endif
+}
+__device__ __forceinline__ float sah_half_min(float v) {
+  uint32_t a, b;
+  sah_half_both(sah_float_to_bits(v), a, b);
+  return __builtin_elementwise_minimum(sah_bits_to_float(a), sah_bits_to_float(b));
+}
+__device__ __forceinline__ float sah_half_sum(float v) {
+  uint32_t a, b;
+  sah_half_both(sah_float_to_bits(v), a, b);
+  return sah_bits_to_float(a) + sah_bits_to_float(b);
+}
+
 template <int CTRL, int ROW_MASK, bool BOUND>
 __device__ __forceinline__ int sah_dpp_i(int v) {
   return __builtin_amdgcn_update_dpp(0, v, CTRL, ROW_MASK, 0xF, BOUND);

@@ -36,6 +36,12 @@ __device__ __forceinline__ float pq_sum_scale(uint32_t absmax_bits) {
 __device__ __forceinline__ void pq_sum_add(long long* p, float x, float scale) {
   atomicAdd((unsigned long long*)p, (unsigned long long)__float2ll_rn(x * scale));
 }
+// The same for keys that are all finite, in three instructions: x * scale is exact in fp64 and below 2^51, so adding
+// 1.5 * 2^52 rounds it to the nearest integer, ties to even, in the low bits of the sum.
+__device__ __forceinline__ void pq_sum_add_finite(long long* p, float x, double scale) {
+  const double m = 6755399441055744.0;
+  atomicAdd((unsigned long long*)p, __builtin_bit_cast(unsigned long long, fma((double)x, scale, m)) - __builtin_bit_cast(unsigned long long, m));
+}
 
 struct pq_assign_params {
   const void* k; int64_t ks_b, ks_h, ks_l;
@@ -293,14 +299,16 @@ __global__ __launch_bounds__(PQB_NT) void k_pq_assign_block(pq_assign_params P) 
 // SPLIT (bf16 keys): -2 c is cut into three bf16 terms of 8 bits each, which together ARE the fp32 number, and the
 // product runs on the bf16 instructions (32 cycles for 16 dimensions x 1 term; in fp32 64 cycles for 2 dimensions):
 // every x * term is exact in fp32, the accumulation is fp32 as before.
-// The split form's rounding is another one (and smaller), so where two centres come within both forms' rounding of each
-// other the key tile is evaluated a second time in fp32: the codes are those of the fp32 form, bit for bit, whichever
-// form the alignment and shape of the keys allow (without: 1e-6 of the codes of an iteration, 5e-4 after ten).
-// Measured (bf16, 8 heads x 16405 keys, 16 sub-vectors of 8, 256 centres, sums included): 204 -> 78 us, 64 of them without
-// the second evaluation (what bounds it: 28 vector and 2 matrix instructions a tile); keys moved by five times their spread,
-// where more centres are near: 94. fp16 (no split: terms of small centres would leave its range) 202 -> 121. 32768 keys,
-// 2 sub-vectors of 64, 64 centres: 218 -> 62. Sums in [centre][d] order and a flush of one centre a lane took 40 (8 dims)
-// to 100 us (64 dims) of these.
+// The split form's rounding is another one (and smaller), so where several centres come within both forms' rounding of the
+// smallest value they are evaluated in the fp32 form's order of operations: the codes are those of the fp32 form, bit for
+// bit, whichever form the alignment and shape of the keys allow (without: 1e-6 of the codes of an iteration, 5e-4 after ten).
+// Measured (bf16, 8 heads x 16277 keys, 16 sub-vectors of 8, 256 centres, sums included): 68 us; 85 with every tile's 16
+// values selected, not their minima over the tiles, the second look by matrix instruction, its test by ballots, the key
+// operand in a structure (which went through scratch memory) and the centres read element by element. What bounds it: issue,
+// 20 vector and 2 matrix instructions a tile (31 us) and 150 vector ones a key tile of eight (25), 10 before and after the
+// loop. fp16 (no split: terms of small centres would leave its range): 121 at 16405 keys. 32768 keys, 2 sub-vectors of 64, 64
+// centres: 218 -> 62 with the split. Sums in [centre][d] order and a flush of one centre a lane took 40 (8 dims) to 100 us
+// (64 dims) of these.
 // The expansion rounds differently from the difference form of the reference ((A - B)^2 summed,
 // pq_utils.py:220-257): a key whose two nearest centres tie to the last bits may take the other one.
 // ---------------------------------------------------------------------------
@@ -338,13 +346,37 @@ __device__ __forceinline__ uint32_t pqm_term(float c, int term) {
   return hi >> 16;
 }
 
+// bit v: a[v] <= b. Two instructions a value: a comparison into the carry, and the mask doubled with the carry in.
+__device__ __forceinline__ uint32_t pqm_mask_le(const sah_f32x16& a, float b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  uint32_t m = 0;
+#define PQM_LE4(x, y, z, w)                                                                                        \
+  asm("v_cmp_le_f32 vcc, %1, %5\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc\n\tv_cmp_le_f32 vcc, %2, %5\n\t"             \
+      "v_addc_co_u32 %0, vcc, %0, %0, vcc\n\tv_cmp_le_f32 vcc, %3, %5\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc\n\t"   \
+      "v_cmp_le_f32 vcc, %4, %5\n\tv_addc_co_u32 %0, vcc, %0, %0, vcc"                                             \
+      : "+&v"(m)                                                                                                   \
+      : "v"(a[x]), "v"(a[y]), "v"(a[z]), "v"(a[w]), "v"(b)                                                         \
+      : "vcc")
+  PQM_LE4(15, 14, 13, 12);
+  PQM_LE4(11, 10, 9, 8);
+  PQM_LE4(7, 6, 5, 4);
+  PQM_LE4(3, 2, 1, 0);
+#undef PQM_LE4
+  return m;
+#else
+  uint32_t m = 0;
+  for (int v = 0; v < 16; ++v) m |= a[v] <= b ? 1u << v : 0u;
+  return m;
+#endif
+}
+
 // (two waves per SIMD at least: with at most 256 registers a wave the compiler keeps the accumulators in ordinary
 // vector registers, which the minimum search reads directly)
 // KS k-steps of two dimensions each: sub-vectors of up to 2 KS dimensions (the operands beyond d_sub are zero), of
 // exactly 2 KS in the split form. SUMS: the per-centre sums of the update step are accumulated here (P.sums given and
 // the LDS holds them). A workgroup takes wg_tiles tiles of 32 keys of one group.
 template <int DT, int KS, bool SUMS, bool SPLIT>
-__global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P, int wg_tiles, int ranges, int n_heads) {
+__global__ __launch_bounds__(PQM_NT, SPLIT && KS <= 16 ? 4 : 2) void k_pq_assign_mfma(pq_assign_params P, int wg_tiles, int ranges, int n_heads) {
   HIP_DYNAMIC_SHARED(unsigned char, pqm_dyn)
   static_assert(!SPLIT || (DT == SAH_BF16 && KS >= 4), "the split form multiplies bf16 keys in sub-vectors of 8 and more");
   if (P.skip_flag && *P.skip_flag) return;
@@ -381,67 +413,84 @@ __global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P
   int* s_cnt = (int*)(s_sum + (size_t)n_cent * d_sub);             // [centre]     above are multiples of 8). A wave adds
                                                                    // one dimension at a time: the centres of its keys
                                                                    // spread over the banks
-  const float sum_scale = SUMS ? pq_sum_scale(*P.absmax_bits) : 1.f;
+  const uint32_t absmax = SUMS ? *P.absmax_bits : 0u;
+  const float sum_scale = SUMS ? pq_sum_scale(absmax) : 1.f;
+  const double sum_scale_d = (double)sum_scale;
+  const bool all_finite = absmax < 0x7f800000u;
 
-  auto norm2 = [&](int c) {
-    if (c >= n_cent) return INFINITY;  // centres beyond n_cent never win
-    float nn = 0.f;
-    for (int d = 0; d < d_sub; ++d) nn = fmaf(cbase[c * d_sub + d], cbase[c * d_sub + d], nn);
-    return nn;
-  };
+  // The centres pass once through LDS (in the place of the sums, which fit them) on their way to operands and norms: one
+  // round trip to memory instead of one per operand element of a thread.
+  float* s_c = SUMS ? (float*)s_sum : nullptr;
+  if (SUMS) {
+    for (int i = tid; i < n_cent * d_sub; i += PQM_NT) s_c[i] = cbase[i];
+    __syncthreads();
+  }
+  auto centre = [&](int c, int d) -> float { return SUMS ? s_c[c * d_sub + d] : cbase[c * d_sub + d]; };
+  int odd = 0;  // a centre that is not finite
+  for (int idx = tid; idx < n_tiles * 32; idx += PQM_NT) {
+    const int v = idx & 15, gg = (idx >> 4) & 1, t = idx >> 5;
+    const int c = t * 32 + 8 * (v >> 2) + 4 * gg + (v & 3);
+    float nn = INFINITY;  // centres beyond n_cent never win
+    if (c < n_cent) {
+      nn = 0.f;
+      for (int d = 0; d < d_sub; ++d) nn = fmaf(centre(c, d), centre(c, d), nn);
+      if (!(nn < INFINITY)) odd = 1;
+    }
+    s_cn[idx] = nn;
+  }
+  if (NORM_IN_A) __syncthreads();
   if constexpr (SPLIT) {
-    for (int idx = tid; idx < n_tiles * TILE_A; idx += PQM_NT) {  // one pair of slots each
-      const int e2 = (idx & 3) * 2, i = (idx >> 2) & 31, gg = (idx >> 7) & 1, op = (idx >> 8) % OPS, t = (idx >> 8) / OPS;
-      const int c = t * 32 + i;
-      uint32_t w = 0;
+    // a pair of dimensions each: its three terms, smallest in the first operands (they meet the accumulator while it holds the
+    // norm alone)
+    uint32_t* a32 = (uint32_t*)s_a;
+    for (int idx = tid; idx < n_tiles * 32 * KS; idx += PQM_NT) {
+      const int e = idx & 3, i = (idx >> 2) & 31, rest = idx >> 7, q8 = rest % (KS / 4), t = rest / (KS / 4);
+      const int c = t * 32 + i, d = 8 * q8 + 2 * e;
+      uint32_t w[3] = {0, 0, 0};
+      if (c < n_cent) {
+        const float lo = -2.0f * centre(c, d), hi = -2.0f * centre(c, d + 1);
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        int d, term;  // smallest terms first: they meet the accumulator while it holds the norm alone
-        if constexpr (KS == 4) {
-          d = e2 + u;
-          term = op ? gg : (gg ? 3 : 2);
-        } else {
-          d = (op % (KS / 8)) * 16 + 8 * gg + e2 + u;
-          term = 2 - op / (KS / 8);
-        }
-        if (NORM_IN_A && term == 3) {
-          if (e2 + u < 3) w |= pqm_term(norm2(c), e2 + u) << (16 * u);
-        } else if (c < n_cent) w |= pqm_term(-2.0f * cbase[c * d_sub + d], term) << (16 * u);
+        for (int term = 0; term < 3; ++term) w[term] = pqm_term(lo, term) | pqm_term(hi, term) << 16;
       }
-      ((uint32_t*)s_a)[idx] = w;
+      uint32_t* at = a32 + (size_t)t * TILE_A + i * 4 + e;  // + 256 * operand + 128 * half
+      if constexpr (KS == 4) {
+        at[0] = w[2];
+        at[256] = w[0];
+        at[384] = w[1];
+        const float nn = s_cn[t * 32 + ((i >> 2) & 1) * 16 + 4 * (i >> 3) + (i & 3)];
+        at[128] = e == 0 ? pqm_term(nn, 0) | pqm_term(nn, 1) << 16 : (e == 1 ? pqm_term(nn, 2) : 0u);
+      } else {
+#pragma unroll
+        for (int term = 0; term < 3; ++term) at[256 * ((q8 >> 1) + (KS / 8) * (2 - term)) + 128 * (q8 & 1)] = w[term];
+      }
     }
   } else {
     for (int idx = tid; idx < n_tiles * TILE_A; idx += PQM_NT) {
       const int s4 = idx % SQ, i = (idx / SQ) & 31, q = (idx / (SQ * 32)) % (KS / SQ), gg = (idx / (SQ * 32 * (KS / SQ))) & 1,
                 t = idx / (64 * KS);
       const int c = t * 32 + i, d = 2 * (q * SQ + s4) + gg;
-      s_a[idx] = (c < n_cent && d < d_sub) ? -2.0f * cbase[c * d_sub + d] : 0.f;
+      s_a[idx] = (c < n_cent && d < d_sub) ? -2.0f * centre(c, d) : 0.f;
     }
   }
-  int odd = 0;  // a centre that is not finite
-  for (int idx = tid; idx < n_tiles * 32; idx += PQM_NT) {
-    const int v = idx & 15, gg = (idx >> 4) & 1, t = idx >> 5;
-    const int c = t * 32 + 8 * (v >> 2) + 4 * gg + (v & 3);
-    s_cn[idx] = norm2(c);
-    if (c < n_cent && !(s_cn[idx] < INFINITY)) odd = 1;
-  }
+  odd = __syncthreads_or(odd);
   if (SUMS) {
     for (int i = tid; i < n_cent * d_sub; i += PQM_NT) s_sum[i] = 0;
     for (int i = tid; i < n_cent; i += PQM_NT) s_cnt[i] = 0;
+    __syncthreads();
   }
-  odd = __syncthreads_or(odd);
 
   const int64_t kbase = (int64_t)b * P.ks_b + (int64_t)hk * P.ks_h + (int64_t)s_idx * d_sub;
+  uint8_t* codes = P.codes + ((int64_t)bh * P.code_pitch + P.code_offset + (int64_t)tg * wg_tiles * 32) * P.n_sub + s_idx;  // of the workgroup's first key
   constexpr int NB = SPLIT ? (KS >= 8 ? KS / 8 : 1) : 1;  // key operands of 16 dimensions
   auto key_offset = [&](int n) { return kbase + (int64_t)(P.key_offset + (n < P.n_keys ? n : P.n_keys - 1)) * P.ks_l; };
-  uint4 nb[NB];  // SPLIT: the next tile's keys, requested while this one is searched
+  sah_u4 nb[NB];  // SPLIT: the next tile's keys, requested while this one is searched
   auto request = [&](int n) {
     const uint16_t* kp = (const uint16_t*)P.k + key_offset(n);
     if constexpr (KS == 4) {
-      nb[0] = *(const uint4*)kp;
+      nb[0] = *(const sah_u4*)kp;
     } else {
 #pragma unroll
-      for (int q = 0; q < NB; ++q) nb[q] = *(const uint4*)(kp + 16 * q + 8 * g);
+      for (int q = 0; q < NB; ++q) nb[q] = *(const sah_u4*)(kp + 16 * q + 8 * g);
     }
   };
   if constexpr (SPLIT) request((tg * wg_tiles + wave) * 32 + j);
@@ -451,13 +500,14 @@ __global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P
     const int n = n0 + j;
     const bool valid = n < P.n_keys;
     float xs[SPLIT ? 1 : KS];  // this lane's dims 2 s + g of its key
-    uint4 xb[NB];              // SPLIT: dims 16 q + 8 g .. + 7 (sub-vectors of 8: both halves hold all)
-    uint4 x0;                  // key operand of the first instruction: with the norm in A, ones against its terms
+    sah_u4 xb[NB];             // SPLIT: dims 16 q + 8 g .. + 7 (sub-vectors of 8: both halves hold all)
+    sah_u4 x0;                 // key operand of the first instruction: with the norm in A, ones against its terms
     if constexpr (SPLIT) {
 #pragma unroll
       for (int q = 0; q < NB; ++q) xb[q] = nb[q];
       request(n + 32 * PQM_NW);
-      x0 = KS == 4 && g ? make_uint4(0x3f803f80u, 0x3f80u, 0u, 0u) : xb[0];
+      x0 = xb[0];
+      if (KS == 4 && g) x0 = sah_u4{0x3f803f80u, 0x3f80u, 0u, 0u};
     } else {
       const int64_t off = key_offset(n);
 #pragma unroll
@@ -478,7 +528,7 @@ __global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P
       if constexpr (SPLIT) {
         const uint4* ap = (const uint4*)s_a + (size_t)t * 64 * OPS + g * 32 + j;
 #pragma unroll
-        for (int op = 0; op < OPS; ++op) acc = sah_mfma_32x32x16<SAH_BF16>(ap[op * 64], op ? xb[op % NB] : x0, acc);
+        for (int op = 0; op < OPS; ++op) acc = sah_mfma_32x32x16<SAH_BF16>(ap[op * 64], __builtin_bit_cast(uint4, op ? xb[op % NB] : x0), acc);
       } else if constexpr (KS >= 4) {
         const float4* ap = (const float4*)(s_a + (size_t)(t * 2 + g) * 32 * KS) + j;
 #pragma unroll
@@ -495,15 +545,17 @@ __global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P
         for (int s = 0; s < KS; ++s) acc = sah_mfma_32x32x2_f32(ap[s], xs[s], acc);
       }
     };
-    // The smallest value, its tile, and that tile's 16 values, from which the slot is found once at the end: 27 vector
-    // instructions a tile (eight three-way minima, one comparison, 18 selects; SPLIT: 28, with the second smallest of the
-    // tiles' minima) where a search for the slot takes 48. Strictly smaller in ascending tiles, lowest slot: the first
-    // minimum is kept. A value that is not a number makes the tile's minimum one: such key tiles are evaluated again below.
+    // The smallest value and its tile; a value that is not a number makes its tile's minimum one, and such key tiles are
+    // evaluated again below. Without the split form also that tile's 16 values, from which the slot is found once at the end
+    // (27 vector instructions a tile; a search for the slot takes 48): strictly smaller in ascending tiles, lowest slot, so
+    // that the first minimum is kept. In the split form instead every slot's minimum over the tiles, two tiles to a three-way
+    // minimum, and the second smallest of the tiles' minima (20 instructions a tile): together they tell whether any other
+    // centre came near the smallest value, and with none near the smallest value's slot is the one whose minimum it is.
     float best = INFINITY, second = INFINITY;
     int bt = 0;
     bool nan = false;
     sah_f32x16 kept = {};
-    auto take_min = [&](const sah_f32x16& acc, int t) {
+    auto tile_min = [&](const sah_f32x16& acc, int t) -> bool {
       float m = acc[0];
 #pragma unroll
       for (int v = 1; v < 16; ++v) m = PQM_MIN(m, acc[v]);
@@ -512,29 +564,54 @@ __global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P
       const bool less = m < best;
       best = less ? m : best;
       bt = less ? t : bt;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) kept[v] = less ? acc[v] : kept[v];
+      return less;
     };
-    // two accumulators: a tile's products are issued before the minimum of the tile before is taken, which so never waits
-    // for a product just started
     sah_f32x16 acc0, acc1;
-    product(acc0, 0);
-    int t = 0;
-    for (; t + 2 < n_tiles; t += 2) {
-      product(acc1, t + 1);
-      take_min(acc0, t);
-      product(acc0, t + 2);
-      take_min(acc1, t + 1);
-    }
-    if (t + 1 < n_tiles) {
-      product(acc1, t + 1);
-      take_min(acc0, t);
-      take_min(acc1, t + 1);
+    if constexpr (SPLIT) {
+      product(acc0, 0);
+      tile_min(acc0, 0);
+      kept = acc0;
+      int t = 1;
+      for (; t + 1 < n_tiles; t += 2) {
+        product(acc0, t);
+        product(acc1, t + 1);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) kept[v] = PQM_MIN(PQM_MIN(kept[v], acc0[v]), acc1[v]);
+        tile_min(acc0, t);
+        tile_min(acc1, t + 1);
+      }
+      if (t < n_tiles) {
+        product(acc0, t);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) kept[v] = PQM_MIN(kept[v], acc0[v]);
+        tile_min(acc0, t);
+      }
     } else {
-      take_min(acc0, t);
+      auto take_min = [&](const sah_f32x16& acc, int t) {
+        const bool less = tile_min(acc, t);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) kept[v] = less ? acc[v] : kept[v];
+      };
+      // two accumulators: a tile's products are issued before the minimum of the tile before is taken, which so never waits
+      // for a product just started
+      product(acc0, 0);
+      int t = 0;
+      for (; t + 2 < n_tiles; t += 2) {
+        product(acc1, t + 1);
+        take_min(acc0, t);
+        product(acc0, t + 2);
+        take_min(acc1, t + 1);
+      }
+      if (t + 1 < n_tiles) {
+        product(acc1, t + 1);
+        take_min(acc0, t);
+        take_min(acc1, t + 1);
+      } else {
+        take_min(acc0, t);
+      }
     }
     int slot = 0, bidx;
-    bool again;  // uniform: the key tile is evaluated in fp32
+    bool again;  // uniform: the key tile is evaluated in fp32, centres or keys not finite
     if constexpr (SPLIT) {
       // The split form's values round differently from the fp32 form's, and the codes are the fp32 form's whichever form
       // ran. They agree where no other centre comes within twice the two forms' difference of the smallest value. With
@@ -545,39 +622,57 @@ __global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P
       float x2 = 0.f;
 #pragma unroll
       for (int q = 0; q < NB; ++q) {
-        const uint32_t w[4] = {xb[q].x, xb[q].y, xb[q].z, xb[q].w};
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float lo = sah_bits_to_float(w[e] << 16), hi = sah_bits_to_float(w[e] & 0xffff0000u);
-          x2 = fmaf(lo, lo, fmaf(hi, hi, x2));
-        }
+        for (int e = 0; e < 4; ++e) x2 = sah_dot2<SAH_BF16>(xb[q][e], xb[q][e], x2);
       }
-      if (KS != 4) x2 += __shfl_xor(x2, 32);
-      const float ob = __shfl_xor(best, 32);
-      best = ob < best ? ob : best;
+      if (KS != 4) x2 = sah_half_sum(x2);
+      best = sah_half_min(best);
       float r2 = best + x2;
       r2 = r2 < 0.f ? 0.f : r2;
-      const float reach = sqrtf(x2) + sqrtf(r2);
+      const float reach = __builtin_amdgcn_sqrtf(x2) + __builtin_amdgcn_sqrtf(r2);
       constexpr float FORMS = KS == 4 ? 16.f : KS == 8 ? 24.f : KS == 16 ? 34.f : KS == 32 ? 48.f : 68.f;
       const float lim = best + 7.0f * 0x1p-24f * FORMS * reach * reach;  // (not finite where the key is not)
-      // the centres within it, of this lane's 16 of the winning tile and of the other tiles' minima: exactly one wins
-      uint64_t one = 0, two = 0;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const bool near = kept[v] <= lim;
-        slot = near ? v : slot;
-        const uint64_t m = __ballot(near);
-        two |= one & m;
-        one |= m;
+      // The centres within it, of the minima of this lane's 16 slots (bit v of `in`) and of the other tiles (bit 16): exactly
+      // one wins. (In vector registers throughout: ballots combined by the scalar unit cost 10 us of a launch.)
+      uint32_t in = pqm_mask_le(kept, lim);
+      const uint32_t info = in | (second <= lim ? 1u << 16 : 0u) | (uint32_t)bt << 20;
+      uint32_t lo_half, hi_half;  // of the lanes g = 0 and g = 1 of the key
+      sah_half_both(info, lo_half, hi_half);
+      const bool from_lo = (lo_half & 0xffffu) != 0;
+      const uint32_t src = from_lo ? lo_half : hi_half;
+      slot = __builtin_ctz(src | 0x10000u);
+      bidx = (int)(src >> 20) * 32 + 8 * (slot >> 2) + (from_lo ? 0 : 4) + (slot & 3);  // tile, slot -> centre
+      const bool open = __popc(lo_half & 0x1ffffu) + __popc(hi_half & 0x1ffffu) != 1;
+      const bool any_open = __ballot(open) != 0;  // uniform
+      again = odd || (any_open && __ballot(!(lim < INFINITY)) != 0);
+      if (any_open && !again) {
+        // The fp32 form's values, for the keys with several centres in reach, of every centre in a slot that holds one: the fp32
+        // matrix instruction is a chain of fused multiply-adds in ascending dimensions (checked bit for bit on the hardware),
+        // so a lane can evaluate one centre.
+        if (!open) in = 0;
+        float fb = INFINITY;
+        int fi = 0x7fffffff;
+        const int64_t koff = key_offset(n);
+        while (in) {
+          const int v = __builtin_ctz(in);
+          in &= in - 1;
+          const int c0 = 8 * (v >> 2) + 4 * g + (v & 3);
+          for (int t = 0; t < n_tiles && t * 32 + c0 < n_cent; ++t) {
+            const int c = t * 32 + c0;
+            float val = s_cn[(t * 2 + g) * 16 + v];
+#pragma unroll 8
+            for (int d = 0; d < 2 * KS; ++d) val = fmaf(-2.0f * cbase[c * d_sub + d], sah_load<DT>(P.k, koff + d), val);
+            if (val < fb || (val == fb && c < fi)) {  // the first minimum
+              fb = val;
+              fi = c;
+            }
+          }
+        }
+        const float ob = __shfl_xor(fb, 32);
+        const int oi = __shfl_xor(fi, 32);
+        if (ob < fb || (ob == fb && oi < fi)) fi = oi;
+        if (open) bidx = fi;
       }
-      const uint64_t m = __ballot(second <= lim);
-      two |= one & m;
-      one |= m;
-      const uint32_t lo1 = (uint32_t)one, hi1 = (uint32_t)(one >> 32);
-      again = odd || ((uint32_t)two | (uint32_t)(two >> 32) | ~(lo1 ^ hi1)) != 0;
-      bidx = bt * 32 + 8 * (slot >> 2) + 4 * g + (slot & 3);  // tile, slot -> centre
-      const int oi = __shfl_xor(bidx, 32);
-      bidx = ((one >> lane) & 1) ? bidx : oi;
     } else {
 #pragma unroll
       for (int v = 15; v >= 0; --v) slot = kept[v] == best ? v : slot;
@@ -587,7 +682,7 @@ __global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P
       if (ob < best || (ob == best && oi < bidx)) bidx = oi;
       again = odd || __ballot(nan) != 0;
     }
-    if (again) {  // in fp32, operands straight from memory; a value that is not a number loses to any other
+    if (again) {  // all centres in fp32, operands straight from memory; a value that is not a number loses to any other
       best = INFINITY;
       bidx = 0;
       const int64_t off = key_offset(n);
@@ -628,25 +723,29 @@ __global__ __launch_bounds__(PQM_NT, 2) void k_pq_assign_mfma(pq_assign_params P
       if (ob < best || (ob == best && oi < bidx)) bidx = oi;
     }
     if (valid) {
-      if (g == 0) P.codes[(((int64_t)bh * P.code_pitch) + P.code_offset + n) * P.n_sub + s_idx] = (uint8_t)bidx;
+      if (g == 0) codes[(uint32_t)((kt * 32 + j) * P.n_sub)] = (uint8_t)bidx;
       if (SUMS) {
         if constexpr (SPLIT) {
-          auto add2 = [&](uint32_t w, int d) {  // two dimensions of a packed word
-            pq_sum_add(&s_sum[d * n_cent + bidx], sah_bits_to_float(w << 16), sum_scale);
-            pq_sum_add(&s_sum[(d + 1) * n_cent + bidx], sah_bits_to_float(w & 0xffff0000u), sum_scale);
-          };
-          if constexpr (KS == 4) {
-            add2(g ? xb[0].z : xb[0].x, 4 * g);
-            add2(g ? xb[0].w : xb[0].y, 4 * g + 2);
-          } else {
+          auto add_all = [&](auto&& add) {
+            auto add2 = [&](uint32_t w, int d) {  // two dimensions of a packed word
+              add(&s_sum[d * n_cent + bidx], sah_bits_to_float(w << 16));
+              add(&s_sum[(d + 1) * n_cent + bidx], sah_bits_to_float(w & 0xffff0000u));
+            };
+            if constexpr (KS == 4) {
+              add2(g ? xb[0].z : xb[0].x, 4 * g);
+              add2(g ? xb[0].w : xb[0].y, 4 * g + 2);
+            } else {
 #pragma unroll
-            for (int q = 0; q < NB; ++q) {
-              add2(xb[q].x, 16 * q + 8 * g);
-              add2(xb[q].y, 16 * q + 8 * g + 2);
-              add2(xb[q].z, 16 * q + 8 * g + 4);
-              add2(xb[q].w, 16 * q + 8 * g + 6);
+              for (int q = 0; q < NB; ++q) {
+                add2(xb[q].x, 16 * q + 8 * g);
+                add2(xb[q].y, 16 * q + 8 * g + 2);
+                add2(xb[q].z, 16 * q + 8 * g + 4);
+                add2(xb[q].w, 16 * q + 8 * g + 6);
+              }
             }
-          }
+          };
+          if (all_finite) add_all([&](long long* p, float x) { pq_sum_add_finite(p, x, sum_scale_d); });  // uniform
+          else add_all([&](long long* p, float x) { pq_sum_add(p, x, sum_scale); });
         } else {
 #pragma unroll
           for (int s = 0; s < KS; ++s)
