@@ -21,7 +21,7 @@ int sah_members_attention(const sah_attention_args* a);
 
 /* A whole Lloyd run: sah_pq_keys_absmax, then max_iter times sah_pq_kmeans_assign and sah_pq_kmeans_update, in one call
  * and without host-made random numbers. given_start != 0: centres hold the start. Otherwise the start is vector
- * start_idx[g][c] (written here, scratch of the caller) of every group: one vector of each of n_cent equal strata of
+ * start_idx[g][c] (scratch of the caller, no output) of every group: one vector of each of n_cent equal strata of
  * [0, n_keys), chosen by number g * n_cent + c of torch.rand(float64) with a CPU generator seeded with start_seed. In
  * iteration i an empty centre takes vector number (i * n_groups + g) * n_cent + c of torch.randint(0, n_keys) with a CPU
  * generator seeded with reseed_seed (below 2^28 keys; beyond, where torch draws 64 bits, still the 32-bit number modulo
@@ -40,7 +40,7 @@ typedef struct sah_pq_kmeans_args {
   float* shift2;                  /* [n_groups] */
   int32_t* state;                 /* [4] */
   uint32_t* absmax_bits;          /* [1] */
-  int32_t* start_idx;             /* [n_groups, n_cent]; may be NULL with given_start */
+  int32_t* start_idx;             /* [n_groups, n_cent], scratch; may be NULL with given_start */
   int32_t* reseed_idx;            /* [max_iter, n_groups, n_cent] or NULL */
   uint64_t start_seed, reseed_seed;
   float tol;

@@ -376,6 +376,22 @@ __device__ __forceinline__ float sah_agent_load_f32(const float* p) {
   return *(const volatile float*)p;
 #endif
 }
+template <typename T>
+__device__ __forceinline__ T sah_agent_load(const T* p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#else
+  return *(const volatile T*)p;
+#endif
+}
+template <typename T>
+__device__ __forceinline__ void sah_agent_store(T* p, T v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#else
+  *(volatile T*)p = v;
+#endif
+}
 // every store this thread has issued has reached its point of coherence
 __device__ __forceinline__ void sah_stores_done() {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -405,6 +421,13 @@ __device__ __forceinline__ void sah_wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Workgroup barrier for data that passes through LDS: __syncthreads() without its wait for the wave's stores to memory.
+__device__ __forceinline__ void sah_lds_barrier() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#endif
 }
 
 // ---------------------------------------------------------------------------

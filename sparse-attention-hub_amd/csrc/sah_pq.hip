@@ -289,6 +289,184 @@ __global__ __launch_bounds__(PQB_NT) void k_pq_assign_block(pq_assign_params P) 
   }
 }
 
+struct pq_update_params {
+  const void* k; int64_t ks_b, ks_h, ks_l;
+  int Hkv, n_sub, d_sub, n_cent, key_offset;
+  float* centres;
+  long long* sums; int* counts;
+  const uint32_t* absmax_bits;
+  const int* reseed_idx;   // NULL: vector i of an empty centre is number reseed_first + g * n_cent + c of the generator
+  uint32_t reseed_seed;    // seeded with reseed_seed, modulo n_keys (torch.randint of the whole run, drawn where needed)
+  int64_t reseed_first;
+  int n_keys;
+  int clear;               // sums and counts are left zero for the next assignment
+  float* shift2;
+  float tol;
+  int* state;
+  int n_groups;
+};
+
+struct pq_update_lds {
+  float red[PQ_MAX_CENT / SAH_WAVE];
+  mt_lds mt;
+};
+// vector of the group that an empty centre takes (thread c: centre c; ridx of the others: any); all threads call
+template <int NT>
+__device__ __forceinline__ int pq_reseed_vector(const pq_update_params& P, int g, int cn, pq_update_lds& S) {
+  static_assert(NT >= PQ_MAX_CENT, "a thread per centre");
+  const int tid = threadIdx.x;
+  int ridx = 0;
+  if (P.reseed_idx) {
+    if (tid < P.n_cent && cn == 0) ridx = P.reseed_idx[(int64_t)g * P.n_cent + tid];
+  } else if (__syncthreads_or(tid < P.n_cent && cn == 0)) {  // rare: the generator runs only where a centre is empty
+    const int64_t first = P.reseed_first + (int64_t)g * P.n_cent;
+    const int64_t mine = first + (tid < P.n_cent ? tid : 0);
+    const int last = (int)((first + P.n_cent - 1) / MT_N);
+    mt_seed(S.mt, P.reseed_seed);
+    for (int blk = 0; blk <= last; ++blk) {
+      mt_next(S.mt, blk & 1);
+      if (mine / MT_N == blk) ridx = (int)(mt_temper(S.mt.st[(blk & 1) ^ 1][mine % MT_N]) % (uint32_t)P.n_keys);
+    }
+  }
+  return ridx;
+}
+// the group's share of the verdict: thread c < n_cent brings the distance centre c has moved
+__device__ __forceinline__ void pq_update_verdict(const pq_update_params& P, int g, float move, pq_update_lds& S) {
+  const int tid = threadIdx.x;
+  move = sah_wave_sum(move);
+  if ((tid & (SAH_WAVE - 1)) == 0 && tid < PQ_MAX_CENT) S.red[tid / SAH_WAVE] = move;
+  __syncthreads();
+  if (tid == 0) {
+    float tot = 0.f;
+    for (int i = 0; i < PQ_MAX_CENT / SAH_WAVE; ++i) tot += S.red[i];
+    const float sh2 = tot * tot;
+    P.shift2[g] = sh2;
+    // the verdict's two counters only: the converged count is in before the ticket is taken, nothing else is handed over
+    if (sh2 < P.tol) atomicAdd(&P.state[0], 1);
+    sah_stores_done();
+    const int ticket = atomicAdd(&P.state[1], 1);
+    if (ticket == P.n_groups - 1) {
+      // last group of this iteration, every other has read the done flag: publish the verdict, reset the counters
+      const int conv = atomicAdd(&P.state[0], 0);
+      if (conv == P.n_groups) P.state[2] = 1;
+      P.state[0] = 0;
+      P.state[1] = 0;
+    }
+  }
+}
+__device__ __forceinline__ int64_t pq_update_key(const pq_update_params& P, int g, int ridx) {
+  const int s = g % P.n_sub, bh = g / P.n_sub;
+  return (int64_t)(bh / P.Hkv) * P.ks_b + (int64_t)(bh % P.Hkv) * P.ks_h + (int64_t)(P.key_offset + ridx) * P.ks_l + (int64_t)s * P.d_sub;
+}
+
+// The update of a group by the workgroup (NT threads) of an assignment that ends last: sums and counts come with accesses that
+// see what the others have added, requested together and at consecutive addresses, and are left zero; the new centres element
+// by element, the distances by a thread per centre in ascending dimensions (as k_pq_update).
+static __host__ __device__ size_t pq_update_here_bytes(int n_cent, int d_sub) {
+  return (sizeof(pq_update_lds) + 15) / 16 * 16 + (size_t)n_cent * 16 + (size_t)n_cent * (d_sub + 1) * 4;
+}
+template <int DT, int NT>
+__device__ __forceinline__ void pq_update_here(const pq_update_params& P, int g, unsigned char* lds) {
+  const int tid = threadIdx.x;
+  const int d_sub = P.d_sub, n_cent = P.n_cent, n_el = n_cent * d_sub;
+  pq_update_lds& S = *(pq_update_lds*)lds;
+  double* s_un = (double*)(lds + (sizeof(pq_update_lds) + 15) / 16 * 16);  // [n_cent] 1 / (scale * members)
+  int* s_from = (int*)(s_un + n_cent);                                     // [n_cent] vector an empty centre takes, -1: none
+  float* s_df = (float*)(s_from + 2 * n_cent);                             // [n_cent][d_sub + 1]
+  float* cc = P.centres + (int64_t)g * n_el;
+  long long* ss = P.sums + (int64_t)g * n_el;
+  int* cp = P.counts + (int64_t)g * n_cent;
+  constexpr int B = 4;  // elements a thread requests at a time
+  long long sv[B];
+  float ov[B];
+  auto request = [&](int i0) {
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      const int i = i0 + u * NT < n_el ? i0 + u * NT : n_el - 1;
+      sv[u] = sah_agent_load(&ss[i]);
+      ov[u] = cc[i];
+    }
+  };
+  const int cn = tid < n_cent ? sah_agent_load(&cp[tid]) : 1;
+  request(tid);
+  const int ridx = pq_reseed_vector<NT>(P, g, cn, S);
+  if (tid < n_cent) {
+    s_un[tid] = 1.0 / ((double)pq_sum_scale(*P.absmax_bits) * (double)(cn > 0 ? cn : 1));
+    s_from[tid] = cn > 0 ? -1 : ridx;
+    sah_agent_store(&cp[tid], 0);
+  }
+  __syncthreads();
+  for (int i0 = tid; i0 < n_el; i0 += B * NT) {
+    if (i0 != tid) request(i0);
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      const int i = i0 + u * NT;
+      if (i < n_el) {
+        const int c = i / d_sub, d = i - c * d_sub, from = s_from[c];
+        const float nv = from < 0 ? (float)((double)sv[u] * s_un[c]) : sah_load<DT>(P.k, pq_update_key(P, g, from) + d);
+        s_df[c * (d_sub + 1) + d] = nv - ov[u];
+        cc[i] = nv;
+        sah_agent_store(&ss[i], 0ll);
+      }
+    }
+  }
+  __syncthreads();
+  float move = 0.f;
+  if (tid < n_cent) {
+    float acc = 0.f;
+    for (int d = 0; d < d_sub; ++d) {
+      const float df = s_df[tid * (d_sub + 1) + d];
+      acc = fmaf(df, df, acc);
+    }
+    move = sqrtf(acc);
+  }
+  pq_update_verdict(P, g, move, S);
+}
+
+// The update in a launch of its own: one workgroup per group, a thread per centre. What bounds it is latency (a group's 18 KB):
+// the sums of eight dimensions are requested together.
+template <int DT>
+__global__ __launch_bounds__(PQ_NT) void k_pq_update(pq_update_params P) {
+  __shared__ pq_update_lds S;
+  if (P.state[2]) return;
+  const int tid = threadIdx.x, g = blockIdx.x;
+  const int d_sub = P.d_sub, n_cent = P.n_cent;
+  float move = 0.f;
+  const int cn = tid < n_cent ? P.counts[(int64_t)g * n_cent + tid] : 1;
+  const int ridx = pq_reseed_vector<PQ_NT>(P, g, cn, S);
+  if (tid < n_cent) {
+    const int c = tid;
+    float* cc = P.centres + ((int64_t)g * n_cent + c) * d_sub;
+    long long* ss = P.sums + ((int64_t)g * n_cent + c) * d_sub;
+    const double unscale = 1.0 / ((double)pq_sum_scale(*P.absmax_bits) * (double)(cn > 0 ? cn : 1));
+    float acc = 0.f;
+    const int64_t roff = pq_update_key(P, g, ridx);
+    for (int d0 = 0; d0 < d_sub; d0 += 8) {
+      long long sv[8];
+      float ov[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int d = d0 + u < d_sub ? d0 + u : d_sub - 1;
+        sv[u] = ss[d];
+        ov[u] = cc[d];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int d = d0 + u;
+        if (d >= d_sub) break;
+        const float nv = (cn > 0) ? (float)((double)sv[u] * unscale) : sah_load<DT>(P.k, roff + d);
+        const float df = nv - ov[u];
+        acc = fmaf(df, df, acc);
+        cc[d] = nv;
+        if (P.clear) ss[d] = 0;
+      }
+    }
+    if (P.clear) P.counts[(int64_t)g * n_cent + c] = 0;
+    move = sqrtf(acc);
+  }
+  pq_update_verdict(P, g, move, S);
+}
+
 // ---------------------------------------------------------------------------
 // Lloyd assignment on the matrix cores. argmin_c ||x - c||^2 = argmin_c (||c||^2 - 2 x.c): the key x centre
 // contraction is a 32 x 32 matrix product whose accumulator starts at ||c||^2 and whose A operand is -2 c, so the
@@ -302,7 +480,7 @@ __global__ __launch_bounds__(PQB_NT) void k_pq_assign_block(pq_assign_params P) 
 // The split form's rounding is another one (and smaller), so where several centres come within both forms' rounding of the
 // smallest value they are evaluated in the fp32 form's order of operations: the codes are those of the fp32 form, bit for
 // bit, whichever form the alignment and shape of the keys allow (without: 1e-6 of the codes of an iteration, 5e-4 after ten).
-// Measured (bf16, 8 heads x 16277 keys, 16 sub-vectors of 8, 256 centres, sums included): 68 us; 85 with every tile's 16
+// Measured (bf16, 8 heads x 16277 keys, 16 sub-vectors of 8, 256 centres, sums included): 68 us (76 with the update); 85 with every tile's 16
 // values selected, not their minima over the tiles, the second look by matrix instruction, its test by ballots, the key
 // operand in a structure (which went through scratch memory) and the centres read element by element. What bounds it: issue,
 // 20 vector and 2 matrix instructions a tile (31 us) and 150 vector ones a key tile of eight (25), 10 before and after the
@@ -331,7 +509,8 @@ static size_t pqm_lds_bytes(int n_cent, int d_sub, int ks, bool sums, bool split
   const size_t n_tiles = (size_t)(n_cent + 31) / 32;
   size_t bytes = n_tiles * 64 * (split ? 16 * (size_t)pqm_split_ops(ks) : 4 * (size_t)ks) + n_tiles * 32 * 4;
   if (sums) bytes += (size_t)n_cent * d_sub * 8 + (size_t)n_cent * 4;
-  return bytes;
+  const size_t update = sums ? pq_update_here_bytes(n_cent, d_sub) : 0;  // (runs in the same LDS)
+  return bytes > update ? bytes : update;
 }
 
 // term 0, 1, 2 of a float as bf16 bits: eight significant bits each, their sum is the float (a float that is not finite
@@ -376,7 +555,8 @@ __device__ __forceinline__ uint32_t pqm_mask_le(const sah_f32x16& a, float b) {
 // exactly 2 KS in the split form. SUMS: the per-centre sums of the update step are accumulated here (P.sums given and
 // the LDS holds them). A workgroup takes wg_tiles tiles of 32 keys of one group.
 template <int DT, int KS, bool SUMS, bool SPLIT>
-__global__ __launch_bounds__(PQM_NT, SPLIT && KS <= 16 ? 4 : 2) void k_pq_assign_mfma(pq_assign_params P, int wg_tiles, int ranges, int n_heads) {
+__global__ __launch_bounds__(PQM_NT, KS <= 16 ? 4 : 2) void k_pq_assign_mfma(pq_assign_params P, pq_update_params U, uint32_t* arrivals,
+                                                                                           int wg_tiles, int ranges, int n_heads) {
   HIP_DYNAMIC_SHARED(unsigned char, pqm_dyn)
   static_assert(!SPLIT || (DT == SAH_BF16 && KS >= 4), "the split form multiplies bf16 keys in sub-vectors of 8 and more");
   if (P.skip_flag && *P.skip_flag) return;
@@ -765,6 +945,17 @@ __global__ __launch_bounds__(PQM_NT, SPLIT && KS <= 16 ? 4 : 2) void k_pq_assign
   }
   for (int c = tid; c < n_cent; c += PQM_NT)
     if (s_cnt[c]) atomicAdd(&P.counts[(int64_t)grp * n_cent + c], s_cnt[c]);
+  if (!arrivals) return;
+  // The workgroup of the group that arrives last carries out the update: 8 us of this kernel, where a launch of its own takes
+  // 9.3 and the way from kernel to kernel.
+  sah_stores_done();  // (the atomics' too)
+  __syncthreads();
+  int* s_last = s_cnt;
+  if (tid == 0) *s_last = sah_last_arrival(arrivals + (int64_t)grp * n_cent, (uint32_t)ranges) ? 1 : 0;
+  __syncthreads();
+  const bool last = *s_last != 0;
+  __syncthreads();  // the LDS goes on to the update
+  if (last) pq_update_here<DT, PQM_NT>(U, grp, pqm_dyn);
 }
 
 // Per-centre sums and counts from the codes an assignment wrote, for shapes whose sums do not fit beside the
@@ -815,7 +1006,8 @@ __global__ __launch_bounds__(PQS_NT) void k_pq_sums(pq_assign_params P, int d_ch
 }
 
 template <int DT, int KS, bool SPLIT>
-static int pq_launch_mfma_ks(const sah_pq_assign_args* a, const pq_assign_params& P, bool fused, size_t lds) {
+static int pq_launch_mfma_ks(const sah_pq_assign_args* a, const pq_assign_params& P, const pq_update_params& U, uint32_t* arrivals, bool fused,
+                             size_t lds) {
   const int tiles = (a->n_keys + 31) / 32;
   const int64_t all = (int64_t)tiles * a->n_sub * a->B * a->Hkv;
   int64_t wg_tiles = (all + PQM_WGS - 1) / PQM_WGS;
@@ -830,24 +1022,25 @@ static int pq_launch_mfma_ks(const sah_pq_assign_args* a, const pq_assign_params
   sah_timed timed("k_pq_assign_mfma", a->stream);
   if (fused) {
     if (int rc = sah_allow_lds((const void*)k_pq_assign_mfma<DT, KS, true, SPLIT>, PQM_MAX_LDS, "sah_pq_kmeans_assign")) return rc;
-    hipLaunchKernelGGL((k_pq_assign_mfma<DT, KS, true, SPLIT>), g, blk, lds, st, P, per, ranges, heads);
+    hipLaunchKernelGGL((k_pq_assign_mfma<DT, KS, true, SPLIT>), g, blk, lds, st, P, U, arrivals, per, ranges, heads);
   } else {
     if (int rc = sah_allow_lds((const void*)k_pq_assign_mfma<DT, KS, false, SPLIT>, PQM_MAX_LDS, "sah_pq_kmeans_assign")) return rc;
-    hipLaunchKernelGGL((k_pq_assign_mfma<DT, KS, false, SPLIT>), g, blk, lds, st, P, per, ranges, heads);
+    hipLaunchKernelGGL((k_pq_assign_mfma<DT, KS, false, SPLIT>), g, blk, lds, st, P, U, nullptr, per, ranges, heads);
   }
   return sah_launch_status("sah_pq_kmeans_assign");
 }
 
 template <int DT, int KS>
-static int pq_launch_mfma_form(const sah_pq_assign_args* a, const pq_assign_params& P, bool split, bool fused, size_t lds) {
+static int pq_launch_mfma_form(const sah_pq_assign_args* a, const pq_assign_params& P, const pq_update_params& U, uint32_t* arrivals, bool split,
+                               bool fused, size_t lds) {
   if constexpr (DT == SAH_BF16 && KS >= 4) {
-    if (split) return pq_launch_mfma_ks<DT, KS, true>(a, P, fused, lds);
+    if (split) return pq_launch_mfma_ks<DT, KS, true>(a, P, U, arrivals, fused, lds);
   }
-  return pq_launch_mfma_ks<DT, KS, false>(a, P, fused, lds);
+  return pq_launch_mfma_ks<DT, KS, false>(a, P, U, arrivals, fused, lds);
 }
 
 template <int DT>
-static int pq_launch_mfma(const sah_pq_assign_args* a, const pq_assign_params& P) {
+static int pq_launch_mfma(const sah_pq_assign_args* a, const pq_assign_params& P, const pq_update_params* U, uint32_t* arrivals, bool* updated) {
   int ks = 2;
   while (2 * ks < a->d_sub) ks *= 2;  // 2, 4, 8, 16, 32, 64 k-steps: sub-vectors of up to 4 ... 128 dimensions
   const bool want_sums = a->sums != nullptr;
@@ -859,14 +1052,17 @@ static int pq_launch_mfma(const sah_pq_assign_args* a, const pq_assign_params& P
                      pqm_lds_bytes(a->n_cent, a->d_sub, ks, false, true) <= PQM_MAX_LDS;
   const bool fused = want_sums && pqm_lds_bytes(a->n_cent, a->d_sub, ks, true, split) <= PQM_FUSED_LDS;
   const size_t lds = pqm_lds_bytes(a->n_cent, a->d_sub, ks, fused, split);
+  const pq_update_params u = U ? *U : pq_update_params{};
+  if (!U || !fused) arrivals = nullptr;
+  if (updated) *updated = arrivals != nullptr;
   int rc;
   switch (ks) {
-    case 2: rc = pq_launch_mfma_form<DT, 2>(a, P, split, fused, lds); break;
-    case 4: rc = pq_launch_mfma_form<DT, 4>(a, P, split, fused, lds); break;
-    case 8: rc = pq_launch_mfma_form<DT, 8>(a, P, split, fused, lds); break;
-    case 16: rc = pq_launch_mfma_form<DT, 16>(a, P, split, fused, lds); break;
-    case 32: rc = pq_launch_mfma_form<DT, 32>(a, P, split, fused, lds); break;
-    default: rc = pq_launch_mfma_form<DT, 64>(a, P, split, fused, lds); break;
+    case 2: rc = pq_launch_mfma_form<DT, 2>(a, P, u, arrivals, split, fused, lds); break;
+    case 4: rc = pq_launch_mfma_form<DT, 4>(a, P, u, arrivals, split, fused, lds); break;
+    case 8: rc = pq_launch_mfma_form<DT, 8>(a, P, u, arrivals, split, fused, lds); break;
+    case 16: rc = pq_launch_mfma_form<DT, 16>(a, P, u, arrivals, split, fused, lds); break;
+    case 32: rc = pq_launch_mfma_form<DT, 32>(a, P, u, arrivals, split, fused, lds); break;
+    default: rc = pq_launch_mfma_form<DT, 64>(a, P, u, arrivals, split, fused, lds); break;
   }
   if (rc || !want_sums || fused) return rc;
   // the sums from the codes just written, in a launch of their own
@@ -880,158 +1076,69 @@ static int pq_launch_mfma(const sah_pq_assign_args* a, const pq_assign_params& P
   return sah_launch_status("sah_pq_kmeans_assign(sums)");
 }
 
-struct pq_update_params {
-  const void* k; int64_t ks_b, ks_h, ks_l;
-  int Hkv, n_sub, d_sub, n_cent, key_offset;
-  float* centres;
-  long long* sums; int* counts;
-  const uint32_t* absmax_bits;
-  const int* reseed_idx;   // NULL: vector i of an empty centre is number reseed_first + g * n_cent + c of the generator
-  uint32_t reseed_seed;    // seeded with reseed_seed, modulo n_keys (torch.randint of the whole run, drawn where needed)
-  int64_t reseed_first;
-  int n_keys;
-  int clear;               // sums and counts are left zero for the next assignment
-  float* shift2;
-  float tol;
-  int* state;
-  int n_groups;
-};
-
-// One workgroup per group, a thread per centre. What bounds it is latency (a group's 18 KB): the sums of eight
-// dimensions are requested together.
-template <int DT>
-__global__ __launch_bounds__(PQ_NT) void k_pq_update(pq_update_params P) {
-  __shared__ float s_red[PQ_NT / SAH_WAVE];
-  __shared__ mt_lds s_mt;
-  if (P.state[2]) return;
-  const int tid = threadIdx.x;
-  const int g = blockIdx.x;
-  const int s = g % P.n_sub;
-  const int bh = g / P.n_sub;
-  const int hk = bh % P.Hkv;
-  const int b = bh / P.Hkv;
-  const int d_sub = P.d_sub, n_cent = P.n_cent;
-  float move = 0.f;
-  int cn = 1, ridx = 0;
-  if (tid < n_cent) {
-    cn = P.counts[(int64_t)g * n_cent + tid];
-    if (cn == 0 && P.reseed_idx) ridx = P.reseed_idx[(int64_t)g * n_cent + tid];
-  }
-  if (!P.reseed_idx && __syncthreads_or(cn == 0)) {  // rare: the generator runs only where a centre is empty
-    const int64_t first = P.reseed_first + (int64_t)g * n_cent;
-    const int64_t mine = first + (tid < n_cent ? tid : 0);
-    const int last = (int)((first + n_cent - 1) / MT_N);
-    mt_seed(s_mt, P.reseed_seed);
-    for (int blk = 0; blk <= last; ++blk) {
-      mt_next(s_mt, blk & 1);
-      if (mine / MT_N == blk) ridx = (int)(mt_temper(s_mt.st[(blk & 1) ^ 1][mine % MT_N]) % (uint32_t)P.n_keys);
-    }
-  }
-  if (tid < n_cent) {
-    const int c = tid;
-    float* cc = P.centres + ((int64_t)g * n_cent + c) * d_sub;
-    long long* ss = P.sums + ((int64_t)g * n_cent + c) * d_sub;
-    const double unscale = 1.0 / ((double)pq_sum_scale(*P.absmax_bits) * (double)(cn > 0 ? cn : 1));
-    float acc = 0.f;
-    const int64_t roff =
-        (int64_t)b * P.ks_b + (int64_t)hk * P.ks_h + (int64_t)(P.key_offset + ridx) * P.ks_l + (int64_t)s * d_sub;
-    for (int d0 = 0; d0 < d_sub; d0 += 8) {
-      long long sv[8];
-      float ov[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int d = d0 + u < d_sub ? d0 + u : d_sub - 1;
-        sv[u] = ss[d];
-        ov[u] = cc[d];
-      }
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int d = d0 + u;
-        if (d >= d_sub) break;
-        const float nv = (cn > 0) ? (float)((double)sv[u] * unscale) : sah_load<DT>(P.k, roff + d);
-        const float df = nv - ov[u];
-        acc = fmaf(df, df, acc);
-        cc[d] = nv;
-        if (P.clear) ss[d] = 0;
-      }
-    }
-    if (P.clear) P.counts[(int64_t)g * n_cent + c] = 0;
-    move = sqrtf(acc);
-  }
-  move = sah_wave_sum(move);
-  if ((tid & (SAH_WAVE - 1)) == 0) s_red[tid / SAH_WAVE] = move;
-  __syncthreads();
-  if (tid == 0) {
-    float tot = 0.f;
-    for (int i = 0; i < PQ_NT / SAH_WAVE; ++i) tot += s_red[i];
-    const float sh2 = tot * tot;
-    P.shift2[g] = sh2;
-    // the verdict's two counters only: the converged count is in before the ticket is taken, nothing else is handed over
-    if (sh2 < P.tol) atomicAdd(&P.state[0], 1);
-    sah_stores_done();
-    const int ticket = atomicAdd(&P.state[1], 1);
-    if (ticket == P.n_groups - 1) {
-      // last group of this iteration, every other has read the done flag: publish the verdict, reset the counters
-      const int conv = atomicAdd(&P.state[0], 0);
-      if (conv == P.n_groups) P.state[2] = 1;
-      P.state[0] = 0;
-      P.state[1] = 0;
-    }
-  }
-}
-
 // Start vectors of every group: number (g, c) of a seeded torch.rand in float64 picks one vector of stratum c of
-// [0, n_keys) (n_cent equal strata). One workgroup draws the whole sequence (0.4 us per 312 numbers; on the host, copy
-// included, 128 groups x 256 centres took 0.5 ms and more).
-#define PQI_NT 320
-__global__ __launch_bounds__(PQI_NT) void k_pq_start(uint32_t seed, int n_groups, int n_cent, int n_keys, double stratum, int* idx) {
-  __shared__ mt_lds S;
-  mt_seed(S, seed);
-  const int64_t total = (int64_t)n_groups * n_cent;
-  int from = 0;
-  for (int64_t first = 0; first < total; first += MT_N / 2, from ^= 1) {
-    mt_next(S, from);
-    const int64_t i = first + threadIdx.x;
-    if (threadIdx.x < MT_N / 2 && i < total) {
-      const uint32_t hi = mt_temper(S.st[from ^ 1][2 * threadIdx.x]), lo = mt_temper(S.st[from ^ 1][2 * threadIdx.x + 1]);
-      const double u = (double)((((uint64_t)hi << 32) | lo) & ((1ull << 53) - 1)) * 0x1p-53;
-      const int c = (int)(i % n_cent);
-      const long long b = (long long)floor((double)c * stratum);
-      long long e = (long long)floor((double)(c + 1) * stratum);
-      if (e > n_keys) e = n_keys;
-      const long long width = e - b > 1 ? e - b : 1;
-      const long long v = b + (long long)floor(u * (double)width);
-      idx[i] = (int)(v < n_keys - 1 ? v : n_keys - 1);
+// [0, n_keys) (n_cent equal strata). One workgroup draws the whole sequence, two words a number.
+struct pq_start_params {
+  int64_t total;  // n_groups * n_cent
+  int n_cent, n_keys;
+  double stratum;
+  int* idx;
+};
+struct pq_start_lds {
+  mts_lds mt;
+  int2 stratum[PQ_MAX_CENT];  // first vector, width
+};
+__device__ __forceinline__ void pq_start_draw(pq_start_lds& S, const mt_state& seeded, const pq_start_params& P) {
+  for (int c = threadIdx.x; c < P.n_cent; c += MTS_NT) {
+    const int b = (int)floor((double)c * P.stratum);
+    const double e_all = floor((double)(c + 1) * P.stratum);
+    const int e = e_all > (double)P.n_keys ? P.n_keys : (int)e_all;
+    S.stratum[c] = make_int2(b, e - b > 1 ? e - b : 1);
+  }
+  const int t_mod = (int)(threadIdx.x % MTS_USE) % P.n_cent, step_mod = MTS_USE % P.n_cent;
+  const int first_mod = MT_N / 2 % P.n_cent, call_mod = MTS_STEP / 2 % P.n_cent;
+  int c_first = 0;  // stratum of the first number of a call
+  mt_stream(S.mt, seeded, 2 * P.total, [&](auto&& word, int64_t first, int count, int t) {
+    int c = c_first + t_mod;
+    if (c >= P.n_cent) c -= P.n_cent;
+    for (int n = t; n < count / 2; n += MTS_USE) {
+      const uint32_t hi = mt_temper(word(2 * n)), lo = mt_temper(word(2 * n + 1));
+      const double u = fma((double)(hi & 0x1fffffu), 0x1p32, (double)lo) * 0x1p-53;  // exact: 53 bits
+      const int2 st = S.stratum[c];
+      const int v = st.x + (int)floor(u * (double)st.y);
+      P.idx[first / 2 + n] = v < P.n_keys - 1 ? v : P.n_keys - 1;
+      c += step_mod;
+      if (c >= P.n_cent) c -= P.n_cent;
     }
-  }
+    c_first += first ? call_mod : first_mod;  // (the last call's numbers need no successor)
+    if (c_first >= P.n_cent) c_first -= P.n_cent;
+  });
 }
 
-// Reseed vectors of a whole run: numbers 0 .. total - 1 of the sequence k_pq_update draws from, by one workgroup
-// (0.63 us per 624 numbers). For runs of so many numbers that the groups with an empty centre, each drawing the sequence
-// again up to its own, would take longer.
-__global__ __launch_bounds__(PQI_NT) void k_pq_reseed(uint32_t seed, int64_t total, int n_keys, int* idx) {
-  __shared__ mt_lds S;
-  mt_seed(S, seed);
-  int from = 0;
-  for (int64_t first = 0; first < total; first += MT_N, from ^= 1) {
-    mt_next(S, from);
-    for (int i = threadIdx.x; i < MT_N; i += PQI_NT)
-      if (first + i < total) idx[first + i] = (int)(mt_temper(S.st[from ^ 1][i]) % (uint32_t)n_keys);
-  }
+// Reseed vectors of a whole run: numbers 0 .. total - 1 of the sequence the update draws from, by one workgroup. For runs of
+// so many numbers that the groups with an empty centre, each drawing the sequence again up to its own, would take longer.
+__global__ __launch_bounds__(MTS_NT) void k_pq_reseed(mt_state seeded, int64_t total, int n_keys, int* idx) {
+  __shared__ mts_lds S;
+  mt_stream(S, seeded, total, [&](auto&& word, int64_t first, int count, int t) {
+    for (int i = t; i < count; i += MTS_USE) idx[first + i] = (int)(mt_temper(word(i)) % (uint32_t)n_keys);
+  });
 }
 
-// centres[g][c][:] = vector idx[g][c] of the group, as fp32
+// centres[g][c][:] = vector idx[g][c] of the group, as fp32. A workgroup per group; idx[g][0] becomes the group's arrival
+// counter (zero) of the assignments that follow.
+#define PQG_NT 1024
 template <int DT>
-__global__ __launch_bounds__(PQ_NT) void k_pq_gather(const void* k, int64_t ks_b, int64_t ks_h, int64_t ks_l, int Hkv, int n_sub,
-                                                     int d_sub, int n_cent, int key_offset, int64_t total, const int* idx,
-                                                     float* centres) {
-  const int64_t i = (int64_t)blockIdx.x * PQ_NT + threadIdx.x;
-  if (i >= total) return;
-  const int64_t gc = i / d_sub;
-  const int d = (int)(i - gc * d_sub);
-  const int g = (int)(gc / n_cent), s = g % n_sub, bh = g / n_sub;
-  centres[i] = sah_load<DT>(k, (int64_t)(bh / Hkv) * ks_b + (int64_t)(bh % Hkv) * ks_h + (int64_t)(key_offset + idx[gc]) * ks_l +
-                                   (int64_t)s * d_sub + d);
+__global__ __launch_bounds__(PQG_NT) void k_pq_gather(const void* k, int64_t ks_b, int64_t ks_h, int64_t ks_l, int Hkv, int n_sub,
+                                                      int d_sub, int n_cent, int key_offset, int* idx, float* centres) {
+  const int g = blockIdx.x, s = g % n_sub, bh = g / n_sub;
+  const int64_t base = (int64_t)(bh / Hkv) * ks_b + (int64_t)(bh % Hkv) * ks_h + (int64_t)s * d_sub;
+  int* mine = idx + (int64_t)g * n_cent;
+  for (int i = threadIdx.x; i < n_cent * d_sub; i += PQG_NT) {
+    const int c = i / d_sub, d = i - c * d_sub;
+    centres[(int64_t)g * n_cent * d_sub + i] = sah_load<DT>(k, base + (int64_t)(key_offset + mine[c]) * ks_l + d);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) mine[0] = 0;
 }
 
 struct pq_adc_params {
@@ -1381,20 +1488,20 @@ static int pq_check_common(const char* what, int B, int Hkv, int n_sub, int d_su
 // floats order like their bit patterns, so an integer atomic max does it). *out must be zero before the launch.
 // VEC elements a load: 16 bytes where the rows allow it (an element at a time, with a 64-bit division each, a 33 MB
 // cache took 72 us; its bytes take 7; with one atomic per wave 51, as here 17).
-template <int DT, int VEC>
-__global__ __launch_bounds__(PQ_NT) void k_pq_absmax(const void* k, int64_t ks_b, int64_t ks_h, int64_t ks_l, int Hkv, int D,
-                                                     int key_offset, int n_keys, uint32_t* out) {
-  const int bh = blockIdx.y;
+// share `part` of `parts` of head bh, by one workgroup of NT threads
+template <int DT, int VEC, int NT>
+__device__ __forceinline__ void pq_absmax_part(const void* k, int64_t ks_b, int64_t ks_h, int64_t ks_l, int Hkv, int D, int key_offset,
+                                               int n_keys, uint32_t* out, int bh, int part, int parts, uint32_t* s_best) {
   const int64_t base = (int64_t)(bh / Hkv) * ks_b + (int64_t)(bh % Hkv) * ks_h + (int64_t)key_offset * ks_l;
   const int upr = D / VEC;  // loads per row
   const int64_t total = (int64_t)n_keys * upr;
-  const int64_t step = (int64_t)gridDim.x * PQ_NT;
+  const int64_t step = (int64_t)parts * NT;
   uint32_t best = 0u;
   auto take = [&](uint32_t bits) {
     bits &= 0x7fffffffu;
     if (bits <= 0x7f800000u) best = bits > best ? bits : best;  // NaN is skipped
   };
-  int64_t i = (int64_t)blockIdx.x * PQ_NT + threadIdx.x;
+  int64_t i = (int64_t)part * NT + threadIdx.x;
   int64_t n = i / upr;
   int c = (int)(i - n * upr);
   const int64_t dn = step / upr;
@@ -1433,30 +1540,71 @@ __global__ __launch_bounds__(PQ_NT) void k_pq_absmax(const void* k, int64_t ks_b
     best = other > best ? other : best;
   }
   // one atomic per workgroup: all go to one address, 5 ns each (8192 of them, one per wave, took 41 us)
-  __shared__ uint32_t s_best[PQ_NT / SAH_WAVE];
   if ((threadIdx.x & (SAH_WAVE - 1)) == 0) s_best[threadIdx.x / SAH_WAVE] = best;
   __syncthreads();
   if (threadIdx.x == 0) {
 #pragma unroll
-    for (int w = 1; w < PQ_NT / SAH_WAVE; ++w) best = s_best[w] > best ? s_best[w] : best;
+    for (int w = 1; w < NT / SAH_WAVE; ++w) best = s_best[w] > best ? s_best[w] : best;
     if (best) atomicMax(out, best);
   }
 }
 
+template <int DT, int VEC>
+__global__ __launch_bounds__(PQ_NT) void k_pq_absmax(const void* k, int64_t ks_b, int64_t ks_h, int64_t ks_l, int Hkv, int D,
+                                                     int key_offset, int n_keys, uint32_t* out) {
+  __shared__ uint32_t s_best[PQ_NT / SAH_WAVE];
+  pq_absmax_part<DT, VEC, PQ_NT>(k, ks_b, ks_h, ks_l, Hkv, D, key_offset, n_keys, out, blockIdx.y, blockIdx.x, gridDim.x, s_best);
+}
+
+// What a run needs before its first assignment and what does not need each other: workgroup 0 draws the start vectors, the
+// others find the largest |element| (`parts` workgroups a head). 54 us (8 heads x 16277 keys of 128, 128 groups of 256 centres);
+// one after the other 78 and 16.
+template <int DT, int VEC>
+__global__ __launch_bounds__(MTS_NT) void k_pq_prepare(mt_state seeded, pq_start_params S, const void* k, int64_t ks_b, int64_t ks_h,
+                                                       int64_t ks_l, int Hkv, int D, int key_offset, int n_keys, uint32_t* out, int parts) {
+  __shared__ pq_start_lds s_start;
+  if (blockIdx.x == 0) {
+    pq_start_draw(s_start, seeded, S);
+    return;
+  }
+  const int w = (int)blockIdx.x - 1;
+  pq_absmax_part<DT, VEC, MTS_NT>(k, ks_b, ks_h, ks_l, Hkv, D, key_offset, n_keys, out, w / parts, w % parts, parts, s_start.mt.x);
+}
+
+// workgroups of nt threads per head, and whether the keys can be read 16 bytes at a time
+static int pq_absmax_parts(const sah_pq_absmax_args* a, int nt, bool* vec) {
+  const int v = a->dtype == SAH_F32 ? 4 : 8;
+  *vec = a->D % v == 0 && a->ks_b % v == 0 && a->ks_h % v == 0 && a->ks_l % v == 0 && (uintptr_t)a->k % 16 == 0;
+  const int64_t total = (int64_t)a->n_keys * (*vec ? a->D / v : a->D), heads = (int64_t)a->B * a->Hkv;
+  int64_t parts = (total + nt * 8 - 1) / (nt * 8);
+  const int64_t most = ((int64_t)1024 * PQ_NT / nt + heads - 1) / heads;
+  return (int)(parts < 1 ? 1 : (parts > most ? most : parts));
+}
 template <int DT>
 static void pq_absmax_launch(const sah_pq_absmax_args* a) {
   constexpr int VEC = DT == SAH_F32 ? 4 : 8;
-  const bool vec = a->D % VEC == 0 && a->ks_b % VEC == 0 && a->ks_h % VEC == 0 && a->ks_l % VEC == 0 && (uintptr_t)a->k % 16 == 0;
-  const int64_t total = (int64_t)a->n_keys * (vec ? a->D / VEC : a->D);
-  int64_t gx = (total + PQ_NT * 8 - 1) / (PQ_NT * 8);
-  const int64_t most = (1024 + (int64_t)a->B * a->Hkv - 1) / ((int64_t)a->B * a->Hkv);
-  gx = gx < 1 ? 1 : (gx > most ? most : gx);
-  dim3 g((unsigned)gx, a->B * a->Hkv), blk(PQ_NT);
+  bool vec;
+  const int parts = pq_absmax_parts(a, PQ_NT, &vec);
+  dim3 g((unsigned)parts, a->B * a->Hkv), blk(PQ_NT);
   hipStream_t st = (hipStream_t)a->stream;
   if (vec)
     hipLaunchKernelGGL((k_pq_absmax<DT, VEC>), g, blk, 0, st, a->k, a->ks_b, a->ks_h, a->ks_l, a->Hkv, a->D, a->key_offset, a->n_keys, a->absmax_bits);
   else
     hipLaunchKernelGGL((k_pq_absmax<DT, 1>), g, blk, 0, st, a->k, a->ks_b, a->ks_h, a->ks_l, a->Hkv, a->D, a->key_offset, a->n_keys, a->absmax_bits);
+}
+template <int DT>
+static void pq_prepare_launch(const sah_pq_absmax_args* a, const pq_start_params& S, uint32_t seed) {
+  constexpr int VEC = DT == SAH_F32 ? 4 : 8;
+  bool vec;
+  const int parts = pq_absmax_parts(a, MTS_NT, &vec);
+  dim3 g((unsigned)(parts * a->B * a->Hkv + 1)), blk(MTS_NT);
+  hipStream_t st = (hipStream_t)a->stream;
+  if (vec)
+    hipLaunchKernelGGL((k_pq_prepare<DT, VEC>), g, blk, 0, st, mt_seeded(seed), S, a->k, a->ks_b, a->ks_h, a->ks_l, a->Hkv, a->D, a->key_offset,
+                       a->n_keys, a->absmax_bits, parts);
+  else
+    hipLaunchKernelGGL((k_pq_prepare<DT, 1>), g, blk, 0, st, mt_seeded(seed), S, a->k, a->ks_b, a->ks_h, a->ks_l, a->Hkv, a->D, a->key_offset,
+                       a->n_keys, a->absmax_bits, parts);
 }
 
 extern "C" int sah_pq_keys_absmax(const sah_pq_absmax_args* a) {
@@ -1475,7 +1623,10 @@ extern "C" int sah_pq_keys_absmax(const sah_pq_absmax_args* a) {
   return sah_launch_status("sah_pq_keys_absmax");
 }
 
-extern "C" int sah_pq_kmeans_assign(const sah_pq_assign_args* a) {
+// sah_pq_kmeans_assign; with U and the groups' arrival counters (arrivals[g * n_cent], zero) the kernel that sums also carries
+// out the update where it can, and says so in *updated
+static int pq_assign(const sah_pq_assign_args* a, const pq_update_params* U, uint32_t* arrivals, bool* updated) {
+  if (updated) *updated = false;
   if (!a) return sah_fail(SAH_ENULL, "sah_pq_kmeans_assign: args is NULL");
   int rc = pq_check_common("sah_pq_kmeans_assign", a->B, a->Hkv, a->n_sub, a->d_sub, a->n_cent);
   if (rc) return rc;
@@ -1532,9 +1683,9 @@ extern "C" int sah_pq_kmeans_assign(const sah_pq_assign_args* a) {
   if (!a->round_dist && (wide || (a->n_keys >= 1024 && (a->d_sub == 4 || a->d_sub == 8 || a->d_sub == 16)))) {
     // Lloyd iterations over a whole context: the contraction goes to the matrix cores
     switch (a->dtype) {
-      case SAH_F32: return pq_launch_mfma<SAH_F32>(a, P);
-      case SAH_BF16: return pq_launch_mfma<SAH_BF16>(a, P);
-      case SAH_F16: return pq_launch_mfma<SAH_F16>(a, P);
+      case SAH_F32: return pq_launch_mfma<SAH_F32>(a, P, U, arrivals, updated);
+      case SAH_BF16: return pq_launch_mfma<SAH_BF16>(a, P, U, arrivals, updated);
+      case SAH_F16: return pq_launch_mfma<SAH_F16>(a, P, U, arrivals, updated);
       default: return sah_fail(SAH_EDTYPE, "sah_pq_kmeans_assign: dtype %d", a->dtype);
     }
   }
@@ -1549,6 +1700,8 @@ extern "C" int sah_pq_kmeans_assign(const sah_pq_assign_args* a) {
   }
   return sah_launch_status("sah_pq_kmeans_assign");
 }
+
+extern "C" int sah_pq_kmeans_assign(const sah_pq_assign_args* a) { return pq_assign(a, nullptr, nullptr, nullptr); }
 
 static int pq_update_launch(const pq_update_params& P, int dtype, void* stream, const char* what) {
   dim3 g(P.n_groups), blk(PQ_NT);
@@ -1594,16 +1747,20 @@ extern "C" int sah_pq_kmeans(const sah_pq_kmeans_args* a) {
                     (long long)a->code_offset, a->n_keys);
   const int n_groups = a->B * a->Hkv * a->n_sub;
   hipStream_t st = (hipStream_t)a->stream;
+  sah_pq_absmax_args m = {a->k, a->ks_b, a->ks_h, a->ks_l, a->dtype, a->B, a->Hkv, a->n_sub * a->d_sub, a->key_offset, a->n_keys,
+                          a->absmax_bits, a->stream};
   if (!a->given_start) {
     if (a->n_keys < a->n_cent) return sah_fail(SAH_EINVAL, "sah_pq_kmeans: fewer keys than centres");
-    const int64_t total = (int64_t)n_groups * a->n_cent * a->d_sub;
+    if ((int64_t)a->B * a->Hkv > 65535) return sah_fail(SAH_EINVAL, "sah_pq_kmeans: more than 65535 heads");
+    const pq_start_params sp = {(int64_t)n_groups * a->n_cent, a->n_cent, a->n_keys, (double)a->n_keys / (double)a->n_cent, a->start_idx};
     sah_timed timed("k_pq_start", a->stream);
-    hipLaunchKernelGGL(k_pq_start, dim3(1), dim3(PQI_NT), 0, st, (uint32_t)a->start_seed, n_groups, a->n_cent, a->n_keys,
-                       (double)a->n_keys / (double)a->n_cent, a->start_idx);
-    dim3 g((unsigned)((total + PQ_NT - 1) / PQ_NT)), blk(PQ_NT);
+    dim3 g(n_groups), blk(PQG_NT);
 #define SAH_PQG(DTC)                                                                                                          \
-  hipLaunchKernelGGL(k_pq_gather<DTC>, g, blk, 0, st, a->k, a->ks_b, a->ks_h, a->ks_l, a->Hkv, a->n_sub, a->d_sub, a->n_cent, \
-                     a->key_offset, total, a->start_idx, a->centres)
+  do {                                                                                                                        \
+    pq_prepare_launch<DTC>(&m, sp, (uint32_t)a->start_seed);                                                                  \
+    hipLaunchKernelGGL(k_pq_gather<DTC>, g, blk, 0, st, a->k, a->ks_b, a->ks_h, a->ks_l, a->Hkv, a->n_sub, a->d_sub, a->n_cent, \
+                       a->key_offset, a->start_idx, a->centres);                                                              \
+  } while (0)
     switch (a->dtype) {
       case SAH_F32: SAH_PQG(SAH_F32); break;
       case SAH_BF16: SAH_PQG(SAH_BF16); break;
@@ -1612,10 +1769,9 @@ extern "C" int sah_pq_kmeans(const sah_pq_kmeans_args* a) {
     }
 #undef SAH_PQG
     if ((rc = sah_launch_status("sah_pq_kmeans(start)"))) return rc;
+  } else if ((rc = sah_pq_keys_absmax(&m))) {
+    return rc;
   }
-  sah_pq_absmax_args m = {a->k, a->ks_b, a->ks_h, a->ks_l, a->dtype, a->B, a->Hkv, a->n_sub * a->d_sub, a->key_offset, a->n_keys,
-                          a->absmax_bits, a->stream};
-  if ((rc = sah_pq_keys_absmax(&m))) return rc;
   sah_pq_assign_args as = {};
   as.k = a->k; as.ks_b = a->ks_b; as.ks_h = a->ks_h; as.ks_l = a->ks_l;
   as.dtype = a->dtype; as.B = a->B; as.Hkv = a->Hkv; as.n_sub = a->n_sub; as.d_sub = a->d_sub; as.n_cent = a->n_cent;
@@ -1630,17 +1786,18 @@ extern "C" int sah_pq_kmeans(const sah_pq_kmeans_args* a) {
   const int64_t n_all = (int64_t)n_groups * a->n_cent;
   if (a->reseed_idx && a->max_iter) {
     sah_timed timed("k_pq_reseed", a->stream);
-    hipLaunchKernelGGL(k_pq_reseed, dim3(1), dim3(PQI_NT), 0, st, (uint32_t)a->reseed_seed, n_all * a->max_iter, a->n_keys,
+    hipLaunchKernelGGL(k_pq_reseed, dim3(1), dim3(MTS_NT), 0, st, mt_seeded((uint32_t)a->reseed_seed), n_all * a->max_iter, a->n_keys,
                        a->reseed_idx);
     if ((rc = sah_launch_status("sah_pq_kmeans(reseed)"))) return rc;
   }
   P.absmax_bits = a->absmax_bits;
   P.shift2 = a->shift2; P.tol = a->tol; P.state = a->state; P.n_groups = n_groups;
   for (int it = 0; it < a->max_iter; ++it) {
-    if ((rc = sah_pq_kmeans_assign(&as))) return rc;
     P.reseed_first = it * n_all;
     P.reseed_idx = a->reseed_idx ? a->reseed_idx + it * n_all : nullptr;
-    if ((rc = pq_update_launch(P, a->dtype, a->stream, "sah_pq_kmeans"))) return rc;
+    bool updated;
+    if ((rc = pq_assign(&as, &P, a->given_start ? nullptr : (uint32_t*)a->start_idx, &updated))) return rc;
+    if (!updated && (rc = pq_update_launch(P, a->dtype, a->stream, "sah_pq_kmeans"))) return rc;
   }
   return SAH_OK;
 }

@@ -112,3 +112,19 @@ def test_a_centre_that_is_not_a_number_loses_alone(cuda, dtype, d):
         c[:, at, d - 1] = float("nan")
         far[:, at] = 1e6
     assert torch.equal(_assign(N, cuda, k, 2, d, c), _assign(N, cuda, k, 2, d, far))
+
+
+# numbers drawn: the generator hands out 312 at first, then 227 at a time, to 256 threads
+@pytest.mark.parametrize("groups,n_cent", [(1, 1), (1, 256), (4, 78), (1, 227), (7, 77), (49, 11), (3, 255), (256, 3), (16, 256)])
+def test_start_vectors_are_the_seeded_stratified_draw(cuda, groups, n_cent):
+    from sparse_attention_hub_amd.sparse_attention.research_attention.maskers.fixed.implementations.utils.pq_utils import (
+        gather_sub_vectors, kmeans_keys_batched, seeded_initial_centres,
+    )
+
+    n, d = 613, 8
+    k = torch.randn(1, groups, n, d, generator=torch.Generator().manual_seed(groups)).to(torch.bfloat16)
+    codes = torch.zeros((1, groups, n, 1), dtype=torch.uint8, device=cuda)
+    centres, _ = kmeans_keys_batched(k.to(cuda), 0, 1, n_cent, 0, codes, n, seed=41)  # no iteration: the start itself
+    torch.cuda.synchronize()
+    want = gather_sub_vectors(k, 0, 1, seeded_initial_centres(groups, n, n_cent, 41, torch.device("cpu")))
+    assert torch.equal(centres.cpu().reshape(-1), want.float().reshape(-1))
