@@ -49,6 +49,19 @@ typedef struct sah_pq_kmeans_args {
 } sah_pq_kmeans_args;
 int sah_pq_kmeans(const sah_pq_kmeans_args* a);
 
+/* sah_amask_classify whose answer the host has when the call returns, without a cleared output, a copy and a wait for the
+ * stream: the kernel writes the flags into host memory, and the call watches that word (after 2 ms, behind long work of the
+ * stream, it waits for the stream instead). mask.flags is not used. scratch: two words of device memory, zero before the
+ * first call and left zero; host_word: pinned host memory the device can write, zero before the first call. Both serve one
+ * call at a time. Refused while the stream is being captured. */
+typedef struct sah_amask_read_args {
+  sah_amask_classify_args mask;
+  uint32_t* scratch;
+  uint64_t* host_word;
+  int32_t flags;  /* out */
+} sah_amask_read_args;
+int sah_amask_read(sah_amask_read_args* a);
+
 #ifdef __cplusplus
 }
 #endif

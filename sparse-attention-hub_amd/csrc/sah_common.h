@@ -423,13 +423,6 @@ __device__ __forceinline__ void sah_wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Workgroup barrier for data that passes through LDS: __syncthreads() without its wait for the wave's stores to memory.
-__device__ __forceinline__ void sah_lds_barrier() {
-#if defined(__HIP_DEVICE_COMPILE__)
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-#endif
-}
-
 // ---------------------------------------------------------------------------
 // device side: cross-lane helpers
 // ---------------------------------------------------------------------------

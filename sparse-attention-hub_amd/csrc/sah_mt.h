@@ -105,7 +105,7 @@ __device__ __forceinline__ void mt_stream(mts_lds& S, const mt_state& seeded, in
     }
     done = made;
     made += MTS_STEP;
-    sah_lds_barrier();  // (what consume stores to memory need not have arrived)
+    __syncthreads();
   }
 }
 

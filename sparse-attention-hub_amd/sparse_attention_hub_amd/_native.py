@@ -62,6 +62,7 @@ EXPECTED_SYMBOLS = (
 EXTENSION_SYMBOLS = {
     "sah_members_attention": 1,
     "sah_pq_kmeans": 1,
+    "sah_amask_read": 1,
 }
 
 
@@ -389,6 +390,10 @@ class AmaskClassifyArgs(C.Structure):
         ("flags", C.c_void_p),
         ("stream", C.c_void_p),
     ]
+
+
+class AmaskReadArgs(C.Structure):
+    _fields_ = [("mask", AmaskClassifyArgs), ("scratch", C.c_void_p), ("host_word", C.c_void_p), ("flags", C.c_int32)]
 
 
 AMASK_NONZERO, AMASK_GENERAL = 1, 2

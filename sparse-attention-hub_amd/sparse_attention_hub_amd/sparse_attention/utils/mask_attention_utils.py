@@ -90,13 +90,32 @@ def additive_mask_args(attention_mask: Optional[torch.Tensor], queries: torch.Te
     return am, am.data_ptr(), sb, sh, am.stride(2)
 
 
+class _AnswerWords(threading.local):
+    """Per thread and device: two words of device memory and one of pinned host memory, through which `sah_amask_read` answers
+    (one call of a thread at a time; the call returns with the answer, so no stream uses them afterwards)."""
+
+    def __init__(self) -> None:
+        self.words = {}
+
+
+_ANSWERS = _AnswerWords()
+
+
+def _answer_words(device: torch.device):
+    words = _ANSWERS.words.get(device.index)
+    if words is None:
+        words = _ANSWERS.words[device.index] = (torch.zeros(2, dtype=torch.int32, device=device),
+                                                torch.zeros(1, dtype=torch.int64, pin_memory=True))
+    return words
+
+
 class AdditiveMaskFacts:
     """What the additive mask of the current forward pass holds, established once per mask tensor.
 
     HuggingFace builds one mask per forward pass and hands the same tensor to every layer; for a single decode
     query of an unpadded batch its eager mask is all zeros, and adding zeros to scores and logits changes nothing
     (reference: hashattention_top_k.py:367-368, oracle_top_k.py:71-72, utils/mask_attention_utils.py:221-225).
-    `all_zero` asks the device once per tensor (one small launch and one read-back, over the mask's whole width: a
+    `all_zero` asks the device once per tensor (one small launch, answered into host memory, over the mask's whole width: a
     mask that is zero everywhere is zero on the columns of any key count) and remembers the answer for as long as
     the same, unmodified tensor keeps arriving; the tensor is kept referenced meanwhile, so its memory cannot be
     handed to another tensor that would then be mistaken for it."""
@@ -112,11 +131,12 @@ class AdditiveMaskFacts:
             return self._flags
         if am.dim() != 4 or am.stride(-1) != 1 or not am.is_cuda or am.numel() == 0:
             return N.AMASK_NONZERO | N.AMASK_GENERAL  # nothing established: every consumer reads the mask itself
-        out = torch.zeros(1, dtype=torch.int32, device=am.device)
-        N.call("sah_amask_classify", N.AmaskClassifyArgs(
+        scratch, word = _answer_words(am.device)
+        args = N.AmaskReadArgs(N.AmaskClassifyArgs(
             am.data_ptr(), am.stride(0), am.stride(1), am.stride(2), N.dtype_code(am.dtype),
-            am.shape[0], am.shape[1], am.shape[2], am.shape[3], out.data_ptr(), N.stream_ptr(am.device)))
-        self._flags = int(out.item())
+            am.shape[0], am.shape[1], am.shape[2], am.shape[3], None, N.stream_ptr(am.device)), scratch.data_ptr(), word.data_ptr())
+        N.call("sah_amask_read", args)
+        self._flags = args.flags
         self._tensor, self._version = am, am._version
         return self._flags
 

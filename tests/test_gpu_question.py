@@ -631,3 +631,40 @@ def test_captured_masked_steps_share_nothing(cuda, chain):
             side.synchronize()
             assert torch.equal(out, want)
             assert torch.equal(step(), want)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1), (1, 1, 1, 7), (3, 1, 1, 8193), (2, 1, 48, 4099), (1, 4, 700, 1025)])  # one workgroup,
+def test_what_a_mask_holds_is_read_back(cuda, dtype, shape):  # and several; rows that start at odd elements
+    from sparse_attention_hub_amd import _native as N
+    from sparse_attention_hub_amd.sparse_attention.utils.mask_attention_utils import AdditiveMaskFacts
+
+    lowest = float(torch.finfo(dtype).min)
+    B, H, L, n = shape
+    zero = torch.zeros(B, H, L, n + 3, dtype=dtype, device=cuda)[..., 1: n + 1]
+    other = torch.cuda.Stream()
+    other.wait_stream(torch.cuda.current_stream())
+    for at in ((0, 0, 0, 0), (B - 1, H - 1, L - 1, n - 1), (B // 2, H // 2, L // 2, n // 2)):
+        for value, want in ((0.0, 0), (-0.0, 0), (lowest, N.AMASK_NONZERO), (-float("inf"), N.AMASK_NONZERO),
+                            (-1.0, N.AMASK_NONZERO | N.AMASK_GENERAL), (float("nan"), N.AMASK_NONZERO | N.AMASK_GENERAL)):
+            m = zero.clone(memory_format=torch.preserve_format)
+            m[at] = value
+            other.wait_stream(torch.cuda.current_stream())
+            assert AdditiveMaskFacts().flags(m) == want, (at, value)
+            with torch.cuda.stream(other):
+                assert AdditiveMaskFacts().flags(m) == want, (at, value)
+        assert AdditiveMaskFacts().flags(zero) == 0
+
+
+def test_a_mask_is_not_read_back_under_capture(cuda):
+    from sparse_attention_hub_amd.sparse_attention.utils.mask_attention_utils import AdditiveMaskFacts
+
+    m = torch.zeros(1, 1, 1, 64, device=cuda)
+    assert AdditiveMaskFacts().flags(m) == 0
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream), torch.cuda.graph(graph, stream=stream):
+        m.add_(0.0)
+        with pytest.raises(RuntimeError, match="captured"):
+            AdditiveMaskFacts().flags(m)
+    assert AdditiveMaskFacts().flags(m) == 0
