@@ -15,8 +15,10 @@
 #include <mutex>
 
 // KEYED: the logits come from the score keys of an exact q.k scoring pass (P.score_keys); K is not read
+// Registers of the split form: five workgroups a CU (96 a lane); four for fp32, whose batch of K and V rows takes 64 of them:
+// with 96 the batch went through scratch memory (128 rows of 10400 entries of 65536 keys: 243 us, 207 so; 32 rows of 4000: 27, 24).
 template <int DT, int D, bool ROW, bool DROP, bool FULL, bool KEYED = false>
-__global__ __launch_bounds__(ROW ? ATT_ROW_NT : ATT_NT, ROW ? 1 : 5) void k_sparse_attn(att_params P) {
+__global__ __launch_bounds__(ROW ? ATT_ROW_NT : ATT_NT, ROW ? 1 : (DT == SAH_F32 ? 4 : 5)) void k_sparse_attn(att_params P) {
   sah_touch_kernargs<sizeof(att_params)>();
   constexpr int NW = (ROW ? ATT_ROW_NT : ATT_NT) / SAH_WAVE;
   __shared__ float s_m[NW];
