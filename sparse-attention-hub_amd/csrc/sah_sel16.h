@@ -553,26 +553,36 @@ __device__ __forceinline__ int sf_select_impl(sf_lds& S, unsigned char* dyn, con
     }
     int* cols = R.cols + (int64_t)r * R.cap;
     int pos = cnt0 + out_base + incl_a - mine_all;
+    // four chunks to a word of emission masks; a lane walks its own bits (chunk by chunk the walk is as long as the sum of
+    // the busiest lanes' counts: 41.3 us instead of 40.5 for the PQCache step of 128 rows of 32768 keys, 33.5 and 32.8 of 32 rows)
 #pragma unroll
-    for (int u = 0; u < NREG; ++u) {
-      const int c = c0 + u;
-      if (c < c1) {
-        uint32_t em = (em_all[u >> 2] >> (8 * (u & 3))) & 0xffu;
-        const int col0 = c * SF_CHUNK + lane * 8 + col_offset;
-        if (em && to_memory && write_bitmap) {
-          atomicOr(&s_bm[col0 >> 5], em << (col0 & 31));
-          if ((col0 & 31) > 24) atomicOr(&s_bm[(col0 >> 5) + 1], em >> (32 - (col0 & 31)));
-        }
-        const bool my_chunk = c % parts == part;
-        while (em) {
-          const int t = __builtin_ctz(em);
-          em &= em - 1;
-          if (pos < R.cap) {
-            s_cols[pos] = col0 + t;
-            if (my_chunk) cols[pos] = col0 + t;
+    for (int q = 0; q < (NREG + 3) / 4; ++q) {
+      const int cq = c0 + 4 * q;
+      uint32_t here = 0;  // bits of the chunks this part writes to the row in memory
+#pragma unroll
+      for (int u = 0; u < 4; ++u) here |= (cq + u) % parts == part ? 0xffu << (8 * u) : 0u;
+      uint32_t em = em_all[q];
+      if (to_memory && write_bitmap) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const uint32_t e = (em >> (8 * u)) & 0xffu;
+          const int col0 = (cq + u) * SF_CHUNK + lane * 8 + col_offset;
+          if (e) {
+            atomicOr(&s_bm[col0 >> 5], e << (col0 & 31));
+            if ((col0 & 31) > 24) atomicOr(&s_bm[(col0 >> 5) + 1], e >> (32 - (col0 & 31)));
           }
-          ++pos;
         }
+      }
+      const int col_q = cq * SF_CHUNK + lane * 8 + col_offset;
+      while (em) {
+        const int bit = __builtin_ctz(em);
+        em &= em - 1;
+        if (pos < R.cap) {
+          const int col = col_q + (bit >> 3) * SF_CHUNK + (bit & 7);
+          s_cols[pos] = col;
+          if ((here >> bit) & 1u) cols[pos] = col;
+        }
+        ++pos;
       }
     }
     if (to_memory && tid == 0) R.cnt[r] = cnt0 + total;
