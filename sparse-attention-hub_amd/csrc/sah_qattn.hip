@@ -3,7 +3,7 @@
 // In a question pass every KV head has G x Lq mask rows, each with its own columns. Gathering them row by row
 // (k_sparse_attn) reads K and V once per entry: 1536 rows of 2278 entries, head_dim 128, are 1.8 GB through the caches,
 // 195 us. Together the rows of a head touch nearly every key, so here the whole of K and V passes once per 128 (or 64)
-// rows, the products run dense on the matrix cores and the rows' bitmaps decide which entries count: 63 us (74 with the
+// rows, the products run dense on the matrix cores and the rows' bitmaps decide which entries count: 63 us (64 with the
 // causal mask) and 9 for the merge. Work grows with rows x keys instead of rows x entries: see members_attention_pays().
 //
 // A workgroup: 4 waves over stages of 64 keys, K and V staged in LDS by loads that write there themselves (two buffers,
@@ -30,6 +30,7 @@
 typedef uint32_t qa_u4 __attribute__((ext_vector_type(4)));
 typedef uint32_t qa_u2 __attribute__((ext_vector_type(2)));
 typedef qa_u2 qa_u2_any __attribute__((aligned(2)));  // 8 bytes at an address that is only element aligned
+typedef qa_u4 qa_u4_any __attribute__((aligned(2)));
 typedef qa_u2 qa_u2_word __attribute__((aligned(4)));
 
 struct qa_params {
@@ -143,33 +144,59 @@ __global__ __launch_bounds__(QA_NT, 2) void k_members_attn_mfma(att_params P, qa
       vo[u] = (uint32_t)src * (uint32_t)P.vs_l * 2u + 16u * (lpos ^ (4 * ((key >> SH) & (D / 32 - 1))));
     }
   };
-  // the bits and the mask of a stage's tiles (this wave's), requested ahead of the rows: they are waited for first
+  // the bits and the mask of a stage's tiles (this wave's), requested before they are used
   constexpr int TW = KW == 1 ? 2 : 1;  // tiles of a stage per wave
   uint32_t bits[TW];
-  qa_u2 mv[AM ? TW : 1][4];
-  auto fetch_bits = [&](int st) {
+  auto fetch_bits = [&](int st) __attribute__((always_inline)) {
 #pragma unroll
     for (int t = 0; t < TW; ++t) {
       const int wi = 2 * st + (KW == 1 ? t : kw);
       bits[t] = DENSE ? sah_range_bits(wi, 0, P.Lk) : (wi < P.rows.n_words ? bm[wi] : 0u);
-      if (AM) {
-        const int key0 = wi * 32;
-        if (key0 + 32 <= P.Lk) {  // uniform
+    }
+  };
+  // Whether a tile's mask is all zeros, as most are, is asked in whole lines: four lanes take the 64 bytes of a row, an
+  // instruction 16 rows. A lane's own elements (16 bytes a row and instruction: four times the cache lines, 1536 rows x 32768
+  // keys under the causal mask 72 us instead of 64) are fetched where that answer is no, and ahead of their use once it has
+  // been no in the stage before (a bias on every key: 17 us more than the causal mask).
+  qa_u4 mv[AM ? TW : 1][2];  // lines of rows lane / 4 and 16 + lane / 4, or (own, uniform) this lane's elements
+  bool own = false;
+  const uint16_t* az[2] = {nullptr, nullptr};
+  if (AM) {
 #pragma unroll
-          for (int q4 = 0; q4 < 4; ++q4) mv[t][q4] = *(const qa_u2_any*)(am + key0 + 8 * q4);
-        } else {
+    for (int i = 0; i < 2; ++i) {
+      const int vz_own = (rt * RW + rw) * 32 + 16 * i + (lane >> 2);
+      const int vz = vz_own < nvec ? vz_own : nvec - 1;
+      az[i] = (const uint16_t*)P.amask + (int64_t)b * P.ms_b + (int64_t)(hk * G + vz / P.Lq) * P.ms_h + (int64_t)(vz % P.Lq) * P.ms_l + 8 * (lane & 3);
+    }
+  }
+  auto fetch_own = [&](int wi, qa_u4 (&m4)[2]) __attribute__((always_inline)) {
+    const int key0 = wi * 32;
+    qa_u2 m[4];
+    if (key0 + 32 <= P.Lk) {  // uniform
 #pragma unroll
-          for (int q4 = 0; q4 < 4; ++q4) {
-            uint32_t two[2] = {0u, 0u};
+      for (int q4 = 0; q4 < 4; ++q4) m[q4] = *(const qa_u2_any*)(am + key0 + 8 * q4);
+    } else {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-              const int kk = key0 + 8 * q4 + e;
-              if (kk + 4 * g < P.Lk) two[e >> 1] |= (uint32_t)am[kk] << (16 * (e & 1));
-            }
-            mv[t][q4] = qa_u2{two[0], two[1]};
-          }
+      for (int q4 = 0; q4 < 4; ++q4) {
+        uint32_t two[2] = {0u, 0u};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int kk = key0 + 8 * q4 + e;
+          if (kk + 4 * g < P.Lk) two[e >> 1] |= (uint32_t)am[kk] << (16 * (e & 1));
         }
+        m[q4] = qa_u2{two[0], two[1]};
       }
+    }
+    m4[0] = qa_u4{m[0].x, m[0].y, m[1].x, m[1].y};
+    m4[1] = qa_u4{m[2].x, m[2].y, m[3].x, m[3].y};
+  };
+  auto fetch_mask = [&](int st, int t) __attribute__((always_inline)) {
+    const int wi = 2 * st + (KW == 1 ? t : kw);
+    if (own) {
+      fetch_own(wi, mv[t]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) mv[t][i] = *(const qa_u4_any*)(az[i] + wi * 32);
     }
   };
   auto fetch = [&](int st, int buf) __attribute__((always_inline)) {
@@ -200,7 +227,8 @@ __global__ __launch_bounds__(QA_NT, 2) void k_members_attn_mfma(att_params P, qa
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[t][e] = 0.f;
 
-  auto tile = [&](int buf, int t32, uint32_t word, const qa_u2 (&am16)[4]) __attribute__((always_inline)) {
+  // biased: the tile's mask is not all zeros (uniform)
+  auto tile = [&](int buf, int t32, uint32_t word, bool biased, const qa_u4 (&am16)[2]) __attribute__((always_inline)) {
     if (__ballot(word != 0u) == 0) return;  // no row of this wave has a column here
     // element e of the product is key 8 (e / 4) + 4 g + e % 4 of the tile; it starts at 0 or, where the row does not hold
     // the key, at -inf (four elements per table entry)
@@ -215,16 +243,11 @@ __global__ __launch_bounds__(QA_NT, 2) void k_members_attn_mfma(att_params P, qa
 #pragma unroll
     for (int st = 0; st < KS; ++st) s = sah_mfma_32x32x16<DT>(*(const uint4*)(kp + (k_from ^ (16 * st))), qf[st], s);
     // most tiles of a mask are zeros: the maximum is then kept in the mask's scale, the products stay as they are
-    bool biased = false;  // uniform
     if (AM) {
-      uint32_t any = 0u;
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) any |= am16[q4].x | am16[q4].y;
-      biased = __ballot((any & 0x7fff7fffu) != 0u) != 0;
       if (biased) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
-          const uint32_t two = am16[e >> 2][(e >> 1) & 1];
+          const uint32_t two = am16[e >> 3][(e >> 1) & 3];
           float a4;
           if (DT == SAH_BF16) a4 = sah_bits_to_float((e & 1) ? (two & 0xffff0000u) : (two << 16));
           else a4 = sah_f16_to_float((uint16_t)(two >> (16 * (e & 1))));
@@ -301,21 +324,37 @@ __global__ __launch_bounds__(QA_NT, 2) void k_members_attn_mfma(att_params P, qa
   };
   auto stage = [&](int buf, int st) __attribute__((always_inline)) {  // buf: a constant in the loop below, LDS offsets are immediates
     uint32_t w[TW];
-    qa_u2 am_now[AM ? TW : 1][4];
+    bool biased[TW];  // uniform: the tile's mask is not all zeros
+    bool any_biased = false;
 #pragma unroll
     for (int t = 0; t < TW; ++t) {
       w[t] = bits[t];
-      if (AM)
+      biased[t] = false;
+      if (AM) {
+        uint32_t any = 0u;
 #pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4) am_now[t][q4] = mv[t][q4];
+        for (int i = 0; i < 2; ++i) any |= mv[t][i].x | mv[t][i].y | mv[t][i].z | mv[t][i].w;
+        biased[t] = __ballot((any & 0x7fff7fffu) != 0u) != 0;
+        any_biased = any_biased || biased[t];
+      }
     }
-    if (st + 1 < st1) {
+    const bool was_own = own;
+    const bool more = st + 1 < st1;
+    if (more) {
       fetch_bits(st + 1);
+      own = any_biased || (st + 2) * QA_STAGE > P.Lk;  // the stage in which the mask's rows end goes by elements
       fetch(st + 1, buf ^ 1);  // the other buffer: read for the last time before the previous barrier
     }
-    if (rows_live) {
 #pragma unroll
-      for (int t = 0; t < TW; ++t) tile(buf, KW == 1 ? t : kw, w[t], am_now[AM ? t : 0]);
+    for (int t = 0; t < TW; ++t) {
+      qa_u4 am_now[2];
+      if (AM) {
+        am_now[0] = mv[t][0];
+        am_now[1] = mv[t][1];
+        if (biased[t] && !was_own) fetch_own(2 * st + (KW == 1 ? t : kw), am_now);
+        if (more) fetch_mask(st + 1, t);
+      }
+      if (rows_live) tile(buf, KW == 1 ? t : kw, w[t], biased[t], am_now);
     }
     sah_stores_done();  // this wave's loads into LDS have landed
     __syncthreads();
@@ -324,6 +363,11 @@ __global__ __launch_bounds__(QA_NT, 2) void k_members_attn_mfma(att_params P, qa
   if (tid < 16) s_seed[tid] = make_float4(tid & 1 ? 0.f : -INFINITY, tid & 2 ? 0.f : -INFINITY, tid & 4 ? 0.f : -INFINITY, tid & 8 ? 0.f : -INFINITY);
   offsets(QA_STAGE);
   fetch_bits(st0);
+  if (AM) {
+    own = (st0 + 1) * QA_STAGE > P.Lk;
+#pragma unroll
+    for (int t = 0; t < TW; ++t) fetch_mask(st0, t);
+  }
   fetch(st0, 0);  // every split has at least one stage
   sah_stores_done();
   __syncthreads();

@@ -143,6 +143,50 @@ def test_attention_of_many_query_vectors(cuda, dtype, kind, shape, density):
     assert worst <= 1.0, worst
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("heads", [False, True])  # a mask for all heads, or one for each
+@pytest.mark.parametrize("pattern", ["lone", "runs"])  # every third 32-key tile with one element in one row; six tiles of eight
+@pytest.mark.parametrize("shape,pad", [((2, 8, 2, 33, 1025, 128), 0), ((2, 8, 2, 40, 2047, 64), 1), ((4, 8, 2, 32, 1024, 128), 0)])
+def test_attention_under_a_mask_of_few_tiles(cuda, dtype, heads, pattern, shape, pad):
+    """Whether a tile's mask is all zeros is asked in whole lines, the elements come behind that answer: every row and place of
+    a tile once, rows at odd elements, -0 in place of 0. Bound as above."""
+    import sparse_attention_hub_amd.sparse_attention as sa
+    from sparse_attention_hub_amd import _native as N
+    from sparse_attention_hub_amd.sparse_attention.utils.mask_attention_utils import get_masked_attention_output
+
+    B, Hq, Hkv, Lq, Lk, D = shape
+    q, k, v = make_qkv(B, Hq, Hkv, Lq, Lk, D, dtype, seed=4, device=cuda)
+    am = torch.zeros(B, Hq if heads else 1, Lq, Lk + pad, dtype=dtype)
+    am[..., 1::2] = -0.0
+    for t in range((Lk + 31) // 32):
+        if pattern == "lone" and t % 3 == 1:
+            am[:, :, (5 * t) % Lq, min(32 * t + (11 * t) % 32, Lk - 1)] = 2.0
+        if pattern == "runs" and t % 8 < 6:
+            am[:, :, :, 32 * t:32 * t + 32] += torch.linspace(-2.0, 2.0, Lq).view(1, 1, -1, 1).to(dtype)
+    am = am.to(cuda)[..., :Lk]
+    g = torch.Generator().manual_seed(2)
+    member = torch.rand(B, Hq, Lq, Lk, generator=g) < 0.4
+    member[..., 0] = True
+    mask = sa.Mask.create_mask_from_dense_mask((B, Hq, Lq, Lk), member.to(dtype).to(cuda), dtype)
+    N.timing_enable(True)
+    out = get_masked_attention_output(None, q, k, v, am, None, D ** -0.5, 0.0, mask)
+    torch.cuda.synchronize()
+    assert "k_members_attn_mfma" in launched(N)
+
+    G = Hq // Hkv
+    qq, kk, vv = q.double().cpu(), k.double().cpu().repeat_interleave(G, 1), v.double().cpu().repeat_interleave(G, 1)
+    z = (qq @ kk.transpose(-1, -2) * D ** -0.5 + am.double().cpu()).masked_fill(~member, -float("inf"))
+    p = torch.softmax(z, -1)
+    ref = (p @ vv).transpose(1, 2)
+    mass = (p @ vv.abs()).transpose(1, 2)
+    half = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    logit = D * 2.0 ** -23 * float((qq.abs() @ kk.abs().transpose(-1, -2)).max()) * D ** -0.5
+    tiny = 2.0 ** -25 if dtype == torch.float16 else 0.0
+    bound = half * ref.abs() * 1.01 + (2.0 ** -19 + 2 * logit) * mass + tiny
+    worst = float(((out.double().cpu() - ref).abs() / bound).max())
+    assert worst <= 1.0, worst
+
+
 @pytest.mark.parametrize("chain", ["oracle", "hash"])
 @pytest.mark.parametrize("shape,heavy,dense", [  # one round of rows, and a share of a round too many; rows and entries enough
     ((1, 8, 2, 32, 8192, 128), 250, False), ((1, 8, 2, 48, 2048, 128), 60, False), ((2, 32, 8, 40, 4096, 128), 400, True)])
