@@ -344,9 +344,10 @@ __global__ __launch_bounds__(QM_NT, 2) void k_qk_scores_mfma(qk_params P, int ch
       *(sah_u4*)&s_q[buf][(idx / (D / 8)) * QP + (idx % (D / 8)) * 8] = qr[u];
     }
     if (tid < QM_VECS) {
-      const int v = c * QM_VECS + tid;
+      const int v_own = c * QM_VECS + tid;
+      const int v = v_own < nvec ? v_own : nvec - 1;
       const int h = hk * G + v / P.Lq, qi = v % P.Lq;
-      s_row[buf][tid] = v < nvec ? (b * P.Hq + h) * P.Lq + qi : -1;
+      s_row[buf][tid] = v_own < nvec ? (b * P.Hq + h) * P.Lq + qi : -1;
       if (AM) s_moff[buf][tid] = (int64_t)b * P.ms_b + (int64_t)h * P.ms_h + (int64_t)qi * P.ms_l;
     }
   };
@@ -372,6 +373,25 @@ __global__ __launch_bounds__(QM_NT, 2) void k_qk_scores_mfma(qk_params P, int ch
     if (more) fetch(c + 1);
     const int n_vt = nvec - c * QM_VECS > 32 ? 2 : 1;
     for (int vt = 0; vt < n_vt; ++vt) {
+      const int k8 = (lane & 7) * 8;  // eight keys of a row per lane, eight rows per load of the mask and per store
+      const int j = j0 + k8;
+      // the mask, under way while the products are computed: asked for at its use, each of the four loads waited for all stores
+      // before it
+      sah_u4 mv[AM ? 4 : 1];
+      if (AM) {
+#pragma unroll
+        for (int it = 0; it < 4; ++it) {
+          const uint16_t* mp = (const uint16_t*)P.amask + s_moff[buf][vt * 32 + it * 8 + (lane >> 3)] + j;
+          if (j0 + QM_KEYS <= P.Lk) {  // uniform
+            mv[it] = *(const sah_u4_any*)mp;
+          } else {
+            mv[it] = sah_u4{0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int t = 0; t < 8; ++t)
+              if (j + t < P.Lk) mv[it][t >> 1] |= (uint32_t)mp[t] << (16 * (t & 1));
+          }
+        }
+      }
       sah_f32x16 acc0, acc1;
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc0[v] = acc1[v] = 0.f;
@@ -390,9 +410,6 @@ __global__ __launch_bounds__(QM_NT, 2) void k_qk_scores_mfma(qk_params P, int ch
         *(uint2*)(orow + 32 + 8 * q4) = make_uint2(sah_pack2_hw<DT>(acc1[4 * q4], acc1[4 * q4 + 1]), sah_pack2_hw<DT>(acc1[4 * q4 + 2], acc1[4 * q4 + 3]));
       }
       sah_wave_lds_sync();
-      // eight keys of a row per lane, eight rows per store
-      const int k8 = (lane & 7) * 8;
-      const int j = j0 + k8;
 #pragma unroll
       for (int it = 0; it < 4; ++it) {
         const int rl = it * 8 + (lane >> 3);
@@ -401,16 +418,7 @@ __global__ __launch_bounds__(QM_NT, 2) void k_qk_scores_mfma(qk_params P, int ch
         uint32_t w[4] = {sc.x, sc.y, sc.z, sc.w};
         const bool whole = row >= 0 && j + 8 <= P.Lk;
         if (AM) {
-          const uint16_t* mp = (const uint16_t*)P.amask + s_moff[buf][vt * 32 + rl] + j;
-          uint32_t m[4] = {0u, 0u, 0u, 0u};
-          if (whole) {
-            const sah_u4 mv = *(const sah_u4_any*)mp;
-            m[0] = mv.x; m[1] = mv.y; m[2] = mv.z; m[3] = mv.w;
-          } else if (row >= 0) {
-#pragma unroll
-            for (int t = 0; t < 8; ++t)
-              if (j + t < P.Lk) m[t >> 1] |= (uint32_t)mp[t] << (16 * (t & 1));
-          }
+          const sah_u4 m = mv[it];
           if (__ballot((m[0] | m[1] | m[2] | m[3]) != 0)) {  // most of a mask is zeros: nothing to add, nothing to round
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
