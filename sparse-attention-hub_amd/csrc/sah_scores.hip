@@ -277,7 +277,8 @@ __global__ __launch_bounds__(SC_NT) void k_qk_scores(qk_params P) {
 // The kernel above streams K once per four query vectors: at 192 vectors (48 queries, 4 heads a group) K passes 48 times
 // and the vector unit does the dot products (1536 rows x 32768 keys, head_dim 128: 520 us). Here K passes once: a wave
 // keeps 64 keys as matrix operands in registers for the whole kernel, the query vectors come by in chunks of 64 through
-// LDS (two buffers, one barrier per chunk), S^T = K Q^T in 32x32x16 steps: 44 us, 47 with the causal mask, 57 with the
+// LDS (two buffers, one barrier per chunk), S^T = K Q^T in 32x32x16 steps: 41 us with the causal mask (42 while a mask row per
+// vector in LDS left room for two workgroups a CU instead of three; 47 with the mask asked for at its use), 57 with the
 // remainders of the scores beside the keys. What bounds it
 // is memory: 67 MB of K in and 100 MB of keys out take 35 us at the rate of a large copy; chunks of 32 vectors and three
 // or four waves per SIMD change nothing. The accumulator has four consecutive keys of one vector in a lane; rounded to the storage type they cross the
@@ -308,7 +309,6 @@ __global__ __launch_bounds__(QM_NT, 2) void k_qk_scores_mfma(qk_params P, int ch
   constexpr int UPT = QM_VECS * (D / 8) / QM_NT;  // 16-byte units of a chunk per thread
   __shared__ uint16_t s_q[2][QM_VECS * QP];
   __shared__ uint16_t s_o[QM_NW][32 * OP];
-  __shared__ int s_row[2][QM_VECS];        // mask row of a vector, -1 beyond the last
   __shared__ int64_t s_moff[2][AM ? QM_VECS : 1];
   const int tid = threadIdx.x;
   const int lane = tid & (SAH_WAVE - 1);
@@ -323,6 +323,7 @@ __global__ __launch_bounds__(QM_NT, 2) void k_qk_scores_mfma(qk_params P, int ch
   const int c0 = blockIdx.z * chunks_per_wg;
   const int c1 = c0 + chunks_per_wg < n_chunks ? c0 + chunks_per_wg : n_chunks;
   if (c0 >= c1) return;
+  const int row0 = (b * P.Hq + hk * G) * P.Lq;  // mask row of the head's first vector; the others follow
 
   // a chunk's query vectors on their way to LDS; vectors beyond the last repeat it and are never stored
   sah_u4 qr[UPT];
@@ -343,12 +344,11 @@ __global__ __launch_bounds__(QM_NT, 2) void k_qk_scores_mfma(qk_params P, int ch
       const int idx = tid + u * QM_NT;
       *(sah_u4*)&s_q[buf][(idx / (D / 8)) * QP + (idx % (D / 8)) * 8] = qr[u];
     }
-    if (tid < QM_VECS) {
+    if (AM && tid < QM_VECS) {
       const int v_own = c * QM_VECS + tid;
       const int v = v_own < nvec ? v_own : nvec - 1;
       const int h = hk * G + v / P.Lq, qi = v % P.Lq;
-      s_row[buf][tid] = v_own < nvec ? (b * P.Hq + h) * P.Lq + qi : -1;
-      if (AM) s_moff[buf][tid] = (int64_t)b * P.ms_b + (int64_t)h * P.ms_h + (int64_t)qi * P.ms_l;
+      s_moff[buf][tid] = (int64_t)b * P.ms_b + (int64_t)h * P.ms_h + (int64_t)qi * P.ms_l;
     }
   };
 
@@ -414,7 +414,8 @@ __global__ __launch_bounds__(QM_NT, 2) void k_qk_scores_mfma(qk_params P, int ch
       for (int it = 0; it < 4; ++it) {
         const int rl = it * 8 + (lane >> 3);
         const uint4 sc = *(const uint4*)&s_o[wave][rl * OP + k8];
-        const int row = s_row[buf][vt * 32 + rl];
+        const int v = c * QM_VECS + vt * 32 + rl;
+          const int row = v < nvec ? row0 + v : -1;
         uint32_t w[4] = {sc.x, sc.y, sc.z, sc.w};
         const bool whole = row >= 0 && j + 8 <= P.Lk;
         if (AM) {
@@ -459,7 +460,8 @@ __global__ __launch_bounds__(QM_NT, 2) void k_qk_scores_mfma(qk_params P, int ch
         for (int it = 0; it < 4; ++it) {
           const int rl = it * 8 + (lane >> 3);
           const uint4 rm = *(const uint4*)&s_o[wave][rl * OP + k8];
-          const int row = s_row[buf][vt * 32 + rl];
+          const int v = c * QM_VECS + vt * 32 + rl;
+          const int row = v < nvec ? row0 + v : -1;
           uint16_t* rout = (uint16_t*)P.resid_out + (int64_t)row * P.key_pitch + j;
           if (row >= 0 && j + 8 <= P.Lk) {
             *(uint4*)rout = rm;
