@@ -596,7 +596,7 @@ __global__ __launch_bounds__(PQM_NT, KS <= 16 ? 4 : 2) void k_pq_assign_mfma(pq_
   const uint32_t absmax = SUMS ? *P.absmax_bits : 0u;
   const float sum_scale = SUMS ? pq_sum_scale(absmax) : 1.f;
   const double sum_scale_d = (double)sum_scale;
-  const bool all_finite = absmax < 0x7f800000u;
+  const bool no_inf = absmax < 0x7f800000u;
 
   // The centres pass once through LDS (in the place of the sums, which fit them) on their way to operands and norms: one
   // round trip to memory instead of one per operand element of a thread.
@@ -924,7 +924,8 @@ __global__ __launch_bounds__(PQM_NT, KS <= 16 ? 4 : 2) void k_pq_assign_mfma(pq_
               }
             }
           };
-          if (all_finite) add_all([&](long long* p, float x) { pq_sum_add_finite(p, x, sum_scale_d); });  // uniform
+          // uniform; the largest |element| passes over NaN, but a key that holds one has had its tile evaluated again
+          if (no_inf && !again) add_all([&](long long* p, float x) { pq_sum_add_finite(p, x, sum_scale_d); });
           else add_all([&](long long* p, float x) { pq_sum_add(p, x, sum_scale); });
         } else {
 #pragma unroll

@@ -61,8 +61,9 @@ def test_assignment(cuda, dtype, shape, sums):
         assert torch.equal(C.cpu(), torch.zeros_like(C.cpu()).scatter_add_(1, got, torch.ones_like(got, dtype=torch.int32)))
 
 
-def _assign(N, dev, k, n_sub, d, c):
-    """Codes (heads, keys, sub-vectors) of keys (1, H, n, .) against centres (H n_sub, n_cent, d)."""
+def _assign(N, dev, k, n_sub, d, c, top=None):
+    """Codes (heads, keys, sub-vectors) of keys (1, H, n, .) against centres (H n_sub, n_cent, d); with the largest |element|
+    `top` also the centres' sums and counts."""
     H, n = k.shape[1], k.shape[2]
     codes = torch.full((H, n, n_sub), 255, dtype=torch.uint8, device=dev)
     flag = torch.zeros(1, dtype=torch.int32, device=dev)
@@ -71,9 +72,13 @@ def _assign(N, dev, k, n_sub, d, c):
     a.B, a.Hkv, a.n_sub, a.d_sub, a.n_cent, a.key_offset, a.n_keys = 1, H, n_sub, d, c.shape[1], 0, n
     a.centres = c.data_ptr(); a.codes = codes.data_ptr(); a.code_pitch = n; a.code_offset = 0
     a.skip_flag = flag.data_ptr(); a.stream = N.stream_ptr(dev)
+    if top is not None:
+        S = torch.zeros(c.shape, dtype=torch.int64, device=dev)
+        C = torch.zeros(c.shape[:2], dtype=torch.int32, device=dev)
+        a.sums = S.data_ptr(); a.counts = C.data_ptr(); a.absmax_bits = top.data_ptr()
     N.call("sah_pq_kmeans_assign", a)
     torch.cuda.synchronize()
-    return codes.cpu()
+    return codes.cpu() if top is None else (codes.cpu(), S.cpu(), C.cpu())
 
 
 @pytest.mark.parametrize("d,n_sub,n_cent", [(8, 16, 256), (8, 2, 33), (16, 4, 128), (32, 2, 64), (64, 2, 64), (128, 1, 65)])
@@ -96,6 +101,39 @@ def test_the_split_form_gives_the_codes_of_the_fp32_form(cuda, d, n_sub, n_cent)
     wide = torch.zeros(1, H, n, n_sub * d + 4, dtype=torch.bfloat16, device=cuda)
     wide[..., : n_sub * d] = k
     assert torch.equal(_assign(N, cuda, k, n_sub, d, c), _assign(N, cuda, wide[..., : n_sub * d], n_sub, d, c))
+
+
+@pytest.mark.parametrize("d,n_sub,n_cent", [(8, 2, 64), (16, 2, 33), (64, 2, 64), (128, 1, 256)])  # the last: sums apart
+def test_an_element_that_is_not_a_number_adds_nothing(cuda, d, n_sub, n_cent):
+    """NaN as the only values that are not finite, which the largest |element| passes over: it counts as 0 in its centre's
+    sums in the split form, the fp32 form and the launch of its own, and a whole run's centres are the same in both forms."""
+    from sparse_attention_hub_amd import _native as N
+    from sparse_attention_hub_amd.sparse_attention.research_attention.maskers.fixed.implementations.utils.pq_utils import kmeans_keys_batched
+
+    n, H = 1500, 2
+    g = torch.Generator().manual_seed(d)
+    k = torch.randn(1, H, n, n_sub * d, generator=g)
+    k[0, 0, 300, 3], k[0, 1, 301, 0], k[0, 1, 1499, d - 1] = float("nan"), float("nan"), float("nan")
+    k[0, 0, 700:732, :d] = float("nan")
+    k = k.bfloat16()
+    wide = torch.zeros(1, H, n, n_sub * d + 4, dtype=torch.bfloat16, device=cuda)
+    forms = (k.to(cuda), wide[..., : n_sub * d].copy_(k))
+    c = torch.randn(H * n_sub, n_cent, d, generator=g).to(cuda)
+    x = torch.nan_to_num(k.view(H, n, n_sub, d).permute(0, 2, 1, 3).reshape(-1, n, d).double())
+    top = x.abs().max().float().view(1)
+    fixed = torch.round(x * 2.0 ** (40 - math.frexp(float(top))[1])).to(torch.int64)  # exact: a power of two and 8 bits
+    for form in forms:
+        codes, S, C = _assign(N, cuda, form, n_sub, d, c, top.to(cuda))
+        at = codes.permute(0, 2, 1).reshape(-1, n).long()
+        assert torch.equal(S, torch.zeros_like(S).scatter_add_(1, at.unsqueeze(-1).expand(-1, -1, d), fixed))
+        assert torch.equal(C, torch.zeros_like(C).scatter_add_(1, at, torch.ones_like(at, dtype=torch.int32)))
+    runs = []
+    for form in forms:
+        codes = torch.zeros((1, H, n, n_sub), dtype=torch.uint8, device=cuda)
+        centres, _ = kmeans_keys_batched(form, 0, n_sub, n_cent, 4, codes, n, seed=41)
+        torch.cuda.synchronize()
+        runs.append((centres.cpu(), codes.cpu()))
+    assert torch.equal(torch.nan_to_num(runs[0][0], nan=1e30), torch.nan_to_num(runs[1][0], nan=1e30)) and torch.equal(runs[0][1], runs[1][1])
 
 
 @pytest.mark.parametrize("d", [4, 8, 16, 64])
