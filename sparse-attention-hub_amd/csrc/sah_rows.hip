@@ -455,6 +455,7 @@ __global__ __launch_bounds__(AMR_NT) void k_amask_read(const void* amask, int64_
     if (!sah_last_arrival(scratch + 1, gridDim.x)) return;
     f = sah_agent_load(scratch);
     sah_agent_store(scratch, 0u);
+    sah_stores_done();  // both words are zero before the host knows: its next call may come by another stream
   }
 #if defined(__HIP_DEVICE_COMPILE__)
   __hip_atomic_store(host_word, (uint64_t)seq << 32 | f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);

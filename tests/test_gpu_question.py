@@ -700,6 +700,25 @@ def test_what_a_mask_holds_is_read_back(cuda, dtype, shape):  # and several; row
         assert AdditiveMaskFacts().flags(zero) == 0
 
 
+def test_the_next_mask_may_be_read_by_another_stream(cuda):
+    """The device words an answer went through are zero when the call returns, not only when its kernel has ended: the
+    thread's next question uses them from whatever stream it comes."""
+    from sparse_attention_hub_amd import _native as N
+    from sparse_attention_hub_amd.sparse_attention.utils import mask_attention_utils as U
+
+    masks = [torch.zeros(1, 1, 64, 8192, device=cuda) for _ in range(2)]  # many workgroups
+    masks[1][0, 0, 63, 8191] = -1.0
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    for s in streams:
+        s.wait_stream(torch.cuda.current_stream())
+    for i in range(60):
+        with torch.cuda.stream(streams[i % 3]):
+            assert U.AdditiveMaskFacts().flags(masks[i % 2]) == (i % 2) * (N.AMASK_NONZERO | N.AMASK_GENERAL)
+        if i % 5 == 0:
+            with torch.cuda.stream(streams[(i + 1) % 3]):
+                assert U._ANSWERS.words[cuda.index or 0][0].tolist() == [0, 0]
+
+
 def test_a_mask_is_not_read_back_under_capture(cuda):
     from sparse_attention_hub_amd.sparse_attention.utils.mask_attention_utils import AdditiveMaskFacts
 
