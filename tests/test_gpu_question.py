@@ -731,3 +731,36 @@ def test_a_mask_is_not_read_back_under_capture(cuda):
         with pytest.raises(RuntimeError, match="captured"):
             AdditiveMaskFacts().flags(m)
     assert AdditiveMaskFacts().flags(m) == 0
+
+
+def test_a_first_question_under_capture_leaves_nothing_behind(cuda):
+    """A thread whose first question comes under capture is refused before it has words to be answered through: the ones it
+    makes afterwards belong to no graph, are clear, and a replay does not touch them."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    from sparse_attention_hub_amd import _native as N
+    from sparse_attention_hub_amd.sparse_attention.utils import mask_attention_utils as U
+
+    zeros = torch.zeros(1, 1, 64, 8192, device=cuda)  # many workgroups
+    other = zeros.clone()
+    other[0, 0, 63, 8191] = -1.0
+    kept = torch.zeros(1, dtype=torch.int64, pin_memory=True)  # another pinned block of that size is there to be handed out
+    del kept
+    torch.cuda.synchronize()
+
+    def first():
+        assert not U._ANSWERS.words
+        graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+        with torch.cuda.stream(stream), torch.cuda.graph(graph, stream=stream):
+            zeros.add_(0.0)
+            with pytest.raises(RuntimeError, match="captured"):
+                U.AdditiveMaskFacts().flags(zeros)
+        assert not U._ANSWERS.words
+        for _ in range(3):
+            assert U.AdditiveMaskFacts().flags(zeros) == 0
+            assert U.AdditiveMaskFacts().flags(other) == N.AMASK_NONZERO | N.AMASK_GENERAL
+            graph.replay()
+            torch.cuda.synchronize()
+
+    with ThreadPoolExecutor(1) as pool:
+        pool.submit(first).result()
