@@ -108,8 +108,9 @@ def _answer_words(device: torch.device):
             if torch.cuda.is_current_stream_capturing():
                 # (as sah_amask_read itself refuses.) Words made now would lie in the graph's memory, cleared by replays alone.
                 raise N.NativeLibraryError("what a mask holds cannot be read back while the stream is captured")
-        words = _ANSWERS.words[device.index] = (torch.zeros(2, dtype=torch.int32, device=device),
-                                                torch.zeros(1, dtype=torch.int64, pin_memory=True))
+            scratch = torch.zeros(2, dtype=torch.int32, device=device)
+            torch.cuda.current_stream().synchronize()  # once: a question refused now is followed by one of another stream
+        words = _ANSWERS.words[device.index] = (scratch, torch.zeros(1, dtype=torch.int64, pin_memory=True))
     return words
 
 

@@ -764,3 +764,29 @@ def test_a_first_question_under_capture_leaves_nothing_behind(cuda):
 
     with ThreadPoolExecutor(1) as pool:
         pool.submit(first).result()
+
+
+def test_words_are_clear_before_another_stream_asks(cuda):
+    """The device words a thread's first question makes are cleared on its stream; if that question is refused, nothing else
+    orders the next one, of another stream, behind the clearing."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    from sparse_attention_hub_amd.sparse_attention.utils import mask_attention_utils as U
+
+    zeros = torch.zeros(1, 1, 64, 8192, device=cuda)  # many workgroups
+    torch.cuda.synchronize()
+
+    def first():
+        a, b = torch.cuda.Stream(), torch.cuda.Stream()
+        with torch.cuda.stream(a):
+            block = torch.full((2,), 7, dtype=torch.int32, device=cuda)
+            a.synchronize()
+            del block  # the next small allocation of this stream
+            torch.cuda._sleep(20_000_000)
+            with pytest.raises(ValueError, match="65535"):
+                U.AdditiveMaskFacts().flags(zeros.expand(1, 1100, 64, 8192))
+        with torch.cuda.stream(b):
+            assert U.AdditiveMaskFacts().flags(zeros) == 0
+
+    with ThreadPoolExecutor(1) as pool:
+        pool.submit(first).result()
