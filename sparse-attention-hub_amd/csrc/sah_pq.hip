@@ -499,6 +499,11 @@ __global__ __launch_bounds__(PQ_NT) void k_pq_update(pq_update_params P) {
 #define PQM_FUSED_LDS (80 * 1024)  // operands + sums up to this much LDS: sums in the same kernel, two workgroups a CU
 #define PQM_MAX_LDS (144 * 1024)  // operands at most (128 dimensions x 256 centres in fp32: 129 KB); the rest of a CU is static LDS
 #define PQM_MIN(a, b) __builtin_elementwise_minimum(a, b)  // three-way minimum instruction, no quieting of its operands
+// Slots of a lane whose centres are evaluated one by one; with more in some lane (repeated keys, whose centres are equal) the key
+// tile goes to the matrix instructions again. Six iterations at 8 heads x 16277 keys, 16 sub-vectors of 8, 256 centres (in us):
+// all keys equal 2178 (8656 one by one, however many), the first 60 % of them zeros 2206 (7139), random keys 508 (503). A slot
+// costs 10 us a launch there, the tile again 43; 2 sub-vectors of 64 and 64 centres: 7 and 42. 1: random keys 2 to 8 % slower.
+#define PQM_NEAR 3
 
 // 16-byte operands per lane and centre tile of the split form: terms x dimensions in slots of 16 (sub-vectors of 8: two
 // instructions; beyond: three per 16 dimensions)
@@ -557,7 +562,7 @@ __device__ __forceinline__ uint32_t pqm_mask_le(const sah_f32x16& a, float b) {
 template <int DT, int KS, bool SUMS, bool SPLIT>
 __global__ __launch_bounds__(PQM_NT, KS <= 16 ? 4 : 2) void k_pq_assign_mfma(pq_assign_params P, pq_update_params U, uint32_t* arrivals,
                                                                                            int wg_tiles, int ranges, int n_heads) {
-  HIP_DYNAMIC_SHARED(unsigned char, pqm_dyn)
+  SAH_DYNAMIC_LDS(pqm_dyn)
   static_assert(!SPLIT || (DT == SAH_BF16 && KS >= 4), "the split form multiplies bf16 keys in sub-vectors of 8 and more");
   if (P.skip_flag && *P.skip_flag) return;
   const int tid = threadIdx.x;
@@ -824,7 +829,7 @@ __global__ __launch_bounds__(PQM_NT, KS <= 16 ? 4 : 2) void k_pq_assign_mfma(pq_
       bidx = (int)(src >> 20) * 32 + 8 * (slot >> 2) + (from_lo ? 0 : 4) + (slot & 3);  // tile, slot -> centre
       const bool open = __popc(lo_half & 0x1ffffu) + __popc(hi_half & 0x1ffffu) != 1;
       const bool any_open = __ballot(open) != 0;  // uniform
-      again = odd || (any_open && __ballot(!(lim < INFINITY)) != 0);
+      again = odd || (any_open && __ballot(!(lim < INFINITY) || (open && __popc(in) > PQM_NEAR)) != 0);
       if (any_open && !again) {
         // The fp32 form's values, for the keys with several centres in reach, of every centre in a slot that holds one: the fp32
         // matrix instruction is a chain of fused multiply-adds in ascending dimensions (checked bit for bit on the hardware),
@@ -968,7 +973,7 @@ __global__ __launch_bounds__(PQM_NT, KS <= 16 ? 4 : 2) void k_pq_assign_mfma(pq_
 // grid.z splits the dimensions into slices of d_chunk; slice 0 also counts the members
 template <int DT>
 __global__ __launch_bounds__(PQS_NT) void k_pq_sums(pq_assign_params P, int d_chunk) {
-  HIP_DYNAMIC_SHARED(unsigned char, pqs_dyn)
+  SAH_DYNAMIC_LDS(pqs_dyn)
   if (P.skip_flag && *P.skip_flag) return;
   const int tid = threadIdx.x;
   const int s_idx = blockIdx.x % P.n_sub;
@@ -1235,7 +1240,7 @@ __global__ __launch_bounds__(ADC_NT) void k_pq_adc(pq_adc_params P, const void* 
   constexpr int NQ = (DT == SAH_F32) ? 2 : 4;
   typedef typename std::conditional<DT == SAH_F32, uint32_t, uint16_t>::type key_t;
   typedef uint2 entry_t;
-  HIP_DYNAMIC_SHARED(unsigned char, adc_dyn)
+  SAH_DYNAMIC_LDS(adc_dyn)
   const int tid = threadIdx.x;
   const int bh = blockIdx.y;
   const int vg = blockIdx.z;

@@ -103,6 +103,30 @@ def test_the_split_form_gives_the_codes_of_the_fp32_form(cuda, d, n_sub, n_cent)
     assert torch.equal(_assign(N, cuda, k, n_sub, d, c), _assign(N, cuda, wide[..., : n_sub * d], n_sub, d, c))
 
 
+@pytest.mark.parametrize("d,n_sub,n_cent", [(8, 2, 256), (16, 2, 130), (64, 2, 64), (128, 1, 64)])
+@pytest.mark.parametrize("copies", [2, 3, 4, 5, 9, 33, 64])
+def test_equal_centres(cuda, d, n_sub, n_cent, copies):
+    """Every centre `copies` times, in as many slots of the search: few are evaluated one by one, many by the matrix
+    instructions again. The first of them is taken, in both forms, with the same sums; some keys are equal to a centre."""
+    from sparse_attention_hub_amd import _native as N
+
+    n, H = 1500, 2
+    g = torch.Generator().manual_seed(copies)
+    base = torch.randn(H * n_sub, max(1, n_cent // copies), d, generator=g).bfloat16().float()
+    c = base.repeat(1, n_cent // base.shape[1] + 1, 1)[:, :n_cent].contiguous().to(cuda)
+    k = torch.randn(1, H, n, n_sub * d, generator=g)
+    for h in range(H):
+        for s in range(n_sub):
+            k[0, h, 700:900, s * d: (s + 1) * d] = base[h * n_sub + s, torch.randint(0, base.shape[1], (200,), generator=g)]
+    k = k.bfloat16()
+    wide = torch.zeros(1, H, n, n_sub * d + 4, dtype=torch.bfloat16, device=cuda)
+    forms = (k.to(cuda), wide[..., : n_sub * d].copy_(k))
+    top = k.float().abs().max().view(1).to(cuda)
+    (codes, S, C), other = (_assign(N, cuda, f, n_sub, d, c, top) for f in forms)
+    assert int(codes.max()) < base.shape[1]
+    assert torch.equal(codes, other[0]) and torch.equal(S, other[1]) and torch.equal(C, other[2])
+
+
 @pytest.mark.parametrize("d,n_sub,n_cent", [(8, 2, 64), (16, 2, 33), (64, 2, 64), (128, 1, 256)])  # the last: sums apart
 def test_an_element_that_is_not_a_number_adds_nothing(cuda, d, n_sub, n_cent):
     """NaN as the only values that are not finite, which the largest |element| passes over: it counts as 0 in its centre's
