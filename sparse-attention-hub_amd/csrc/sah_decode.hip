@@ -143,7 +143,7 @@ template <int DT, bool MF, bool CP, bool SILU>
 __global__ __launch_bounds__(HSW_NT) void k_hash_decode(hdec_params P) {
   sah_touch_kernargs<sizeof(hdec_params)>();
   __shared__ hsw_lds S;
-  HIP_DYNAMIC_SHARED(unsigned char, hdec_dyn)
+  SAH_DYNAMIC_LDS(hdec_dyn)
   hdec_row<DT, MF, CP, SILU>(P, blockIdx.x, S, hdec_dyn, nullptr);
 }
 
@@ -163,7 +163,7 @@ __global__ __launch_bounds__(HSW_NT) void k_hash_decode_attn(hdec_params P, att_
   __shared__ float s_l[HSW_NW];
   __shared__ float s_acc[HSW_NW][D];
   __shared__ int s_last;
-  HIP_DYNAMIC_SHARED(unsigned char, hdec_dyn)
+  SAH_DYNAMIC_LDS(hdec_dyn)
   sah_touch_kernargs<sizeof(hdec_params) + sizeof(att_params) + 32>();
   const int G = A.Hq / A.Hkv;
   const int GP = G * parts;

@@ -132,7 +132,7 @@ __global__ __launch_bounds__(GEMV_NT) void k_hash_sig_gemv(sig_pair PP) {
 // GELU's error function included, end up inside the hot loop and the code outgrows the instruction cache)
 template <int DT, int ACT>
 __global__ __launch_bounds__(SGM_NT, 4) void k_hash_sig_mfma(sig_params P, int n_chunks, int tiles_per_wg) {
-  HIP_DYNAMIC_SHARED(unsigned char, sgm_dyn)
+  SAH_DYNAMIC_LDS(sgm_dyn)
   const int tid = threadIdx.x;
   const int lane = tid & (SAH_WAVE - 1);
   const int wave = sah_wave_id();

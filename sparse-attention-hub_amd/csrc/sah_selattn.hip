@@ -44,7 +44,7 @@ __global__ __launch_bounds__(SF_NT) void k_select16_attn(selattn_params P, att_p
   __shared__ float s_l[NW];
   __shared__ float s_acc[NW][D];
   __shared__ int s_last;
-  HIP_DYNAMIC_SHARED(unsigned char, sa_dyn)
+  SAH_DYNAMIC_LDS(sa_dyn)
   // Workgroup -> (row, part). Consecutive workgroup ids go round-robin to the 8 dies; a tile is a GQA group, tile t
   // runs on die t % 8 and all G x parts workgroups of the group take adjacent slots of that die: the sink / local K / V
   // rows the G heads have in common and the score keys the parts of a row have in common are fetched once per die.

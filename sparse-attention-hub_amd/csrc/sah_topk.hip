@@ -348,7 +348,7 @@ template <int KB>
 __global__ __launch_bounds__(SEL_NT) void k_select_topk(sah_rows R, sel_layout L, const void* keys, int64_t pitch,
                                                         int n_cand, int col_offset, int k, uint32_t excluded_key) {
   __shared__ sel_shared S;
-  HIP_DYNAMIC_SHARED(unsigned char, sel_dyn)
+  SAH_DYNAMIC_LDS(sel_dyn)
   const int r = blockIdx.x;
   if (KB == 16) {
     key_src_mem16 src{(const uint16_t*)keys + (int64_t)r * pitch};
@@ -362,7 +362,7 @@ __global__ __launch_bounds__(SEL_NT) void k_select_topk(sah_rows R, sel_layout L
 __global__ __launch_bounds__(SEL_NT) void k_hamming_topk(sah_rows R, sel_layout L, const uint2* kcodes, int64_t pitch,
                                                          const uint2* qcodes, int lq, int k) {
   __shared__ sel_shared S;
-  HIP_DYNAMIC_SHARED(unsigned char, sel_dyn)
+  SAH_DYNAMIC_LDS(sel_dyn)
   const int r = blockIdx.x;
   key_src_hamming src{kcodes + (int64_t)(r / lq) * pitch, qcodes[r]};
   select_row<key_src_hamming, 7, uint8_t>(S, sel_dyn, L, R, r, src, R.n_keys, 0, k, 0u);
@@ -371,7 +371,7 @@ __global__ __launch_bounds__(SEL_NT) void k_hamming_topk(sah_rows R, sel_layout 
 __global__ __launch_bounds__(HSW_NT) void k_hamming_topk_swar(sah_rows R, const uint2* kcodes, int64_t pitch,
                                                               const uint2* qcodes, int lq, int k) {
   __shared__ hsw_lds S;
-  HIP_DYNAMIC_SHARED(unsigned char, hsw_dyn)
+  SAH_DYNAMIC_LDS(hsw_dyn)
   const int r = blockIdx.x;
   const int tid = threadIdx.x;
   const int n_ch = (R.n_keys + 255) / 256;
@@ -401,7 +401,7 @@ __global__ __launch_bounds__(NW * SAH_WAVE, SQ_WAVES_PER_SIMD(NW, CPW)) void k_s
     int window) {
   sah_touch_kernargs<sizeof(sah_rows) + 56>();
   __shared__ sq_lds S;
-  HIP_DYNAMIC_SHARED(unsigned char, sq_dyn)
+  SAH_DYNAMIC_LDS(sq_dyn)
   const int r = blockIdx.x;
   sq_select_row<NW, CPW>(S, sq_dyn, R, r, keys + (int64_t)r * pitch, n_cand, col_offset, k < n_cand ? k : n_cand, excluded_key,
                          fresh, sink, window);
@@ -414,7 +414,7 @@ __global__ __launch_bounds__(SF_NT) void k_select16_row(sah_rows R, const uint16
                                                         int k, uint32_t excluded_key, int fresh, int sink, int window) {
   sah_touch_kernargs<sizeof(sah_rows) + 56>();
   __shared__ sf_lds S;
-  HIP_DYNAMIC_SHARED(unsigned char, sf_dyn)
+  SAH_DYNAMIC_LDS(sf_dyn)
   const int r = blockIdx.x;
   sf_select_row<CPW>(S, sf_dyn, R, r, keys + (int64_t)r * pitch, n_cand, col_offset, k < n_cand ? k : n_cand, excluded_key, fresh,
                      sink, window);
