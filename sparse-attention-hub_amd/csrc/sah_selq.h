@@ -6,9 +6,9 @@
 // sampled rank to either side. Every key is compared with the bracket's two ends, and the few per cent inside are looked at
 // one by one: counted value by value, which gives T exactly or shows that the bracket missed it, and kept in LDS until they
 // can be compared with T. Rows for which that does not work (active columns that rank among them, a bracket of more than
-// SQ_FINE key values, a missed T) take the general way: the bracket's keys picked from the registers, the bracket taken from
-// a histogram of all keys if need be. Then, and where a lane has more of the bracket's keys than slots, every key is
-// compared with T.
+// SQ_FINE key values, a missed T, waves that hold little else than keys of the bracket) take the general way: the bracket's
+// keys picked from the registers, the bracket taken from a histogram of all keys if need be. Then, and where a lane has more of
+// the bracket's keys than slots, every key is compared with T.
 // Winners above T are written by every wave independently; the ties taken are the lowest columns. The list is unordered
 // inside a row; its order is a pure function of the inputs.
 #pragma once
@@ -35,7 +35,7 @@ struct sq_lds {
   int lo_bin, hi_bin, lo_above;  // bins of the two sample ranks; keys in the bins above lo_bin
   int above;                     // keys above the bracket
   int sel_bin, sel_need;
-  int over;                      // a lane ran out of slots
+  int over;                      // 1: a lane ran out of slots; 2: and a wave left its keys to be counted from the registers
 };
 
 // words of the histograms' and the slots' common place
@@ -79,6 +79,7 @@ __device__ __forceinline__ void sq_select_row(sq_lds& S, unsigned char* dyn, con
                                               int window) {
   constexpr int NT = NW * SAH_WAVE;
   constexpr int SLOTS = SQ_SLOTS(CPW);
+  constexpr bool LONG = CPW >= 8;           // what rows of few different keys lose grows with their length
   constexpr int NWD = (CPW + 3) / 4;        // 32-bit words of a lane's candidate masks: word w holds chunks 4 w .. 4 w + 3
   const int tid = threadIdx.x;
   const int lane = tid & (SAH_WAVE - 1);
@@ -258,9 +259,40 @@ __device__ __forceinline__ void sq_select_row(sq_lds& S, unsigned char* dyn, con
     __syncthreads();
   };
 
+  // Many of a wave's 64 lanes with one key (hidden columns, rows of few keys): their adds to one counter go one after the other,
+  // 2.4 cycles each. crowd: whether an eighth of the lanes hold the same word as the first or the 32nd one, and its lower key;
+  // the lanes with that index then add once, together (all lanes call). 1056 rows x 131000 candidates, k 6550, and how long
+  // without: the first 90 % hidden 247 us (709), 97 % 242 (480), the same share hidden here and there 233 (682) and 235 (470),
+  // one key throughout 272 (506); no two columns alike 148 (144).
+  auto crowd = [&](uint32_t word, uint32_t& key) -> bool {
+    uint32_t w = (uint32_t)__builtin_amdgcn_readlane((int)word, 0);
+    uint64_t all = __ballot(word == w);
+    if (__popcll(all) < SAH_WAVE / 8) {
+      w = (uint32_t)__builtin_amdgcn_readlane((int)word, SAH_WAVE / 2);
+      all = __ballot(word == w);
+    }
+    key = w & 0xffffu;
+    return __popcll(all) >= SAH_WAVE / 8;
+  };
+  auto add_crowd = [&](uint32_t* counters, uint32_t index, uint32_t of_crowd, bool counted) {
+    const bool same = counted && index == of_crowd;
+    const uint64_t all = __ballot(same);
+    if (counted && (!same || lane == __builtin_ctzll(all))) atomicAdd(&counters[index], same ? (uint32_t)__popcll(all) : 1u);
+  };
+  uint32_t* my_f = s_fi + (lane & (SQ_COPIES - 1)) * SQ_FINE;
+
+  uint32_t of_crowd;
+  const bool crowds = LONG && crowd(kreg[0].x, of_crowd);  // uniform across the wave
   for_chunks([&](int, const uint32_t (&kk)[4], int u) {
-    const uint32_t key = key_of(kk, u & 7);
-    atomicAdd(&s_co[key >> (SQ_SHIFT + 1)], (key >> SQ_SHIFT) & 1u ? 0x10000u : 1u);
+    const uint32_t key = key_of(kk, u & 7), bin = key >> SQ_SHIFT;
+    const uint32_t n = bin & 1u ? 0x10000u : 1u;
+    if (crowds) {
+      const bool same = bin == of_crowd >> SQ_SHIFT;
+      const uint64_t all = __ballot(same);
+      if (!same || lane == __builtin_ctzll(all)) atomicAdd(&s_co[bin >> 1], same ? n * (uint32_t)__popcll(all) : n);
+    } else {
+      atomicAdd(&s_co[bin >> 1], n);
+    }
   });
   __syncthreads();
   {
@@ -286,8 +318,9 @@ __device__ __forceinline__ void sq_select_row(sq_lds& S, unsigned char* dyn, con
   for (int w = 0; w < NWD; ++w) gt[w] = eq[w] = act[w] = 0u;
   // candidate of bit b of mask word w
   auto bit_cand = [&](int w, int b) -> int { return first_cand(c0 + 4 * w) + ((b & 24) << 6) + (b & 7); };
-  uint32_t* my_f = s_fi + (lane & (SQ_COPIES - 1)) * SQ_FINE;
   bool found = false, done = false;  // uniform: T is known, and the masks are
+  bool tried = false;                // uniform: the short way's masks have been made, what lies above the bracket is counted
+  bool counted = false;              // uniform across the wave: its keys of the bracket are
   if (!exact && (uint32_t)lo > ek) {
     // ---- the short way: keys above the bracket into gt, the bracket's keys one by one
     uint32_t in[NWD];
@@ -308,35 +341,51 @@ __device__ __forceinline__ void sq_select_row(sq_lds& S, unsigned char* dyn, con
     int n = 0, n_above = 0;
 #pragma unroll
     for (int w = 0; w < NWD; ++w) {
+      if (LONG) n += __popc(in[w]);
       n_above += __popc(gt[w]);
-      uint32_t m = in[w];
-      while (m) {
-        uint32_t kv[SQ_GATHER];
-        uint32_t left = m;
+    }
+    tried = true;
+    // (requested one by one, 1056 rows x 131000 of one key: 507 us; at three eighths in place of three quarters, rows that rise
+    // with the column lose more than rows of two keys gain)
+    counted = !LONG || __ballot(n <= SLOTS || n <= 6 * (c1 - c0)) != 0;
+    if (counted) {
+      n = 0;
 #pragma unroll
-        for (int i = 0; i < SQ_GATHER; ++i) {
-          kv[i] = keys[left ? bit_cand(w, __builtin_ctz(left)) : 0];  // (not active: the key in memory is the key)
-          left &= left - 1;
-        }
+      for (int w = 0; w < NWD; ++w) {
+        uint32_t m = in[w];
+        while (m) {
+          uint32_t kv[SQ_GATHER];
+          uint32_t left = m;
 #pragma unroll
-        for (int i = 0; i < SQ_GATHER; ++i) {
-          if (m) {
-            atomicAdd(&my_f[kv[i] - (uint32_t)lo], 1u);
-            if (n < SLOTS) s_slot[n * NT + tid] = (uint16_t)kv[i];
-            ++n;
+          for (int i = 0; i < SQ_GATHER; ++i) {
+            kv[i] = keys[left ? bit_cand(w, __builtin_ctz(left)) : 0];  // (not active: the key in memory is the key)
+            left &= left - 1;
           }
-          m &= m - 1;
+#pragma unroll
+          for (int i = 0; i < SQ_GATHER; ++i) {
+            if (m) {
+              atomicAdd(&my_f[kv[i] - (uint32_t)lo], 1u);
+              if (n < SLOTS) s_slot[n * NT + tid] = (uint16_t)kv[i];
+              ++n;
+            }
+            m &= m - 1;
+          }
         }
       }
     }
-    if (n > SLOTS) S.over = 1;
+    if (n > SLOTS) {  // (every lane of a wave that has not counted)
+      if (LONG) atomicMax(&S.over, counted ? 1 : 2);
+      else S.over = 1;
+    }
     const int na = sah_wave_sum_i(n_above);
     if (lane == 0 && na) atomicAdd(&S.above, na);
     __syncthreads();
-    pick(S.above);
-    found = S.sel_bin >= 0;
-    exact = !found;
-    done = found && !S.over;
+    if (!LONG || S.over < 2) {
+      pick(S.above);
+      found = S.sel_bin >= 0;
+      exact = !found;
+      done = found && !S.over;
+    }
     if (done) {
       const uint32_t t = (uint32_t)(lo + S.sel_bin);
       n = 0;
@@ -359,8 +408,11 @@ __device__ __forceinline__ void sq_select_row(sq_lds& S, unsigned char* dyn, con
   }
   if (!found) {
     // ---- the general way to T
+    uint32_t of_crowd;
+    const bool crowds = crowd(kreg[0].x, of_crowd);
     for (;;) {  // at most twice, uniform
       if (exact) {
+        counted = false;
         __syncthreads();  // the counts of the attempt before have been read
         clear(s_co, SQ_COARSE_WORDS);
         clear(s_fi, SQ_COPIES * SQ_FINE);
@@ -370,8 +422,12 @@ __device__ __forceinline__ void sq_select_row(sq_lds& S, unsigned char* dyn, con
         }
         __syncthreads();
         for_chunks([&](int, const uint32_t (&kk)[4], int) {
+          const bool crowded = crowds && crowd(kk[0], of_crowd);  // uniform across the wave
 #pragma unroll
-          for (int t = 0; t < 8; ++t) atomicAdd(&s_co[key_of(kk, t) >> SQ_ALL_SHIFT], 1u);
+          for (int t = 0; t < 8; ++t) {
+            if (crowded) add_crowd(s_co, key_of(kk, t) >> SQ_ALL_SHIFT, of_crowd >> SQ_ALL_SHIFT, true);
+            else atomicAdd(&s_co[key_of(kk, t) >> SQ_ALL_SHIFT], 1u);
+          }
         });
         __syncthreads();
         const int mine = coarse_sum(false);
@@ -385,7 +441,7 @@ __device__ __forceinline__ void sq_select_row(sq_lds& S, unsigned char* dyn, con
       const uint32_t lo2 = (uint32_t)lo * 0x00010001u, span2 = (uint32_t)span * 0x00010001u;
       const uint32_t last2 = (uint32_t)(lo + span - 1) * 0x00010001u;
       uint32_t n_above = 0;
-      for_chunks([&](int, const uint32_t (&kk)[4], int) {
+      if (!counted) for_chunks([&](int, const uint32_t (&kk)[4], int) {
         uint32_t d[4], g[4];
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
@@ -394,6 +450,11 @@ __device__ __forceinline__ void sq_select_row(sq_lds& S, unsigned char* dyn, con
           g[p] = sah_pk_gt01_u16(span2, d[p]);
         }
         uint32_t in = sq_join(g) & 0xffu;
+        if (crowds && crowd(d[0], of_crowd) && of_crowd < (uint32_t)span) {  // uniform across the wave
+#pragma unroll
+          for (int t = 0; t < 8; ++t) add_crowd(s_fi, key_of(d, t), of_crowd, key_of(g, t) != 0u);
+          return;
+        }
         while (in) {
           const int t = __builtin_ctz(in);
           in &= in - 1;
@@ -402,7 +463,7 @@ __device__ __forceinline__ void sq_select_row(sq_lds& S, unsigned char* dyn, con
           atomicAdd(&my_f[t & 1 ? two >> 16 : two & 0xffffu], 1u);
         }
       });
-      if (!exact) {
+      if (!exact && !tried) {
         const int na = sah_wave_sum_i((int)((n_above & 0xffffu) + (n_above >> 16)));
         if (lane == 0 && na) atomicAdd(&S.above, na);
       }

@@ -18,6 +18,9 @@ def _keys(kind, n_rows, pitch, g):
         return torch.randint(1, 8, (n_rows, pitch), generator=g, device=g.device) * 16 + 0x8000
     if kind == "equal":
         return torch.full((n_rows, pitch), 0x8123, device=g.device)
+    if kind[:6] in ("hidden", "hiding"):  # that share of the columns, the first or any, at the excluded key of hidden ones
+        share, seen = int(kind[6:]) / 100, _keys("float", n_rows, pitch, g)
+        return torch.where((j < share * pitch) if kind[:6] == "hidden" else (torch.rand(n_rows, pitch, generator=g, device=g.device) < share), 0x0080, seen)
     if kind == "zero":  # the smallest key, which missing candidates carry too
         return torch.where(torch.rand(n_rows, pitch, generator=g, device=g.device) < 0.02, 7, 0)
     # "striped": what is large depends on the place inside a group of eight, from which the sample takes one
@@ -48,9 +51,26 @@ def _keys(kind, n_rows, pitch, g):
 ])
 @pytest.mark.parametrize("offset", [0, 13])
 def test_rows_share_a_compute_unit(cuda, n_cand, k, kind, n_active, ek, offset):
+    _select(cuda, 258, n_cand, k, kind, n_active, ek, offset)
+
+
+@pytest.mark.parametrize("n_rows", [3, 258])  # sixteen waves a row, and eight
+@pytest.mark.parametrize("n_cand,k,kind", [
+    (16384, 900, "float"), (16385, 900, "float"), (32768, 1638, "few"), (32769, 1638, "float"), (65536, 3000, "striped"),
+    (65537, 3000, "float"),
+    (20481, 1200, "hidden90"), (20481, 1200, "hiding97"),
+    (33000, 300, "equal"), (33280, 1500, "equal"),  # the last wave's two chunks fit its slots, the others' do not
+    (36800, 1900, "hidden90"), (41000, 1500, "hidden97"), (41000, 3000, "hiding97"), (65500, 2000, "few"), (66000, 3500, "hiding90"),
+    (66100, 1, "equal"), (98000, 4800, "hidden97"), (131072, 9000, "hidden90"), (131072, 6000, "equal"), (131072, 60000, "few"),
+])
+def test_rows_of_repeated_keys(cuda, n_rows, n_cand, k, kind):
+    """Lanes that add to one counter do it together, waves full of the bracket's keys count them where they are."""
+    _select(cuda, n_rows, n_cand, k, kind, 200, 0x0080, 5)
+
+
+def _select(cuda, n_rows, n_cand, k, kind, n_active, ek, offset):
     from sparse_attention_hub_amd import _native as N
 
-    n_rows = 258
     n_keys = n_cand + offset
     pitch = (n_cand + 7) // 8 * 8
     g = torch.Generator(device=cuda).manual_seed(n_cand + k)
