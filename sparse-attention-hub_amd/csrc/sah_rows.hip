@@ -354,9 +354,17 @@ extern "C" int sah_rows_to_dense(const sah_dense_rows_args* a) {
 #define AMC_NT 256
 #define AMC_PER_THREAD 8
 
+// one element's share of the answer. Hidden: as low as the lowest finite value of the dtype (what HuggingFace's masks put on a
+// hidden column) or -inf; NaN: general
+template <int DT>
+__device__ __forceinline__ int amask_flags(float x) {
+  constexpr float lowest = DT == SAH_F32 ? -3.4028234663852886e38f : (DT == SAH_BF16 ? -3.3895313892515355e38f : -65504.0f);
+  return x == 0.f ? 0 : ((x <= lowest) ? SAH_AMASK_NONZERO : (SAH_AMASK_NONZERO | SAH_AMASK_GENERAL));
+}
+
 template <int DT>
 __global__ __launch_bounds__(AMC_NT) void k_amask_classify(const void* amask, int64_t ms_b, int64_t ms_h, int64_t ms_l, int Hm,
-                                                           int Lq, int Lk, float lowest, int* flags) {
+                                                           int Lq, int Lk, int* flags) {
   const int row = blockIdx.y;  // (b * Hm + h) * Lq + q
   const int q = row % Lq, h = (row / Lq) % Hm, b = row / (Lq * Hm);
   const int64_t base = b * ms_b + h * ms_h + q * ms_l;
@@ -365,10 +373,7 @@ __global__ __launch_bounds__(AMC_NT) void k_amask_classify(const void* amask, in
 #pragma unroll
   for (int i = 0; i < AMC_PER_THREAD; ++i) {
     const int c = c0 + i;
-    if (c < Lk) {
-      const float x = sah_load<DT>(amask, base + c);
-      if (x != 0.f) f |= (x <= lowest) ? SAH_AMASK_NONZERO : (SAH_AMASK_NONZERO | SAH_AMASK_GENERAL);  // NaN: general
-    }
+    if (c < Lk) f |= amask_flags<DT>(sah_load<DT>(amask, base + c));
   }
   if (__ballot(f != 0)) {
     // one atomic per wave that saw anything
@@ -386,22 +391,15 @@ extern "C" int sah_amask_classify(const sah_amask_classify_args* a) {
   const dim3 g((unsigned)((a->Lk + AMC_NT * AMC_PER_THREAD - 1) / (AMC_NT * AMC_PER_THREAD)), (unsigned)rows), blk(AMC_NT);
   hipStream_t st = (hipStream_t)a->stream;
   sah_timed timed("k_amask_classify", a->stream);
-  // "as low as the lowest finite value of the dtype" (what HuggingFace's masks put on a hidden column) or -inf
+#define SAH_AMC(DTC) \
+  hipLaunchKernelGGL(k_amask_classify<DTC>, g, blk, 0, st, a->amask, a->ms_b, a->ms_h, a->ms_l, a->Hm, a->Lq, a->Lk, a->flags)
   switch (a->dtype) {
-    case SAH_F32:
-      hipLaunchKernelGGL(k_amask_classify<SAH_F32>, g, blk, 0, st, a->amask, a->ms_b, a->ms_h, a->ms_l, a->Hm, a->Lq, a->Lk,
-                         -3.4028234663852886e38f, a->flags);
-      break;
-    case SAH_BF16:
-      hipLaunchKernelGGL(k_amask_classify<SAH_BF16>, g, blk, 0, st, a->amask, a->ms_b, a->ms_h, a->ms_l, a->Hm, a->Lq, a->Lk,
-                         -3.3895313892515355e38f, a->flags);
-      break;
-    case SAH_F16:
-      hipLaunchKernelGGL(k_amask_classify<SAH_F16>, g, blk, 0, st, a->amask, a->ms_b, a->ms_h, a->ms_l, a->Hm, a->Lq, a->Lk, -65504.0f,
-                         a->flags);
-      break;
+    case SAH_F32: SAH_AMC(SAH_F32); break;
+    case SAH_BF16: SAH_AMC(SAH_BF16); break;
+    case SAH_F16: SAH_AMC(SAH_F16); break;
     default: return sah_fail(SAH_EDTYPE, "sah_amask_classify: dtype %d", a->dtype);
   }
+#undef SAH_AMC
   return sah_launch_status("sah_amask_classify");
 }
 
@@ -415,15 +413,13 @@ extern "C" int sah_amask_classify(const sah_amask_classify_args* a) {
 #define AMR_MAX_WGS 256
 template <int DT>
 __global__ __launch_bounds__(AMR_NT) void k_amask_read(const void* amask, int64_t ms_b, int64_t ms_h, int64_t ms_l, int Hm, int Lq, int Lk,
-                                                       int rows, float lowest, uint32_t* scratch, uint64_t* host_word, uint32_t seq) {
+                                                       int rows, uint32_t* scratch, uint64_t* host_word, uint32_t seq) {
   __shared__ uint32_t s_f;
   const int tid = threadIdx.x;
   if (tid == 0) s_f = 0u;
   __syncthreads();
   uint32_t f = 0u;
-  auto look = [&](float x) {
-    if (x != 0.f) f |= (x <= lowest) ? SAH_AMASK_NONZERO : (SAH_AMASK_NONZERO | SAH_AMASK_GENERAL);  // NaN: general
-  };
+  auto look = [&](float x) { f |= (uint32_t)amask_flags<DT>(x); };
   const int upr = (Lk + 7) / 8;  // units of eight elements a row
   const int64_t units = (int64_t)rows * upr, step = (int64_t)gridDim.x * AMR_NT;
   for (int64_t u = (int64_t)blockIdx.x * AMR_NT + tid; u < units; u += step) {
@@ -479,15 +475,14 @@ extern "C" int sah_amask_read(sah_amask_read_args* r) {
   volatile uint64_t* word = r->host_word;
   const uint32_t seq = (uint32_t)(*word >> 32) + 1u;
   {
-    sah_timed timed("k_amask_classify", a->stream);
-    // "as low as the lowest finite value of the dtype" (what HuggingFace's masks put on a hidden column) or -inf
-#define SAH_AMR(DTC, LOWEST)                                                                                                    \
+    sah_timed timed("k_amask_classify", a->stream);  // (one name for the question, whichever kernel answers)
+#define SAH_AMR(DTC)                                                                                                            \
   hipLaunchKernelGGL(k_amask_read<DTC>, dim3((unsigned)wgs), dim3(AMR_NT), 0, st, a->amask, a->ms_b, a->ms_h, a->ms_l, a->Hm, a->Lq, \
-                     a->Lk, (int)rows, LOWEST, r->scratch, r->host_word, seq)
+                     a->Lk, (int)rows, r->scratch, r->host_word, seq)
     switch (a->dtype) {
-      case SAH_F32: SAH_AMR(SAH_F32, -3.4028234663852886e38f); break;
-      case SAH_BF16: SAH_AMR(SAH_BF16, -3.3895313892515355e38f); break;
-      case SAH_F16: SAH_AMR(SAH_F16, -65504.0f); break;
+      case SAH_F32: SAH_AMR(SAH_F32); break;
+      case SAH_BF16: SAH_AMR(SAH_BF16); break;
+      case SAH_F16: SAH_AMR(SAH_F16); break;
       default: return sah_fail(SAH_EDTYPE, "sah_amask_read: dtype %d", a->dtype);
     }
 #undef SAH_AMR

@@ -700,6 +700,22 @@ def test_what_a_mask_holds_is_read_back(cuda, dtype, shape):  # and several; row
         assert AdditiveMaskFacts().flags(zero) == 0
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("shape", [(1, 1, 1, 7), (2, 1, 48, 4099), (1, 4, 3, 2049)])
+def test_what_a_mask_holds_into_device_memory(cuda, dtype, shape):
+    """`sah_amask_classify`: the answer of `sah_amask_read` in a word of device memory, which it adds to."""
+    from sparse_attention_hub_amd import _native as N
+    from sparse_attention_hub_amd.sparse_attention.utils.mask_attention_utils import AdditiveMaskFacts
+
+    B, H, L, n = shape
+    m = torch.zeros(B, H, L, n + 3, dtype=dtype, device=cuda)[..., 1: n + 1]
+    for value in (0.0, -0.0, float(torch.finfo(dtype).min), -float("inf"), -1.0, float("nan")):
+        m[B - 1, H - 1, L - 1, n - 1] = value
+        flags = torch.zeros(1, dtype=torch.int32, device=cuda)
+        N.call("sah_amask_classify", N.AmaskClassifyArgs(m.data_ptr(), *m.stride()[:3], N.dtype_code(dtype), B, H, L, n, flags.data_ptr(), N.stream_ptr(cuda)))
+        assert int(flags) == AdditiveMaskFacts().flags(m), value
+
+
 def test_the_next_mask_may_be_read_by_another_stream(cuda):
     """The device words an answer went through are zero when the call returns, not only when its kernel has ended: the
     thread's next question uses them from whatever stream it comes."""
