@@ -415,7 +415,7 @@ __global__ __launch_bounds__(QM_NT, 2) void k_qk_scores_mfma(qk_params P, int ch
         const int rl = it * 8 + (lane >> 3);
         const uint4 sc = *(const uint4*)&s_o[wave][rl * OP + k8];
         const int v = c * QM_VECS + vt * 32 + rl;
-          const int row = v < nvec ? row0 + v : -1;
+        const int row = v < nvec ? row0 + v : -1;
         uint32_t w[4] = {sc.x, sc.y, sc.z, sc.w};
         const bool whole = row >= 0 && j + 8 <= P.Lk;
         if (AM) {
