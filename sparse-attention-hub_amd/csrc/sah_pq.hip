@@ -480,12 +480,12 @@ __global__ __launch_bounds__(PQ_NT) void k_pq_update(pq_update_params P) {
 // The split form's rounding is another one (and smaller), so where several centres come within both forms' rounding of the
 // smallest value they are evaluated in the fp32 form's order of operations: the codes are those of the fp32 form, bit for
 // bit, whichever form the alignment and shape of the keys allow (without: 1e-6 of the codes of an iteration, 5e-4 after ten).
-// Measured (bf16, 8 heads x 16277 keys, 16 sub-vectors of 8, 256 centres, sums included): 68 us (76 with the update); 85 with every tile's 16
-// values selected, not their minima over the tiles, the second look by matrix instruction, its test by ballots, the key
+// Measured (bf16, 8 heads x 16277 keys, 16 sub-vectors of 8, 256 centres, sums included): 65 us (72 with the update); 85 with every
+// tile's 16 values selected, not their minima over the tiles, the second look by matrix instruction, its test by ballots, the key
 // operand in a structure (which went through scratch memory) and the centres read element by element. What bounds it: issue,
 // 20 vector and 2 matrix instructions a tile (31 us) and 150 vector ones a key tile of eight (25), 10 before and after the
 // loop. fp16 (no split: terms of small centres would leave its range): 121 at 16405 keys. 32768 keys, 2 sub-vectors of 64, 64
-// centres: 218 -> 62 with the split. Sums in [centre][d] order and a flush of one centre a lane took 40 (8 dims) to 100 us
+// centres: 218 -> 47 with the split. Sums in [centre][d] order and a flush of one centre a lane took 40 (8 dims) to 100 us
 // (64 dims) of these.
 // The expansion rounds differently from the difference form of the reference ((A - B)^2 summed,
 // pq_utils.py:220-257): a key whose two nearest centres tie to the last bits may take the other one.
@@ -952,8 +952,8 @@ __global__ __launch_bounds__(PQM_NT, KS <= 16 ? 4 : 2) void k_pq_assign_mfma(pq_
   for (int c = tid; c < n_cent; c += PQM_NT)
     if (s_cnt[c]) atomicAdd(&P.counts[(int64_t)grp * n_cent + c], s_cnt[c]);
   if (!arrivals) return;
-  // The workgroup of the group that arrives last carries out the update: 8 us of this kernel, where a launch of its own takes
-  // 9.3 and the way from kernel to kernel.
+  // The workgroup of the group that arrives last carries out the update: 7 us of this kernel, where a launch of its own takes
+  // 8.7 and the way from kernel to kernel.
   sah_stores_done();  // (the atomics' too)
   __syncthreads();
   int* s_last = s_cnt;

@@ -388,12 +388,16 @@ __global__ __launch_bounds__(HSW_NT) void k_hamming_topk_swar(sah_rows R, const 
 }
 
 // Registers for four, three or two workgroups of eight waves a CU (16 waves: one or two): a row alone on a CU leaves the
-// vector unit idle at every barrier and while its keys arrive. 1536 rows x 32768 candidates, k 1638, bf16 scores: 41 us, 25 of
+// vector unit idle at every barrier and while its keys arrive. 1536 rows x 32768 candidates, k 1638, bf16 scores: 42 us, 25 of
 // them the issue of 1270 vector instructions a wave, the rest 100 MB of keys; one workgroup of 16 waves a CU with the passes
-// of sah_sel16.h takes 65 us (fp16 scores, whose threshold lies in no top bin: 39 and 122). 512 x 131072, k 2621: 57 and 93;
-// 1536 x 4096: 20 and 37; 1056 x 32801 signature scores: 46 and 68; rows of one key throughout: 133 and 157. Nine chunks a
-// wave for rows a little longer than 32768, five for those beyond 16384: 16 and 8 leave registers for fewer workgroups
-// (1056 x 32801: 59 us).
+// of sah_sel16.h takes 65 us (fp16 scores, whose threshold lies in no top bin: 41 and 122). 512 x 131072, k 2621: 59 and 93;
+// 1536 x 4096: 16 and 37; 1056 x 32801 signature scores: 45 and 68; rows of one key throughout: 65 and 157.
+// The forms, at 1056 rows of bf16 scores (in us): a form of more chunks than the row has costs registers, so that fewer rows share
+// a CU, and passes over empty ones: 16300 candidates in four chunks a wave 19.8, in five 20.9, in eight 23.9; 20000 in five 23.9,
+// in eight 27.4; 32700 in eight 33.1, in nine 34.4; 36800 in nine 38.1, in sixteen 49.4. Five and nine stand for rows a little
+// longer than 16384 and 32768 (a context and its question); between 36865 and 65536 sixteen serve all (37000: 51.9, 65400: 66.1).
+// Eight waves a row against sixteen: from 257 rows on 32700 x 258 14.6 and 14.9, 65400 x 258 24.7 and 28.5, 41000 x 1056 54 and
+// 67; at most one row a CU, sixteen: 16405 x 256 10.2 and 10.8, 32700 x 128 10.8 and 12.1, 65400 x 128 16.0 and 18.7.
 #define SQ_WAVES_PER_SIMD(NW, CPW) ((CPW) <= 5 ? 8 : (CPW) <= 9 && (NW) == 8 ? 6 : 4)
 template <int NW, int CPW>
 __global__ __launch_bounds__(NW * SAH_WAVE, SQ_WAVES_PER_SIMD(NW, CPW)) void k_select16(
@@ -407,8 +411,10 @@ __global__ __launch_bounds__(NW * SAH_WAVE, SQ_WAVES_PER_SIMD(NW, CPW)) void k_s
                          fresh, sink, window);
 }
 
-// CPW = 4: few short rows, which the latency of one row's passes bounds (128 rows x 12011: 9.0 us here, 10.3 in the form above;
-// 32 x 32678: 11.6 and 11.2). CPW = 0: rows too long for the registers of a workgroup; their keys are read in every pass.
+// CPW = 4: few rows of up to 16384 candidates, which the latency of one row's passes bounds. 8 x 12011 bf16 scores: 8.0 us, 9.1 in
+// the form above with 16 waves (8.3 with eight); 128 x 16300: 9.1 and 9.6. Longer ones go there, for what signature scores gain:
+// 128 x 16405 bf16 scores 9.6 us here and 9.9 there, signature scores 12.0 and 10.7, 32700: 11.7 and 10.8, 16.6 and 12.2.
+// CPW = 0: rows too long for the registers of a workgroup; their keys are read in every pass.
 template <int CPW>
 __global__ __launch_bounds__(SF_NT) void k_select16_row(sah_rows R, const uint16_t* keys, int64_t pitch, int n_cand, int col_offset,
                                                         int k, uint32_t excluded_key, int fresh, int sink, int window) {

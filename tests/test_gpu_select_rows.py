@@ -1,6 +1,7 @@
-"""`sah_select_topk` on 16-bit keys through the C ABI with more mask rows than compute units, where several rows share one:
-every register form (candidates around each limit), the bracket taken from a sample and what happens when it misses the
-threshold, lanes with more bracket keys than slots, ties, active columns that rank. Checked against a stable sort."""
+"""`sah_select_topk` on 16-bit keys through the C ABI: more mask rows than compute units, where several share one, and few, which
+have one to themselves. Every register form (candidates around each limit), the bracket taken from a sample and what happens
+when it misses the threshold, lanes with more bracket keys than slots, ties, active columns that rank, repeated keys. Checked
+against a stable sort."""
 import pytest
 import torch
 
