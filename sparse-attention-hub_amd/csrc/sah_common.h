@@ -166,6 +166,20 @@ __device__ __forceinline__ float sah_round(float f) {
   return f;
 }
 
+// The same in one instruction for bf16: the converter packs two values, the rounded one above a zero is the float. (The
+// zero is opaque, or the compiler converts the value into the low half and shifts it up.)
+template <int DT>
+__device__ __forceinline__ float sah_round1(float f) {
+  if (DT != SAH_BF16) return sah_round<DT>(f);
+  typedef __bf16 v2 __attribute__((ext_vector_type(2)));
+  float zero = 0.f;
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm("" : "+s"(zero));
+#endif
+  const v2 p = {(__bf16)zero, (__bf16)f};
+  return __builtin_bit_cast(float, p);
+}
+
 // two values rounded to the 16-bit storage type DT and packed, lo in the low half
 template <int DT>
 __device__ __forceinline__ uint32_t sah_pack2_hw(float lo, float hi) {

@@ -122,7 +122,6 @@ __global__ __launch_bounds__(GEMV_NT) void k_hash_sig_gemv(sig_pair PP) {
 // ---------------------------------------------------------------------------
 #define SGM_NT 512
 #define SGM_NW (SGM_NT / SAH_WAVE)
-#define SGM_TILE (32 * SGM_NW)  // vectors per workgroup tile
 #define SGM_MAXW 128            // widest layer
 #define SGM_MAXK (SGM_MAXW / 16)
 #define SGM_MAXM (SGM_MAXW / 32)
@@ -130,8 +129,9 @@ __global__ __launch_bounds__(GEMV_NT) void k_hash_sig_gemv(sig_pair PP) {
 
 // ACT: the activation, fixed at compile time (one kernel each: with the choice left to run time the four epilogues,
 // GELU's error function included, end up inside the hot loop and the code outgrows the instruction cache)
+// A workgroup takes tiles [wg * wg_tiles, (wg + 1) * wg_tiles) of 32 vectors of its head, its waves every eighth of them.
 template <int DT, int ACT>
-__global__ __launch_bounds__(SGM_NT, 4) void k_hash_sig_mfma(sig_params P, int n_chunks, int tiles_per_wg) {
+__global__ __launch_bounds__(SGM_NT, 4) void k_hash_sig_mfma(sig_params P, int n_chunks, int wg_tiles) {
   SAH_DYNAMIC_LDS(sgm_dyn)
   const int tid = threadIdx.x;
   const int lane = tid & (SAH_WAVE - 1);
@@ -168,7 +168,9 @@ __global__ __launch_bounds__(SGM_NT, 4) void k_hash_sig_mfma(sig_params P, int n
   float* s_bias = (float*)((uint16_t*)sgm_dyn + ((w_elems + 1) & ~1));
   {
     int din = P.D;
-    for (int l = 0; l < P.n_layers; ++l) {
+#pragma unroll
+    for (int l = 0; l < SAH_MAX_MLP_LAYERS; ++l) {
+      if (l >= P.n_layers) break;
       const int dout = P.d_out[l];
       const int rows = (dout + 31) & ~31;
       const int upr = din >> 2;  // 8-byte units per row
@@ -191,20 +193,23 @@ __global__ __launch_bounds__(SGM_NT, 4) void k_hash_sig_mfma(sig_params P, int n
 
   const char* xbase = (const char*)P.x + ((int64_t)b * P.xs_b + (int64_t)hx * P.xs_h + 8 * g) * 2;
   uint2* codes = (uint2*)P.codes + ((int64_t)b * P.Hq + h) * P.code_pitch + P.code_offset;
-
-  for (int t = 0; t < tiles_per_wg; ++t) {
-    const int v0 = (chunk * tiles_per_wg + t) * SGM_TILE + wave * 32;  // first vector of this wave
-    if (v0 >= P.L) break;                                               // uniform across the wave
-    int vec = v0 + i32;
-    const bool live = vec < P.L;
-    if (!live) vec = P.L - 1;  // computed and dropped
-    // B operand of the first layer: 8 consecutive elements of the vector per 16-element step
-    uint4 bop[SGM_MAXK];
+  const int k0 = P.D >> 4;
+  // B operand of the first layer: 8 consecutive elements of the vector per 16-element step (a vector past the end: the
+  // last one again, computed and dropped)
+  uint4 bop[SGM_MAXK];
+  auto request = [&](int t) {
+    const int vec = t * 32 + i32 < P.L ? t * 32 + i32 : P.L - 1;
     const char* xrow = xbase + (int64_t)vec * P.xs_l * 2;
-    const int k0 = P.D >> 4;
 #pragma unroll
     for (int s = 0; s < SGM_MAXK; ++s) bop[s] = s < k0 ? *(const uint4*)(xrow + s * 32) : make_uint4(0u, 0u, 0u, 0u);
+  };
 
+  int t_end = (P.L + 31) >> 5;
+  if (t_end > (chunk + 1) * wg_tiles) t_end = (chunk + 1) * wg_tiles;
+  int t = chunk * wg_tiles + wave;
+  if (t >= t_end) return;
+  request(t);
+  for (; t < t_end; t += SGM_NW) {  // uniform across the wave
     int ksteps = k0;
 #pragma unroll
     for (int l = 0; l < SAH_MAX_MLP_LAYERS; ++l) {
@@ -228,8 +233,8 @@ __global__ __launch_bounds__(SGM_NT, 4) void k_hash_sig_mfma(sig_params P, int n
         return acc;
       };
       if (!last) {
-        // bias, activation, rounding as torch rounds them; the result is the next layer's B operand. Two tiles at a
-        // time: their accumulators, this layer's operand and the next one's are all that is live (four waves per SIMD)
+        // bias, activation, rounding as torch rounds them; the result is the next layer's B operand. One tile at a
+        // time: its accumulator, this layer's operand and the next one's are all that is live (four waves per SIMD)
         uint4 nxt[SGM_MAXK];
 #pragma unroll
         for (int q = 0; q < SGM_MAXM; ++q) {
@@ -241,10 +246,10 @@ __global__ __launch_bounds__(SGM_NT, 4) void k_hash_sig_mfma(sig_params P, int n
               const float4 b4 = *(const float4*)(bl + q * 32 + 8 * v4);  // four biases in one read
               const float bb[4] = {b4.x, b4.y, b4.z, b4.w};
 #pragma unroll
-              for (int t = 0; t < 4; ++t) {
-                float z = sah_round<DT>(acc[4 * v4 + t]);
-                z = sah_round<DT>(z + bb[t]);
-                y[4 * v4 + t] = sig_act_fast(ACT, z);  // rounded by the packing below
+              for (int e = 0; e < 4; ++e) {
+                float z = sah_round1<DT>(acc[4 * v4 + e]);
+                z = sah_round1<DT>(z + bb[e]);
+                y[4 * v4 + e] = sig_act_fast(ACT, z);  // rounded by the packing below
               }
             }
           } else {
@@ -262,20 +267,142 @@ __global__ __launch_bounds__(SGM_NT, 4) void k_hash_sig_mfma(sig_params P, int n
       } else {
         // sign planes: this lane holds 16 of the vector's bits, lane ^ 32 the other 16
         sah_f32x16 acc0 = tile(0);
+        request(t + SGM_NW);  // (the operand registers are free: the next vectors arrive during the epilogue)
         uint32_t pos = 0u, nz = 0u;
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-          float z = sah_round<DT>(acc0[v]);
-          z = sah_round<DT>(z + bl[8 * (v >> 2) + (v & 3)]);
+          float z = sah_round1<DT>(acc0[v]);
+          z = sah_round1<DT>(z + bl[8 * (v >> 2) + (v & 3)]);
           const int bit = 8 * (v >> 2) + 4 * g + (v & 3);
           pos |= (z > 0.f ? 1u : 0u) << bit;
           nz |= (z != 0.f ? 1u : 0u) << bit;
         }
         pos |= __shfl_xor(pos, 32);
         nz |= __shfl_xor(nz, 32);
-        if (g == 0 && live) codes[v0 + i32] = make_uint2(pos, nz);
+        if (g == 0 && t * 32 + i32 < P.L) codes[t * 32 + i32] = make_uint2(pos, nz);
       }
     }
+  }
+}
+
+// The usual MLP: head_dim 128, layers of 128, 128 and 32 outputs. Its shape is known at compile time, and the matrix
+// instructions of a tile stand between the vector instructions of the epilogue of the tile before it: two elements to a matrix
+// instruction. Spaced like this they take 6 to 7 cycles of the SIMD's issue; eight in a row take 12 each at four waves a
+// SIMD (and 32 at one), since a wave that waits for the matrix unit keeps the issue port. Roundings are one instruction each
+// (sah_round1). What bounds it: vector issue, 1262 instructions per 32 vectors, 256 of them exponentials and reciprocals at half
+// rate: 88 % of the cycles of its steady state. 8 x 32 heads x 32768 keys: 1050 -> 900 us, 32 heads x 32801 keys 165 -> 137.
+#define SGU_PITCH (128 + SGM_PAD)
+#define SGU_ROWS (128 + 128 + 32)
+template <int DT, int ACT>
+__global__ __launch_bounds__(SGM_NT, 4) void k_hash_sig_usual(sig_params P, int n_chunks, int wg_tiles) {
+  __shared__ uint4 s_raw[SGU_ROWS * SGU_PITCH / 8];  // W^T of the three layers
+  __shared__ float s_bias[SGU_ROWS];
+  const int tid = threadIdx.x;
+  const int lane = tid & (SAH_WAVE - 1);
+  const int wave = sah_wave_id();
+  const int i32 = lane & 31;
+  const int g = lane >> 5;
+  int idx = blockIdx.x;  // as above
+  const int hq = idx % P.group;
+  idx /= P.group;
+  const int chunk = idx % n_chunks;
+  idx /= n_chunks;
+  const int Hx = P.Hq / P.group;
+  const int hx = idx % Hx;
+  const int b = idx / Hx;
+  const int h = hx * P.group + hq;
+
+  const char* xbase = (const char*)P.x + ((int64_t)b * P.xs_b + (int64_t)hx * P.xs_h + 8 * g) * 2;
+  uint2* codes = (uint2*)P.codes + ((int64_t)b * P.Hq + h) * P.code_pitch + P.code_offset;
+  uint4 bop[8], nxt[8];
+  auto request = [&](int t) {  // (past the end: the last vector again, dropped)
+    const int vec = t * 32 + i32 < P.L ? t * 32 + i32 : P.L - 1;
+    const char* xrow = xbase + (int64_t)vec * P.xs_l * 2;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) bop[s] = *(const uint4*)(xrow + s * 32);
+  };
+  int t = chunk * wg_tiles + wave;
+  request(t);
+
+  {  // stage the weights: rows of the second and third layer in the order of their operands
+    uint16_t* const s_w = (uint16_t*)s_raw;
+#pragma unroll
+    for (int l = 0; l < 3; ++l) {
+      const int dout = l < 2 ? 128 : 32;
+      const uint16_t* wt = (const uint16_t*)P.Wt[l] + (int64_t)h * dout * 128;
+#pragma unroll
+      for (int u = tid; u < dout * 32; u += SGM_NT) {
+        const int row = u >> 5, c4 = u & 31, sub = c4 & 3;
+        const int dsub = (l > 0 && (sub == 1 || sub == 2)) ? (sub ^ 3) : sub;
+        *(uint2*)(s_w + (l * 128 + row) * SGU_PITCH + (c4 >> 2) * 16 + dsub * 4) = *(const uint2*)(wt + row * 128 + c4 * 4);
+      }
+      if (tid < dout) s_bias[l * 128 + tid] = sah_load<DT>(P.bias[l], (int64_t)h * dout + tid);
+    }
+  }
+  __syncthreads();
+
+  int t_end = (P.L + 31) >> 5;
+  if (t_end > (chunk + 1) * wg_tiles) t_end = (chunk + 1) * wg_tiles;
+  const uint16_t* const wl = (const uint16_t*)s_raw + i32 * SGU_PITCH + 8 * g;
+  const float* const bl = s_bias + 4 * g;
+  auto a_op = [&](int l, int q, int s) { return *(const uint4*)(wl + (l * 128 + q * 32) * SGU_PITCH + s * 16); };
+  for (; t < t_end; t += SGM_NW) {  // uniform across the wave
+    sah_f32x16 acc = {};
+#pragma unroll
+    for (int s = 0; s < 8; ++s) acc = sah_mfma_32x32x16<DT>(a_op(0, 0, s), bop[s], acc);
+#pragma unroll
+    for (int l = 0; l < 2; ++l) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        // the tile after this one: of the same layer, or the next layer's first, whose operands are there but for the last two
+        const int nl = q < 3 ? l : l + 1, nq = q < 3 ? q + 1 : 0;
+        sah_f32x16 ahead = {};
+        uint4 a = a_op(nl, nq, 0);
+        float2 bias = *(const float2*)(bl + l * 128 + q * 32);
+        uint32_t word[8];
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+          uint4 a2 = a;
+          float2 bias2 = bias;
+          if (s < 7) {
+            a2 = a_op(nl, nq, s + 1);
+            bias2 = *(const float2*)(bl + l * 128 + q * 32 + 8 * ((s + 1) >> 1) + 2 * ((s + 1) & 1));
+          }
+          if (q < 3) ahead = sah_mfma_32x32x16<DT>(a, bop[s], ahead);
+          else if (s < 6) ahead = sah_mfma_32x32x16<DT>(a, nxt[s], ahead);
+          const float z0 = sah_round1<DT>(sah_round1<DT>(acc[2 * s]) + bias.x);
+          const float z1 = sah_round1<DT>(sah_round1<DT>(acc[2 * s + 1]) + bias.y);
+          word[s] = sah_pack2_hw<DT>(sig_act_fast(ACT, z0), sig_act_fast(ACT, z1));
+          if (q < 3 || s < 6) {
+            a = a2;
+          }
+          bias = bias2;
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        nxt[2 * q] = make_uint4(word[0], word[1], word[2], word[3]);
+        nxt[2 * q + 1] = make_uint4(word[4], word[5], word[6], word[7]);
+        if (q == 3) {
+          ahead = sah_mfma_32x32x16<DT>(a, nxt[6], ahead);
+          ahead = sah_mfma_32x32x16<DT>(a_op(nl, nq, 7), nxt[7], ahead);
+        }
+        acc = ahead;
+      }
+#pragma unroll
+      for (int s = 0; s < 8; ++s) bop[s] = nxt[s];
+    }
+    request(t + SGM_NW);  // (the operand registers are free)
+    uint32_t pos = 0u, nz = 0u;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const float z = sah_round1<DT>(sah_round1<DT>(acc[v]) + bl[256 + 8 * (v >> 2) + (v & 3)]);
+      pos |= (z > 0.f ? 1u : 0u) << (8 * (v >> 2) + (v & 3));
+      nz |= (z != 0.f ? 1u : 0u) << (8 * (v >> 2) + (v & 3));
+    }
+    pos <<= 4 * g;
+    nz <<= 4 * g;
+    pos |= __shfl_xor(pos, 32);
+    nz |= __shfl_xor(nz, 32);
+    if (g == 0 && t * 32 + i32 < P.L) codes[t * 32 + i32] = make_uint2(pos, nz);
   }
 }
 
@@ -304,17 +431,44 @@ static bool sig_mfma_ok(const sah_hash_sig_args* a) {
   return sgm_lds_bytes(a) <= 150 * 1024;
 }
 
+// Workgroups per head: of all counts the one that should take least time. Two workgroups fit a CU; a round takes a workgroup's
+// tiles, half of that from the waves that have one more than the others, and staging the weights as long as eight tiles.
+// 32 heads (in us, before: 256-vector tiles, eight to a workgroup; now): 1024 keys 47 -> 13, 8112 keys 92 -> 41, 16405 keys
+// 145 -> 86, 32801 keys (17 workgroups a head, 544 on 512 places) 165 -> 137.
+static int sgm_chunks(int64_t heads, int n_tiles) {
+  const int slots = 512, most = (n_tiles + SGM_NW - 1) / SGM_NW;  // a tile a wave
+  int best = 1;
+  int64_t best_cost = INT64_MAX;
+  for (int c = 1; c <= most && c <= 4 * slots; ++c) {
+    const int tiles = (n_tiles + c - 1) / c, per_wave = (tiles + SGM_NW - 1) / SGM_NW;
+    const int64_t cost = ((heads * c + slots - 1) / slots) * (tiles + SGM_NW * per_wave + 2 * SGM_NW);
+    if (cost < best_cost) {
+      best = c;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
 template <int DT, int ACT>
 static int sig_launch_mfma_a(const sah_hash_sig_args* a, const sig_params& P) {
-  if (int rc = sah_allow_lds((const void*)k_hash_sig_mfma<DT, ACT>, 150 * 1024, "sah_hash_signatures")) return rc;
-  const int n_tiles = (a->L + SGM_TILE - 1) / SGM_TILE;
-  const int tiles_per_wg = n_tiles < 8 ? n_tiles : 8;   // the staged weights serve up to 8 tiles
-  const int n_chunks = (n_tiles + tiles_per_wg - 1) / tiles_per_wg;
-  const int64_t n_wg = (int64_t)a->B * a->Hq * n_chunks;
+  const int64_t heads = (int64_t)a->B * a->Hq;
+  const int n_tiles = (a->L + 31) / 32;
+  int n_chunks = sgm_chunks(heads, n_tiles);
+  const int wg_tiles = (n_tiles + n_chunks - 1) / n_chunks;
+  n_chunks = (n_tiles + wg_tiles - 1) / wg_tiles;
+  const int64_t n_wg = heads * n_chunks;
   if (n_wg > 0x7fffffff) return sah_fail(SAH_ESHAPE, "sah_hash_signatures: too many workgroups");
   sah_timed timed("k_hash_sig_mfma", a->stream);
-  hipLaunchKernelGGL((k_hash_sig_mfma<DT, ACT>), dim3((unsigned)n_wg), dim3(SGM_NT), sgm_lds_bytes(a), (hipStream_t)a->stream, P,
-                     n_chunks, tiles_per_wg);
+  const dim3 grid((unsigned)n_wg), block(SGM_NT);
+  // (GELU's error function does not fit the registers beside two tiles)
+  constexpr int UACT = ACT == SAH_ACT_GELU ? SAH_ACT_RELU : ACT;
+  if (ACT == UACT && a->D == 128 && a->n_layers == 3 && a->d_out[0] == 128 && a->d_out[1] == 128 && a->d_out[2] == 32) {
+    hipLaunchKernelGGL((k_hash_sig_usual<DT, UACT>), grid, block, 0, (hipStream_t)a->stream, P, n_chunks, wg_tiles);
+  } else {
+    if (int rc = sah_allow_lds((const void*)k_hash_sig_mfma<DT, ACT>, 150 * 1024, "sah_hash_signatures")) return rc;
+    hipLaunchKernelGGL((k_hash_sig_mfma<DT, ACT>), grid, block, sgm_lds_bytes(a), (hipStream_t)a->stream, P, n_chunks, wg_tiles);
+  }
   return sah_launch_status("sah_hash_signatures");
 }
 
