@@ -429,17 +429,44 @@ extern "C" int sah_hash_decode_attention(const sah_hash_decode_args* a, const sa
 // ---------------------------------------------------------------------------
 // Compact form of the key-code stream: sign planes and the list of columns with a zero component.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_hash_compact(const uint2* codes, int64_t code_pitch, int from, int to, uint32_t* pos,
-                                                      int64_t pos_pitch, uint4* exc, int exc_cap, int* exc_cnt,
-                                                      uint32_t full_plane) {
+// A workgroup takes 2048 columns of a row and its place in the list by one atomic: an atomic per entry, all of a row's at one
+// address, took the kernel 25 us for 128 rows of 12011 keys (1.6 % of them with a zero component), now 8.
+#define HCP_NT 256
+#define HCP_PER 8
+__global__ __launch_bounds__(HCP_NT) void k_hash_compact(const uint2* codes, int64_t code_pitch, int from, int to, uint32_t* pos,
+                                                         int64_t pos_pitch, uint4* exc, int exc_cap, int* exc_cnt, uint32_t full_plane) {
+  __shared__ int s_cnt, s_base;
   const int r = blockIdx.y;
-  const int j = from + blockIdx.x * 256 + threadIdx.x;
-  if (j >= to) return;
-  const uint2 c = codes[(int64_t)r * code_pitch + j];
-  pos[(int64_t)r * pos_pitch + j] = c.x;
-  if (c.y != full_plane) {
-    const int slot = atomicAdd(&exc_cnt[r], 1);
-    if (slot < exc_cap) exc[(int64_t)r * exc_cap + slot] = make_uint4((uint32_t)j, c.y, c.x, 0u);
+  const int j0 = from + blockIdx.x * (HCP_NT * HCP_PER) + threadIdx.x;
+  if (threadIdx.x == 0) s_cnt = 0;
+  __syncthreads();
+  uint2 c[HCP_PER];
+#pragma unroll
+  for (int u = 0; u < HCP_PER; ++u) {
+    const int j = j0 + u * HCP_NT;
+    c[u] = codes[(int64_t)r * code_pitch + (j < to ? j : to - 1)];
+  }
+  int mine = 0;
+#pragma unroll
+  for (int u = 0; u < HCP_PER; ++u) {
+    const int j = j0 + u * HCP_NT;
+    if (j < to) {
+      pos[(int64_t)r * pos_pitch + j] = c[u].x;
+      mine += c[u].y != full_plane ? 1 : 0;
+    }
+  }
+  int at = mine ? atomicAdd(&s_cnt, mine) : 0;
+  __syncthreads();
+  if (threadIdx.x == 0) s_base = s_cnt ? atomicAdd(&exc_cnt[r], s_cnt) : 0;
+  __syncthreads();
+  at += s_base;
+#pragma unroll
+  for (int u = 0; u < HCP_PER; ++u) {
+    const int j = j0 + u * HCP_NT;
+    if (j < to && c[u].y != full_plane) {
+      if (at < exc_cap) exc[(int64_t)r * exc_cap + at] = make_uint4((uint32_t)j, c[u].y, c[u].x, 0u);
+      ++at;
+    }
   }
 }
 
@@ -452,7 +479,7 @@ extern "C" int sah_hash_compact_codes(const sah_hash_compact_args* a) {
   if (a->exc_cap < 1 || ((uintptr_t)a->exc % 16)) return sah_fail(SAH_EINVAL, "sah_hash_compact_codes: exception list unaligned or empty");
   if (a->to == a->from) return SAH_OK;
   sah_timed timed("k_hash_compact", a->stream);
-  hipLaunchKernelGGL(k_hash_compact, dim3((a->to - a->from + 255) / 256, a->n_rows), dim3(256), 0, (hipStream_t)a->stream,
+  hipLaunchKernelGGL(k_hash_compact, dim3((a->to - a->from + HCP_NT * HCP_PER - 1) / (HCP_NT * HCP_PER), a->n_rows), dim3(HCP_NT), 0, (hipStream_t)a->stream,
                      (const uint2*)a->codes, a->code_pitch, a->from, a->to, a->pos_codes, a->pos_pitch, (uint4*)a->exc,
                      a->exc_cap, a->exc_cnt, a->full_plane);
   return sah_launch_status("sah_hash_compact_codes");

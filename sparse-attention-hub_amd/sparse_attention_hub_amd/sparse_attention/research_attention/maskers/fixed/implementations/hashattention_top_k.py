@@ -86,13 +86,13 @@ class PackedSignatureCache:
 
     def ensure_compact_buffers(self) -> None:
         """Buffers of the compact form, sized for the current capacity (8192 columns of slack for the
-        kernel's whole-chunk reads)."""
+        kernel's whole-chunk reads, whose scores count nowhere)."""
         if self.pos is not None:
             return
         B, H = self.codes.shape[0], self.codes.shape[1]
         dev = self.codes.device
         pitch = self.capacity + 8192
-        self.pos = torch.zeros((B, H, pitch), dtype=torch.int32, device=dev)
+        self.pos = torch.empty((B, H, pitch), dtype=torch.int32, device=dev)
         self.exc = torch.empty((B, H, max(1024, self.capacity // 16), 4), dtype=torch.int32, device=dev)
         self.exc_cnt = torch.zeros((B, H), dtype=torch.int32, device=dev)
         self.n_compact = 0
