@@ -62,6 +62,20 @@ typedef struct sah_amask_read_args {
 } sah_amask_read_args;
 int sah_amask_read(sah_amask_read_args* a);
 
+/* sah_hash_decode_attention under an additive mask (attention.amask, of the queries' type) that holds nothing but 0, the
+ * type's lowest value and -inf, in one kernel: the selection ranks a column at the lowest value below every other one (as the
+ * sum of score and mask does) and leaves out one at -inf, whose weight is 0. fits says whether one kernel runs the step: fp32
+ * or bf16, skip_bitmap set, no key_sig, the compact form given, and what else sah_hash_decode_attention needs for it; with ask != 0
+ * the call only says so, otherwise a step that does not fit is refused. */
+typedef struct sah_hash_decode_masked_args {
+  const sah_hash_decode_args* decode;
+  const sah_attention_args* attention;
+  uint32_t* tickets;
+  int32_t ask;
+  int32_t fits;  /* out */
+} sah_hash_decode_masked_args;
+int sah_hash_decode_masked(sah_hash_decode_masked_args* m);
+
 #ifdef __cplusplus
 }
 #endif

@@ -50,20 +50,48 @@ struct hdec_params {
   uint32_t full_plane;
 };
 
+// Columns c0 .. c0 + 7 of a mask row: bit c of `hidden` the type's lowest value, of `never` -inf
+template <int DT>
+__device__ __forceinline__ void hdec_hidden_byte(const void* mask, int c0, int n, uint32_t& hidden, uint32_t& never) {
+  auto take = [&](int c, float x) {
+    hidden |= (x != 0.f && x != -INFINITY ? 1u : 0u) << c;
+    never |= (x == -INFINITY ? 1u : 0u) << c;
+  };
+  if (DT != SAH_F32 && c0 + 8 <= n) {
+    const sah_u4 w = *(const sah_u4_any*)((const char*)mask + (int64_t)c0 * 2);  // (the row may start at any element)
+    if (((w.x | w.y | w.z | w.w) & 0x7fff7fffu) == 0u) return;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      take(2 * t, sah_bits_to_float(w[t] << 16));
+      take(2 * t + 1, sah_bits_to_float(w[t] & 0xffff0000u));
+    }
+  } else {
+#pragma unroll
+    for (int c = 0; c < 8; ++c)
+      if (c0 + c < n) take(c, sah_load<DT>(mask, c0 + c));
+  }
+}
+
 // The mask row r of one decode step; returns its entry count. s_cols (optional, LDS, R.cap ints): copy of the
 // row's column list for a caller that continues with it in the same kernel (complete after its next barrier).
 // CP: the codes are read in their compact form (one sign plane per column + exception list).
 // SILU: both MLPs use SiLU and have the usual shape, 128 -> 128 -> 128 -> 32 (checked by the host): the matrix-core form
 // then carries no other activation's code and knows every width at compile time
-template <int DT, bool MF, bool CP, bool SILU = false>
-__device__ __forceinline__ int hdec_row(const hdec_params& P, int r, hsw_lds& S, unsigned char* hdec_dyn, int* s_cols) {
+// HID: the step runs under an additive mask of nothing but 0, the type's lowest value and -inf; `mask` is the row's. Its columns
+// become two bitmaps while the MLP computes: the ones at the lowest value rank below every other column (a score added to
+// the lowest value of bf16 or fp32 is that value again), the ones at -inf, whose weight is 0 wherever another column has one,
+// count as active. (s_bm then holds more than the row: update_bitmap must be 0.)
+template <int DT, bool MF, bool CP, bool SILU = false, bool HID = false>
+__device__ __forceinline__ int hdec_row(const hdec_params& P, int r, hsw_lds& S, unsigned char* hdec_dyn, int* s_cols,
+                                        const void* mask = nullptr) {
   typedef typename hdec_sig<MF>::lds hdec_sig_lds;
   const sah_rows& R = P.R;
   const int tid = threadIdx.x;
   const int n = R.n_keys;
   const int n_ch = (n + 255) / 256;
   uint32_t* s_bm = (uint32_t*)hdec_dyn;
-  uint32_t* s_key = s_bm + n_ch * 8;
+  uint32_t* s_hid = s_bm + n_ch * 8;  // HID only
+  uint32_t* s_key = s_hid + (HID ? n_ch * 8 : 0);
   // the MLP scratch shares the space of the staged scores: the MLPs are over before staging starts
   hdec_sig_lds* s_sig = (hdec_sig_lds*)s_key;
 
@@ -86,8 +114,22 @@ __device__ __forceinline__ int hdec_row(const hdec_params& P, int r, hsw_lds& S,
       if (s_cols) s_cols[i] = i < s_hi ? i : lo2 + (i - s_hi);
       if (R.w) R.w[(int64_t)r * R.cap + i] = 1.0f;
     }
-    for (int wi = tid; wi < n_ch * 8; wi += HSW_NT)
-      s_bm[wi] = wi < R.n_words ? (sah_range_bits(wi, 0, s_hi) | sah_range_bits(wi, lo, hi)) : 0u;
+    if constexpr (HID) {
+      // by the half of the workgroup that has no MLP to run
+      if (tid >= HDEC_GROUP) {
+        for (int u = tid - HDEC_GROUP; u < n_ch * 32; u += HSW_NT - HDEC_GROUP) {
+          const int wi = u >> 2;
+          uint32_t hidden = 0u, never = 0u;
+          hdec_hidden_byte<DT>(mask, u * 8, n, hidden, never);
+          never |= ((wi < R.n_words ? (sah_range_bits(wi, 0, s_hi) | sah_range_bits(wi, lo, hi)) : 0u) >> (8 * (u & 3))) & 0xffu;
+          ((unsigned char*)s_hid)[u] = (unsigned char)hidden;
+          ((unsigned char*)s_bm)[u] = (unsigned char)never;
+        }
+      }
+    } else {
+      for (int wi = tid; wi < n_ch * 8; wi += HSW_NT)
+        s_bm[wi] = wi < R.n_words ? (sah_range_bits(wi, 0, s_hi) | sah_range_bits(wi, lo, hi)) : 0u;
+    }
   };
 
   // ---- 2. signatures of the query and of the newest key
@@ -135,8 +177,8 @@ __device__ __forceinline__ int hdec_row(const hdec_params& P, int r, hsw_lds& S,
 
   // ---- 3. top-k over the remaining columns
   // the row's active columns are the sink and local ranges just built, nothing else
-  return hsw_select_row<CP>(R, r, kc, q, P.k, fixed < R.cap ? fixed : R.cap, s_bm, s_key, S, buf, early, P.update_bitmap != 0,
-                            s_cols, CP ? &cs : nullptr, s_hi, n_local > 0 ? lo2 : n);
+  return hsw_select_row<CP, HID>(R, r, kc, q, P.k, fixed < R.cap ? fixed : R.cap, s_bm, s_key, S, buf, early, P.update_bitmap != 0,
+                                 s_cols, CP ? &cs : nullptr, s_hi, n_local > 0 ? lo2 : n, s_hid);
 }
 
 template <int DT, bool MF, bool CP, bool SILU>
@@ -155,7 +197,9 @@ __global__ __launch_bounds__(HSW_NT) void k_hash_decode(hdec_params P) {
 // parts > 1 (fewer rows than CUs): every row is given `parts` workgroups. Each builds the whole row by itself (the
 // same arithmetic, so the lists are identical and both write the same values to the row in memory), attends to its
 // share of the list, and the one that arrives last merges the partial results (att_merge_parts).
-template <int DT, bool MF, bool CP, int D, bool SILU>
+// HID: under an additive mask that only hides columns (A.amask; hdec_row). Four layers of a padded batch of 4 at 12K keys, 1024
+// chosen: 193 us with the scores in memory (hashing 7, scores 5, selection and attention 29 a layer), 159 so (31 a layer).
+template <int DT, bool MF, bool CP, int D, bool SILU, bool HID>
 __global__ __launch_bounds__(HSW_NT) void k_hash_decode_attn(hdec_params P, att_params A, int cols_offset, int parts, float* work,
                                                              uint32_t* tickets) {
   __shared__ hsw_lds S;
@@ -177,9 +221,10 @@ __global__ __launch_bounds__(HSW_NT) void k_hash_decode_attn(hdec_params P, att_
   const int h = hk * G + within % G;
   const int r = b * A.Hq + h;
   int* s_cols = (int*)(hdec_dyn + cols_offset);
-  const int cnt = hdec_row<DT, MF, CP, SILU>(P, r, S, hdec_dyn, s_cols);
+  const void* mask = HID ? (const char*)A.amask + ((int64_t)b * A.ms_b + (int64_t)h * A.ms_h) * (DT == SAH_F32 ? 4 : 2) : nullptr;
+  const int cnt = hdec_row<DT, MF, CP, SILU, HID>(P, r, S, hdec_dyn, s_cols, mask);
   __syncthreads();  // the column list in LDS is complete
-  // the whole-row attention over the list in LDS: no additive mask, no weights, no logits output on this path
+  // the whole-row attention over the list in LDS: no weights, no logits output on this path
   {
     constexpr int KPI = SAH_WAVE / (D / 8);
     const int wave = sah_wave_id();
@@ -190,7 +235,7 @@ __global__ __launch_bounds__(HSW_NT) void k_hash_decode_attn(hdec_params P, att_
     att_wave_state st;
     st.clear();
     const float unit = A.unit_inv_w;
-    att_walk<DT, D, false, true>(
+    att_walk<DT, D, false, !HID, true, HID>(
         A, r, b, h, hk, 0, first, bound, SAH_WAVE, [&](int i) { return s_cols[i]; }, [&](int) { return unit; }, st);
     att_park<D, HSW_NW>(st, wave, s_m, s_l, s_acc);
     __syncthreads();
@@ -201,10 +246,10 @@ __global__ __launch_bounds__(HSW_NT) void k_hash_decode_attn(hdec_params P, att_
   }
 }
 
-static size_t hdec_lds_bytes(int n_keys) {
+static size_t hdec_lds_bytes(int n_keys, bool hidden = false) {
   const int n_ch = (n_keys + 255) / 256;
   const size_t a = sizeof(hdec_sig<false>::lds), b = sizeof(hdec_sig<true>::lds);
-  const size_t bm = (size_t)n_ch * 8 * 4, key = (size_t)n_ch * 64 * 4, sig = 2 * (a > b ? a : b);
+  const size_t bm = (size_t)n_ch * 8 * 4 * (hidden ? 2 : 1), key = (size_t)n_ch * 64 * 4, sig = 2 * (a > b ? a : b);
   return bm + (key > sig ? key : sig);
 }
 
@@ -360,22 +405,30 @@ extern "C" int sah_hash_decode_topk(const sah_hash_decode_args* a) {
   }
 }
 
-template <int DT, bool MF, bool CP, int D, bool SILU>
+template <int DT, bool MF, bool CP, int D, bool SILU, bool HID = false>
 static int hdec_attn_launch_s(const sah_hash_decode_args* a, const hdec_params& P, const att_params& A, size_t lds, int cols_offset,
                               int parts, float* work, uint32_t* tickets) {
-  if (int rc = sah_allow_lds((const void*)k_hash_decode_attn<DT, MF, CP, D, SILU>, 150 * 1024, "sah_hash_decode_attention")) return rc;
+  if (int rc = sah_allow_lds((const void*)k_hash_decode_attn<DT, MF, CP, D, SILU, HID>, 150 * 1024, "sah_hash_decode_attention")) return rc;
   const int G = A.Hq / A.Hkv;
   const int n_tiles = P.R.n_rows / G;
   const int n_wg = (n_tiles + ATT_XCDS - 1) / ATT_XCDS * ATT_XCDS * G * parts;
   sah_timed timed("k_hash_decode_attn", a->stream);
-  hipLaunchKernelGGL((k_hash_decode_attn<DT, MF, CP, D, SILU>), dim3(n_wg), dim3(HSW_NT), lds, (hipStream_t)a->stream, P, A, cols_offset,
-                     parts, work, tickets);
+  hipLaunchKernelGGL((k_hash_decode_attn<DT, MF, CP, D, SILU, HID>), dim3(n_wg), dim3(HSW_NT), lds, (hipStream_t)a->stream, P, A,
+                     cols_offset, parts, work, tickets);
   return sah_launch_status("sah_hash_decode_attention");
 }
 
 template <int DT, bool MF, bool CP, int D>
 static int hdec_attn_launch_t(const sah_hash_decode_args* a, const hdec_params& P, const att_params& A, size_t lds, int cols_offset,
                               int parts, float* work, uint32_t* tickets) {
+  if constexpr (CP && DT != SAH_F16) {
+    if (A.amask) {
+      if constexpr (MF) {
+        if (hdec_silu(P)) return hdec_attn_launch_s<DT, MF, CP, D, true, true>(a, P, A, lds, cols_offset, parts, work, tickets);
+      }
+      return hdec_attn_launch_s<DT, MF, CP, D, false, true>(a, P, A, lds, cols_offset, parts, work, tickets);
+    }
+  }
   if constexpr (MF) {
     if (hdec_silu(P)) return hdec_attn_launch_s<DT, MF, CP, D, true>(a, P, A, lds, cols_offset, parts, work, tickets);
   }
@@ -389,6 +442,48 @@ static int hdec_attn_launch(const sah_hash_decode_args* a, const hdec_params& P,
                : hdec_attn_launch_t<DT, MF, false, D>(a, P, A, lds, cols_offset, parts, work, tickets);
 }
 
+// One step: its LDS, its workgroups per row, and whether one kernel can run it (t->amask aside)
+struct hdec_attn_plan {
+  size_t cols_offset, lds;
+  int parts;
+  bool one_kernel;
+};
+
+static hdec_attn_plan hdec_attn_shape(const sah_hash_decode_args* a, const sah_attention_args* t, const att_params& A,
+                                      const uint32_t* tickets, bool hidden) {
+  hdec_attn_plan p;
+  p.cols_offset = (hdec_lds_bytes(a->rows.n_keys, hidden) + 15) & ~(size_t)15;
+  p.lds = p.cols_offset + (size_t)a->rows.cap * 4;
+  // rows fewer than CUs: several workgroups per row, if the caller brought the tickets and the workspace for it
+  p.parts = att_row_parts(a->rows.n_rows);
+  const bool shared_rows = p.parts > 1 && tickets && t->work && t->work_floats >= (int64_t)a->rows.n_rows * p.parts * (t->D + 2);
+  if (!shared_rows) p.parts = 1;
+  p.one_kernel =
+      hdec_fusable(a) && (shared_rows || A.n_split == 0) && !t->dense && !t->closed_form && !t->logits_out && !t->rows.w && t->Lq == 1 &&
+      t->dropout_p == 0.f &&
+      t->rows.cols == a->rows.cols && t->rows.cnt == a->rows.cnt && t->rows.cap == a->rows.cap &&
+      t->rows.n_rows == a->rows.n_rows && t->stream == a->stream && t->dtype == a->query_sig->dtype &&
+      (t->D == 128 || t->D == 64) && p.lds <= 150 * 1024;
+  return p;
+}
+
+static int hdec_attn_run(const sah_hash_decode_args* a, const sah_attention_args* t, const att_params& A, const hdec_attn_plan& p,
+                         uint32_t* tickets) {
+  const bool has_key = a->key_sig && a->key_sig->L > 0;
+  hdec_params P;
+  hdec_fill(a, P);
+  const bool mf = hdec_sig_kind(a, has_key) == 2;
+#define SAH_HDA(DTC, MFC)                                                                                       \
+  (t->D == 128 ? hdec_attn_launch<DTC, MFC, 128>(a, P, A, p.lds, (int)p.cols_offset, p.parts, t->work, tickets) \
+               : hdec_attn_launch<DTC, MFC, 64>(a, P, A, p.lds, (int)p.cols_offset, p.parts, t->work, tickets))
+  switch (t->dtype) {
+    case SAH_F32: return SAH_HDA(SAH_F32, false);
+    case SAH_BF16: return mf ? SAH_HDA(SAH_BF16, true) : SAH_HDA(SAH_BF16, false);
+    default: return mf ? SAH_HDA(SAH_F16, true) : SAH_HDA(SAH_F16, false);
+  }
+#undef SAH_HDA
+}
+
 extern "C" int sah_hash_decode_attention(const sah_hash_decode_args* a, const sah_attention_args* t, uint32_t* tickets) {
   if (!a || !t) return sah_fail(SAH_ENULL, "sah_hash_decode_attention: args is NULL");
   int rc = hdec_validate(a);
@@ -396,34 +491,30 @@ extern "C" int sah_hash_decode_attention(const sah_hash_decode_args* a, const sa
   att_params A;
   rc = att_prepare(t, A);
   if (rc) return rc;
-  const bool has_key = a->key_sig && a->key_sig->L > 0;
-  const size_t cols_offset = (hdec_lds_bytes(a->rows.n_keys) + 15) & ~(size_t)15;
-  const size_t lds = cols_offset + (size_t)a->rows.cap * 4;
-  // rows fewer than CUs: several workgroups per row, if the caller brought the tickets and the workspace for it
-  const int parts = att_row_parts(a->rows.n_rows);
-  const bool shared_rows = parts > 1 && tickets && t->work && t->work_floats >= (int64_t)a->rows.n_rows * parts * (t->D + 2);
-  const bool one_kernel =
-      hdec_fusable(a) && (shared_rows || A.n_split == 0) && !t->dense && !t->closed_form && !t->amask && !t->logits_out && !t->rows.w && t->Lq == 1 &&
-      t->dropout_p == 0.f &&
-      t->rows.cols == a->rows.cols && t->rows.cnt == a->rows.cnt && t->rows.cap == a->rows.cap &&
-      t->rows.n_rows == a->rows.n_rows && t->stream == a->stream && t->dtype == a->query_sig->dtype &&
-      (t->D == 128 || t->D == 64) && lds <= 150 * 1024;
-  if (!one_kernel) {
+  const hdec_attn_plan p = hdec_attn_shape(a, t, A, tickets, false);
+  if (!p.one_kernel || t->amask) {
     if ((rc = sah_hash_decode_topk(a))) return rc;
     return sah_sparse_attention(t);
   }
-  hdec_params P;
-  hdec_fill(a, P);
-  const bool mf = hdec_sig_kind(a, has_key) == 2;
-#define SAH_HDA(DTC, MFC)                                                                    \
-  (t->D == 128 ? hdec_attn_launch<DTC, MFC, 128>(a, P, A, lds, (int)cols_offset, shared_rows ? parts : 1, t->work, tickets)  \
-               : hdec_attn_launch<DTC, MFC, 64>(a, P, A, lds, (int)cols_offset, shared_rows ? parts : 1, t->work, tickets))
-  switch (t->dtype) {
-    case SAH_F32: return SAH_HDA(SAH_F32, false);
-    case SAH_BF16: return mf ? SAH_HDA(SAH_BF16, true) : SAH_HDA(SAH_BF16, false);
-    default: return mf ? SAH_HDA(SAH_F16, true) : SAH_HDA(SAH_F16, false);
-  }
-#undef SAH_HDA
+  return hdec_attn_run(a, t, A, p, tickets);
+}
+
+extern "C" int sah_hash_decode_masked(sah_hash_decode_masked_args* m) {
+  if (!m) return sah_fail(SAH_ENULL, "sah_hash_decode_masked: args is NULL");
+  const sah_hash_decode_args* a = m->decode;
+  const sah_attention_args* t = m->attention;
+  if (!a || !t || !t->amask) return sah_fail(SAH_ENULL, "sah_hash_decode_masked: decode / attention / attention.amask is NULL");
+  int rc = hdec_validate(a);
+  if (rc) return rc;
+  att_params A;
+  rc = att_prepare(t, A);
+  if (rc) return rc;
+  const hdec_attn_plan p = hdec_attn_shape(a, t, A, m->tickets, true);
+  // (fp16: a score added to the lowest value is not that value again)
+  m->fits = p.one_kernel && t->dtype != SAH_F16 && a->skip_bitmap && !(a->key_sig && a->key_sig->L > 0) && hdec_compact_ok(a) ? 1 : 0;
+  if (m->ask) return SAH_OK;
+  if (!m->fits) return sah_fail(SAH_ESHAPE, "sah_hash_decode_masked: not a step that one kernel runs");
+  return hdec_attn_run(a, t, A, p, m->tickets);
 }
 
 // ---------------------------------------------------------------------------

@@ -159,11 +159,16 @@ __device__ __forceinline__ void hsw_prefetch(const hsw_compact& cs, int n, hsw_b
 // active_below / active_from (both >= 0): the caller knows that the row's active columns are exactly
 // [0, active_below) and [active_from, n) (the sink and local columns of a fresh decode row); chunks that lie between
 // the two ranges then skip the bitmap test of every word.
-template <bool CP = false>
+// HID: an additive mask hides the columns of the bitmap s_hid (as s_bm, complete at the same barrier): they rank below every
+// other column, as equals; their byte is 1 and a score's is score + 34.
+template <bool CP = false, bool HID = false>
 __device__ __forceinline__ int hsw_select_row(const sah_rows& R, int r, const uint2* kc, const uint2 q, int k, int cnt0,
                                               uint32_t* s_bm, uint32_t* s_key, hsw_lds& S, hsw_bufs_t<CP>& buf,
                                               bool prefetched = false, bool update_bitmap = true, int* s_cols = nullptr,
-                                              const hsw_compact* cs = nullptr, int active_below = -1, int active_from = -1) {
+                                              const hsw_compact* cs = nullptr, int active_below = -1, int active_from = -1,
+                                              const uint32_t* s_hid = nullptr) {
+  static_assert(CP || !HID, "hidden columns: compact stream only");
+  constexpr uint32_t ZERO = HID ? 34u : 33u;  // byte of score 0
   int* s_gt = S.gt;
   int* s_eq = S.eq;
   const int tid = threadIdx.x;
@@ -186,14 +191,22 @@ __device__ __forceinline__ int hsw_select_row(const sah_rows& R, int r, const ui
   const bool ranges_known = active_below >= 0 && active_from >= 0;
   // may chunk c hold an active column? (uniform across the wave)
   auto chunk_may_be_active = [&](int c) { return !ranges_known || c * 256 < active_below || (c + 1) * 256 > active_from; };
+  auto bytes_of = [](uint32_t nib) { return (nib | (nib << 7) | (nib << 14) | (nib << 21)) & 0x01010101u; };  // bit t -> byte t
   auto stage = [&](uint32_t word, int wi, bool check) {
     uint32_t kw = word;
-    if (check) {
+    if constexpr (HID) {
+      const int j0 = wi * 4;
+      const uint32_t nib = (s_bm[j0 >> 5] >> (j0 & 31)) & 0xFu, hid = (s_hid[j0 >> 5] >> (j0 & 31)) & 0xFu;
+      if (__ballot((nib | hid) != 0)) {
+        const uint32_t one = bytes_of(nib | hid);
+        kw = (word & ~((one << 8) - one)) | bytes_of(hid & ~nib);
+      }
+    } else if (check) {
       const int j0 = wi * 4;
       // Most chunks of a long row hold no active column at all: uniform test, the expansion is skipped
       const uint32_t nib = (s_bm[j0 >> 5] >> (j0 & 31)) & 0xFu;  // nibble -> byte mask
       if (__ballot(nib != 0)) {
-        const uint32_t one = (nib | (nib << 7) | (nib << 14) | (nib << 21)) & 0x01010101u;
+        const uint32_t one = bytes_of(nib);
         kw = word & ~((one << 8) - one);
       }
     }
@@ -204,7 +217,7 @@ __device__ __forceinline__ int hsw_select_row(const sah_rows& R, int r, const ui
   };
   if constexpr (CP) {
     // ---- compact stream: every component taken as non-zero, score = popc(q.y) - 2 popc((q.x ^ k.x) & q.y)
-    const uint32_t s_full = (uint32_t)__popc(q.y) + 33u;
+    const uint32_t s_full = (uint32_t)__popc(q.y) + ZERO;
     const uint32_t s_full4 = s_full * 0x01010101u;
     // a query without zero components (the usual case) needs no mask on the differing bits; uniform
     const bool q_dense = q.y == 0xFFFFFFFFu;
@@ -250,8 +263,8 @@ __device__ __forceinline__ int hsw_select_row(const sah_rows& R, int r, const ui
     __syncthreads();  // every word is staged
     unsigned char* s_byte = (unsigned char*)s_key;
     auto patch = [&](int col, uint32_t kx, uint32_t ky) {
-      if (col < n && !((s_bm[col >> 5] >> (col & 31)) & 1u)) {
-        const uint32_t s_new = (uint32_t)(sig_score(q, make_uint2(kx, ky)) + 33);
+      if (col < n && !(((HID ? s_bm[col >> 5] | s_hid[col >> 5] : s_bm[col >> 5]) >> (col & 31)) & 1u)) {
+        const uint32_t s_new = (uint32_t)(sig_score(q, make_uint2(kx, ky)) + (int)ZERO);
         const uint32_t s_old = s_byte[col];
         s_byte[col] = (unsigned char)s_new;
 #pragma unroll

@@ -63,6 +63,7 @@ EXTENSION_SYMBOLS = {
     "sah_members_attention": 1,
     "sah_pq_kmeans": 1,
     "sah_amask_read": 1,
+    "sah_hash_decode_masked": 1,
 }
 
 
@@ -397,6 +398,10 @@ class AmaskReadArgs(C.Structure):
 
 
 AMASK_NONZERO, AMASK_GENERAL = 1, 2
+
+
+class HashDecodeMaskedArgs(C.Structure):
+    _fields_ = [("decode", C.c_void_p), ("attention", C.c_void_p), ("tickets", C.c_void_p), ("ask", C.c_int32), ("fits", C.c_int32)]
 
 
 class AttentionWeightsArgs(C.Structure):

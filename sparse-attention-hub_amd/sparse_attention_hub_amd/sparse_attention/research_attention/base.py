@@ -83,12 +83,16 @@ class ResearchAttention(SparseAttention):
             raise ValueError("sparse_meta_data must be provided in kwargs while calling custom_attention()")
         sparse_meta_data: Dict[Any, Any] = kwargs.pop("sparse_meta_data")
 
+        only_hides = False
         if (attention_mask is not None and attention_mask.is_cuda and attention_mask.dim() == 4
-                and attention_mask.shape[-1] >= keys.shape[2] and attention_mask.dtype in (torch.float32, torch.bfloat16, torch.float16)
-                and self._mask_facts.all_zero(attention_mask)):
-            # an additive mask of zeros (HuggingFace's eager mask of an unpadded decode step) adds nothing anywhere:
-            # established once per mask tensor, i.e. once per forward pass, not per layer
-            attention_mask = None
+                and attention_mask.shape[-1] >= keys.shape[2] and attention_mask.dtype in (torch.float32, torch.bfloat16, torch.float16)):
+            flags = self._mask_facts.flags(attention_mask)
+            # (a lowest value of another type than the queries' is none of theirs)
+            only_hides = not flags & _native.AMASK_GENERAL and attention_mask.dtype == queries.dtype
+            if flags == 0:
+                # an additive mask of zeros (HuggingFace's eager mask of an unpadded decode step) adds nothing anywhere:
+                # established once per mask tensor, i.e. once per forward pass, not per layer
+                attention_mask = None
 
         metrics = MicroMetricLogger()
         want_density = metrics.is_metric_enabled("research_attention_density")
@@ -112,7 +116,7 @@ class ResearchAttention(SparseAttention):
                 plan = self._plans.get(key)
                 if plan is None or plan.owner != owner:
                     plan = self._plans[key] = DecodePlan(self.maskers, self._plan_kind, queries, keys, masked, owner)
-            out = plan.run(queries, keys, values, scaling, sparse_meta_data, kwargs.get("layer_idx"), attention_mask)
+            out = plan.run(queries, keys, values, scaling, sparse_meta_data, kwargs.get("layer_idx"), attention_mask, only_hides)
             if out is not None:
                 return out, None
 

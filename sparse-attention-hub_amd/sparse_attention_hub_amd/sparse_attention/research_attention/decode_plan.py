@@ -94,6 +94,7 @@ class DecodePlan:
         self.hamming = N.HammingTopkArgs()
         self.hash_decode = N.HashDecodeArgs()
         self.scores = N.HammingScoresArgs()
+        self.hash_masked = N.HashDecodeMaskedArgs()
         self.compact = N.HashCompactArgs()
         self.qk = N.QkScoresArgs()
         self.pq_assign = N.PqAssignArgs()
@@ -136,11 +137,78 @@ class DecodePlan:
             self.residbuf = (torch.empty_like(self.keybuf)
                              if self.kind == "oracle" and not self.masked and kdt == torch.int16 and self.D in (64, 128) else None)
 
+    def _use_compact(self, hd: "N.HashDecodeArgs", cache: PackedSignatureCache, hashed: int, stream: int, commit: list) -> None:
+        """The compact form of the first `hashed` codes for `hd`, brought up to date by a launch of the chain's."""
+        cache.ensure_compact_buffers()
+        if hashed > cache.n_compact:
+            cp = self.compact
+            cp.codes, cp.code_pitch, cp.n_rows = cache.codes.data_ptr(), cache.capacity, self.n_rows
+            cp.from_, cp.to = cache.n_compact, hashed
+            cp.pos_codes, cp.pos_pitch = cache.pos.data_ptr(), cache.pos.shape[2]
+            cp.exc, cp.exc_cap, cp.exc_cnt = cache.exc.data_ptr(), cache.exc.shape[2], cache.exc_cnt.data_ptr()
+            cp.full_plane, cp.stream = cache.full_plane, stream
+            self.chain.compact = C.addressof(cp)
+            commit.append((cache, "n_compact", hashed))
+            commit.append((cache, "compact_stream", stream))
+        hd.pos_codes, hd.pos_pitch = cache.pos.data_ptr(), cache.pos.shape[2]
+        hd.exc, hd.exc_cap, hd.exc_cnt = cache.exc.data_ptr(), cache.exc.shape[2], cache.exc_cnt.data_ptr()
+        hd.full_plane = cache.full_plane
+
+    def _hash_masked(self, rows, cache: PackedSignatureCache, hashed: int, k_eff: int, sink: int, window: int, stream: int,
+                     mask_args: Tuple, only_hides: bool, commit: list) -> None:
+        """A HashAttention step under an additive mask; the chain holds the signatures of new keys and of the query, `self.att`
+        the attention."""
+        chain, at = self.chain, self.att
+        # A mask that only hides columns: one kernel. The compact form it reads is kept by steps like this one; a step that
+        # would read what another stream has written, or that is captured and would have to write it, takes the other way.
+        if (only_hides and self.dtype != torch.float16 and cache.compact_stream in (None, stream)
+                and (cache.n_compact >= hashed or not torch.cuda.is_current_stream_capturing())):
+            hd, hm = self.hash_decode, self.hash_masked
+            hd.rows, hd.sink, hd.window, hd.k, hd.stream = rows, sink, window, k_eff, stream
+            hd.query_sig, hd.key_sig, hd.skip_bitmap = chain.sig_b, None, 1
+            hd.kcodes, hd.code_pitch = cache.codes.data_ptr(), cache.capacity
+            hm.decode, hm.attention, hm.tickets = C.addressof(hd), C.addressof(at), self.tickets.data_ptr()
+            done = []
+            self._use_compact(hd, cache, hashed, stream, done)
+            hm.ask = 1
+            N.call("sah_hash_decode_masked", hm)
+            if hm.fits:
+                chain.sig_b = chain.attention = None
+                if chain.sig_a or chain.compact:
+                    N.call("sah_run_chain", chain)
+                hm.ask = 0
+                N.call("sah_hash_decode_masked", hm)
+                commit.extend(done)
+                return
+            chain.compact = None
+        # The mask takes part in the scores: they go through memory as sortable keys, and the selection writes the sink +
+        # local rows itself (the codes of keys that are still inside the window, perhaps not hashed yet, belong to columns it
+        # leaves out).
+        Lk = rows.n_keys
+        self._ensure_keybuf(Lk)
+        sc = self.scores
+        sc.kcodes, sc.code_pitch, sc.qcodes = cache.codes.data_ptr(), cache.capacity, self.qcodes.data_ptr()
+        sc.B, sc.Hq, sc.Lq, sc.n_keys = self.B, self.Hq, self.Lq, Lk
+        sc.amask, sc.ms_b, sc.ms_h, sc.ms_l = mask_args
+        sc.dtype, sc.keys_out, sc.key_pitch, sc.stream = self.dt, self.keybuf.data_ptr(), self.keybuf_pitch, stream
+        se = self.select
+        se.rows, se.keys, se.key_pitch, se.key_bits = rows, self.keybuf.data_ptr(), self.keybuf_pitch, self.key_bits
+        se.n_cand, se.col_offset, se.k, se.excluded_key, se.stream = Lk, 0, k_eff, self._excluded_inf, stream
+        se.skip_bitmap, se.fresh, se.fresh_sink, se.fresh_window = 1, 1, sink, window
+        # signatures, then the masked scores, then selection and attention
+        chain.attention = None
+        N.call("sah_run_chain", chain)
+        N.call("sah_hamming_scores", sc)
+        chain.sig_a = chain.sig_b = None
+        chain.select, chain.attention = C.addressof(se), C.addressof(at)
+        N.call("sah_run_chain", chain)
+
     # --------------------------------------------------------------------- run
     def run(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scaling: float,
             sparse_meta_data: Dict[Any, Any], layer_idx: Optional[int],
-            attention_mask: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
-        """One layer-step; returns the attention output (B, Lq, Hq, D) or None if not applicable."""
+            attention_mask: Optional[torch.Tensor] = None, only_hides: bool = False) -> Optional[torch.Tensor]:
+        """One layer-step; returns the attention output (B, Lq, Hq, D) or None if not applicable. `only_hides`: the mask is known
+        to hold nothing but zeros and entries at the lowest value of its type or -inf."""
         masked = self.masked
         if masked and (self.Lq != 1 or attention_mask.dim() != 4):
             return None
@@ -214,19 +282,6 @@ class DecodePlan:
             bq.xs_b, bq.xs_h, bq.xs_l, bq.stream = q.stride(0), q.stride(1), q.stride(2), stream
             chain.sig_b = C.addressof(bq)
             if masked:
-                # an additive mask takes part in the scores: they go through memory as sortable keys, and the
-                # selection writes the sink + local rows itself (the codes of keys that are still inside the window,
-                # perhaps not hashed yet, belong to columns it leaves out)
-                self._ensure_keybuf(Lk)
-                sc = self.scores
-                sc.kcodes, sc.code_pitch, sc.qcodes = cache.codes.data_ptr(), cache.capacity, self.qcodes.data_ptr()
-                sc.B, sc.Hq, sc.Lq, sc.n_keys = self.B, self.Hq, Lq, Lk
-                sc.amask, sc.ms_b, sc.ms_h, sc.ms_l = am_ptr, am_b, am_h, am_l
-                sc.dtype, sc.keys_out, sc.key_pitch, sc.stream = self.dt, self.keybuf.data_ptr(), self.keybuf_pitch, stream
-                se = self.select
-                se.rows, se.keys, se.key_pitch, se.key_bits = rows, self.keybuf.data_ptr(), self.keybuf_pitch, self.key_bits
-                se.n_cand, se.col_offset, se.k, se.excluded_key, se.stream = Lk, 0, k_eff, self._excluded_inf, stream
-                se.skip_bitmap, se.fresh, se.fresh_sink, se.fresh_window = 1, 1, sink, window
                 chain.sink_local = None
             elif Lq == 1:
                 # the whole mask-building half of the step as one entry point (one kernel when shapes allow);
@@ -240,20 +295,7 @@ class DecodePlan:
                 if use_compact:
                     # keys hashed since the compact form was last brought up to date (by this step's launch in
                     # front of the kernel, by the first call of the layer, by the general path) are added to it
-                    cache.ensure_compact_buffers()
-                    hashed = Lk if hash_now else cache.n
-                    if hashed > cache.n_compact:
-                        cp = self.compact
-                        cp.codes, cp.code_pitch, cp.n_rows = cache.codes.data_ptr(), cache.capacity, self.n_rows
-                        cp.from_, cp.to = cache.n_compact, hashed
-                        cp.pos_codes, cp.pos_pitch = cache.pos.data_ptr(), cache.pos.shape[2]
-                        cp.exc, cp.exc_cap, cp.exc_cnt = cache.exc.data_ptr(), cache.exc.shape[2], cache.exc_cnt.data_ptr()
-                        cp.full_plane, cp.stream = cache.full_plane, stream
-                        chain.compact = C.addressof(cp)
-                        commit.append((cache, "n_compact", hashed))
-                    hd.pos_codes, hd.pos_pitch = cache.pos.data_ptr(), cache.pos.shape[2]
-                    hd.exc, hd.exc_cap, hd.exc_cnt = cache.exc.data_ptr(), cache.exc.shape[2], cache.exc_cnt.data_ptr()
-                    hd.full_plane = cache.full_plane
+                    self._use_compact(hd, cache, Lk if hash_now else cache.n, stream, commit)
                 hd.kcodes, hd.code_pitch, hd.k, hd.stream = cache.codes.data_ptr(), cache.capacity, k_eff, stream
                 hd.skip_bitmap = 1  # only the attention kernel reads these rows, and it reads the column lists
                 chain.hash_decode = C.addressof(hd)
@@ -380,13 +422,10 @@ class DecodePlan:
         chain.attention = C.addressof(at)
         chain.tickets = self.tickets.data_ptr()
         if masked and self.kind == "hash":
-            # signatures, then the masked scores, then selection and attention
-            chain.attention = None
+            self._hash_masked(rows, cache, Lk if hash_now else cache.n, k_eff, sink, window, stream, (am_ptr, am_b, am_h, am_l),
+                              only_hides, commit)
+        else:
             N.call("sah_run_chain", chain)
-            N.call("sah_hamming_scores", self.scores)
-            chain.sig_a = chain.sig_b = None
-            chain.select, chain.attention = C.addressof(self.select), C.addressof(at)
-        N.call("sah_run_chain", chain)
         for obj, name, value in commit:
             setattr(obj, name, value)
         return out

@@ -60,6 +60,7 @@ class PackedSignatureCache:
         # columns with a zero component [B, Hq, exc_cap, 4] and their number [B, Hq]; valid for `n_compact` keys
         self.pos = self.exc = self.exc_cnt = None
         self.n_compact = 0
+        self.compact_stream = None  # the stream of the launch that last wrote the compact form
 
     @property
     def capacity(self) -> int:

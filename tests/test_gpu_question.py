@@ -806,3 +806,97 @@ def test_words_are_clear_before_another_stream_asks(cuda):
 
     with ThreadPoolExecutor(1) as pool:
         pool.submit(first).result()
+
+
+def _hide(m, kind, n, window, lowest):
+    """What the rows of a padded batch hide: left padding; all but a few columns, fewer than the selection takes; all of them;
+    columns here and there, at the lowest value and at -inf."""
+    for b in range(m.shape[0]):
+        if kind == "padded":
+            m[b, ..., : (b + 1) * n // (m.shape[0] + 2)] = lowest
+        elif kind == "few":
+            m[b, ..., : n - window - 20 - b] = lowest
+        elif kind == "none visible":
+            m[b] = lowest if b % 2 == 0 else 0.0
+        else:
+            m[b, ..., b::3] = lowest
+            m[b, ..., 1::7] = -float("inf")
+    return m
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
+@pytest.mark.parametrize("kind", ["padded", "few", "none visible", "mixed"])
+@pytest.mark.parametrize("shape", [(3, 8, 2, 1201, 128), (1, 14, 2, 333, 64), (17, 16, 8, 515, 64), (2, 4, 4, 34001, 64)])
+def test_hash_steps_under_a_mask_that_hides_columns(cuda, dtype, kind, shape):
+    """The one-kernel step against the masker-by-masker path; signatures with components that are zero among the keys'."""
+    import sparse_attention_hub_amd.sparse_attention as sa
+    from sparse_attention_hub_amd import _native as N
+    from sparse_attention_hub_amd.sparse_attention.utils.hashattention_utils import random_hat_weights
+
+    B, Hq, Hkv, Lk, D = shape
+    window = 70
+    wts = random_hat_weights(1, Hq, D, 32, 3, 128, dtype=dtype, seed=1)
+    cfgs = [sa.SinkMaskerConfig(sink_size=9), sa.LocalMaskerConfig(window_size=window), sa.HashAttentionTopKMaskerConfig(
+        heavy_size=50, hat_bits=32, hat_mlp_layers=3, hat_mlp_hidden_size=128,
+        hat_mlp_activation="silu" if D == 128 else "relu", hat_weights=wts)]
+    _, k, v = make_qkv(B, Hq, Hkv, 1, Lk, D, dtype, seed=5, device=cuda)
+    k[:, :, ::5] = 0.0  # (zero keys: relu leaves signature components that are zero)
+    lowest = float(torch.finfo(dtype).min)
+    outs = []
+    for planned in (True, False):
+        ra = sa.ResearchAttention.create_from_config(sa.ResearchAttentionConfig(masker_configs=cfgs))
+        ra.return_attention_weights = False
+        if not planned:
+            ra._plan_kind = None
+        meta, got = {}, []
+        for i, n in enumerate((Lk - 64, Lk - 64, Lk - 63, Lk)):  # the first call fills the layer's cache
+            q = make_qkv(B, Hq, Hkv, 1, 1, D, dtype, seed=100 + i, device=cuda)[0]
+            m = _hide(torch.zeros((B, 1, 1, n + 3)), kind, n, window, lowest)
+            N.timing_enable(True)
+            out, _ = ra.custom_attention(None, q, k[:, :, :n], v[:, :, :n], m.to(dtype).to(cuda), D ** -0.5, 0.0,
+                                         sparse_meta_data=meta, layer_idx=0)
+            torch.cuda.synchronize()
+            assert ("k_hash_decode_attn" in launched(N)) == (planned and i > 0 and dtype != torch.float16)
+            got.append(out.double().cpu())
+        outs.append(torch.stack(got))
+    a, b = outs
+    # as above; fp16 and rows of which every entry is hidden leave nothing to select by but sums beyond the type's range
+    ok = torch.isfinite(b)
+    assert torch.equal(ok, torch.isfinite(a)) and (bool(ok.all()) or kind == "none visible")
+    unit = {torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10, torch.float32: 2.0 ** -18}[dtype]
+    assert bool(((a - b).abs() <= unit * b.abs() + (1e-6 if dtype == torch.float32 else 2.0 ** -18))[ok].all())
+
+
+def test_a_masked_step_does_not_read_what_another_stream_writes(cuda):
+    """The compact codes are written by the first planned step; a step on another stream, nothing between the two, takes the way
+    that does not read them."""
+    import sparse_attention_hub_amd.sparse_attention as sa
+    from sparse_attention_hub_amd import _native as N
+    from sparse_attention_hub_amd.sparse_attention.utils.hashattention_utils import random_hat_weights
+
+    B, Hq, Hkv, Lk, D = 2, 8, 2, 900, 128
+    _, k, v = make_qkv(B, Hq, Hkv, 1, Lk, D, torch.bfloat16, seed=5, device=cuda)
+    q = make_qkv(B, Hq, Hkv, 1, 1, D, torch.bfloat16, seed=1, device=cuda)[0]
+    m = _hide(torch.zeros((B, 1, 1, Lk)), "padded", Lk, 70, float(torch.finfo(torch.bfloat16).min)).to(torch.bfloat16).to(cuda)
+    ra = sa.ResearchAttention.create_from_config(sa.ResearchAttentionConfig(masker_configs=[
+        sa.SinkMaskerConfig(sink_size=9), sa.LocalMaskerConfig(window_size=70), sa.HashAttentionTopKMaskerConfig(
+            heavy_size=50, hat_bits=32, hat_mlp_layers=3, hat_mlp_hidden_size=128, hat_mlp_activation="silu",
+            hat_weights=random_hat_weights(1, Hq, D, 32, 3, 128, dtype=torch.bfloat16, seed=1))]))
+    ra.return_attention_weights = False
+    meta = {}
+
+    def step():
+        return ra.custom_attention(None, q, k, v, m, D ** -0.5, 0.0, sparse_meta_data=meta, layer_idx=0)[0]
+
+    step()
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    N.timing_enable(True)
+    a = step()
+    with torch.cuda.stream(side):
+        b = step()
+    torch.cuda.synchronize()
+    seen = N.timing_collect()
+    N.timing_enable(False)
+    assert seen["k_hash_decode_attn"][0] == 1 and seen["k_hamming_scores"][0] == 1
+    assert bool(((a.double() - b.double()).abs() <= 2.0 ** -7 * b.double().abs() + 2.0 ** -18).all())
