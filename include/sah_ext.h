@@ -51,7 +51,7 @@ int sah_pq_kmeans(const sah_pq_kmeans_args* a);
 
 /* sah_amask_classify whose answer the host has when the call returns, without a cleared output, a copy and a wait for the
  * stream: the kernel writes the flags into host memory, and the call watches that word (after 2 ms, behind long work of the
- * stream, it waits for the stream instead). mask.flags is not used. scratch: two words of device memory, zero before the
+ * stream, now and then). mask.flags is not used. scratch: two words of device memory, zero before the
  * first call and left zero; host_word: pinned host memory the device can write, zero before the first call. Both serve one
  * call at a time. Refused while the stream is being captured. */
 typedef struct sah_amask_read_args {
@@ -61,6 +61,15 @@ typedef struct sah_amask_read_args {
   int32_t flags;  /* out */
 } sah_amask_read_args;
 int sah_amask_read(sah_amask_read_args* a);
+
+/* The same as two calls, for a caller that puts other work on its way between question and answer. scratch and host_word serve
+ * one question at a time, from ask to answer, and stay allocated that long, as does the mask. */
+typedef struct sah_amask_question {
+  sah_amask_read_args read;
+  uint32_t asked;  /* of the library */
+} sah_amask_question;
+int sah_amask_ask(sah_amask_question* q);
+int sah_amask_answer(sah_amask_question* q);
 
 /* sah_hash_decode_attention under an additive mask (attention.amask, of the queries' type) that holds nothing but 0, the
  * type's lowest value and -inf, in one kernel: the selection ranks a column at the lowest value below every other one (as the

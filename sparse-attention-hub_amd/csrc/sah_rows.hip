@@ -2,6 +2,7 @@
 // conversion. Integer work; one workgroup per mask row, bitmap kept coherent
 // with the column list so later maskers can test membership in O(1).
 #include <chrono>
+#include <thread>
 #include "sah_common.h"
 
 static thread_local char g_err[512];
@@ -458,46 +459,66 @@ __global__ __launch_bounds__(AMR_NT) void k_amask_read(const void* amask, int64_
 #endif
 }
 
-extern "C" int sah_amask_read(sah_amask_read_args* r) {
-  if (!r) return sah_fail(SAH_ENULL, "sah_amask_read: args is NULL");
+static int amr_ask(const char* who, sah_amask_read_args* r, uint32_t* asked) {
   const sah_amask_classify_args* a = &r->mask;
-  if (!a->amask || !r->scratch || !r->host_word) return sah_fail(SAH_ENULL, "sah_amask_read: amask / scratch / host_word is NULL");
-  if (a->B <= 0 || a->Hm <= 0 || a->Lq <= 0 || a->Lk <= 0) return sah_fail(SAH_EINVAL, "sah_amask_read: B, Hm, Lq, Lk must be > 0");
+  if (!a->amask || !r->scratch || !r->host_word) return sah_fail(SAH_ENULL, "%s: amask / scratch / host_word is NULL", who);
+  if (a->B <= 0 || a->Hm <= 0 || a->Lq <= 0 || a->Lk <= 0) return sah_fail(SAH_EINVAL, "%s: B, Hm, Lq, Lk must be > 0", who);
   const int64_t rows = (int64_t)a->B * a->Hm * a->Lq;
-  if (rows > 65535) return sah_fail(SAH_ESHAPE, "sah_amask_read: %lld mask rows exceed 65535", (long long)rows);
+  if (rows > 65535) return sah_fail(SAH_ESHAPE, "%s: %lld mask rows exceed 65535", who, (long long)rows);
   hipStream_t st = (hipStream_t)a->stream;
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(st, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone)
-    return sah_fail((int)hipErrorStreamCaptureUnsupported, "sah_amask_read: what a mask holds cannot be read back while the stream is captured");
+    return sah_fail((int)hipErrorStreamCaptureUnsupported, "%s: what a mask holds cannot be read back while the stream is captured", who);
   const int64_t units = rows * ((a->Lk + 7) / 8);
   int64_t wgs = (units + 2 * AMR_NT - 1) / (2 * AMR_NT);
   wgs = wgs > AMR_MAX_WGS ? AMR_MAX_WGS : wgs;
-  volatile uint64_t* word = r->host_word;
+  const volatile uint64_t* word = r->host_word;
   const uint32_t seq = (uint32_t)(*word >> 32) + 1u;
-  {
-    sah_timed timed("k_amask_classify", a->stream);  // (one name for the question, whichever kernel answers)
+  sah_timed timed("k_amask_classify", a->stream);  // (one name for the question, whichever kernel answers)
 #define SAH_AMR(DTC)                                                                                                            \
   hipLaunchKernelGGL(k_amask_read<DTC>, dim3((unsigned)wgs), dim3(AMR_NT), 0, st, a->amask, a->ms_b, a->ms_h, a->ms_l, a->Hm, a->Lq, \
                      a->Lk, (int)rows, r->scratch, r->host_word, seq)
-    switch (a->dtype) {
-      case SAH_F32: SAH_AMR(SAH_F32); break;
-      case SAH_BF16: SAH_AMR(SAH_BF16); break;
-      case SAH_F16: SAH_AMR(SAH_F16); break;
-      default: return sah_fail(SAH_EDTYPE, "sah_amask_read: dtype %d", a->dtype);
-    }
-#undef SAH_AMR
-    if (int rc = sah_launch_status("sah_amask_read")) return rc;
+  switch (a->dtype) {
+    case SAH_F32: SAH_AMR(SAH_F32); break;
+    case SAH_BF16: SAH_AMR(SAH_BF16); break;
+    case SAH_F16: SAH_AMR(SAH_F16); break;
+    default: return sah_fail(SAH_EDTYPE, "%s: dtype %d", who, a->dtype);
   }
+#undef SAH_AMR
+  *asked = seq;
+  return sah_launch_status(who);
+}
+
+static int amr_answer(const char* who, sah_amask_read_args* r, uint32_t seq) {
+  const volatile uint64_t* word = r->host_word;
   const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(2);
   while ((uint32_t)(*word >> 32) != seq) {
-    if (std::chrono::steady_clock::now() > until) {
-      const hipError_t e = hipStreamSynchronize(st);
-      if (e != hipSuccess) return sah_fail((int)e, "sah_amask_read: %s", hipGetErrorString(e));
-      break;
-    }
+    if (std::chrono::steady_clock::now() < until) continue;
+    // behind long work: the stream may by now hold more of it than the question, so it is not waited for
+    const hipError_t e = hipStreamQuery((hipStream_t)r->mask.stream);
+    if (e == hipSuccess) break;
+    if (e != hipErrorNotReady) return sah_fail((int)e, "%s: %s", who, hipGetErrorString(e));
+    std::this_thread::sleep_for(std::chrono::microseconds(20));
   }
   const uint64_t got = *word;
-  if ((uint32_t)(got >> 32) != seq) return sah_fail(SAH_EINVAL, "sah_amask_read: host_word is not memory the device can write");
+  if ((uint32_t)(got >> 32) != seq) return sah_fail(SAH_EINVAL, "%s: host_word is not memory the device can write", who);
   r->flags = (int32_t)(uint32_t)got;
   return SAH_OK;
+}
+
+extern "C" int sah_amask_read(sah_amask_read_args* r) {
+  if (!r) return sah_fail(SAH_ENULL, "sah_amask_read: args is NULL");
+  uint32_t seq = 0;
+  if (int rc = amr_ask("sah_amask_read", r, &seq)) return rc;
+  return amr_answer("sah_amask_read", r, seq);
+}
+
+extern "C" int sah_amask_ask(sah_amask_question* q) {
+  if (!q) return sah_fail(SAH_ENULL, "sah_amask_ask: args is NULL");
+  return amr_ask("sah_amask_ask", &q->read, &q->asked);
+}
+
+extern "C" int sah_amask_answer(sah_amask_question* q) {
+  if (!q || !q->read.host_word) return sah_fail(SAH_ENULL, "sah_amask_answer: args or host_word is NULL");
+  return amr_answer("sah_amask_answer", &q->read, q->asked);
 }

@@ -63,6 +63,8 @@ EXTENSION_SYMBOLS = {
     "sah_members_attention": 1,
     "sah_pq_kmeans": 1,
     "sah_amask_read": 1,
+    "sah_amask_ask": 1,
+    "sah_amask_answer": 1,
     "sah_hash_decode_masked": 1,
 }
 
@@ -395,6 +397,10 @@ class AmaskClassifyArgs(C.Structure):
 
 class AmaskReadArgs(C.Structure):
     _fields_ = [("mask", AmaskClassifyArgs), ("scratch", C.c_void_p), ("host_word", C.c_void_p), ("flags", C.c_int32)]
+
+
+class AmaskQuestion(C.Structure):
+    _fields_ = [("read", AmaskReadArgs), ("asked", C.c_uint32)]
 
 
 AMASK_NONZERO, AMASK_GENERAL = 1, 2

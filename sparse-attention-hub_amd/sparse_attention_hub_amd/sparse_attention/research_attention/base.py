@@ -19,7 +19,9 @@ from ... import _native
 from ...metric_logging import MicroMetricLogger
 from ..base import SparseAttention, SparseAttentionConfig
 from ..utils.mask import Mask
-from ..utils.mask_attention_utils import AdditiveMaskFacts, get_masked_attention_output, get_true_attention_output
+from ..utils.mask_attention_utils import (
+    AdditiveMaskFacts, MaskQuestion, get_masked_attention_output, get_true_attention_output, mask_covers,
+)
 from ..utils.native_rows import NativeRows
 from .decode_plan import DecodePlan, plan_kind
 from .maskers.base import MaskerConfig, ResearchMasker
@@ -83,42 +85,21 @@ class ResearchAttention(SparseAttention):
             raise ValueError("sparse_meta_data must be provided in kwargs while calling custom_attention()")
         sparse_meta_data: Dict[Any, Any] = kwargs.pop("sparse_meta_data")
 
-        only_hides = False
-        if (attention_mask is not None and attention_mask.is_cuda and attention_mask.dim() == 4
-                and attention_mask.shape[-1] >= keys.shape[2] and attention_mask.dtype in (torch.float32, torch.bfloat16, torch.float16)):
-            flags = self._mask_facts.flags(attention_mask)
-            # (a lowest value of another type than the queries' is none of theirs)
-            only_hides = not flags & _native.AMASK_GENERAL and attention_mask.dtype == queries.dtype
-            if flags == 0:
-                # an additive mask of zeros (HuggingFace's eager mask of an unpadded decode step) adds nothing anywhere:
-                # established once per mask tensor, i.e. once per forward pass, not per layer
-                attention_mask = None
-
         metrics = MicroMetricLogger()
         want_density = metrics.is_metric_enabled("research_attention_density")
         want_error = metrics.is_metric_enabled("research_attention_output_error")
+        # the decode fast path: the whole chain as one native call over cached argument blocks
+        plannable = (not (want_density or want_error)  # the metrics read the finished mask: masker-by-masker path
+                     and not self.return_attention_weights and self._plan_kind is not None
+                     and not isinstance(kwargs.get("s_aux"), torch.Tensor) and queries.dim() == 4
+                     and not (dropout > 0.0 and module is not None and getattr(module, "training", False)))
 
-        if (not (want_density or want_error)  # the metrics read the finished mask: masker-by-masker path
-                and not self.return_attention_weights and (attention_mask is None or queries.shape[2] == 1) and self._plan_kind is not None
-                and not isinstance(kwargs.get("s_aux"), torch.Tensor) and queries.dim() == 4
-                and not (dropout > 0.0 and module is not None and getattr(module, "training", False))):
-            # decode fast path: the whole chain as one native call over cached argument blocks
-            _native.require_device(queries, "queries")
-            masked = attention_mask is not None
-            key = (queries.device, queries.dtype, tuple(queries.shape), keys.shape[1], masked)
-            # A masked step's buffers belong to the stream and thread of their plan, as those of the masker-by-masker path
-            # belong to the call: a step on another stream is not ordered with the ones that use them. A captured one's
-            # belong to its graph alone: what its plan clears is clear when the graph runs, not now.
-            owner = (_native.stream_ptr(queries.device), threading.get_ident()) if masked else None
-            if masked and torch.cuda.is_current_stream_capturing():
-                plan = DecodePlan(self.maskers, self._plan_kind, queries, keys, True)
-            else:
-                plan = self._plans.get(key)
-                if plan is None or plan.owner != owner:
-                    plan = self._plans[key] = DecodePlan(self.maskers, self._plan_kind, queries, keys, masked, owner)
-            out = plan.run(queries, keys, values, scaling, sparse_meta_data, kwargs.get("layer_idx"), attention_mask, only_hides)
-            if out is not None:
-                return out, None
+        attention_mask, only_hides, out, question = self._under_mask(
+            queries, keys, values, attention_mask, scaling, sparse_meta_data, kwargs.get("layer_idx"), plannable)
+        if out is None and plannable and (attention_mask is None or queries.shape[2] == 1):
+            out = self._plan_step(queries, keys, values, attention_mask, scaling, sparse_meta_data, kwargs.get("layer_idx"), only_hides)
+        if out is not None:
+            return out, None
 
         mask_shape = (queries.shape[0], queries.shape[1], queries.shape[2], keys.shape[2])
         mask = Mask.create_empty_mask(mask_shape, dtype=queries.dtype, device=queries.device)
@@ -175,12 +156,69 @@ class ResearchAttention(SparseAttention):
                 sinks=s_aux, scaling=scaling, dropout=dropout, sparse_attention_mask=mask,
                 return_attention_weights=False, **kwargs,
             )
+        if question is not None:
+            self._mask_facts.take(question)
         if want_error:
             # relative distance to dense attention over all keys, by the same kernel in dense mode (reference :150-168)
             true_out, _ = get_true_attention_output(module, queries, keys, values, attention_mask, scaling, dropout, **kwargs)
             error = torch.norm(true_out.float() - out.float()) / torch.norm(true_out.float())
             metrics.log("research_attention_output_error", float(error.item()), metadata={"layer_idx": kwargs["layer_idx"]})
         return out, weights
+
+    def _under_mask(self, queries: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, attention_mask: Optional[torch.Tensor],
+                    scaling: float, sparse_meta_data: Dict[Any, Any], layer_idx: Optional[int], plannable: bool):
+        """(the mask that counts, does it only hide columns, the step's output if it has been made, a question still open).
+
+        An additive mask of zeros (HuggingFace's eager mask of an unpadded decode step) adds nothing anywhere and is left out;
+        one that only hides columns has a faster way. Which it is, is established once per mask tensor, i.e. once per forward
+        pass, not per layer, and the first layer does not wait for the answer with nothing under way: a decode step's mask is
+        taken to be like the last step's, the step is launched and the answer read; a step launched on a wrong guess is
+        launched again (what it adds to the caches does not depend on the mask). A mask of several queries, all but always
+        nonzero, is taken as it is, which is right whatever it holds."""
+        am = attention_mask
+        if (am is None or not am.is_cuda or am.dim() != 4 or am.shape[-1] < keys.shape[2]
+                or am.dtype not in (torch.float32, torch.bfloat16, torch.float16)):
+            return am, False, None, None
+        facts = self._mask_facts
+        same_type = am.dtype == queries.dtype  # (a lowest value of another type is none of the queries')
+        flags = facts.known(am)
+        if flags is None:
+            guess = facts.guess(am)
+            question = MaskQuestion(am)
+            if plannable and guess is not None and (guess == 0 or queries.shape[2] == 1):
+                hides = not guess & _native.AMASK_GENERAL and same_type
+                try:
+                    out = self._plan_step(queries, keys, values, am if guess else None, scaling, sparse_meta_data, layer_idx, hides)
+                except Exception:
+                    out = None  # (what is wrong with the call under its own mask, if anything, is said then)
+                flags = facts.take(question)
+                if out is not None and (flags == guess or (guess and not (hides and flags & _native.AMASK_GENERAL))):
+                    return am, hides, out, None
+            elif am.shape[2] > 1 and guess != 0 and mask_covers(am, queries, keys.shape[2]):
+                return am, False, None, question
+            else:
+                flags = facts.take(question)
+        if flags == 0:
+            return None, False, None, None
+        return am, not flags & _native.AMASK_GENERAL and same_type, None, None
+
+    def _plan_step(self, queries: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, attention_mask: Optional[torch.Tensor],
+                   scaling: float, sparse_meta_data: Dict[Any, Any], layer_idx: Optional[int], only_hides: bool) -> Optional[torch.Tensor]:
+        """One step through the cached plan of its geometry, or None where the plan does not cover it."""
+        _native.require_device(queries, "queries")
+        masked = attention_mask is not None
+        key = (queries.device, queries.dtype, tuple(queries.shape), keys.shape[1], masked)
+        # A masked step's buffers belong to the stream and thread of their plan, as those of the masker-by-masker path
+        # belong to the call: a step on another stream is not ordered with the ones that use them. A captured one's
+        # belong to its graph alone: what its plan clears is clear when the graph runs, not now.
+        owner = (_native.stream_ptr(queries.device), threading.get_ident()) if masked else None
+        if masked and torch.cuda.is_current_stream_capturing():
+            plan = DecodePlan(self.maskers, self._plan_kind, queries, keys, True)
+        else:
+            plan = self._plans.get(key)
+            if plan is None or plan.owner != owner:
+                plan = self._plans[key] = DecodePlan(self.maskers, self._plan_kind, queries, keys, masked, owner)
+        return plan.run(queries, keys, values, scaling, sparse_meta_data, layer_idx, attention_mask, only_hides)
 
     @classmethod
     def create_from_config(cls, config: SparseAttentionConfig) -> "ResearchAttention":

@@ -71,6 +71,12 @@ def unit_inverse_weight(dtype: torch.dtype) -> float:
     return 1.0  # bf16 / fp16: 1 + 1e-6 rounds back to 1
 
 
+def mask_covers(am: torch.Tensor, queries: torch.Tensor, n_keys: int) -> bool:
+    """Has the 4-dimensional mask a row for every query, as wide as the keys?"""
+    return (am.shape[-1] >= n_keys and am.shape[2] == queries.shape[2] and am.shape[0] in (1, queries.shape[0])
+            and am.shape[1] in (1, queries.shape[1]))
+
+
 def additive_mask_args(attention_mask: Optional[torch.Tensor], queries: torch.Tensor, n_keys: int):
     """(tensor kept alive, ptr, stride_b, stride_h, stride_q) of the additive mask or all-None/0."""
     if attention_mask is None:
@@ -78,8 +84,7 @@ def additive_mask_args(attention_mask: Optional[torch.Tensor], queries: torch.Te
     am = attention_mask
     if am.dim() != 4:
         raise ValueError(f"attention_mask must have 4 dimensions, got shape {tuple(am.shape)}")
-    B, H, Lq = queries.shape[0], queries.shape[1], queries.shape[2]
-    if am.shape[-1] < n_keys or am.shape[2] != Lq or am.shape[0] not in (1, B) or am.shape[1] not in (1, H):
+    if not mask_covers(am, queries, n_keys):
         raise ValueError(f"attention_mask shape {tuple(am.shape)} does not cover queries {tuple(queries.shape)} x {n_keys} keys")
     if am.dtype != queries.dtype:
         am = am.to(queries.dtype)
@@ -91,11 +96,12 @@ def additive_mask_args(attention_mask: Optional[torch.Tensor], queries: torch.Te
 
 
 class _AnswerWords(threading.local):
-    """Per thread and device: two words of device memory and one of pinned host memory, through which `sah_amask_read` answers
-    (one call of a thread at a time; the call returns with the answer, so no stream uses them afterwards)."""
+    """Per thread and device: two words of device memory and one of pinned host memory, through which a mask's question is
+    answered, and the thread's question that waits for its answer (one at a time; nobody returns to a caller in between)."""
 
     def __init__(self) -> None:
         self.words = {}
+        self.open = {}
 
 
 _ANSWERS = _AnswerWords()
@@ -114,36 +120,76 @@ def _answer_words(device: torch.device):
     return words
 
 
+class MaskQuestion:
+    """What does this mask hold? Asked of the device when made; `settle` waits for the answer."""
+
+    def __init__(self, am: torch.Tensor) -> None:
+        dev = am.device
+        scratch, word = _answer_words(dev)
+        earlier = _ANSWERS.open.get(dev.index)
+        if earlier is not None:
+            earlier.settle()
+        # (mask and words stay allocated until the answer)
+        self.mask, self.version, self.flags, self._words = am, am._version, None, (scratch, word)
+        args = N.AmaskQuestion(N.AmaskReadArgs(N.AmaskClassifyArgs(
+            am.data_ptr(), am.stride(0), am.stride(1), am.stride(2), N.dtype_code(am.dtype),
+            am.shape[0], am.shape[1], am.shape[2], am.shape[3], None, N.stream_ptr(dev)), scratch.data_ptr(), word.data_ptr()))
+        N.call("sah_amask_ask", args)
+        self._args = args
+        _ANSWERS.open[dev.index] = self
+
+    def settle(self) -> int:
+        if self.flags is None:
+            _ANSWERS.open.pop(self.mask.device.index, None)
+            N.call("sah_amask_answer", self._args)
+            self.flags = self._args.read.flags
+        return self.flags
+
+    def __del__(self) -> None:
+        # a thread that ends on a call that failed in between: the words go only after the kernel has written them
+        if getattr(self, "_args", None) is not None and self.flags is None:
+            try:
+                N.call("sah_amask_answer", self._args)
+            except Exception:
+                pass
+
+
 class AdditiveMaskFacts:
     """What the additive mask of the current forward pass holds, established once per mask tensor.
 
     HuggingFace builds one mask per forward pass and hands the same tensor to every layer; for a single decode
     query of an unpadded batch its eager mask is all zeros, and adding zeros to scores and logits changes nothing
     (reference: hashattention_top_k.py:367-368, oracle_top_k.py:71-72, utils/mask_attention_utils.py:221-225).
-    `all_zero` asks the device once per tensor (one small launch, answered into host memory, over the mask's whole width: a
-    mask that is zero everywhere is zero on the columns of any key count) and remembers the answer for as long as
+    The device is asked once per tensor (one small launch, answered into host memory, over the mask's whole width: a
+    mask that is zero everywhere is zero on the columns of any key count) and the answer remembered for as long as
     the same, unmodified tensor keeps arriving; the tensor is kept referenced meanwhile, so its memory cannot be
     handed to another tensor that would then be mistaken for it."""
 
     def __init__(self) -> None:
-        self._tensor: Optional[torch.Tensor] = None
-        self._version = -1
-        self._flags = 0
+        self._seen: Tuple[Optional[torch.Tensor], int, int] = (None, -1, 0)  # tensor, its version, flags
+        self._last: Dict[bool, int] = {}  # one query or several -> flags of the last such mask
 
-    def flags(self, attention_mask: torch.Tensor) -> int:
-        am = attention_mask
-        if am is self._tensor and am._version == self._version:
-            return self._flags
+    def known(self, am: torch.Tensor) -> Optional[int]:
+        tensor, version, flags = self._seen
+        if am is tensor and am._version == version:
+            return flags
         if am.dim() != 4 or am.stride(-1) != 1 or not am.is_cuda or am.numel() == 0:
             return N.AMASK_NONZERO | N.AMASK_GENERAL  # nothing established: every consumer reads the mask itself
-        scratch, word = _answer_words(am.device)
-        args = N.AmaskReadArgs(N.AmaskClassifyArgs(
-            am.data_ptr(), am.stride(0), am.stride(1), am.stride(2), N.dtype_code(am.dtype),
-            am.shape[0], am.shape[1], am.shape[2], am.shape[3], None, N.stream_ptr(am.device)), scratch.data_ptr(), word.data_ptr())
-        N.call("sah_amask_read", args)
-        self._flags = args.flags
-        self._tensor, self._version = am, am._version
-        return self._flags
+        return None
+
+    def guess(self, am: torch.Tensor) -> Optional[int]:
+        """The flags of the last mask for as many queries (one, or several)."""
+        return self._last.get(am.shape[2] == 1)
+
+    def take(self, question: MaskQuestion) -> int:
+        flags = question.settle()
+        self._seen = (question.mask, question.version, flags)
+        self._last[question.mask.shape[2] == 1] = flags
+        return flags
+
+    def flags(self, attention_mask: torch.Tensor) -> int:
+        known = self.known(attention_mask)
+        return self.take(MaskQuestion(attention_mask)) if known is None else known
 
     def all_zero(self, attention_mask: torch.Tensor) -> bool:
         return self.flags(attention_mask) == 0

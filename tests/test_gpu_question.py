@@ -900,3 +900,64 @@ def test_a_masked_step_does_not_read_what_another_stream_writes(cuda):
     N.timing_enable(False)
     assert seen["k_hash_decode_attn"][0] == 1 and seen["k_hamming_scores"][0] == 1
     assert bool(((a.double() - b.double()).abs() <= 2.0 ** -7 * b.double().abs() + 2.0 ** -18).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("chain", ["fixed", "hash", "oracle", "pq"])
+def test_steps_launched_on_a_guess_about_their_mask(cuda, dtype, chain):
+    """A step's first layer is launched as if its mask were like the last step's: every order of zero, hiding and general masks,
+    new keys in between, against an instance that has no last step; then masks of several queries, and of one row for several."""
+    import sparse_attention_hub_amd.sparse_attention as sa
+    from sparse_attention_hub_amd.sparse_attention.utils.hashattention_utils import random_hat_weights
+
+    B, Hq, Hkv, Lk, D = 2, 8, 2, 900, 64
+    cfgs = [sa.SinkMaskerConfig(sink_size=9), sa.LocalMaskerConfig(window_size=70)]
+    if chain == "hash":
+        cfgs.append(sa.HashAttentionTopKMaskerConfig(
+            heavy_size=50, hat_bits=32, hat_mlp_layers=3, hat_mlp_hidden_size=128, hat_mlp_activation="silu",
+            hat_weights=random_hat_weights(1, Hq, D, 32, 3, 128, dtype=dtype, seed=1)))
+    elif chain == "oracle":
+        cfgs.append(sa.OracleTopKConfig(heavy_size=50))
+    elif chain == "pq":
+        cfgs.append(sa.PQCacheConfig(heavy_size=50, pq_group_factor=8, pq_bits=4, kmeans_iter=3, init_offset=9, metric="euclidean"))
+
+    def make():
+        ra = sa.ResearchAttention.create_from_config(sa.ResearchAttentionConfig(masker_configs=cfgs))
+        ra.return_attention_weights = False
+        return ra
+
+    lowest = float(torch.finfo(dtype).min)
+    _, k, v = make_qkv(B, Hq, Hkv, 1, Lk, D, dtype, seed=5, device=cuda)
+    guessing, meta, meta_ref = make(), {}, {}
+    unit = {torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}[dtype]
+    order = "z" + "zhzghhggzgz"  # the first call fills the cache
+    for i, kind in enumerate(order):
+        n = Lk - 100 + 9 * i
+        q = make_qkv(B, Hq, Hkv, 1, 1, D, dtype, seed=100 + i, device=cuda)[0]
+        m = torch.zeros((B, 1, 1, n))
+        if kind != "z":
+            m[0, ..., :200] = lowest
+        if kind == "g":
+            m[..., 1::3] -= 1.5
+            m.clamp_(min=lowest)
+        m = m.to(dtype).to(cuda)
+        args = (None, q, k[:, :, :n], v[:, :, :n], m, D ** -0.5, 0.0)
+        got = guessing.custom_attention(*args, sparse_meta_data=meta, layer_idx=0)[0].double()
+        want = make().custom_attention(*args, sparse_meta_data=meta_ref, layer_idx=0)[0].double()
+        assert guessing._mask_facts.known(m) == {"z": 0, "h": 1, "g": 3}[kind]
+        assert bool(((got - want).abs() <= unit * want.abs() + 2.0 ** -18).all()), (i, kind)
+    for shape, kind in (((B, 1, 5, Lk), "h"), ((1, 1, 5, Lk), "z"), ((B, Hq, 5, Lk), "g"), ((1, 1, 1, Lk), "z")):
+        q = make_qkv(B, Hq, Hkv, 5, 1, D, dtype, seed=7, device=cuda)[0]
+        m = torch.zeros(shape)
+        if kind != "z":
+            m[..., :100] = lowest if kind == "h" else -1.0
+        m = m.to(dtype).to(cuda)
+        args = (None, q, k, v, m, D ** -0.5, 0.0)
+        got = guessing.custom_attention(*args, sparse_meta_data=dict(meta), layer_idx=0)[0].double()
+        want = make().custom_attention(*args, sparse_meta_data=dict(meta), layer_idx=0)[0].double()
+        assert guessing._mask_facts.known(m) == {"z": 0, "h": 1, "g": 3}[kind]
+        assert bool(((got - want).abs() <= unit * want.abs() + 2.0 ** -18).all()), (shape, kind)
+    # a mask that covers nothing of the call is refused if it holds something, whatever was guessed
+    bad = torch.full((1, 1, 3, Lk), -1.0, dtype=dtype, device=cuda)
+    with pytest.raises(ValueError, match="does not cover"):
+        guessing.custom_attention(None, q, k, v, bad, D ** -0.5, 0.0, sparse_meta_data=meta, layer_idx=0)
