@@ -559,10 +559,14 @@ __device__ __forceinline__ uint32_t pqm_mask_le(const sah_f32x16& a, float b) {
 // KS k-steps of two dimensions each: sub-vectors of up to 2 KS dimensions (the operands beyond d_sub are zero), of
 // exactly 2 KS in the split form. SUMS: the per-centre sums of the update step are accumulated here (P.sums given and
 // the LDS holds them). A workgroup takes wg_tiles tiles of 32 keys of one group.
-template <int DT, int KS, bool SUMS, bool SPLIT>
+// PIPE: the centre tiles go by in pairs, a multiple of four of them; a pair's products are under way while the minima of the
+// pair before are taken, each matrix instruction between ten vector ones, and a key tile's last pair has the next key tile's
+// first behind it, which so computes while the key tile is concluded.
+template <int DT, int KS, bool SUMS, bool SPLIT, bool PIPE>
 __global__ __launch_bounds__(PQM_NT, KS <= 16 ? 4 : 2) void k_pq_assign_mfma(pq_assign_params P, pq_update_params U, uint32_t* arrivals,
                                                                                            int wg_tiles, int ranges, int n_heads) {
   SAH_DYNAMIC_LDS(pqm_dyn)
+  static_assert(!PIPE || (SPLIT && KS <= 8), "the pipelined loop holds a key in one operand");
   static_assert(!SPLIT || (DT == SAH_BF16 && KS >= 4), "the split form multiplies bf16 keys in sub-vectors of 8 and more");
   if (P.skip_flag && *P.skip_flag) return;
   const int tid = threadIdx.x;
@@ -679,122 +683,18 @@ __global__ __launch_bounds__(PQM_NT, KS <= 16 ? 4 : 2) void k_pq_assign_mfma(pq_
     }
   };
   if constexpr (SPLIT) request((tg * wg_tiles + wave) * 32 + j);
-  for (int kt = wave; kt < wg_tiles; kt += PQM_NW) {
-    const int n0 = (tg * wg_tiles + kt) * 32;
-    if (n0 >= P.n_keys) break;  // uniform across the wave
-    const int n = n0 + j;
+  // From a key tile's minima to its codes and sums. kept: every slot's minimum over the tiles (SPLIT) or the 16 values of the
+  // tile of the smallest; xb / xs: its keys.
+  auto conclude = [&](int kt, int n, const sah_u4 (&xb)[NB], const float (&xs)[SPLIT ? 1 : KS], const sah_f32x16& kept, float best,
+                      float second, int bt, bool nan) __attribute__((always_inline)) {
+    // (the lane is opaque here: what follows from it is computed again for every key tile, in a few instructions, instead of
+    // being held in registers that the products need)
+    int own = tid & (SAH_WAVE - 1);
+#if defined(__HIP_DEVICE_COMPILE__)
+    if (PIPE) asm volatile("" : "+v"(own));
+#endif
+    const int j = own & 31, g = own >> 5;
     const bool valid = n < P.n_keys;
-    float xs[SPLIT ? 1 : KS];  // this lane's dims 2 s + g of its key
-    sah_u4 xb[NB];             // SPLIT: dims 16 q + 8 g .. + 7 (sub-vectors of 8: both halves hold all)
-    sah_u4 x0;                 // key operand of the first instruction: with the norm in A, ones against its terms
-    if constexpr (SPLIT) {
-#pragma unroll
-      for (int q = 0; q < NB; ++q) xb[q] = nb[q];
-      request(n + 32 * PQM_NW);
-      x0 = xb[0];
-      if (KS == 4 && g) x0 = sah_u4{0x3f803f80u, 0x3f80u, 0u, 0u};
-    } else {
-      const int64_t off = key_offset(n);
-#pragma unroll
-      for (int s = 0; s < KS; ++s) xs[s] = (2 * s + g < d_sub) ? sah_load<DT>(P.k, off + 2 * s + g) : 0.f;
-    }
-    // accumulator of centre tile t: seeded with the norms, then the matrix instructions
-    auto product = [&](sah_f32x16& acc, int t) {
-      if constexpr (NORM_IN_A) {
-        acc = sah_f32x16{};
-      } else {
-        const float4* cn4 = (const float4*)(s_cn + (t * 2 + g) * 16);
-#pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4) {
-          const float4 c4 = cn4[q4];
-          acc[4 * q4] = c4.x; acc[4 * q4 + 1] = c4.y; acc[4 * q4 + 2] = c4.z; acc[4 * q4 + 3] = c4.w;
-        }
-      }
-      if constexpr (SPLIT) {
-        const uint4* ap = (const uint4*)s_a + (size_t)t * 64 * OPS + g * 32 + j;
-#pragma unroll
-        for (int op = 0; op < OPS; ++op) acc = sah_mfma_32x32x16<SAH_BF16>(ap[op * 64], __builtin_bit_cast(uint4, op ? xb[op % NB] : x0), acc);
-      } else if constexpr (KS >= 4) {
-        const float4* ap = (const float4*)(s_a + (size_t)(t * 2 + g) * 32 * KS) + j;
-#pragma unroll
-        for (int q = 0; q < KS / 4; ++q) {
-          const float4 a4 = ap[q * 32];
-          acc = sah_mfma_32x32x2_f32(a4.x, xs[4 * q], acc);
-          acc = sah_mfma_32x32x2_f32(a4.y, xs[4 * q + 1], acc);
-          acc = sah_mfma_32x32x2_f32(a4.z, xs[4 * q + 2], acc);
-          acc = sah_mfma_32x32x2_f32(a4.w, xs[4 * q + 3], acc);
-        }
-      } else {
-        const float* ap = s_a + ((t * 2 + g) * 32 + j) * KS;
-#pragma unroll
-        for (int s = 0; s < KS; ++s) acc = sah_mfma_32x32x2_f32(ap[s], xs[s], acc);
-      }
-    };
-    // The smallest value and its tile; a value that is not a number makes its tile's minimum one, and such key tiles are
-    // evaluated again below. Without the split form also that tile's 16 values, from which the slot is found once at the end
-    // (27 vector instructions a tile; a search for the slot takes 48): strictly smaller in ascending tiles, lowest slot, so
-    // that the first minimum is kept. In the split form instead every slot's minimum over the tiles, two tiles to a three-way
-    // minimum, and the second smallest of the tiles' minima (20 instructions a tile): together they tell whether any other
-    // centre came near the smallest value, and with none near the smallest value's slot is the one whose minimum it is.
-    float best = INFINITY, second = INFINITY;
-    int bt = 0;
-    bool nan = false;
-    sah_f32x16 kept = {};
-    auto tile_min = [&](const sah_f32x16& acc, int t) -> bool {
-      float m = acc[0];
-#pragma unroll
-      for (int v = 1; v < 16; ++v) m = PQM_MIN(m, acc[v]);
-      if (SPLIT) second = __builtin_amdgcn_fmed3f(best, second, m);
-      else nan |= m != m;
-      const bool less = m < best;
-      best = less ? m : best;
-      bt = less ? t : bt;
-      return less;
-    };
-    sah_f32x16 acc0, acc1;
-    if constexpr (SPLIT) {
-      product(acc0, 0);
-      tile_min(acc0, 0);
-      kept = acc0;
-      int t = 1;
-      for (; t + 1 < n_tiles; t += 2) {
-        product(acc0, t);
-        product(acc1, t + 1);
-#pragma unroll
-        for (int v = 0; v < 16; ++v) kept[v] = PQM_MIN(PQM_MIN(kept[v], acc0[v]), acc1[v]);
-        tile_min(acc0, t);
-        tile_min(acc1, t + 1);
-      }
-      if (t < n_tiles) {
-        product(acc0, t);
-#pragma unroll
-        for (int v = 0; v < 16; ++v) kept[v] = PQM_MIN(kept[v], acc0[v]);
-        tile_min(acc0, t);
-      }
-    } else {
-      auto take_min = [&](const sah_f32x16& acc, int t) {
-        const bool less = tile_min(acc, t);
-#pragma unroll
-        for (int v = 0; v < 16; ++v) kept[v] = less ? acc[v] : kept[v];
-      };
-      // two accumulators: a tile's products are issued before the minimum of the tile before is taken, which so never waits
-      // for a product just started
-      product(acc0, 0);
-      int t = 0;
-      for (; t + 2 < n_tiles; t += 2) {
-        product(acc1, t + 1);
-        take_min(acc0, t);
-        product(acc0, t + 2);
-        take_min(acc1, t + 1);
-      }
-      if (t + 1 < n_tiles) {
-        product(acc1, t + 1);
-        take_min(acc0, t);
-        take_min(acc1, t + 1);
-      } else {
-        take_min(acc0, t);
-      }
-    }
     int slot = 0, bidx;
     bool again;  // uniform: the key tile is evaluated in fp32, centres or keys not finite
     if constexpr (SPLIT) {
@@ -917,8 +817,9 @@ __global__ __launch_bounds__(PQM_NT, KS <= 16 ? 4 : 2) void k_pq_assign_mfma(pq_
               add(&s_sum[(d + 1) * n_cent + bidx], sah_bits_to_float(w & 0xffff0000u));
             };
             if constexpr (KS == 4) {
-              add2(g ? xb[0].z : xb[0].x, 4 * g);
-              add2(g ? xb[0].w : xb[0].y, 4 * g + 2);
+              const uint32_t upper = 0u - (uint32_t)g;  // (a choice between elements would become an index into scratch memory)
+              add2((xb[0].z & upper) | (xb[0].x & ~upper), 4 * g);
+              add2((xb[0].w & upper) | (xb[0].y & ~upper), 4 * g + 2);
             } else {
 #pragma unroll
               for (int q = 0; q < NB; ++q) {
@@ -940,6 +841,234 @@ __global__ __launch_bounds__(PQM_NT, KS <= 16 ? 4 : 2) void k_pq_assign_mfma(pq_
         if (g == 0) atomicAdd(&s_cnt[bidx], 1);
       }
     }
+  };
+  if constexpr (PIPE) {
+    auto first_op = [&](const sah_u4& x) { return KS == 4 && g ? sah_u4{0x3f803f80u, 0x3f80u, 0u, 0u} : x; };
+    auto in_range = [&](int kt) { return kt < wg_tiles && (tg * wg_tiles + kt) * 32 < P.n_keys; };  // uniform across the wave
+    int kt = wave;
+    if (in_range(kt)) {
+      float best, second;
+      int bt;
+      sah_f32x16 kept;
+      sah_u4 cur[NB];  // the keys in hand (nb: the next ones)
+      cur[0] = nb[0];
+      request((tg * wg_tiles + kt + PQM_NW) * 32 + j);
+      // the products of a pair of centre tiles: start, and for every operand its two loads and two matrix instructions
+      auto start = [&](int t, sah_f32x16& n0, sah_f32x16& n1) __attribute__((always_inline)) {
+        if constexpr (NORM_IN_A) {
+          n0 = n1 = sah_f32x16{};
+        } else {
+          const float4* cn4 = (const float4*)(s_cn + (t * 2 + g) * 16);
+#pragma unroll
+          for (int q4 = 0; q4 < 4; ++q4) {
+            const float4 c4 = cn4[q4], d4 = cn4[8 + q4];
+            n0[4 * q4] = c4.x; n0[4 * q4 + 1] = c4.y; n0[4 * q4 + 2] = c4.z; n0[4 * q4 + 3] = c4.w;
+            n1[4 * q4] = d4.x; n1[4 * q4 + 1] = d4.y; n1[4 * q4 + 2] = d4.z; n1[4 * q4 + 3] = d4.w;
+          }
+        }
+      };
+      auto load = [&](int t, int op, uint4 (&o)[2]) __attribute__((always_inline)) {
+        const uint4* ap = (const uint4*)s_a + (size_t)t * 64 * OPS + g * 32 + j;
+        o[0] = ap[op * 64];
+        o[1] = ap[(OPS + op) * 64];
+      };
+      auto mm = [&](const sah_u4& x, const uint4& o, sah_f32x16& acc) __attribute__((always_inline)) {
+        acc = sah_mfma_32x32x16<SAH_BF16>(o, __builtin_bit_cast(uint4, x), acc);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      auto take = [&](float m, int t) __attribute__((always_inline)) {
+        second = __builtin_amdgcn_fmed3f(best, second, m);
+        const bool less = m < best;
+        best = less ? m : best;
+        bt = less ? t : bt;
+      };
+      // the minima of tiles t and t + 1 (c0, c1), the products of tiles t_next and t_next + 1 (n0, n1) with the keys x
+      auto step = [&](auto first_c, const sah_f32x16& c0, const sah_f32x16& c1, int t, sah_f32x16& n0, sah_f32x16& n1, int t_next,
+                      const sah_u4& x, const sah_u4& x0) __attribute__((always_inline)) {
+        constexpr bool FIRST = decltype(first_c)::value;
+        uint4 o[2];
+        start(t_next, n0, n1);
+        load(t_next, 0, o);
+        if (FIRST) {
+          best = second = INFINITY;
+          bt = 0;
+        }
+        float m = c0[0];
+#pragma unroll
+        for (int v = 1; v < 8; ++v) m = PQM_MIN(m, c0[v]);
+        __builtin_amdgcn_sched_barrier(0);
+        mm(x0, o[0], n0);
+#pragma unroll
+        for (int v = 8; v < 16; ++v) m = PQM_MIN(m, c0[v]);
+        take(m, t);
+        __builtin_amdgcn_sched_barrier(0);
+        mm(x0, o[1], n1);
+        load(t_next, 1, o);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) kept[v] = FIRST ? PQM_MIN(c0[v], c1[v]) : PQM_MIN(PQM_MIN(kept[v], c0[v]), c1[v]);
+        __builtin_amdgcn_sched_barrier(0);
+        mm(x, o[0], n0);
+        m = c1[0];
+#pragma unroll
+        for (int v = 1; v < 8; ++v) m = PQM_MIN(m, c1[v]);
+        __builtin_amdgcn_sched_barrier(0);
+        mm(x, o[1], n1);
+        if constexpr (OPS == 3) load(t_next, 2, o);
+#pragma unroll
+        for (int v = 8; v < 16; ++v) m = PQM_MIN(m, c1[v]);
+        take(m, t + 1);
+        if constexpr (OPS == 3) {
+          __builtin_amdgcn_sched_barrier(0);
+          mm(x, o[0], n0);
+          mm(x, o[1], n1);
+        }
+      };
+      sah_f32x16 a0, a1, b0, b1;
+      {
+        start(0, a0, a1);
+#pragma unroll
+        for (int op = 0; op < OPS; ++op) {
+          uint4 o[2];
+          load(0, op, o);
+          mm(op ? cur[0] : first_op(cur[0]), o[0], a0);
+          mm(op ? cur[0] : first_op(cur[0]), o[1], a1);
+        }
+      }
+      for (;;) {
+        const int n = (tg * wg_tiles + kt) * 32 + j;
+        const sah_u4 cur0 = first_op(cur[0]);
+        step(std::true_type(), a0, a1, 0, b0, b1, 2, cur[0], cur0);
+        int t = 2;  // tiles t, t + 1 in b0, b1
+        for (; t + 2 < n_tiles; t += 4) {
+          step(std::false_type(), b0, b1, t, a0, a1, t + 2, cur[0], cur0);
+          step(std::false_type(), a0, a1, t + 2, b0, b1, t + 4, cur[0], cur0);
+        }
+        step(std::false_type(), b0, b1, t, a0, a1, 0, nb[0], first_op(nb[0]));
+        conclude(kt, n, cur, {0.f}, kept, best, second, bt, false);
+        kt += PQM_NW;
+        if (!in_range(kt)) break;
+        cur[0] = nb[0];
+        request(n + 2 * 32 * PQM_NW);
+      }
+    }
+  } else {
+  for (int kt = wave; kt < wg_tiles; kt += PQM_NW) {
+    const int n0 = (tg * wg_tiles + kt) * 32;
+    if (n0 >= P.n_keys) break;  // uniform across the wave
+    const int n = n0 + j;
+    float xs[SPLIT ? 1 : KS];  // this lane's dims 2 s + g of its key
+    sah_u4 xb[NB];             // SPLIT: dims 16 q + 8 g .. + 7 (sub-vectors of 8: both halves hold all)
+    sah_u4 x0;                 // key operand of the first instruction: with the norm in A, ones against its terms
+    if constexpr (SPLIT) {
+#pragma unroll
+      for (int q = 0; q < NB; ++q) xb[q] = nb[q];
+      request(n + 32 * PQM_NW);
+      x0 = xb[0];
+      if (KS == 4 && g) x0 = sah_u4{0x3f803f80u, 0x3f80u, 0u, 0u};
+    } else {
+      const int64_t off = key_offset(n);
+#pragma unroll
+      for (int s = 0; s < KS; ++s) xs[s] = (2 * s + g < d_sub) ? sah_load<DT>(P.k, off + 2 * s + g) : 0.f;
+    }
+    // accumulator of centre tile t: seeded with the norms, then the matrix instructions
+    auto product = [&](sah_f32x16& acc, int t) {
+      if constexpr (NORM_IN_A) {
+        acc = sah_f32x16{};
+      } else {
+        const float4* cn4 = (const float4*)(s_cn + (t * 2 + g) * 16);
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4) {
+          const float4 c4 = cn4[q4];
+          acc[4 * q4] = c4.x; acc[4 * q4 + 1] = c4.y; acc[4 * q4 + 2] = c4.z; acc[4 * q4 + 3] = c4.w;
+        }
+      }
+      if constexpr (SPLIT) {
+        const uint4* ap = (const uint4*)s_a + (size_t)t * 64 * OPS + g * 32 + j;
+#pragma unroll
+        for (int op = 0; op < OPS; ++op) acc = sah_mfma_32x32x16<SAH_BF16>(ap[op * 64], __builtin_bit_cast(uint4, op ? xb[op % NB] : x0), acc);
+      } else if constexpr (KS >= 4) {
+        const float4* ap = (const float4*)(s_a + (size_t)(t * 2 + g) * 32 * KS) + j;
+#pragma unroll
+        for (int q = 0; q < KS / 4; ++q) {
+          const float4 a4 = ap[q * 32];
+          acc = sah_mfma_32x32x2_f32(a4.x, xs[4 * q], acc);
+          acc = sah_mfma_32x32x2_f32(a4.y, xs[4 * q + 1], acc);
+          acc = sah_mfma_32x32x2_f32(a4.z, xs[4 * q + 2], acc);
+          acc = sah_mfma_32x32x2_f32(a4.w, xs[4 * q + 3], acc);
+        }
+      } else {
+        const float* ap = s_a + ((t * 2 + g) * 32 + j) * KS;
+#pragma unroll
+        for (int s = 0; s < KS; ++s) acc = sah_mfma_32x32x2_f32(ap[s], xs[s], acc);
+      }
+    };
+    // The smallest value and its tile; a value that is not a number makes its tile's minimum one, and such key tiles are
+    // evaluated again below. Without the split form also that tile's 16 values, from which the slot is found once at the end
+    // (27 vector instructions a tile; a search for the slot takes 48): strictly smaller in ascending tiles, lowest slot, so
+    // that the first minimum is kept. In the split form instead every slot's minimum over the tiles, two tiles to a three-way
+    // minimum, and the second smallest of the tiles' minima (20 instructions a tile): together they tell whether any other
+    // centre came near the smallest value, and with none near the smallest value's slot is the one whose minimum it is.
+    float best = INFINITY, second = INFINITY;
+    int bt = 0;
+    bool nan = false;
+    sah_f32x16 kept = {};
+    auto tile_min = [&](const sah_f32x16& acc, int t) -> bool {
+      float m = acc[0];
+#pragma unroll
+      for (int v = 1; v < 16; ++v) m = PQM_MIN(m, acc[v]);
+      if (SPLIT) second = __builtin_amdgcn_fmed3f(best, second, m);
+      else nan |= m != m;
+      const bool less = m < best;
+      best = less ? m : best;
+      bt = less ? t : bt;
+      return less;
+    };
+    sah_f32x16 acc0, acc1;
+    if constexpr (SPLIT) {
+      product(acc0, 0);
+      tile_min(acc0, 0);
+      kept = acc0;
+      int t = 1;
+      for (; t + 1 < n_tiles; t += 2) {
+        product(acc0, t);
+        product(acc1, t + 1);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) kept[v] = PQM_MIN(PQM_MIN(kept[v], acc0[v]), acc1[v]);
+        tile_min(acc0, t);
+        tile_min(acc1, t + 1);
+      }
+      if (t < n_tiles) {
+        product(acc0, t);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) kept[v] = PQM_MIN(kept[v], acc0[v]);
+        tile_min(acc0, t);
+      }
+    } else {
+      auto take_min = [&](const sah_f32x16& acc, int t) {
+        const bool less = tile_min(acc, t);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) kept[v] = less ? acc[v] : kept[v];
+      };
+      // two accumulators: a tile's products are issued before the minimum of the tile before is taken, which so never waits
+      // for a product just started
+      product(acc0, 0);
+      int t = 0;
+      for (; t + 2 < n_tiles; t += 2) {
+        product(acc1, t + 1);
+        take_min(acc0, t);
+        product(acc0, t + 2);
+        take_min(acc1, t + 1);
+      }
+      if (t + 1 < n_tiles) {
+        product(acc1, t + 1);
+        take_min(acc0, t);
+        take_min(acc1, t + 1);
+      } else {
+        take_min(acc0, t);
+      }
+    }
+    conclude(kt, n, xb, xs, kept, best, second, bt, nan);
+  }
   }
   if (!SUMS) return;
   __syncthreads();
@@ -1011,7 +1140,7 @@ __global__ __launch_bounds__(PQS_NT) void k_pq_sums(pq_assign_params P, int d_ch
       if (s_cnt[c]) atomicAdd(&P.counts[(int64_t)grp * n_cent + c], s_cnt[c]);
 }
 
-template <int DT, int KS, bool SPLIT>
+template <int DT, int KS, bool SPLIT, bool PIPE>
 static int pq_launch_mfma_ks(const sah_pq_assign_args* a, const pq_assign_params& P, const pq_update_params& U, uint32_t* arrivals, bool fused,
                              size_t lds) {
   const int tiles = (a->n_keys + 31) / 32;
@@ -1027,11 +1156,11 @@ static int pq_launch_mfma_ks(const sah_pq_assign_args* a, const pq_assign_params
   hipStream_t st = (hipStream_t)a->stream;
   sah_timed timed("k_pq_assign_mfma", a->stream);
   if (fused) {
-    if (int rc = sah_allow_lds((const void*)k_pq_assign_mfma<DT, KS, true, SPLIT>, PQM_MAX_LDS, "sah_pq_kmeans_assign")) return rc;
-    hipLaunchKernelGGL((k_pq_assign_mfma<DT, KS, true, SPLIT>), g, blk, lds, st, P, U, arrivals, per, ranges, heads);
+    if (int rc = sah_allow_lds((const void*)k_pq_assign_mfma<DT, KS, true, SPLIT, PIPE>, PQM_MAX_LDS, "sah_pq_kmeans_assign")) return rc;
+    hipLaunchKernelGGL((k_pq_assign_mfma<DT, KS, true, SPLIT, PIPE>), g, blk, lds, st, P, U, arrivals, per, ranges, heads);
   } else {
-    if (int rc = sah_allow_lds((const void*)k_pq_assign_mfma<DT, KS, false, SPLIT>, PQM_MAX_LDS, "sah_pq_kmeans_assign")) return rc;
-    hipLaunchKernelGGL((k_pq_assign_mfma<DT, KS, false, SPLIT>), g, blk, lds, st, P, U, nullptr, per, ranges, heads);
+    if (int rc = sah_allow_lds((const void*)k_pq_assign_mfma<DT, KS, false, SPLIT, PIPE>, PQM_MAX_LDS, "sah_pq_kmeans_assign")) return rc;
+    hipLaunchKernelGGL((k_pq_assign_mfma<DT, KS, false, SPLIT, PIPE>), g, blk, lds, st, P, U, nullptr, per, ranges, heads);
   }
   return sah_launch_status("sah_pq_kmeans_assign");
 }
@@ -1040,9 +1169,12 @@ template <int DT, int KS>
 static int pq_launch_mfma_form(const sah_pq_assign_args* a, const pq_assign_params& P, const pq_update_params& U, uint32_t* arrivals, bool split,
                                bool fused, size_t lds) {
   if constexpr (DT == SAH_BF16 && KS >= 4) {
-    if (split) return pq_launch_mfma_ks<DT, KS, true>(a, P, U, arrivals, fused, lds);
+    if constexpr (KS <= 8) {
+      if (split && (a->n_cent + 31) / 32 % 4 == 0) return pq_launch_mfma_ks<DT, KS, true, true>(a, P, U, arrivals, fused, lds);
+    }
+    if (split) return pq_launch_mfma_ks<DT, KS, true, false>(a, P, U, arrivals, fused, lds);
   }
-  return pq_launch_mfma_ks<DT, KS, false>(a, P, U, arrivals, fused, lds);
+  return pq_launch_mfma_ks<DT, KS, false, false>(a, P, U, arrivals, fused, lds);
 }
 
 template <int DT>
