@@ -94,8 +94,10 @@ class ResearchAttention(SparseAttention):
                      and not isinstance(kwargs.get("s_aux"), torch.Tensor) and queries.dim() == 4
                      and not (dropout > 0.0 and module is not None and getattr(module, "training", False)))
 
-        attention_mask, only_hides, out, question = self._under_mask(
-            queries, keys, values, attention_mask, scaling, sparse_meta_data, kwargs.get("layer_idx"), plannable)
+        only_hides, out, question = False, None, None
+        if attention_mask is not None:
+            attention_mask, only_hides, out, question = self._under_mask(
+                queries, keys, values, attention_mask, scaling, sparse_meta_data, kwargs.get("layer_idx"), plannable)
         if out is None and plannable and (attention_mask is None or queries.shape[2] == 1):
             out = self._plan_step(queries, keys, values, attention_mask, scaling, sparse_meta_data, kwargs.get("layer_idx"), only_hides)
         if out is not None:
@@ -165,7 +167,7 @@ class ResearchAttention(SparseAttention):
             metrics.log("research_attention_output_error", float(error.item()), metadata={"layer_idx": kwargs["layer_idx"]})
         return out, weights
 
-    def _under_mask(self, queries: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, attention_mask: Optional[torch.Tensor],
+    def _under_mask(self, queries: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, attention_mask: torch.Tensor,
                     scaling: float, sparse_meta_data: Dict[Any, Any], layer_idx: Optional[int], plannable: bool):
         """(the mask that counts, does it only hide columns, the step's output if it has been made, a question still open).
 
@@ -176,7 +178,7 @@ class ResearchAttention(SparseAttention):
         launched again (what it adds to the caches does not depend on the mask). A mask of several queries, all but always
         nonzero, is taken as it is, which is right whatever it holds."""
         am = attention_mask
-        if (am is None or not am.is_cuda or am.dim() != 4 or am.shape[-1] < keys.shape[2]
+        if (not am.is_cuda or am.dim() != 4 or am.shape[-1] < keys.shape[2]
                 or am.dtype not in (torch.float32, torch.bfloat16, torch.float16)):
             return am, False, None, None
         facts = self._mask_facts
