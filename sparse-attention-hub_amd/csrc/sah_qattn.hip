@@ -16,7 +16,7 @@
 // rounding the result is off by 2.4e-7 (2-norm, 4096 keys, bf16; fp16 3.5e-7) where the gather's is by 1.6e-7 (1.8e-7): the
 // order of the fp32 sums. With two terms for bf16 2.3e-6.
 // What bounds it: per wave and 32-key tile 32 matrix instructions (fp16: 24; 1024 and 768 cycles) and about 190 vector ones
-// with 17 exponentials (150; 960 and 800 cycles), which do not overlap on a SIMD. The third term costs 3 us of a pass of 244
+// with 17 exponentials (150; 960 and 800 cycles), which overlap little with two waves on a SIMD, each issuing one in eight cycles. The third term costs 3 us of a pass of 244
 // with the causal mask.
 // Keys are split over workgroups; the partial results (m, l, acc) are merged by a second kernel.
 #include "sah_common.h"
