@@ -483,7 +483,7 @@ __global__ __launch_bounds__(PQ_NT) void k_pq_update(pq_update_params P) {
 // Measured (bf16, 8 heads x 16277 keys, 16 sub-vectors of 8, 256 centres, sums included): 64 us (66 with the update; 65 and 71
 // without the pipeline of PIPE); 85 with every tile's 16 values selected, not their minima over the tiles, the second look by matrix instruction, its test by ballots, the key
 // operand in a structure (which went through scratch memory) and the centres read element by element. What bounds it: 20 vector
-// and 2 matrix instructions a tile, in sum (5 us a tile and key tile: 40), 150 vector ones a key tile of eight (20), 6 before and
+// and 2 matrix instructions a tile, in sum (5 us a centre tile: 40), 150 vector ones a key tile of eight (20), 6 before and
 // after the loop. fp16 (no split: terms of small centres would leave its range): 121 at 16405 keys. 32768 keys, 2 sub-vectors of 64, 64
 // centres: 218 -> 47 with the split. Sums in [centre][d] order and a flush of one centre a lane took 40 (8 dims) to 100 us
 // (64 dims) of these.
