@@ -80,6 +80,7 @@ class PackedSignatureCache:
         self.codes = grown
         self.pos = self.exc = self.exc_cnt = None  # rebuilt from the codes at the next decode step
         self.n_compact = 0
+        self.compact_stream = None
 
     @property
     def full_plane(self) -> int:
