@@ -190,7 +190,7 @@ class ResearchAttention(SparseAttention):
             if plannable and guess is not None and (guess == 0 or queries.shape[2] == 1):
                 hides = not guess & _native.AMASK_GENERAL and same_type
                 try:
-                    out = self._plan_step(queries, keys, values, am if guess else None, scaling, sparse_meta_data, layer_idx, hides)
+                    out = self._plan_step(queries, keys, values, am if guess else None, scaling, sparse_meta_data, layer_idx, hides, guessed=True)
                 except Exception:
                     out = None  # (what is wrong with the call under its own mask, if anything, is said then)
                 flags = facts.take(question)
@@ -205,15 +205,19 @@ class ResearchAttention(SparseAttention):
         return am, not flags & _native.AMASK_GENERAL and same_type, None, None
 
     def _plan_step(self, queries: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, attention_mask: Optional[torch.Tensor],
-                   scaling: float, sparse_meta_data: Dict[Any, Any], layer_idx: Optional[int], only_hides: bool) -> Optional[torch.Tensor]:
-        """One step through the cached plan of its geometry, or None where the plan does not cover it."""
+                   scaling: float, sparse_meta_data: Dict[Any, Any], layer_idx: Optional[int], only_hides: bool,
+                   guessed: bool = False) -> Optional[torch.Tensor]:
+        """One step through the cached plan of its geometry, or None where the plan does not cover it. `guessed`: launched as if
+        its mask were zero, or only hid columns, before the answer is there."""
         _native.require_device(queries, "queries")
         masked = attention_mask is not None
-        key = (queries.device, queries.dtype, tuple(queries.shape), keys.shape[1], masked)
         # A masked step's buffers belong to the stream and thread of their plan, as those of the masker-by-masker path
-        # belong to the call: a step on another stream is not ordered with the ones that use them. A captured one's
+        # belong to the call: a step on another stream is not ordered with the ones that use them. So do those of a step whose
+        # mask is guessed to be zero: it may turn out to be a masked one. A captured step's
         # belong to its graph alone: what its plan clears is clear when the graph runs, not now.
-        owner = (_native.stream_ptr(queries.device), threading.get_ident()) if masked else None
+        owned = masked or guessed
+        key = (queries.device, queries.dtype, tuple(queries.shape), keys.shape[1], masked, owned)
+        owner = (_native.stream_ptr(queries.device), threading.get_ident()) if owned else None
         if masked and torch.cuda.is_current_stream_capturing():
             plan = DecodePlan(self.maskers, self._plan_kind, queries, keys, True)
         else:

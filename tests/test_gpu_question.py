@@ -961,3 +961,42 @@ def test_steps_launched_on_a_guess_about_their_mask(cuda, dtype, chain):
     bad = torch.full((1, 1, 3, Lk), -1.0, dtype=dtype, device=cuda)
     with pytest.raises(ValueError, match="does not cover"):
         guessing.custom_attention(None, q, k, v, bad, D ** -0.5, 0.0, sparse_meta_data=meta, layer_idx=0)
+
+
+@pytest.mark.parametrize("chain", ["fixed", "hash", "oracle", "pq"])
+def test_padded_and_unpadded_sessions_on_two_streams(cuda, chain):
+    """Two sessions of one instance and geometry, unpadded on one stream and padded on the other, nothing between the two: every
+    step gives what it gives alone."""
+    import sparse_attention_hub_amd.sparse_attention as sa
+    from sparse_attention_hub_amd.sparse_attention.utils.hashattention_utils import random_hat_weights
+
+    B, Hq, Hkv, Lk, D = 2, 8, 2, 1500, 128
+    cfgs = [sa.SinkMaskerConfig(sink_size=9), sa.LocalMaskerConfig(window_size=70)]
+    if chain == "hash":
+        cfgs.append(sa.HashAttentionTopKMaskerConfig(
+            heavy_size=50, hat_bits=32, hat_mlp_layers=3, hat_mlp_hidden_size=128, hat_mlp_activation="silu",
+            hat_weights=random_hat_weights(1, Hq, D, 32, 3, 128, dtype=torch.bfloat16, seed=1)))
+    elif chain == "oracle":
+        cfgs.append(sa.OracleTopKConfig(heavy_size=50))
+    elif chain == "pq":
+        cfgs.append(sa.PQCacheConfig(heavy_size=50, pq_group_factor=8, pq_bits=4, kmeans_iter=3, init_offset=9, metric="euclidean"))
+    _, k, v = make_qkv(B, Hq, Hkv, 1, Lk, D, torch.bfloat16, seed=5, device=cuda)
+    qs = [make_qkv(B, Hq, Hkv, 1, 1, D, torch.bfloat16, seed=s, device=cuda)[0] for s in range(12)]
+    zero = torch.zeros((B, 1, 1, Lk))
+    padded = _hide(zero.clone(), "padded", Lk, 70, float(torch.finfo(torch.bfloat16).min))
+    masks = [(padded if i % 2 else zero).to(torch.bfloat16).to(cuda) for i in range(12)]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    results = []
+    for together in (False, True):
+        ra = sa.ResearchAttention.create_from_config(sa.ResearchAttentionConfig(masker_configs=cfgs))
+        ra.return_attention_weights = False
+        metas, outs = ({}, {}), []
+        torch.cuda.synchronize()
+        for i in range(12):  # (the first two fill the layers' caches)
+            with torch.cuda.stream(streams[i % 2]):
+                outs.append(ra.custom_attention(None, qs[i], k, v, masks[i], D ** -0.5, 0.0, sparse_meta_data=metas[i % 2], layer_idx=0)[0])
+            if not together or i < 2:
+                torch.cuda.synchronize()
+        torch.cuda.synchronize()
+        results.append(torch.stack(outs))
+    assert torch.equal(results[0], results[1])

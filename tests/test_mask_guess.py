@@ -1,0 +1,147 @@
+"""What is known, guessed and asked about an additive mask, and whose buffers a step uses meanwhile: host logic, with the
+native calls recorded instead of made."""
+import threading
+
+import pytest
+import torch
+
+from sparse_attention_hub_amd import _native as N
+from sparse_attention_hub_amd import sparse_attention as sa
+from sparse_attention_hub_amd.sparse_attention.research_attention.maskers.fixed.implementations.hashattention_top_k import (
+    PackedSignatureCache,
+)
+from sparse_attention_hub_amd.sparse_attention.utils import mask_attention_utils as U
+from sparse_attention_hub_amd.sparse_attention.utils.hashattention_utils import random_hat_weights
+
+B, HQ, HKV, LK, D = 2, 4, 2, 400, 64
+LOWEST = float(torch.finfo(torch.bfloat16).min)
+
+
+class Recorder:
+    """Native calls by name, the stream they were made on and the buffers that a chain's blocks name."""
+
+    def __init__(self):
+        self.stream, self.capturing, self.fails = 0, False, None
+        self.calls, self.masks = [], {}
+
+    def call(self, name, args):
+        if self.fails is not None and name in ("sah_run_chain", "sah_hash_decode_masked"):
+            raise self.fails
+        if name == "sah_hash_decode_masked":
+            if args.ask:
+                args.fits = 1
+                return
+            hd = N.HashDecodeArgs.from_address(args.decode)
+            self.calls.append((name, self.stream, {hd.rows.cols, hd.rows.cnt, args.tickets, N.HashSigArgs.from_address(hd.query_sig).codes}, hd))
+        elif name == "sah_run_chain":
+            used = {args.tickets}
+            if args.select:
+                se = N.SelectTopkArgs.from_address(args.select)
+                used |= {se.keys, se.rows.cols, se.rows.cnt}
+            if args.hash_decode:
+                hd = N.HashDecodeArgs.from_address(args.hash_decode)
+                used |= {hd.rows.cols, hd.rows.cnt, N.HashSigArgs.from_address(hd.query_sig).codes}
+            if args.attention:
+                at = N.AttentionArgs.from_address(args.attention)
+                used |= {at.rows.cols, at.rows.cnt}
+            self.calls.append((name, self.stream, used, bool(args.compact)))
+        else:
+            if name == "sah_amask_answer":
+                m = self.masks[args.read.mask.amask]
+                args.read.flags = (1 if bool((m != 0).any()) else 0) | (2 if bool(((m != 0) & (m != LOWEST)).any()) else 0)
+            self.calls.append((name, self.stream, set(), None))
+
+    def launches(self):
+        return [c for c in self.calls if c[0] == "sah_hash_decode_masked" or c[0] == "sah_run_chain"]
+
+
+@pytest.fixture
+def device(monkeypatch):
+    r = Recorder()
+    words = threading.local()
+
+    def answer_words(dev):
+        if not hasattr(words, "pair"):
+            words.pair = (torch.zeros(2, dtype=torch.int32), torch.zeros(1, dtype=torch.int64))
+        return words.pair
+
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True, raising=False)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: r.capturing)
+    monkeypatch.setattr(N, "call", r.call)
+    monkeypatch.setattr(N, "stream_ptr", lambda device: r.stream)
+    monkeypatch.setattr(N, "work_floats", lambda *a: 64)
+    monkeypatch.setattr(N, "members_work_floats", lambda *a: 64)
+    monkeypatch.setattr(U, "_answer_words", answer_words)
+    return r
+
+
+def attention(chain):
+    cfgs = [sa.SinkMaskerConfig(sink_size=4), sa.LocalMaskerConfig(window_size=32)]
+    if chain == "oracle":
+        cfgs.append(sa.OracleTopKConfig(heavy_size=20))
+    elif chain == "hash":
+        cfgs.append(sa.HashAttentionTopKMaskerConfig(
+            heavy_size=20, hat_bits=32, hat_mlp_layers=3, hat_mlp_hidden_size=128, hat_mlp_activation="silu",
+            hat_weights=random_hat_weights(1, HQ, D, 32, 3, 128, dtype=torch.bfloat16, seed=1)))
+    ra = sa.ResearchAttention.create_from_config(sa.ResearchAttentionConfig(masker_configs=cfgs))
+    ra.return_attention_weights = False
+    return ra
+
+
+class Session:
+    """One sequence's steps: its caches, and a new mask tensor for every step."""
+
+    def __init__(self, r, ra, chain, n=LK):
+        self.r, self.ra, self.kept = r, ra, []
+        self.meta = {}
+        if chain == "hash":
+            cache = PackedSignatureCache(B, HQ, 32, n + 4096, torch.device("cpu"))
+            cache.n = n
+            self.meta["key"] = {0: cache}
+            self.cache = cache
+        self.q = torch.zeros(B, HQ, 1, D, dtype=torch.bfloat16)
+        self.k = torch.zeros(B, HKV, n + 64, D, dtype=torch.bfloat16)
+
+    def mask(self, kind, n=LK, n_q=1):
+        m = torch.zeros(B, 1, n_q, n, dtype=torch.bfloat16)
+        if kind != "z":
+            m[0, ..., :50] = LOWEST if kind == "h" else -1.0
+        self.r.masks[m.data_ptr()] = m
+        self.kept.append(m)
+        return m
+
+    def step(self, kind, stream=0, n=LK, mask=None):
+        """The launches of one step under a new mask: zero, hiding or general."""
+        before = len(self.r.launches())
+        m = self.mask(kind, n) if mask is None else mask
+        self.r.stream = stream
+        out = self.ra.custom_attention(None, self.q, self.k[:, :, :n], self.k[:, :, :n], m, D ** -0.5, 0.0,
+                                       sparse_meta_data=self.meta, layer_idx=0)[0]
+        self.kept.append((out, list(self.ra._plans.values())))  # (no address is given out twice)
+        return self.r.launches()[before:]
+
+
+@pytest.mark.parametrize("other", ["stream", "thread"])
+@pytest.mark.parametrize("chain", ["fixed", "hash", "oracle"])
+@pytest.mark.parametrize("order", ["zh", "zzh", "hz", "zhzh", "zzhhz", "zhhzz"])  # z: the unpadded session's turn, h: the padded one's
+def test_sessions_that_are_not_ordered_share_no_buffers(device, chain, order, other):
+    """An unpadded session on one stream or thread and a padded one of the same geometry on another: whatever is launched for
+    the padded one, on a guess or not, uses nothing that the unpadded one uses."""
+    ra = attention(chain)
+    plain, padded = Session(device, ra, chain), Session(device, ra, chain)
+    used = {"z": set(), "h": set()}
+    for kind in order:
+        if kind == "z":
+            launches = plain.step("z", 1)
+        elif other == "stream":
+            launches = padded.step("h", 2)
+        else:
+            out = []
+            t = threading.Thread(target=lambda: out.extend(padded.step("h", 1)))
+            t.start()
+            t.join()
+            launches = out
+        assert launches
+        for _, _, buffers, _ in launches:
+            used[kind] |= buffers - {None}
+    assert used["z"] and used["h"] and used["z"].isdisjoint(used["h"])
