@@ -159,7 +159,7 @@ class ResearchAttention(SparseAttention):
                 return_attention_weights=False, **kwargs,
             )
         if question is not None:
-            self._mask_facts.take(question)
+            self._mask_facts.take(question, sparse_meta_data)
         if want_error:
             # relative distance to dense attention over all keys, by the same kernel in dense mode (reference :150-168)
             true_out, _ = get_true_attention_output(module, queries, keys, values, attention_mask, scaling, dropout, **kwargs)
@@ -174,7 +174,7 @@ class ResearchAttention(SparseAttention):
         An additive mask of zeros (HuggingFace's eager mask of an unpadded decode step) adds nothing anywhere and is left out;
         one that only hides columns has a faster way. Which it is, is established once per mask tensor, i.e. once per forward
         pass, not per layer, and the first layer does not wait for the answer with nothing under way: a decode step's mask is
-        taken to be like the last step's, the step is launched and the answer read; a step launched on a wrong guess is
+        taken to be like the session's last step's, the step is launched and the answer read; a step launched on a wrong guess is
         launched again (what it adds to the caches does not depend on the mask). A mask of several queries, all but always
         nonzero, is taken as it is, which is right whatever it holds."""
         am = attention_mask
@@ -185,7 +185,7 @@ class ResearchAttention(SparseAttention):
         same_type = am.dtype == queries.dtype  # (a lowest value of another type is none of the queries')
         flags = facts.known(am)
         if flags is None:
-            guess = facts.guess(am)
+            guess = facts.guess(am, sparse_meta_data)
             question = MaskQuestion(am)
             if plannable and guess is not None and (guess == 0 or queries.shape[2] == 1):
                 hides = not guess & _native.AMASK_GENERAL and same_type
@@ -193,13 +193,13 @@ class ResearchAttention(SparseAttention):
                     out = self._plan_step(queries, keys, values, am if guess else None, scaling, sparse_meta_data, layer_idx, hides, guessed=True)
                 except Exception:
                     out = None  # (what is wrong with the call under its own mask, if anything, is said then)
-                flags = facts.take(question)
+                flags = facts.take(question, sparse_meta_data)
                 if out is not None and (flags == guess or (guess and not (hides and flags & _native.AMASK_GENERAL))):
                     return am, hides, out, None
             elif am.shape[2] > 1 and guess != 0 and mask_covers(am, queries, keys.shape[2]):
                 return am, False, None, question
             else:
-                flags = facts.take(question)
+                flags = facts.take(question, sparse_meta_data)
         if flags == 0:
             return None, False, None, None
         return am, not flags & _native.AMASK_GENERAL and same_type, None, None

@@ -10,6 +10,7 @@ reference, utils/mask.py:733-735).
 """
 from __future__ import annotations
 
+import itertools
 import threading
 from typing import Any, Dict, Optional, Tuple, Union
 
@@ -163,11 +164,16 @@ class AdditiveMaskFacts:
     The device is asked once per tensor (one small launch, answered into host memory, over the mask's whole width: a
     mask that is zero everywhere is zero on the columns of any key count) and the answer remembered for as long as
     the same, unmodified tensor keeps arriving; the tensor is kept referenced meanwhile, so its memory cannot be
-    handed to another tensor that would then be mistaken for it."""
+    handed to another tensor that would then be mistaken for it.
+
+    What a session's last mask held is the guess for its next one. It is kept in the session's own `sparse_meta_data` (sessions
+    with and without padding that take turns are each guessed right), under a number of this object's."""
+
+    _numbers = itertools.count()
 
     def __init__(self) -> None:
         self._seen: Tuple[Optional[torch.Tensor], int, int] = (None, -1, 0)  # tensor, its version, flags
-        self._last: Dict[bool, int] = {}  # one query or several -> flags of the last such mask
+        self._number = next(self._numbers)
 
     def known(self, am: torch.Tensor) -> Optional[int]:
         tensor, version, flags = self._seen
@@ -177,14 +183,17 @@ class AdditiveMaskFacts:
             return N.AMASK_NONZERO | N.AMASK_GENERAL  # nothing established: every consumer reads the mask itself
         return None
 
-    def guess(self, am: torch.Tensor) -> Optional[int]:
-        """The flags of the last mask for as many queries (one, or several)."""
-        return self._last.get(am.shape[2] == 1)
+    def guess(self, am: torch.Tensor, session: Any) -> Optional[int]:
+        """The flags of the session's last mask for as many queries (one, or several)."""
+        if not isinstance(session, dict):
+            return None
+        return session.get("additive_mask_flags", {}).get((self._number, am.shape[2] == 1))
 
-    def take(self, question: MaskQuestion) -> int:
+    def take(self, question: MaskQuestion, session: Any = None) -> int:
         flags = question.settle()
         self._seen = (question.mask, question.version, flags)
-        self._last[question.mask.shape[2] == 1] = flags
+        if isinstance(session, dict):
+            session.setdefault("additive_mask_flags", {})[(self._number, question.mask.shape[2] == 1)] = flags
         return flags
 
     def flags(self, attention_mask: torch.Tensor) -> int:

@@ -145,3 +145,27 @@ def test_sessions_that_are_not_ordered_share_no_buffers(device, chain, order, ot
         for _, _, buffers, _ in launches:
             used[kind] |= buffers - {None}
     assert used["z"] and used["h"] and used["z"].isdisjoint(used["h"])
+
+
+@pytest.mark.parametrize("chain", ["fixed", "oracle"])
+def test_sessions_in_turn_are_launched_once_a_step(device, chain):
+    """The guess is the session's: padded and unpadded ones that one instance serves in turn are each guessed right. A session's
+    own change of mask costs it one launch."""
+    ra = attention(chain)
+    plain, padded = Session(device, ra, chain), Session(device, ra, chain)
+    for _ in range(3):
+        assert len(plain.step("z")) == 1 and len(padded.step("h")) == 1
+    assert [len(plain.step(kind)) for kind in "zhhz"] == [1, 2, 1, 1]  # (a zero mask is right under a plan that takes a mask)
+    answers = [i for i, c in enumerate(device.calls) if c[0] == "sah_amask_answer"]
+    launches = [i for i, c in enumerate(device.calls) if c[0] == "sah_run_chain"]
+    assert launches[-1] < answers[-1]  # the step's answer is read with the step under way
+
+
+def test_an_instance_guesses_nothing_from_another_one(device):
+    first = attention("oracle")
+    session = Session(device, first, "oracle")
+    session.step("z")
+    session.ra = attention("oracle")
+    assert len(session.step("h")) == 1
+    session.meta = None  # a chain that keeps nothing takes this, too
+    assert [len(session.step(kind)) for kind in "hzh"] == [1, 1, 1]
