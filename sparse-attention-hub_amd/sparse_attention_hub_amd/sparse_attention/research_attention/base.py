@@ -224,7 +224,7 @@ class ResearchAttention(SparseAttention):
             plan = self._plans.get(key)
             if plan is None or plan.owner != owner:
                 plan = self._plans[key] = DecodePlan(self.maskers, self._plan_kind, queries, keys, masked, owner)
-        return plan.run(queries, keys, values, scaling, sparse_meta_data, layer_idx, attention_mask, only_hides)
+        return plan.run(queries, keys, values, scaling, sparse_meta_data, layer_idx, attention_mask, only_hides, guessed)
 
     @classmethod
     def create_from_config(cls, config: SparseAttentionConfig) -> "ResearchAttention":

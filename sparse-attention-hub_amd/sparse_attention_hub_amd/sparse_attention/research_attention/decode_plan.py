@@ -27,7 +27,7 @@ from ... import _native as N
 from ..utils.mask_attention_utils import _workspace, additive_mask_args, dense_rows_possible, unit_inverse_weight
 from .maskers.fixed.base import sortable_key_of
 from .maskers.fixed.implementations.basic_fixed import LocalMasker, SinkMasker
-from .maskers.fixed.implementations.hashattention_top_k import HashAttentionTopKMasker, PackedSignatureCache
+from .maskers.fixed.implementations.hashattention_top_k import HashAttentionTopKMasker, PackedSignatureCache, SEVERAL_STREAMS
 from .maskers.fixed.implementations.oracle_top_k import OracleTopK
 from .maskers.fixed.implementations.pq_top_k import PQCache, PQCodebook, adc_lut_buffer
 
@@ -139,7 +139,7 @@ class DecodePlan:
 
     def _use_compact(self, hd: "N.HashDecodeArgs", cache: PackedSignatureCache, hashed: int, stream: int, commit: list) -> None:
         """The compact form of the first `hashed` codes for `hd`, brought up to date by a launch of the chain's."""
-        cache.ensure_compact_buffers()
+        cache.ensure_compact_buffers(stream)
         if hashed > cache.n_compact:
             cp = self.compact
             cp.codes, cp.code_pitch, cp.n_rows = cache.codes.data_ptr(), cache.capacity, self.n_rows
@@ -149,7 +149,8 @@ class DecodePlan:
             cp.full_plane, cp.stream = cache.full_plane, stream
             self.chain.compact = C.addressof(cp)
             commit.append((cache, "n_compact", hashed))
-            commit.append((cache, "compact_stream", stream))
+            # (what two streams have written stays unordered for either)
+            commit.append((cache, "compact_stream", stream if cache.compact_ordered(stream) else SEVERAL_STREAMS))
         hd.pos_codes, hd.pos_pitch = cache.pos.data_ptr(), cache.pos.shape[2]
         hd.exc, hd.exc_cap, hd.exc_cnt = cache.exc.data_ptr(), cache.exc.shape[2], cache.exc_cnt.data_ptr()
         hd.full_plane = cache.full_plane
@@ -163,7 +164,7 @@ class DecodePlan:
         # would read what another stream has written, or that is captured and would have to write it, takes the other way.
         # (a byte and two bits of LDS a key and four bytes an entry: longer rows do not get as far as buffers they cannot use)
         if (only_hides and self.dtype != torch.float16 and rows.n_keys * 5 // 4 + 4 * rows.cap <= 150 * 1024
-                and cache.compact_stream in (None, stream)
+                and cache.compact_ordered(stream)
                 and (cache.n_compact >= hashed or not torch.cuda.is_current_stream_capturing())):
             hd, hm = self.hash_decode, self.hash_masked
             hd.rows, hd.sink, hd.window, hd.k, hd.stream = rows, sink, window, k_eff, stream
@@ -208,9 +209,10 @@ class DecodePlan:
     # --------------------------------------------------------------------- run
     def run(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scaling: float,
             sparse_meta_data: Dict[Any, Any], layer_idx: Optional[int],
-            attention_mask: Optional[torch.Tensor] = None, only_hides: bool = False) -> Optional[torch.Tensor]:
+            attention_mask: Optional[torch.Tensor] = None, only_hides: bool = False, guessed: bool = False) -> Optional[torch.Tensor]:
         """One layer-step; returns the attention output (B, Lq, Hq, D) or None if not applicable. `only_hides`: the mask is known
-        to hold nothing but zeros and entries at the lowest value of its type or -inf."""
+        to hold nothing but zeros and entries at the lowest value of its type or -inf. `guessed`: the step's mask may be another
+        one, under which the step must not read or write what another stream has written."""
         masked = self.masked
         if masked and (self.Lq != 1 or attention_mask.dim() != 4):
             return None
@@ -254,6 +256,8 @@ class DecodePlan:
             if not isinstance(cache, PackedSignatureCache) or Lk < cache.n or Lk - cache.n > _MAX_NEW_KEYS:
                 return None
             if cache.codes.shape[0] != self.B or cache.codes.shape[1] != self.Hq:
+                return None
+            if guessed and not cache.compact_ordered(stream):
                 return None
             blocks = self.layers.get(layer_idx)
             wkey = (id(top.hat_weights), layer_idx)

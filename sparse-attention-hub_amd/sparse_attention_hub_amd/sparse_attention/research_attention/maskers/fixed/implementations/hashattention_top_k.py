@@ -42,6 +42,9 @@ class HashAttentionTopKMaskerConfig(TopKMaskerConfig):
     search_space: Dict[str, Any] = field(default_factory=_default_search_space)
 
 
+SEVERAL_STREAMS = -1  # no stream's handle
+
+
 class PackedSignatureCache:
     """Key signatures of one layer: int32 codes [B, Hq, capacity, 2] (positive plane,
     non-zero plane), `n` of them valid.
@@ -60,7 +63,8 @@ class PackedSignatureCache:
         # columns with a zero component [B, Hq, exc_cap, 4] and their number [B, Hq]; valid for `n_compact` keys
         self.pos = self.exc = self.exc_cnt = None
         self.n_compact = 0
-        self.compact_stream = None  # the stream of the launch that last wrote the compact form
+        # the one stream on which the compact form's buffers were cleared and written; None: there are none, SEVERAL_STREAMS: no one
+        self.compact_stream: Optional[int] = None
 
     @property
     def capacity(self) -> int:
@@ -86,11 +90,16 @@ class PackedSignatureCache:
     def full_plane(self) -> int:
         return (1 << self.bits) - 1
 
-    def ensure_compact_buffers(self) -> None:
-        """Buffers of the compact form, sized for the current capacity (8192 columns of slack for the
-        kernel's whole-chunk reads, whose scores count nowhere)."""
+    def compact_ordered(self, stream: int) -> bool:
+        """Is a launch on `stream` behind everything that wrote the compact form, whatever the caller orders?"""
+        return self.compact_stream in (None, stream)
+
+    def ensure_compact_buffers(self, stream: int) -> None:
+        """Buffers of the compact form, for a launch that writes them on `stream`, the current one; sized for the current
+        capacity (8192 columns of slack for the kernel's whole-chunk reads, whose scores count nowhere)."""
         if self.pos is not None:
             return
+        self.compact_stream = stream
         B, H = self.codes.shape[0], self.codes.shape[1]
         dev = self.codes.device
         pitch = self.capacity + 8192

@@ -21,7 +21,7 @@ class Recorder:
     """Native calls by name, the stream they were made on and the buffers that a chain's blocks name."""
 
     def __init__(self):
-        self.stream, self.capturing, self.fails = 0, False, None
+        self.stream, self.capturing, self.fails, self.fits = 0, False, None, 1
         self.calls, self.masks = [], {}
 
     def call(self, name, args):
@@ -29,7 +29,7 @@ class Recorder:
             raise self.fails
         if name == "sah_hash_decode_masked":
             if args.ask:
-                args.fits = 1
+                args.fits = self.fits
                 return
             hd = N.HashDecodeArgs.from_address(args.decode)
             self.calls.append((name, self.stream, {hd.rows.cols, hd.rows.cnt, args.tickets, N.HashSigArgs.from_address(hd.query_sig).codes}, hd))
@@ -110,10 +110,10 @@ class Session:
         self.kept.append(m)
         return m
 
-    def step(self, kind, stream=0, n=LK, mask=None):
-        """The launches of one step under a new mask: zero, hiding or general."""
+    def step(self, kind, stream=0, n=LK):
+        """The launches of one step under a new mask: zero, hiding, general or none."""
         before = len(self.r.launches())
-        m = self.mask(kind, n) if mask is None else mask
+        m = None if kind == "-" else self.mask(kind, n)
         self.r.stream = stream
         out = self.ra.custom_attention(None, self.q, self.k[:, :, :n], self.k[:, :, :n], m, D ** -0.5, 0.0,
                                        sparse_meta_data=self.meta, layer_idx=0)[0]
@@ -169,3 +169,45 @@ def test_an_instance_guesses_nothing_from_another_one(device):
     assert len(session.step("h")) == 1
     session.meta = None  # a chain that keeps nothing takes this, too
     assert [len(session.step(kind)) for kind in "hzh"] == [1, 1, 1]
+
+
+def compact(launches):
+    """Which of them read the compact codes."""
+    return [c[0] == "sah_hash_decode_masked" or c[3] for c in launches]
+
+
+def one_kernel(launches):
+    return any(c[0] == "sah_hash_decode_masked" for c in launches)
+
+
+def test_compact_codes_of_two_streams_are_no_masked_steps(device):
+    """One stream has written most of the compact codes, another has added to them: a masked step on either would read what the
+    other has written, and goes without them."""
+    s = Session(device, attention("hash"), "hash")
+    assert one_kernel(s.step("h", 1)) and one_kernel(s.step("h", 1))
+    assert not one_kernel(s.step("h", 2))
+    s.step("-", 2, LK + 40)
+    assert s.cache.n_compact == LK + 40
+    assert not one_kernel(s.step("h", 2, LK + 40)) and not one_kernel(s.step("h", 1, LK + 40))
+    s.cache.reserve(s.cache.capacity + 1)  # other buffers, written anew
+    assert one_kernel(s.step("h", 2, LK + 40)) and not one_kernel(s.step("h", 1, LK + 40))
+
+
+def test_compact_buffers_belong_to_the_stream_that_clears_them(device):
+    s = Session(device, attention("hash"), "hash")
+    device.fits = 0
+    assert not one_kernel(s.step("h", 1))  # makes the buffers, and then has no use for them
+    device.fits = 1
+    assert not one_kernel(s.step("h", 2)) and one_kernel(s.step("h", 1))
+
+
+@pytest.mark.parametrize("kind", ["z", "h"])
+def test_a_guess_reads_no_compact_codes_of_another_stream(device, kind):
+    s = Session(device, attention("hash"), "hash")
+    s.step("z", 1)
+    s.step("z", 1)
+    before = len(device.calls)
+    s.step(kind, 2)
+    names = [c[0] for c in device.calls[before:]]
+    assert "sah_run_chain" not in names[:names.index("sah_amask_answer")]
+    assert s.cache.n_compact == LK
