@@ -161,11 +161,11 @@ class DecodePlan:
         the attention."""
         chain, at = self.chain, self.att
         # A mask that only hides columns: one kernel. The compact form it reads is kept by steps like this one; a step that
-        # would read what another stream has written, or that is captured and would have to write it, takes the other way.
+        # would read what another stream has written takes the other way, and so does a captured one: its mask is what the
+        # buffer holds at a replay, which may be anything.
         # (a byte and two bits of LDS a key and four bytes an entry: longer rows do not get as far as buffers they cannot use)
         if (only_hides and self.dtype != torch.float16 and rows.n_keys * 5 // 4 + 4 * rows.cap <= 150 * 1024
-                and cache.compact_ordered(stream)
-                and (cache.n_compact >= hashed or not torch.cuda.is_current_stream_capturing())):
+                and cache.compact_ordered(stream) and not torch.cuda.is_current_stream_capturing()):
             hd, hm = self.hash_decode, self.hash_masked
             hd.rows, hd.sink, hd.window, hd.k, hd.stream = rows, sink, window, k_eff, stream
             hd.query_sig, hd.key_sig, hd.skip_bitmap = chain.sig_b, None, 1

@@ -1000,3 +1000,44 @@ def test_padded_and_unpadded_sessions_on_two_streams(cuda, chain):
         torch.cuda.synchronize()
         results.append(torch.stack(outs))
     assert torch.equal(results[0], results[1])
+
+
+def test_a_replay_takes_the_mask_as_it_is_then(cuda):
+    """A HashAttention step captured under a mask that only hides columns, replayed after a bias has been written into it."""
+    import sparse_attention_hub_amd.sparse_attention as sa
+    from sparse_attention_hub_amd.sparse_attention.utils.hashattention_utils import random_hat_weights
+
+    B, Hq, Hkv, Lk, D = 2, 8, 2, 900, 64
+    lowest = float(torch.finfo(torch.bfloat16).min)
+    _, k, v = make_qkv(B, Hq, Hkv, 1, Lk, D, torch.bfloat16, seed=5, device=cuda)
+    q = make_qkv(B, Hq, Hkv, 1, 1, D, torch.bfloat16, seed=1, device=cuda)[0]
+    kinds = {"h": _hide(torch.zeros((B, 1, 1, Lk)), "padded", Lk, 70, lowest)}
+    kinds["g"] = (kinds["h"] - 3.0 * (torch.arange(Lk) % 5 == 0)).clamp_(min=lowest)
+    kinds = {name: m.to(torch.bfloat16).to(cuda) for name, m in kinds.items()}
+    m = kinds["h"].clone()
+    ra = sa.ResearchAttention.create_from_config(sa.ResearchAttentionConfig(masker_configs=[
+        sa.SinkMaskerConfig(sink_size=9), sa.LocalMaskerConfig(window_size=70), sa.HashAttentionTopKMaskerConfig(
+            heavy_size=50, hat_bits=32, hat_mlp_layers=3, hat_mlp_hidden_size=128, hat_mlp_activation="silu",
+            hat_weights=random_hat_weights(1, Hq, D, 32, 3, 128, dtype=torch.bfloat16, seed=1))]))
+    ra.return_attention_weights = False
+    meta = {}
+
+    def step(mask):
+        return ra.custom_attention(None, q, k, v, mask, D ** -0.5, 0.0, sparse_meta_data=meta, layer_idx=0)[0]
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        want = {name: [step(mask.clone()) for _ in range(2)][1].double() for name, mask in kinds.items()}
+        step(m)
+        step(m)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            out = step(m)
+        for kind in "hghgg":
+            m.copy_(kinds[kind])
+            out.zero_()
+            graph.replay()
+            assert bool(((out.double() - want[kind]).abs() <= 2.0 ** -7 * want[kind].abs() + 2.0 ** -18).all()), kind
+        side.synchronize()
+    assert not bool(((want["h"] - want["g"]).abs() <= 2.0 ** -4 * want["h"].abs()).all())  # the bias does change what is chosen

@@ -110,10 +110,10 @@ class Session:
         self.kept.append(m)
         return m
 
-    def step(self, kind, stream=0, n=LK):
-        """The launches of one step under a new mask: zero, hiding, general or none."""
+    def step(self, kind, stream=0, n=LK, mask=None):
+        """The launches of one step under a new mask (or the given one): zero, hiding, general or none."""
         before = len(self.r.launches())
-        m = None if kind == "-" else self.mask(kind, n)
+        m = mask if mask is not None else None if kind == "-" else self.mask(kind, n)
         self.r.stream = stream
         out = self.ra.custom_attention(None, self.q, self.k[:, :, :n], self.k[:, :, :n], m, D ** -0.5, 0.0,
                                        sparse_meta_data=self.meta, layer_idx=0)[0]
@@ -211,3 +211,13 @@ def test_a_guess_reads_no_compact_codes_of_another_stream(device, kind):
     names = [c[0] for c in device.calls[before:]]
     assert "sah_run_chain" not in names[:names.index("sah_amask_answer")]
     assert s.cache.n_compact == LK
+
+
+def test_a_captured_step_does_not_rely_on_what_its_mask_holds(device):
+    s = Session(device, attention("hash"), "hash")
+    m = s.mask("h")
+    assert one_kernel(s.step("h", 1, mask=m)) and one_kernel(s.step("h", 1, mask=m))
+    device.capturing = True
+    assert not one_kernel(s.step("h", 1, mask=m))
+    device.capturing = False
+    assert one_kernel(s.step("h", 1, mask=m))
