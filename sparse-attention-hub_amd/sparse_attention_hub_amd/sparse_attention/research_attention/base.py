@@ -187,7 +187,8 @@ class ResearchAttention(SparseAttention):
         if flags is None:
             guess = facts.guess(am, sparse_meta_data)
             question = MaskQuestion(am)
-            if plannable and guess is not None and (guess == 0 or queries.shape[2] == 1):
+            covers = mask_covers(am, queries, keys.shape[2])  # (else it has to be zero, or is refused)
+            if plannable and covers and guess is not None and (guess == 0 or queries.shape[2] == 1):
                 hides = not guess & _native.AMASK_GENERAL and same_type
                 try:
                     out = self._plan_step(queries, keys, values, am if guess else None, scaling, sparse_meta_data, layer_idx, hides, guessed=True)
@@ -196,7 +197,7 @@ class ResearchAttention(SparseAttention):
                 flags = facts.take(question, sparse_meta_data)
                 if out is not None and (flags == guess or (guess and not (hides and flags & _native.AMASK_GENERAL))):
                     return am, hides, out, None
-            elif am.shape[2] > 1 and guess != 0 and mask_covers(am, queries, keys.shape[2]):
+            elif am.shape[2] > 1 and guess != 0 and covers:
                 return am, False, None, question
             else:
                 flags = facts.take(question, sparse_meta_data)

@@ -25,8 +25,8 @@ class Recorder:
         self.calls, self.masks = [], {}
 
     def call(self, name, args):
-        if self.fails is not None and name in ("sah_run_chain", "sah_hash_decode_masked"):
-            raise self.fails
+        if self.fails is not None and name == "sah_run_chain":
+            self.fails(N.AttentionArgs.from_address(args.attention).amask)
         if name == "sah_hash_decode_masked":
             if args.ask:
                 args.fits = self.fits
@@ -221,3 +221,20 @@ def test_a_captured_step_does_not_rely_on_what_its_mask_holds(device):
     assert not one_kernel(s.step("h", 1, mask=m))
     device.capturing = False
     assert one_kernel(s.step("h", 1, mask=m))
+
+
+def test_a_mask_that_covers_nothing_of_the_call_is_launched_on_no_guess(device):
+    s = Session(device, attention("oracle"), "oracle")
+    s.step("z")
+    s.step("z")
+    before = len(device.launches())
+    wide = torch.zeros(B + 1, 1, 1, LK, dtype=torch.bfloat16)
+    device.masks[wide.data_ptr()] = wide
+    names = len(device.calls)
+    assert len(s.step("z", mask=wide)) == 1  # adds nothing anywhere
+    assert [c[0] for c in device.calls[names:]][:2] == ["sah_amask_ask", "sah_amask_answer"]
+    other = wide.clone().fill_(LOWEST)
+    device.masks[other.data_ptr()] = other
+    with pytest.raises(ValueError, match="does not cover"):
+        s.step("h", mask=other)
+    assert len(device.launches()) == before + 1
