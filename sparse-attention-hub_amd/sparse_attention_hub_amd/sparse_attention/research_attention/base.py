@@ -190,11 +190,16 @@ class ResearchAttention(SparseAttention):
             covers = mask_covers(am, queries, keys.shape[2])  # (else it has to be zero, or is refused)
             if plannable and covers and guess is not None and (guess == 0 or queries.shape[2] == 1):
                 hides = not guess & _native.AMASK_GENERAL and same_type
+                out, error = None, None
                 try:
                     out = self._plan_step(queries, keys, values, am if guess else None, scaling, sparse_meta_data, layer_idx, hides, guessed=True)
-                except Exception:
-                    out = None  # (what is wrong with the call under its own mask, if anything, is said then)
+                except Exception as e:
+                    error = e
                 flags = facts.take(question, sparse_meta_data)
+                # the error of a right guess is the call's own (memory may have been short for buffers that only a guess needs)
+                if error is not None and flags == guess and not isinstance(error, torch.OutOfMemoryError):
+                    raise error
+                error = None
                 if out is not None and (flags == guess or (guess and not (hides and flags & _native.AMASK_GENERAL))):
                     return am, hides, out, None
             elif am.shape[2] > 1 and guess != 0 and covers:

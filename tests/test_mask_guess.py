@@ -223,6 +223,34 @@ def test_a_captured_step_does_not_rely_on_what_its_mask_holds(device):
     assert one_kernel(s.step("h", 1, mask=m))
 
 
+def test_what_a_launch_on_a_guess_raises(device):
+    """The step's own error if the guess was right, nothing if it was wrong; memory for buffers of the guess's own is no one's."""
+    tries = []
+
+    def fail(amask):
+        tries.append(amask)
+        raise N.NativeLibraryError("device")
+
+    s = Session(device, attention("oracle"), "oracle")
+    s.step("z")
+    device.fails = fail
+    with pytest.raises(N.NativeLibraryError, match="device"):
+        s.step("z")
+    assert tries == [None] and not U._ANSWERS.open
+    device.fails = lambda amask: fail(amask) if amask is None else None
+    assert len(s.step("h")) == 1 and len(tries) == 2
+    device.fails = None
+    s.step("z")
+    s.step("z")
+
+    def out_of_memory(amask):
+        device.fails = None
+        raise torch.OutOfMemoryError("buffers")
+
+    device.fails = out_of_memory
+    assert len(s.step("z")) == 1
+
+
 def test_a_mask_that_covers_nothing_of_the_call_is_launched_on_no_guess(device):
     s = Session(device, attention("oracle"), "oracle")
     s.step("z")
