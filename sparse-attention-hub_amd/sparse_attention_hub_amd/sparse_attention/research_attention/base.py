@@ -102,7 +102,18 @@ class ResearchAttention(SparseAttention):
             out = self._plan_step(queries, keys, values, attention_mask, scaling, sparse_meta_data, kwargs.get("layer_idx"), only_hides)
         if out is not None:
             return out, None
+        try:
+            return self._by_maskers(module, queries, keys, values, attention_mask, scaling, dropout, sparse_meta_data,
+                                    want_density, want_error, kwargs)
+        finally:
+            if question is not None:
+                self._mask_facts.take(question, sparse_meta_data)
 
+    def _by_maskers(self, module: nn.Module, queries: torch.Tensor, keys: torch.Tensor, values: torch.Tensor,
+                    attention_mask: Optional[torch.Tensor], scaling: float, dropout: float, sparse_meta_data: Dict[Any, Any],
+                    want_density: bool, want_error: bool, kwargs: Dict[str, Any]) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
+        """Every masker's `add_mask` in order, then the attention over the finished mask."""
+        metrics = MicroMetricLogger()
         mask_shape = (queries.shape[0], queries.shape[1], queries.shape[2], keys.shape[2])
         mask = Mask.create_empty_mask(mask_shape, dtype=queries.dtype, device=queries.device)
         if self.maskers:
@@ -158,8 +169,6 @@ class ResearchAttention(SparseAttention):
                 sinks=s_aux, scaling=scaling, dropout=dropout, sparse_attention_mask=mask,
                 return_attention_weights=False, **kwargs,
             )
-        if question is not None:
-            self._mask_facts.take(question, sparse_meta_data)
         if want_error:
             # relative distance to dense attention over all keys, by the same kernel in dense mode (reference :150-168)
             true_out, _ = get_true_attention_output(module, queries, keys, values, attention_mask, scaling, dropout, **kwargs)

@@ -98,7 +98,8 @@ def additive_mask_args(attention_mask: Optional[torch.Tensor], queries: torch.Te
 
 class _AnswerWords(threading.local):
     """Per thread and device: two words of device memory and one of pinned host memory, through which a mask's question is
-    answered, and the thread's question that waits for its answer (one at a time; nobody returns to a caller in between)."""
+    answered, and the thread's question that waits for its answer (one at a time; a call that asks takes the answer before it
+    returns or raises)."""
 
     def __init__(self) -> None:
         self.words = {}

@@ -266,3 +266,16 @@ def test_a_mask_that_covers_nothing_of_the_call_is_launched_on_no_guess(device):
     with pytest.raises(ValueError, match="does not cover"):
         s.step("h", mask=other)
     assert len(device.launches()) == before + 1
+
+
+def test_a_call_that_fails_leaves_no_question_open(device, monkeypatch):
+    """A mask of several queries is asked about while the maskers run: the answer is taken whatever becomes of them."""
+    from sparse_attention_hub_amd.sparse_attention.research_attention import base
+
+    s = Session(device, attention("fixed"), "fixed")
+    m = s.mask("h", n_q=3)
+    monkeypatch.setattr(base.Mask, "create_empty_mask", lambda *a, **k: (_ for _ in ()).throw(ValueError("masker")))
+    with pytest.raises(ValueError, match="masker"):
+        s.ra.custom_attention(None, torch.zeros(B, HQ, 3, D, dtype=torch.bfloat16), s.k[:, :, :LK], s.k[:, :, :LK], m, D ** -0.5, 0.0,
+                              sparse_meta_data=s.meta, layer_idx=0)
+    assert not U._ANSWERS.open and s.ra._mask_facts.known(m) == N.AMASK_NONZERO
