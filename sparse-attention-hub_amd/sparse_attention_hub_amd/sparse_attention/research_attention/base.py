@@ -103,78 +103,70 @@ class ResearchAttention(SparseAttention):
         if out is not None:
             return out, None
         try:
-            return self._by_maskers(module, queries, keys, values, attention_mask, scaling, dropout, sparse_meta_data,
-                                    want_density, want_error, kwargs)
+            mask_shape = (queries.shape[0], queries.shape[1], queries.shape[2], keys.shape[2])
+            mask = Mask.create_empty_mask(mask_shape, dtype=queries.dtype, device=queries.device)
+            if self.maskers:
+                # size the row buffers once for the whole chain so no masker has to grow them
+                dims = self.maskers[0]._extract_tensor_dimensions(keys, queries)
+                planned = self._planned_capacity(dims)
+                if planned is not None and planned > 0:
+                    rows = NativeRows(mask_shape[0] * mask_shape[1] * mask_shape[2], mask_shape[3], planned, queries.device)
+                    mask = _EmptyRowsMask(mask_shape, rows, queries.dtype)
+
+            maskers = self.maskers
+            if (len(maskers) >= 2 and type(maskers[0]) is SinkMasker and type(maskers[1]) is LocalMasker
+                    and not mask.is_full_mask()):
+                # Sink directly followed by Local on a still-empty mask: one fused launch writes both ranges
+                mask = fused_sink_local(maskers[0], maskers[1], keys, queries, mask)
+                maskers = maskers[2:]
+
+            # per-call scratch the maskers may share (e.g. the QK score keys of one scoring pass)
+            call_scratch: Dict[str, Any] = {}
+            for masker in maskers:
+                mask = masker.add_mask(
+                    keys=keys,
+                    queries=queries,
+                    values=values,
+                    attention_mask=attention_mask,
+                    scaling=scaling,
+                    dropout=dropout,
+                    sparse_meta_data=sparse_meta_data,
+                    previous_mask=mask,
+                    _call_scratch=call_scratch,
+                    **kwargs,
+                )
+
+            if want_density:
+                # active fraction of the (B, Hq, Lq, Lk) mask, from the per-row counts (reference :121-126)
+                metrics.log("research_attention_density", mask.get_density(), metadata={"layer_idx": kwargs["layer_idx"]})
+
+            s_aux_raw: Any = kwargs.pop("s_aux", None)
+            s_aux: Optional[torch.Tensor] = s_aux_raw if isinstance(s_aux_raw, torch.Tensor) else None
+            weights: Optional[torch.Tensor] = None
+            # a masker of this call scored every key exactly (OracleTopK, AdaptiveSampling): the attention takes its
+            # logits from those scores instead of reading K again
+            kwargs["_score_keys"] = (call_scratch.get("qk_score_keys"), call_scratch.get("qk_score_resid"))
+            if self.return_attention_weights:
+                out, weights = get_masked_attention_output(
+                    module=module, queries=queries, keys=keys, values=values, attention_mask=attention_mask,
+                    sinks=s_aux, scaling=scaling, dropout=dropout, sparse_attention_mask=mask,
+                    return_attention_weights=True, **kwargs,
+                )
+            else:
+                out = get_masked_attention_output(
+                    module=module, queries=queries, keys=keys, values=values, attention_mask=attention_mask,
+                    sinks=s_aux, scaling=scaling, dropout=dropout, sparse_attention_mask=mask,
+                    return_attention_weights=False, **kwargs,
+                )
+            if want_error:
+                # relative distance to dense attention over all keys, by the same kernel in dense mode (reference :150-168)
+                true_out, _ = get_true_attention_output(module, queries, keys, values, attention_mask, scaling, dropout, **kwargs)
+                error = torch.norm(true_out.float() - out.float()) / torch.norm(true_out.float())
+                metrics.log("research_attention_output_error", float(error.item()), metadata={"layer_idx": kwargs["layer_idx"]})
+            return out, weights
         finally:
             if question is not None:
                 self._mask_facts.take(question, sparse_meta_data)
-
-    def _by_maskers(self, module: nn.Module, queries: torch.Tensor, keys: torch.Tensor, values: torch.Tensor,
-                    attention_mask: Optional[torch.Tensor], scaling: float, dropout: float, sparse_meta_data: Dict[Any, Any],
-                    want_density: bool, want_error: bool, kwargs: Dict[str, Any]) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
-        """Every masker's `add_mask` in order, then the attention over the finished mask."""
-        metrics = MicroMetricLogger()
-        mask_shape = (queries.shape[0], queries.shape[1], queries.shape[2], keys.shape[2])
-        mask = Mask.create_empty_mask(mask_shape, dtype=queries.dtype, device=queries.device)
-        if self.maskers:
-            # size the row buffers once for the whole chain so no masker has to grow them
-            dims = self.maskers[0]._extract_tensor_dimensions(keys, queries)
-            planned = self._planned_capacity(dims)
-            if planned is not None and planned > 0:
-                rows = NativeRows(mask_shape[0] * mask_shape[1] * mask_shape[2], mask_shape[3], planned, queries.device)
-                mask = _EmptyRowsMask(mask_shape, rows, queries.dtype)
-
-        maskers = self.maskers
-        if (len(maskers) >= 2 and type(maskers[0]) is SinkMasker and type(maskers[1]) is LocalMasker
-                and not mask.is_full_mask()):
-            # Sink directly followed by Local on a still-empty mask: one fused launch writes both ranges
-            mask = fused_sink_local(maskers[0], maskers[1], keys, queries, mask)
-            maskers = maskers[2:]
-
-        # per-call scratch the maskers may share (e.g. the QK score keys of one scoring pass)
-        call_scratch: Dict[str, Any] = {}
-        for masker in maskers:
-            mask = masker.add_mask(
-                keys=keys,
-                queries=queries,
-                values=values,
-                attention_mask=attention_mask,
-                scaling=scaling,
-                dropout=dropout,
-                sparse_meta_data=sparse_meta_data,
-                previous_mask=mask,
-                _call_scratch=call_scratch,
-                **kwargs,
-            )
-
-        if want_density:
-            # active fraction of the (B, Hq, Lq, Lk) mask, from the per-row counts (reference :121-126)
-            metrics.log("research_attention_density", mask.get_density(), metadata={"layer_idx": kwargs["layer_idx"]})
-
-        s_aux_raw: Any = kwargs.pop("s_aux", None)
-        s_aux: Optional[torch.Tensor] = s_aux_raw if isinstance(s_aux_raw, torch.Tensor) else None
-        weights: Optional[torch.Tensor] = None
-        # a masker of this call scored every key exactly (OracleTopK, AdaptiveSampling): the attention takes its
-        # logits from those scores instead of reading K again
-        kwargs["_score_keys"] = (call_scratch.get("qk_score_keys"), call_scratch.get("qk_score_resid"))
-        if self.return_attention_weights:
-            out, weights = get_masked_attention_output(
-                module=module, queries=queries, keys=keys, values=values, attention_mask=attention_mask,
-                sinks=s_aux, scaling=scaling, dropout=dropout, sparse_attention_mask=mask,
-                return_attention_weights=True, **kwargs,
-            )
-        else:
-            out = get_masked_attention_output(
-                module=module, queries=queries, keys=keys, values=values, attention_mask=attention_mask,
-                sinks=s_aux, scaling=scaling, dropout=dropout, sparse_attention_mask=mask,
-                return_attention_weights=False, **kwargs,
-            )
-        if want_error:
-            # relative distance to dense attention over all keys, by the same kernel in dense mode (reference :150-168)
-            true_out, _ = get_true_attention_output(module, queries, keys, values, attention_mask, scaling, dropout, **kwargs)
-            error = torch.norm(true_out.float() - out.float()) / torch.norm(true_out.float())
-            metrics.log("research_attention_output_error", float(error.item()), metadata={"layer_idx": kwargs["layer_idx"]})
-        return out, weights
 
     def _under_mask(self, queries: torch.Tensor, keys: torch.Tensor, values: torch.Tensor, attention_mask: torch.Tensor,
                     scaling: float, sparse_meta_data: Dict[Any, Any], layer_idx: Optional[int], plannable: bool):
