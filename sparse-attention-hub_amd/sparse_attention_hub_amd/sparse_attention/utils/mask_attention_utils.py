@@ -201,9 +201,6 @@ class AdditiveMaskFacts:
         known = self.known(attention_mask)
         return self.take(MaskQuestion(attention_mask)) if known is None else known
 
-    def all_zero(self, attention_mask: torch.Tensor) -> bool:
-        return self.flags(attention_mask) == 0
-
 
 def _run_attention(
     queries: torch.Tensor,
