@@ -431,12 +431,14 @@ static bool sig_mfma_ok(const sah_hash_sig_args* a) {
   return sgm_lds_bytes(a) <= 150 * 1024;
 }
 
-// Workgroups per head: of all counts the one that should take least time. Two workgroups fit a CU; a round takes a workgroup's
-// tiles, half of that from the waves that have one more than the others, and staging the weights as long as eight tiles.
-// 32 heads (in us, before: 256-vector tiles, eight to a workgroup; now): 1024 keys 47 -> 13, 8112 keys 92 -> 41, 16405 keys
-// 145 -> 86, 32801 keys (17 workgroups a head, 544 on 512 places) 165 -> 137.
-static int sgm_chunks(int64_t heads, int n_tiles) {
-  const int slots = 512, most = (n_tiles + SGM_NW - 1) / SGM_NW;  // a tile a wave
+// Workgroups per head: of all counts the one that should take least time. A CU holds as many workgroups as its 160 KB of LDS
+// do, at most two (registers); a round takes a workgroup's tiles, half of that from the waves that have one more than the
+// others, and staging the weights as long as eight tiles. 32 heads of the usual MLP (us, four launches one after the other, all on
+// one GPU; before: 256-vector tiles, eight to a workgroup; now): 1024 keys 49 -> 15, 8112 keys 96 -> 43, 16405 keys 154 -> 74,
+// 32801 keys (17 workgroups a head, 544 on 512 places) 196 -> 154. Four layers of 128, one workgroup a CU: 3000 keys 129 -> 43 (60
+// with places for two), 16405 keys 170 -> 148 (161).
+static int sgm_chunks(int64_t heads, int n_tiles, size_t lds) {
+  const int slots = lds <= 80 * 1024 ? 512 : 256, most = (n_tiles + SGM_NW - 1) / SGM_NW;  // a tile a wave
   int best = 1;
   int64_t best_cost = INT64_MAX;
   for (int c = 1; c <= most && c <= 4 * slots; ++c) {
@@ -452,22 +454,24 @@ static int sgm_chunks(int64_t heads, int n_tiles) {
 
 template <int DT, int ACT>
 static int sig_launch_mfma_a(const sah_hash_sig_args* a, const sig_params& P) {
+  // (GELU's error function does not fit the registers beside two tiles)
+  constexpr int UACT = ACT == SAH_ACT_GELU ? SAH_ACT_RELU : ACT;
+  const bool usual = ACT == UACT && a->D == 128 && a->n_layers == 3 && a->d_out[0] == 128 && a->d_out[1] == 128 && a->d_out[2] == 32;
+  const size_t lds = sgm_lds_bytes(a);
   const int64_t heads = (int64_t)a->B * a->Hq;
   const int n_tiles = (a->L + 31) / 32;
-  int n_chunks = sgm_chunks(heads, n_tiles);
+  int n_chunks = sgm_chunks(heads, n_tiles, lds);  // (the usual MLP's static LDS is as large)
   const int wg_tiles = (n_tiles + n_chunks - 1) / n_chunks;
   n_chunks = (n_tiles + wg_tiles - 1) / wg_tiles;
   const int64_t n_wg = heads * n_chunks;
   if (n_wg > 0x7fffffff) return sah_fail(SAH_ESHAPE, "sah_hash_signatures: too many workgroups");
   sah_timed timed("k_hash_sig_mfma", a->stream);
   const dim3 grid((unsigned)n_wg), block(SGM_NT);
-  // (GELU's error function does not fit the registers beside two tiles)
-  constexpr int UACT = ACT == SAH_ACT_GELU ? SAH_ACT_RELU : ACT;
-  if (ACT == UACT && a->D == 128 && a->n_layers == 3 && a->d_out[0] == 128 && a->d_out[1] == 128 && a->d_out[2] == 32) {
+  if (usual) {
     hipLaunchKernelGGL((k_hash_sig_usual<DT, UACT>), grid, block, 0, (hipStream_t)a->stream, P, n_chunks, wg_tiles);
   } else {
     if (int rc = sah_allow_lds((const void*)k_hash_sig_mfma<DT, ACT>, 150 * 1024, "sah_hash_signatures")) return rc;
-    hipLaunchKernelGGL((k_hash_sig_mfma<DT, ACT>), grid, block, sgm_lds_bytes(a), (hipStream_t)a->stream, P, n_chunks, wg_tiles);
+    hipLaunchKernelGGL((k_hash_sig_mfma<DT, ACT>), grid, block, lds, (hipStream_t)a->stream, P, n_chunks, wg_tiles);
   }
   return sah_launch_status("sah_hash_signatures");
 }

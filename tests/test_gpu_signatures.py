@@ -8,14 +8,14 @@ from oracle import reference_path as O
 pytestmark = pytest.mark.gpu
 
 
-def _masker(wts, bits, hidden, act):
+def _masker(wts, bits, hidden, act, layers=3):
     from sparse_attention_hub_amd.sparse_attention import HashAttentionTopKMaskerConfig
     from sparse_attention_hub_amd.sparse_attention.research_attention.maskers.fixed.implementations.hashattention_top_k import (
         HashAttentionTopKMasker,
     )
 
     return HashAttentionTopKMasker(HashAttentionTopKMaskerConfig(
-        heavy_size=8, hat_bits=bits, hat_mlp_layers=3, hat_mlp_hidden_size=hidden, hat_mlp_activation=act, hat_weights=wts))
+        heavy_size=8, hat_bits=bits, hat_mlp_layers=layers, hat_mlp_hidden_size=hidden, hat_mlp_activation=act, hat_weights=wts))
 
 
 def _codes(masker, x, heads, pitch, offset):
@@ -67,3 +67,15 @@ def test_a_key_that_is_not_finite_reaches_no_other_key(cuda):
     assert torch.equal(a[:, :, keep], b[:, :, keep])
     # not a number is neither positive nor zero
     assert (b[:, :, bad[1::2].cpu(), 0] == 0).all() and (b[:, :, bad[1::2].cpu(), 1] == -1).all()
+
+
+@pytest.mark.parametrize("L", [129, 3001, 9000])  # weights that leave room for one workgroup a CU
+def test_bulk_signatures_of_four_layers(cuda, L):
+    from sparse_attention_hub_amd.sparse_attention.utils.hashattention_utils import random_hat_weights
+
+    wts = random_hat_weights(1, 4, 128, 32, 4, 128, dtype=torch.bfloat16, seed=1)
+    x = torch.randn(1, 2, L, 128, generator=torch.Generator().manual_seed(L)).to(torch.bfloat16)
+    codes = _codes(_masker(wts, 32, 128, "silu", layers=4), x.to(cuda), 4, L, 0)
+    sig = O.hash_signatures(O.repeat_kv(x, 2), wts[0]["key_matrix"], wts[0]["key_bias"], "silu")
+    agree = (_signs(codes, 32) == sig.float()).float().mean(dim=(0, 1, 3))  # (as above)
+    assert agree.mean().item() >= 0.9995 and agree.min().item() >= 0.9
