@@ -433,17 +433,21 @@ static bool sig_mfma_ok(const sah_hash_sig_args* a) {
 
 // Workgroups per head: of all counts the one that should take least time. A CU holds as many workgroups as its 160 KB of LDS
 // do, at most two (registers); a round takes a workgroup's tiles, half of that from the waves that have one more than the
-// others, and staging the weights as long as eight tiles. 32 heads of the usual MLP (us, four launches one after the other, all on
+// others, and staging the weights as long as eight tiles. SiLU with two workgroups a CU: a quarter of a share is added for the end,
+// where one of the two is done. Long shares in one round lose there to half as long ones in two (256 heads x 8192 keys of bf16 252 ->
+// 241 us, of fp16 with 64 dimensions 284 -> 271; 256 x 32768 keys 916 -> 858); GELU is 1 to 4 % faster with the long ones, ReLU
+// either way. 32 heads of the usual MLP (us, four launches one after the other, all on
 // one GPU; before: 256-vector tiles, eight to a workgroup; now): 1024 keys 49 -> 15, 8112 keys 96 -> 43, 16405 keys 154 -> 74,
 // 32801 keys (17 workgroups a head, 544 on 512 places) 196 -> 154. Four layers of 128, one workgroup a CU: 3000 keys 129 -> 43 (60
 // with places for two), 16405 keys 170 -> 148 (161).
-static int sgm_chunks(int64_t heads, int n_tiles, size_t lds) {
+static int sgm_chunks(int64_t heads, int n_tiles, size_t lds, int act) {
   const int slots = lds <= 80 * 1024 ? 512 : 256, most = (n_tiles + SGM_NW - 1) / SGM_NW;  // a tile a wave
   int best = 1;
   int64_t best_cost = INT64_MAX;
   for (int c = 1; c <= most && c <= 4 * slots; ++c) {
     const int tiles = (n_tiles + c - 1) / c, per_wave = (tiles + SGM_NW - 1) / SGM_NW;
-    const int64_t cost = ((heads * c + slots - 1) / slots) * (tiles + SGM_NW * per_wave + 2 * SGM_NW);
+    const int64_t share = tiles + SGM_NW * per_wave, rounds = (heads * c + slots - 1) / slots;
+    const int64_t cost = 4 * rounds * (share + 2 * SGM_NW) + (slots == 512 && act == SAH_ACT_SILU ? share : 0);
     if (cost < best_cost) {
       best = c;
       best_cost = cost;
@@ -460,7 +464,7 @@ static int sig_launch_mfma_a(const sah_hash_sig_args* a, const sig_params& P) {
   const size_t lds = sgm_lds_bytes(a);
   const int64_t heads = (int64_t)a->B * a->Hq;
   const int n_tiles = (a->L + 31) / 32;
-  int n_chunks = sgm_chunks(heads, n_tiles, lds);  // (the usual MLP's static LDS is as large)
+  int n_chunks = sgm_chunks(heads, n_tiles, lds, ACT);  // (the usual MLP's static LDS is as large)
   const int wg_tiles = (n_tiles + n_chunks - 1) / n_chunks;
   n_chunks = (n_tiles + wg_tiles - 1) / wg_tiles;
   const int64_t n_wg = heads * n_chunks;
