@@ -129,7 +129,8 @@ __global__ __launch_bounds__(GEMV_NT) void k_hash_sig_gemv(sig_pair PP) {
 
 // ACT: the activation, fixed at compile time (one kernel each: with the choice left to run time the four epilogues,
 // GELU's error function included, end up inside the hot loop and the code outgrows the instruction cache)
-// A workgroup takes tiles [wg * wg_tiles, (wg + 1) * wg_tiles) of 32 vectors of its head, its waves every eighth of them.
+// A workgroup takes tiles [wg * wg_tiles, (wg + 1) * wg_tiles) of 32 vectors of its head, its waves every eighth of them. (A tile's
+// vectors are requested at its start: requested during the epilogue of the tile before they cost 1 to 5 %, the registers being full.)
 template <int DT, int ACT>
 __global__ __launch_bounds__(SGM_NT, 4) void k_hash_sig_mfma(sig_params P, int n_chunks, int wg_tiles) {
   SAH_DYNAMIC_LDS(sgm_dyn)
@@ -208,8 +209,8 @@ __global__ __launch_bounds__(SGM_NT, 4) void k_hash_sig_mfma(sig_params P, int n
   if (t_end > (chunk + 1) * wg_tiles) t_end = (chunk + 1) * wg_tiles;
   int t = chunk * wg_tiles + wave;
   if (t >= t_end) return;
-  request(t);
   for (; t < t_end; t += SGM_NW) {  // uniform across the wave
+    request(t);
     int ksteps = k0;
 #pragma unroll
     for (int l = 0; l < SAH_MAX_MLP_LAYERS; ++l) {
@@ -267,7 +268,6 @@ __global__ __launch_bounds__(SGM_NT, 4) void k_hash_sig_mfma(sig_params P, int n
       } else {
         // sign planes: this lane holds 16 of the vector's bits, lane ^ 32 the other 16
         sah_f32x16 acc0 = tile(0);
-        request(t + SGM_NW);  // (the operand registers are free: the next vectors arrive during the epilogue)
         uint32_t pos = 0u, nz = 0u;
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
