@@ -74,8 +74,8 @@ int sah_amask_answer(sah_amask_question* q);
 /* sah_hash_decode_attention under an additive mask (attention.amask, of the queries' type) that holds nothing but 0, the
  * type's lowest value and -inf, in one kernel: the selection ranks a column at the lowest value below every other one (as the
  * sum of score and mask does) and leaves out one at -inf, whose weight is 0. fits says whether one kernel runs the step: fp32
- * or bf16, skip_bitmap set, no key_sig, the compact form given, and what else sah_hash_decode_attention needs for it; with ask != 0
- * the call only says so, otherwise a step that does not fit is refused. */
+ * or bf16, skip_bitmap set, no key_sig (the compact form may be given or not), and what else sah_hash_decode_attention needs for it;
+ * with ask != 0 the call only says so, otherwise a step that does not fit is refused. */
 typedef struct sah_hash_decode_masked_args {
   const sah_hash_decode_args* decode;
   const sah_attention_args* attention;

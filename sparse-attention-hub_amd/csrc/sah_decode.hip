@@ -421,7 +421,7 @@ static int hdec_attn_launch_s(const sah_hash_decode_args* a, const hdec_params& 
 template <int DT, bool MF, bool CP, int D>
 static int hdec_attn_launch_t(const sah_hash_decode_args* a, const hdec_params& P, const att_params& A, size_t lds, int cols_offset,
                               int parts, float* work, uint32_t* tickets) {
-  if constexpr (CP && DT != SAH_F16) {
+  if constexpr (DT != SAH_F16) {
     if (A.amask) {
       if constexpr (MF) {
         if (hdec_silu(P)) return hdec_attn_launch_s<DT, MF, CP, D, true, true>(a, P, A, lds, cols_offset, parts, work, tickets);
@@ -511,7 +511,7 @@ extern "C" int sah_hash_decode_masked(sah_hash_decode_masked_args* m) {
   if (rc) return rc;
   const hdec_attn_plan p = hdec_attn_shape(a, t, A, m->tickets, true);
   // (fp16: a score added to the lowest value is not that value again)
-  m->fits = p.one_kernel && t->dtype != SAH_F16 && a->skip_bitmap && !(a->key_sig && a->key_sig->L > 0) && hdec_compact_ok(a) ? 1 : 0;
+  m->fits = p.one_kernel && t->dtype != SAH_F16 && a->skip_bitmap && !(a->key_sig && a->key_sig->L > 0) ? 1 : 0;
   if (m->ask) return SAH_OK;
   if (!m->fits) return sah_fail(SAH_ESHAPE, "sah_hash_decode_masked: not a step that one kernel runs");
   return hdec_attn_run(a, t, A, p, m->tickets);

@@ -11,7 +11,7 @@ __device__ __forceinline__ int sig_score(uint2 q, uint2 k) {
 }
 
 // ---------------------------------------------------------------------------
-// Signature top-k, SWAR form. Scores fit a byte (score + 33 in [1, 65], 0 = column already
+// Signature top-k, SWAR form. Scores fit a byte (score + 33 in [1, 65], with hidden columns score + 34; 0 = column already
 // active or out of range), so a lane handles 4 consecutive columns as one 32-bit word:
 //   P0  each lane loads its 4 codes (32 B, whole wave: 2 KB contiguous; in the compact form of the stream 16 B of
 //       sign planes, with the few columns that have a zero component corrected afterwards), scores them, zeroes
@@ -37,8 +37,8 @@ __device__ __forceinline__ uint32_t swar_ge(uint32_t w, uint32_t t) {
 
 #define HSW_GC 8      // chunks per mask group of P2 / P3: 8 x 4 columns of a lane = one 32-bit mask
 #define HSW_PROBES 8  // thresholds counted while the scores are staged
-// Probe i: 32, 36, ... 60. Scores + 33 lie in [1, 65] around 33, and a top-k of less than half the row has its
-// threshold above that, so these eight bracket it to 4 values in the usual case; below 32 a second set
+// Probe i: 32, 36, ... 60. The bytes of the scores lie in [1, 66] around 33 (34 with hidden columns), and a top-k of less than
+// half the row has its threshold above that, so these eight bracket it to 4 values in the usual case; below 32 a second set
 // (4, 8, ... 28) is counted from the staged bytes, from 60 up the last bracket is resolved in one 7-way pass.
 __host__ __device__ constexpr uint32_t hsw_probe_at(int i) { return 32u + 4u * (uint32_t)i; }
 
@@ -160,14 +160,13 @@ __device__ __forceinline__ void hsw_prefetch(const hsw_compact& cs, int n, hsw_b
 // [0, active_below) and [active_from, n) (the sink and local columns of a fresh decode row); chunks that lie between
 // the two ranges then skip the bitmap test of every word.
 // HID: an additive mask hides the columns of the bitmap s_hid (as s_bm, complete at the same barrier): they rank below every
-// other column, as equals; their byte is 1 and a score's is score + 34.
+// other column, as equals; their byte is 1 and a score's is score + 34, in [2, 66].
 template <bool CP = false, bool HID = false>
 __device__ __forceinline__ int hsw_select_row(const sah_rows& R, int r, const uint2* kc, const uint2 q, int k, int cnt0,
                                               uint32_t* s_bm, uint32_t* s_key, hsw_lds& S, hsw_bufs_t<CP>& buf,
                                               bool prefetched = false, bool update_bitmap = true, int* s_cols = nullptr,
                                               const hsw_compact* cs = nullptr, int active_below = -1, int active_from = -1,
                                               const uint32_t* s_hid = nullptr) {
-  static_assert(CP || !HID, "hidden columns: compact stream only");
   constexpr uint32_t ZERO = HID ? 34u : 33u;  // byte of score 0
   int* s_gt = S.gt;
   int* s_eq = S.eq;
@@ -300,15 +299,15 @@ __device__ __forceinline__ int hsw_select_row(const sah_rows& R, int r, const ui
         const int j0 = wi * 4;
         uint32_t word;
         if (j0 + 4 <= n) {
-          const uint32_t s0 = (uint32_t)(sig_score(q, make_uint2(ra[u].x, ra[u].y)) + 33);
-          const uint32_t s1 = (uint32_t)(sig_score(q, make_uint2(ra[u].z, ra[u].w)) + 33);
-          const uint32_t s2 = (uint32_t)(sig_score(q, make_uint2(rb[u].x, rb[u].y)) + 33);
-          const uint32_t s3 = (uint32_t)(sig_score(q, make_uint2(rb[u].z, rb[u].w)) + 33);
+          const uint32_t s0 = (uint32_t)(sig_score(q, make_uint2(ra[u].x, ra[u].y)) + (int)ZERO);
+          const uint32_t s1 = (uint32_t)(sig_score(q, make_uint2(ra[u].z, ra[u].w)) + (int)ZERO);
+          const uint32_t s2 = (uint32_t)(sig_score(q, make_uint2(rb[u].x, rb[u].y)) + (int)ZERO);
+          const uint32_t s3 = (uint32_t)(sig_score(q, make_uint2(rb[u].z, rb[u].w)) + (int)ZERO);
           word = s0 | (s1 << 8) | (s2 << 16) | (s3 << 24);
         } else {
           word = 0;  // ragged tail: the few columns of the last, partial group
           for (int t = 0; t < 4; ++t)
-            if (j0 + t < n) word |= (uint32_t)(sig_score(q, kc[j0 + t]) + 33) << (8 * t);
+            if (j0 + t < n) word |= (uint32_t)(sig_score(q, kc[j0 + t]) + (int)ZERO) << (8 * t);
         }
         stage(word, wi, chunk_may_be_active(c0 + u));
       }
@@ -349,7 +348,7 @@ __device__ __forceinline__ int hsw_select_row(const sah_rows& R, int r, const ui
     n_f = 3;
     next_probe = __shfl(tot, n_pass);
   } else if (n_pass == HSW_PROBES) {
-    base = hsw_probe_at(HSW_PROBES - 1);  // 60: scores end at 65, so count(key >= 68) = 0
+    base = hsw_probe_at(HSW_PROBES - 1);  // 60: scores end at 65 or 66, so count(key >= 68) = 0
     n_f = 7;
     next_probe = 0;
   } else {

@@ -220,13 +220,13 @@ class ResearchAttention(SparseAttention):
         masked = attention_mask is not None
         # A masked step's buffers belong to the stream and thread of their plan, as those of the masker-by-masker path
         # belong to the call: a step on another stream is not ordered with the ones that use them. So do those of a step whose
-        # mask is guessed to be zero: it may turn out to be a masked one. A captured step's
-        # belong to its graph alone: what its plan clears is clear when the graph runs, not now.
+        # mask is guessed to be zero: it may turn out to be a masked one. A captured step's belong to its graph alone: what its
+        # plan clears is clear when the graph runs, not now; and its mask is what the buffer holds then, which may be anything.
         owned = masked or guessed
         key = (queries.device, queries.dtype, tuple(queries.shape), keys.shape[1], masked, owned)
         owner = (_native.stream_ptr(queries.device), threading.get_ident()) if owned else None
         if masked and torch.cuda.is_current_stream_capturing():
-            plan = DecodePlan(self.maskers, self._plan_kind, queries, keys, True)
+            plan, only_hides = DecodePlan(self.maskers, self._plan_kind, queries, keys, True), False
         else:
             plan = self._plans.get(key)
             if plan is None or plan.owner != owner:

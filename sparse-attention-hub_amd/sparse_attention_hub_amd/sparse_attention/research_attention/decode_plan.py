@@ -33,6 +33,13 @@ from .maskers.fixed.implementations.pq_top_k import PQCache, PQCodebook, adc_lut
 
 _MAX_NEW_KEYS = 64  # more than this many unseen keys => not a decode step, take the general path
 _COMPACT_CODES = True  # HashAttention decode: the kernel scans 4-byte sign planes + an exception list instead of 8-byte codes
+# HashAttention decode under a mask that hides columns: rows of up to this many keys are scanned in the two-plane form, longer ones
+# in the compact form once a session has made so many such steps. Two planes / compact, us a layer: 256 rows of 2000 keys 25.1 / 25.5,
+# 8192 keys 37.3 / 37.1, 12011 keys 41.6 / 39.9, 32768 keys 55.0 / 49.6; 32 rows 20.4 / 21.5, 24.0 / 23.3, 24.3 / 23.3, 29.5 / 28.3.
+# Building the compact form takes 18 to 45 us a layer, which 8 to 30 steps win back, and a session may end after one: the first
+# step of four layers of 256 rows of 32768 keys 506 -> 380 us (425 before there was one kernel), 128 rows of 12011 keys 260 -> 200 (226).
+_TWO_PLANE_KEYS = 8192
+_TWO_PLANE_STEPS = 16
 _HASH_BLOCK = 64    # HashAttention decode: new keys are hashed this many at a time (never more than the local window)
 
 
@@ -160,19 +167,21 @@ class DecodePlan:
         """A HashAttention step under an additive mask; the chain holds the signatures of new keys and of the query, `self.att`
         the attention."""
         chain, at = self.chain, self.att
-        # A mask that only hides columns: one kernel. The compact form it reads is kept by steps like this one; a step that
-        # would read what another stream has written takes the other way, and so does a captured one: its mask is what the
-        # buffer holds at a replay, which may be anything.
+        # A mask that only hides columns: one kernel. The compact form that it reads for long rows is kept by steps like this one; a
+        # step that would read what another stream has written takes the other way.
         # (a byte and two bits of LDS a key and four bytes an entry: longer rows do not get as far as buffers they cannot use)
         if (only_hides and self.dtype != torch.float16 and rows.n_keys * 5 // 4 + 4 * rows.cap <= 150 * 1024
-                and cache.compact_ordered(stream) and not torch.cuda.is_current_stream_capturing()):
+                and cache.compact_ordered(stream)):
             hd, hm = self.hash_decode, self.hash_masked
             hd.rows, hd.sink, hd.window, hd.k, hd.stream = rows, sink, window, k_eff, stream
             hd.query_sig, hd.key_sig, hd.skip_bitmap = chain.sig_b, None, 1
             hd.kcodes, hd.code_pitch = cache.codes.data_ptr(), cache.capacity
             hm.decode, hm.attention, hm.tickets = C.addressof(hd), C.addressof(at), self.tickets.data_ptr()
             done = []
-            self._use_compact(hd, cache, hashed, stream, done)
+            if rows.n_keys > _TWO_PLANE_KEYS and (cache.pos is not None or cache.masked_steps >= _TWO_PLANE_STEPS):
+                self._use_compact(hd, cache, hashed, stream, done)
+            else:
+                hd.pos_codes = hd.exc = hd.exc_cnt = None
             hm.ask = 1
             N.call("sah_hash_decode_masked", hm)
             if hm.fits:
@@ -182,6 +191,8 @@ class DecodePlan:
                 hm.ask = 0
                 N.call("sah_hash_decode_masked", hm)
                 commit.extend(done)
+                cache.masked_steps += 1
+                cache.compact_stream = stream  # (the first such step says whose the compact form will be)
                 return
             chain.compact = None
         # The mask takes part in the scores: they go through memory as sortable keys, and the selection writes the sink +

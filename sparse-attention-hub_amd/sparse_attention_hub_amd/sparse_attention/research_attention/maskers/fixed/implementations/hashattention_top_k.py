@@ -63,8 +63,10 @@ class PackedSignatureCache:
         # columns with a zero component [B, Hq, exc_cap, 4] and their number [B, Hq]; valid for `n_compact` keys
         self.pos = self.exc = self.exc_cnt = None
         self.n_compact = 0
-        # the one stream on which the compact form's buffers were cleared and written; None: there are none, SEVERAL_STREAMS: no one
+        # the one stream on which the compact form's buffers were cleared and written, or a masked step will write them; None:
+        # there are none, SEVERAL_STREAMS: no one
         self.compact_stream: Optional[int] = None
+        self.masked_steps = 0  # steps of one kernel under a mask that hides columns
 
     @property
     def capacity(self) -> int:

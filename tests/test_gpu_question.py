@@ -1041,3 +1041,67 @@ def test_a_replay_takes_the_mask_as_it_is_then(cuda):
             assert bool(((out.double() - want[kind]).abs() <= 2.0 ** -7 * want[kind].abs() + 2.0 ** -18).all()), kind
         side.synchronize()
     assert not bool(((want["h"] - want["g"]).abs() <= 2.0 ** -4 * want["h"].abs()).all())  # the bias does change what is chosen
+
+
+def _signature_planes(codes):
+    """The +-1 / 0 components of packed codes (..., 2)."""
+    c = codes.to(torch.int64) & 0xFFFFFFFF
+    shifts = torch.arange(32, device=codes.device)
+    return ((((c[..., :1] >> shifts) & 1) * 2 - 1) * ((c[..., 1:] >> shifts) & 1)).float()
+
+
+@pytest.mark.parametrize("form", ["two planes", "compact"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("kind", ["padded", "few", "mixed", "never"])
+@pytest.mark.parametrize("shape", [  # rows in several workgroups and in one; keys on either side of 256, 8192 and 16384
+    (2, 8, 2, 253, 128), (3, 8, 2, 1281, 64), (20, 16, 8, 700, 128), (1, 8, 2, 8191, 128), (1, 8, 2, 16320, 128), (1, 4, 4, 16451, 64)])
+def test_one_kernel_masked_step_against_the_oracle(cuda, monkeypatch, form, dtype, kind, shape):
+    """Both forms of the codes, given the kernel's signatures; `never`: -inf wherever the padded batch is hidden, and in all of
+    a row."""
+    import sparse_attention_hub_amd.sparse_attention as sa
+    from oracle import reference_path as O
+    from sparse_attention_hub_amd import _native as N
+    from sparse_attention_hub_amd.sparse_attention.research_attention import decode_plan
+    from sparse_attention_hub_amd.sparse_attention.utils.hashattention_utils import random_hat_weights
+
+    if form == "compact":
+        monkeypatch.setattr(decode_plan, "_TWO_PLANE_KEYS", 0)
+        monkeypatch.setattr(decode_plan, "_TWO_PLANE_STEPS", 0)
+    else:
+        monkeypatch.setattr(decode_plan, "_TWO_PLANE_KEYS", 1 << 30)
+    B, Hq, Hkv, n, D = shape
+    sink, window, heavy = 9, 70, 50
+    lowest = float(torch.finfo(dtype).min)
+    ra = sa.ResearchAttention.create_from_config(sa.ResearchAttentionConfig(masker_configs=[
+        sa.SinkMaskerConfig(sink_size=sink), sa.LocalMaskerConfig(window_size=window), sa.HashAttentionTopKMaskerConfig(
+            heavy_size=heavy, hat_bits=32, hat_mlp_layers=3, hat_mlp_hidden_size=128, hat_mlp_activation="relu" if D == 64 else "silu",
+            hat_weights=random_hat_weights(1, Hq, D, 32, 3, 128, dtype=dtype, seed=1))]))
+    ra.return_attention_weights = False
+    q, k, v = make_qkv(B, Hq, Hkv, 1, n, D, dtype, seed=5)
+    k[:, :, ::5] = 0.0  # (zero keys: relu leaves signature components that are zero)
+    m = _hide(torch.zeros((B, 1, 1, n)), "padded" if kind == "never" else kind, n, window, -float("inf") if kind == "never" else lowest)
+    if kind == "never" and B > 1:
+        m[B - 1] = -float("inf")
+    m = m.to(dtype)
+    args = [t.to(cuda) for t in (q, k, v, m)]
+    meta = {}
+    for i in range(2):
+        N.timing_enable(True)
+        out = ra.custom_attention(None, *args, D ** -0.5, 0.0, sparse_meta_data=meta, layer_idx=0)[0]
+        torch.cuda.synchronize()
+        names = launched(N)
+        assert i == 0 or "k_hash_decode_attn" in names
+    assert (meta["key"][0].pos is not None) == (form == "compact")
+    qcodes = torch.empty((B, Hq, 1, 2), dtype=torch.int32, device=cuda)
+    ra.maskers[2]._hash(args[0], Hq, Hq, 0, 1, 0, "query", qcodes, 1, 0)
+    state = {"key_sig": _signature_planes(meta["key"][0].codes[:, :, :n]).cpu(), "query_sig": _signature_planes(qcodes).cpu()}
+    want = O.research_attention([("sink", sink), ("local", window), ("hash_topk", heavy, None, None)],
+                                q.float(), k.float(), v.float(), m.float().masked_fill(m == lowest, float(torch.finfo(torch.float32).min)),
+                                D ** -0.5, None, state)[0].double()
+    got = out.cpu().double()
+    ok = torch.isfinite(want)
+    assert bool(ok.all()) or kind == "never"
+    assert torch.equal(ok, torch.isfinite(got))
+    # rounding of the output, and the order of the fp32 sums (values of about 1, at most 129 of them)
+    unit = {torch.bfloat16: 2.0 ** -8, torch.float32: 2.0 ** -23}[dtype]
+    assert bool(((got - want).abs() <= unit * want.abs() + 129 * 2.0 ** -23)[ok].all()), float(((got - want).abs())[ok].max())

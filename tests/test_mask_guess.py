@@ -7,6 +7,7 @@ import torch
 
 from sparse_attention_hub_amd import _native as N
 from sparse_attention_hub_amd import sparse_attention as sa
+from sparse_attention_hub_amd.sparse_attention.research_attention import decode_plan
 from sparse_attention_hub_amd.sparse_attention.research_attention.maskers.fixed.implementations.hashattention_top_k import (
     PackedSignatureCache,
 )
@@ -32,7 +33,8 @@ class Recorder:
                 args.fits = self.fits
                 return
             hd = N.HashDecodeArgs.from_address(args.decode)
-            self.calls.append((name, self.stream, {hd.rows.cols, hd.rows.cnt, args.tickets, N.HashSigArgs.from_address(hd.query_sig).codes}, hd))
+            self.calls.append((name, self.stream, {hd.rows.cols, hd.rows.cnt, args.tickets, N.HashSigArgs.from_address(hd.query_sig).codes},
+                               N.HashDecodeArgs.from_buffer_copy(hd)))
         elif name == "sah_run_chain":
             used = {args.tickets}
             if args.select:
@@ -171,16 +173,17 @@ def test_an_instance_guesses_nothing_from_another_one(device):
     assert [len(session.step(kind)) for kind in "hzh"] == [1, 1, 1]
 
 
-def compact(launches):
-    """Which of them read the compact codes."""
-    return [c[0] == "sah_hash_decode_masked" or c[3] for c in launches]
-
-
 def one_kernel(launches):
     return any(c[0] == "sah_hash_decode_masked" for c in launches)
 
 
-def test_compact_codes_of_two_streams_are_no_masked_steps(device):
+@pytest.fixture
+def compact_at_once(monkeypatch):
+    monkeypatch.setattr(decode_plan, "_TWO_PLANE_KEYS", 0)
+    monkeypatch.setattr(decode_plan, "_TWO_PLANE_STEPS", 0)
+
+
+def test_compact_codes_of_two_streams_are_no_masked_steps(device, compact_at_once):
     """One stream has written most of the compact codes, another has added to them: a masked step on either would read what the
     other has written, and goes without them."""
     s = Session(device, attention("hash"), "hash")
@@ -193,7 +196,7 @@ def test_compact_codes_of_two_streams_are_no_masked_steps(device):
     assert one_kernel(s.step("h", 2, LK + 40)) and not one_kernel(s.step("h", 1, LK + 40))
 
 
-def test_compact_buffers_belong_to_the_stream_that_clears_them(device):
+def test_compact_buffers_belong_to_the_stream_that_clears_them(device, compact_at_once):
     s = Session(device, attention("hash"), "hash")
     device.fits = 0
     assert not one_kernel(s.step("h", 1))  # makes the buffers, and then has no use for them
@@ -279,3 +282,16 @@ def test_a_call_that_fails_leaves_no_question_open(device, monkeypatch):
         s.ra.custom_attention(None, torch.zeros(B, HQ, 3, D, dtype=torch.bfloat16), s.k[:, :, :LK], s.k[:, :, :LK], m, D ** -0.5, 0.0,
                               sparse_meta_data=s.meta, layer_idx=0)
     assert not U._ANSWERS.open and s.ra._mask_facts.known(m) == N.AMASK_NONZERO
+
+
+def test_a_session_of_few_masked_steps_builds_no_compact_codes(device, monkeypatch):
+    s = Session(device, attention("hash"), "hash")
+    for _ in range(20):
+        assert one_kernel(s.step("h"))
+    assert s.cache.pos is None  # rows of this length never need them
+    monkeypatch.setattr(decode_plan, "_TWO_PLANE_KEYS", LK - 1)
+    s = Session(device, attention("hash"), "hash")
+    for i in range(decode_plan._TWO_PLANE_STEPS + 2):
+        launches = s.step("h")
+        assert one_kernel(launches) and len(launches) == (2 if i == decode_plan._TWO_PLANE_STEPS else 1)
+        assert bool(launches[-1][3].pos_codes) == (s.cache.pos is not None) == (i >= decode_plan._TWO_PLANE_STEPS)
