@@ -74,8 +74,8 @@ def unit_inverse_weight(dtype: torch.dtype) -> float:
 
 def mask_covers(am: torch.Tensor, queries: torch.Tensor, n_keys: int) -> bool:
     """Has the 4-dimensional mask a row for every query, as wide as the keys?"""
-    return (am.shape[-1] >= n_keys and am.shape[2] == queries.shape[2] and am.shape[0] in (1, queries.shape[0])
-            and am.shape[1] in (1, queries.shape[1]))
+    m, q = am.shape, queries.shape
+    return m[3] >= n_keys and m[2] == q[2] and m[0] in (1, q[0]) and m[1] in (1, q[1])
 
 
 def additive_mask_args(attention_mask: Optional[torch.Tensor], queries: torch.Tensor, n_keys: int):
@@ -133,9 +133,11 @@ class MaskQuestion:
             earlier.settle()
         # (mask and words stay allocated until the answer)
         self.mask, self.version, self.flags, self._words = am, am._version, None, (scratch, word)
+        b, h, n_q, n = am.shape
+        sb, sh, sq, _ = am.stride()
+        self.one_query = n_q == 1
         args = N.AmaskQuestion(N.AmaskReadArgs(N.AmaskClassifyArgs(
-            am.data_ptr(), am.stride(0), am.stride(1), am.stride(2), N.dtype_code(am.dtype),
-            am.shape[0], am.shape[1], am.shape[2], am.shape[3], None, N.stream_ptr(dev)), scratch.data_ptr(), word.data_ptr()))
+            am.data_ptr(), sb, sh, sq, N.dtype_code(am.dtype), b, h, n_q, n, None, N.stream_ptr(dev)), scratch.data_ptr(), word.data_ptr()))
         N.call("sah_amask_ask", args)
         self._args = args
         _ANSWERS.open[dev.index] = self
@@ -168,13 +170,14 @@ class AdditiveMaskFacts:
     handed to another tensor that would then be mistaken for it.
 
     What a session's last mask held is the guess for its next one. It is kept in the session's own `sparse_meta_data` (sessions
-    with and without padding that take turns are each guessed right), under a number of this object's."""
+    with and without padding that take turns are each guessed right), under names of this object's."""
 
     _numbers = itertools.count()
 
     def __init__(self) -> None:
         self._seen: Tuple[Optional[torch.Tensor], int, int] = (None, -1, 0)  # tensor, its version, flags
-        self._number = next(self._numbers)
+        number = next(self._numbers)
+        self._one, self._several = f"additive_mask_{number}_one_query", f"additive_mask_{number}_several_queries"
 
     def known(self, am: torch.Tensor) -> Optional[int]:
         tensor, version, flags = self._seen
@@ -186,15 +189,13 @@ class AdditiveMaskFacts:
 
     def guess(self, am: torch.Tensor, session: Any) -> Optional[int]:
         """The flags of the session's last mask for as many queries (one, or several)."""
-        if not isinstance(session, dict):
-            return None
-        return session.get("additive_mask_flags", {}).get((self._number, am.shape[2] == 1))
+        return session.get(self._one if am.shape[2] == 1 else self._several) if isinstance(session, dict) else None
 
     def take(self, question: MaskQuestion, session: Any = None) -> int:
         flags = question.settle()
         self._seen = (question.mask, question.version, flags)
         if isinstance(session, dict):
-            session.setdefault("additive_mask_flags", {})[(self._number, question.mask.shape[2] == 1)] = flags
+            session[self._one if question.one_query else self._several] = flags
         return flags
 
     def flags(self, attention_mask: torch.Tensor) -> int:
