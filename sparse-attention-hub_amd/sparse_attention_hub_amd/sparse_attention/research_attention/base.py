@@ -34,6 +34,12 @@ MicroMetricLogger.register_metric("research_attention_density", float)
 MicroMetricLogger.register_metric("research_attention_output_error", float)
 
 
+# Plans of steps whose mask is guessed to be zero that an instance keeps, over geometries, streams and threads: the latest ones made
+# (making one at every step takes longer than the wait that a guess saves). Each holds its rows and 2 to 6 bytes of score keys a row
+# and key.
+_GUESSED_PLANS = 16
+
+
 @dataclass
 class ResearchAttentionConfig(SparseAttentionConfig):
     masker_configs: List[MaskerConfig]
@@ -179,12 +185,12 @@ class ResearchAttention(SparseAttention):
         launched again (what it adds to the caches does not depend on the mask). A mask of several queries, all but always
         nonzero, is taken as it is, which is right whatever it holds."""
         am = attention_mask
-        if (not am.is_cuda or am.dim() != 4 or am.shape[-1] < keys.shape[2]
-                or am.dtype not in (torch.float32, torch.bfloat16, torch.float16)):
-            return am, False, None, None
         facts = self._mask_facts
+        flags = facts.known(am)  # (of the layers behind the first, the usual call)
+        if (am.dim() != 4 or am.shape[-1] < keys.shape[2]
+                or flags is None and am.dtype not in (torch.float32, torch.bfloat16, torch.float16)):
+            return am, False, None, None
         same_type = am.dtype == queries.dtype  # (a lowest value of another type is none of the queries')
-        flags = facts.known(am)
         if flags is None:
             guess = facts.guess(am, sparse_meta_data)
             question = MaskQuestion(am)
@@ -193,7 +199,8 @@ class ResearchAttention(SparseAttention):
                 hides = not guess & _native.AMASK_GENERAL and same_type
                 out, error = None, None
                 try:
-                    out = self._plan_step(queries, keys, values, am if guess else None, scaling, sparse_meta_data, layer_idx, hides, guessed=True)
+                    out = self._plan_step(queries, keys, values, am if guess else None, scaling, sparse_meta_data, layer_idx, hides,
+                                          guessed=True)
                 except Exception as e:
                     error = e
                 flags = facts.take(question, sparse_meta_data)
@@ -222,16 +229,20 @@ class ResearchAttention(SparseAttention):
         # belong to the call: a step on another stream is not ordered with the ones that use them. So do those of a step whose
         # mask is guessed to be zero: it may turn out to be a masked one. A captured step's belong to its graph alone: what its
         # plan clears is clear when the graph runs, not now; and its mask is what the buffer holds then, which may be anything.
-        owned = masked or guessed
-        key = (queries.device, queries.dtype, tuple(queries.shape), keys.shape[1], masked, owned)
-        owner = (_native.stream_ptr(queries.device), threading.get_ident()) if owned else None
-        if masked and torch.cuda.is_current_stream_capturing():
+        owner = (_native.stream_ptr(queries.device), threading.get_ident()) if masked or guessed else None
+        capturing = torch.cuda.is_current_stream_capturing() if masked else None
+        if capturing:
             plan, only_hides = DecodePlan(self.maskers, self._plan_kind, queries, keys, True), False
         else:
+            key = (queries.device, queries.dtype, queries.shape, keys.shape[1], masked, None if masked else owner)
             plan = self._plans.get(key)
             if plan is None or plan.owner != owner:
+                if guessed and not masked:
+                    guesses = [k for k, p in list(self._plans.items()) if p.owner is not None and not p.masked]
+                    if len(guesses) >= _GUESSED_PLANS:
+                        self._plans.pop(guesses[0], None)
                 plan = self._plans[key] = DecodePlan(self.maskers, self._plan_kind, queries, keys, masked, owner)
-        return plan.run(queries, keys, values, scaling, sparse_meta_data, layer_idx, attention_mask, only_hides, guessed)
+        return plan.run(queries, keys, values, scaling, sparse_meta_data, layer_idx, attention_mask, only_hides, guessed, capturing)
 
     @classmethod
     def create_from_config(cls, config: SparseAttentionConfig) -> "ResearchAttention":

@@ -220,10 +220,12 @@ class DecodePlan:
     # --------------------------------------------------------------------- run
     def run(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scaling: float,
             sparse_meta_data: Dict[Any, Any], layer_idx: Optional[int],
-            attention_mask: Optional[torch.Tensor] = None, only_hides: bool = False, guessed: bool = False) -> Optional[torch.Tensor]:
+            attention_mask: Optional[torch.Tensor] = None, only_hides: bool = False, guessed: bool = False,
+            capturing: Optional[bool] = None) -> Optional[torch.Tensor]:
         """One layer-step; returns the attention output (B, Lq, Hq, D) or None if not applicable. `only_hides`: the mask is known
         to hold nothing but zeros and entries at the lowest value of its type or -inf. `guessed`: the step's mask may be another
-        one, under which the step must not read or write what another stream has written."""
+        one, under which the step must not read or write what another stream has written. `capturing`: is the
+        stream, if the caller knows."""
         masked = self.masked
         if masked and (self.Lq != 1 or attention_mask.dim() != 4):
             return None
@@ -413,7 +415,7 @@ class DecodePlan:
         floats = self.work_need
         if self.by_bitmap:
             floats = max(floats, N.members_work_floats(self.B, self.Hq, self.Hkv, Lq, Lk, self.D))
-        work = _workspace(self.device, floats, stream)
+        work = _workspace(self.device, floats, stream, capturing)
         at = self.att
         at.rows = rows
         at.q, at.qs_b, at.qs_h, at.qs_l = q.data_ptr(), q.stride(0), q.stride(1), q.stride(2)

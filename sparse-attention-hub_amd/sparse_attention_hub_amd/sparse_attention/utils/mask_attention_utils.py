@@ -36,13 +36,13 @@ class _Scratch(threading.local):
 _WORK = _Scratch()
 
 
-def _workspace(device: torch.device, floats: int, stream: int) -> torch.Tensor:
+def _workspace(device: torch.device, floats: int, stream: int, capturing: Optional[bool] = None) -> torch.Tensor:
     """Grow-only fp32 scratch of the calling thread for the current stream of `device` (whose handle is `stream`): calls on
     other streams are not ordered with this one's, and another thread's may come between the two kernels of a call. The
     latest few streams' buffers are kept until the thread ends; one that goes was allocated on its stream, so torch's
     allocator hands its memory to later work of that stream. Large ones (many query vectors of a long pass, merged in
     milliseconds) are the call's. A captured call's scratch is its graph's own: replays use it whatever this thread keeps."""
-    if floats > _WORK_FLOATS or torch.cuda.is_current_stream_capturing():
+    if floats > _WORK_FLOATS or (torch.cuda.is_current_stream_capturing() if capturing is None else capturing):
         return torch.empty(floats, dtype=torch.float32, device=device)
     key = (device.index, stream)
     buffers = _WORK.buffers

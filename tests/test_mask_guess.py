@@ -295,3 +295,23 @@ def test_a_session_of_few_masked_steps_builds_no_compact_codes(device, monkeypat
         launches = s.step("h")
         assert one_kernel(launches) and len(launches) == (2 if i == decode_plan._TWO_PLANE_STEPS else 1)
         assert bool(launches[-1][3].pos_codes) == (s.cache.pos is not None) == (i >= decode_plan._TWO_PLANE_STEPS)
+
+
+def test_guesses_of_several_threads_make_one_plan_each(device):
+    """Unpadded sessions of two streams in turn keep their plans; only so many are kept."""
+    from sparse_attention_hub_amd.sparse_attention.research_attention import base
+
+    ra = attention("oracle")
+    sessions = [Session(device, ra, "oracle") for _ in range(2)]
+    for _ in range(2):
+        for stream, s in enumerate(sessions):
+            s.step("z", stream)
+    plans = dict(ra._plans)
+    assert len(plans) == 3  # with the one of steps that are known to have no mask
+    for _ in range(3):
+        for stream, s in enumerate(sessions):
+            s.step("z", stream)
+    assert ra._plans == plans
+    for stream in range(2 * base._GUESSED_PLANS):
+        sessions[0].step("z", stream)
+    assert len(ra._plans) == base._GUESSED_PLANS + 1
