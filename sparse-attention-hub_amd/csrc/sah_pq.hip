@@ -480,8 +480,9 @@ __global__ __launch_bounds__(PQ_NT) void k_pq_update(pq_update_params P) {
 // The split form's rounding is another one (and smaller), so where several centres come within both forms' rounding of the
 // smallest value they are evaluated in the fp32 form's order of operations: the codes are those of the fp32 form, bit for
 // bit, whichever form the alignment and shape of the keys allow (without: 1e-6 of the codes of an iteration, 5e-4 after ten).
-// Measured (bf16, 8 heads x 16277 keys, 16 sub-vectors of 8, 256 centres, sums included): 64 us (66 with the update; 65 and 71
-// without the pipeline of PIPE); 85 with every tile's 16 values selected, not their minima over the tiles, the second look by matrix instruction, its test by ballots, the key
+// Measured (bf16, 8 heads x 16277 keys, 16 sub-vectors of 8, 256 centres, sums and update included, by events on a warm GPU): 66 us
+// (a trace of a few passes, its clock still low, says 70 to 73); 85 with every tile's 16 values selected, not their minima over
+// the tiles, the second look by matrix instruction, its test by ballots, the key
 // operand in a structure (which went through scratch memory) and the centres read element by element. What bounds it: 20 vector
 // and 2 matrix instructions a tile, in sum (5 us a centre tile: 40), 150 vector ones a key tile of eight (20), 6 before and
 // after the loop. fp16 (no split: terms of small centres would leave its range): 121 at 16405 keys. 32768 keys, 2 sub-vectors of 64, 64
@@ -561,12 +562,14 @@ __device__ __forceinline__ uint32_t pqm_mask_le(const sah_f32x16& a, float b) {
 // the LDS holds them). A workgroup takes wg_tiles tiles of 32 keys of one group.
 // PIPE: the centre tiles go by in pairs, a multiple of four of them; a pair's products are under way while the minima of the
 // pair before are taken, each matrix instruction between ten vector ones, and a key tile's last pair has the next key tile's
-// first behind it, which so computes while the key tile is concluded.
+// first behind it, which so computes while the key tile is concluded. Sub-vectors of 8 alone: 8 heads x 16 of them, 256 centres:
+// 4096 keys 30.4 -> 29.5 us, 16405 keys 66.8 -> 66.2, 32768 keys 114.8 -> 113.3 (32 heads x 8192 keys 113.3 -> 114.2, 128 centres x
+// 16405 keys 46.6 -> 47.2); sub-vectors of 16 lost up to 2 % (8 of them, 128 centres, 16405 keys 38.9 -> 39.5).
 template <int DT, int KS, bool SUMS, bool SPLIT, bool PIPE>
 __global__ __launch_bounds__(PQM_NT, KS <= 16 ? 4 : 2) void k_pq_assign_mfma(pq_assign_params P, pq_update_params U, uint32_t* arrivals,
                                                                                            int wg_tiles, int ranges, int n_heads) {
   SAH_DYNAMIC_LDS(pqm_dyn)
-  static_assert(!PIPE || (SPLIT && KS <= 8), "the pipelined loop holds a key in one operand");
+  static_assert(!PIPE || (SPLIT && KS == 4), "the pipelined loop has two operands a tile and the norms among them");
   static_assert(!SPLIT || (DT == SAH_BF16 && KS >= 4), "the split form multiplies bf16 keys in sub-vectors of 8 and more");
   if (P.skip_flag && *P.skip_flag) return;
   const int tid = threadIdx.x;
@@ -843,7 +846,7 @@ __global__ __launch_bounds__(PQM_NT, KS <= 16 ? 4 : 2) void k_pq_assign_mfma(pq_
     }
   };
   if constexpr (PIPE) {
-    auto first_op = [&](const sah_u4& x) { return KS == 4 && g ? sah_u4{0x3f803f80u, 0x3f80u, 0u, 0u} : x; };
+    auto first_op = [&](const sah_u4& x) { return g ? sah_u4{0x3f803f80u, 0x3f80u, 0u, 0u} : x; };
     auto in_range = [&](int kt) { return kt < wg_tiles && (tg * wg_tiles + kt) * 32 < P.n_keys; };  // uniform across the wave
     int kt = wave;
     if (in_range(kt)) {
@@ -853,20 +856,7 @@ __global__ __launch_bounds__(PQM_NT, KS <= 16 ? 4 : 2) void k_pq_assign_mfma(pq_
       sah_u4 cur[NB];  // the keys in hand (nb: the next ones)
       cur[0] = nb[0];
       request((tg * wg_tiles + kt + PQM_NW) * 32 + j);
-      // the products of a pair of centre tiles: start, and for every operand its two loads and two matrix instructions
-      auto start = [&](int t, sah_f32x16& n0, sah_f32x16& n1) __attribute__((always_inline)) {
-        if constexpr (NORM_IN_A) {
-          n0 = n1 = sah_f32x16{};
-        } else {
-          const float4* cn4 = (const float4*)(s_cn + (t * 2 + g) * 16);
-#pragma unroll
-          for (int q4 = 0; q4 < 4; ++q4) {
-            const float4 c4 = cn4[q4], d4 = cn4[8 + q4];
-            n0[4 * q4] = c4.x; n0[4 * q4 + 1] = c4.y; n0[4 * q4 + 2] = c4.z; n0[4 * q4 + 3] = c4.w;
-            n1[4 * q4] = d4.x; n1[4 * q4 + 1] = d4.y; n1[4 * q4 + 2] = d4.z; n1[4 * q4 + 3] = d4.w;
-          }
-        }
-      };
+      // the products of a pair of centre tiles: for every operand its two loads and two matrix instructions
       auto load = [&](int t, int op, uint4 (&o)[2]) __attribute__((always_inline)) {
         const uint4* ap = (const uint4*)s_a + (size_t)t * 64 * OPS + g * 32 + j;
         o[0] = ap[op * 64];
@@ -887,7 +877,7 @@ __global__ __launch_bounds__(PQM_NT, KS <= 16 ? 4 : 2) void k_pq_assign_mfma(pq_
                       const sah_u4& x, const sah_u4& x0) __attribute__((always_inline)) {
         constexpr bool FIRST = decltype(first_c)::value;
         uint4 o[2];
-        start(t_next, n0, n1);
+        n0 = n1 = sah_f32x16{};
         load(t_next, 0, o);
         if (FIRST) {
           best = second = INFINITY;
@@ -913,19 +903,13 @@ __global__ __launch_bounds__(PQM_NT, KS <= 16 ? 4 : 2) void k_pq_assign_mfma(pq_
         for (int v = 1; v < 8; ++v) m = PQM_MIN(m, c1[v]);
         __builtin_amdgcn_sched_barrier(0);
         mm(x, o[1], n1);
-        if constexpr (OPS == 3) load(t_next, 2, o);
 #pragma unroll
         for (int v = 8; v < 16; ++v) m = PQM_MIN(m, c1[v]);
         take(m, t + 1);
-        if constexpr (OPS == 3) {
-          __builtin_amdgcn_sched_barrier(0);
-          mm(x, o[0], n0);
-          mm(x, o[1], n1);
-        }
       };
       sah_f32x16 a0, a1, b0, b1;
       {
-        start(0, a0, a1);
+        a0 = a1 = sah_f32x16{};
 #pragma unroll
         for (int op = 0; op < OPS; ++op) {
           uint4 o[2];
@@ -1169,7 +1153,7 @@ template <int DT, int KS>
 static int pq_launch_mfma_form(const sah_pq_assign_args* a, const pq_assign_params& P, const pq_update_params& U, uint32_t* arrivals, bool split,
                                bool fused, size_t lds) {
   if constexpr (DT == SAH_BF16 && KS >= 4) {
-    if constexpr (KS <= 8) {
+    if constexpr (KS == 4) {
       if (split && (a->n_cent + 31) / 32 % 4 == 0) return pq_launch_mfma_ks<DT, KS, true, true>(a, P, U, arrivals, fused, lds);
     }
     if (split) return pq_launch_mfma_ks<DT, KS, true, false>(a, P, U, arrivals, fused, lds);
