@@ -936,123 +936,123 @@ __global__ __launch_bounds__(PQM_NT, KS <= 16 ? 4 : 2) void k_pq_assign_mfma(pq_
       }
     }
   } else {
-  for (int kt = wave; kt < wg_tiles; kt += PQM_NW) {
-    const int n0 = (tg * wg_tiles + kt) * 32;
-    if (n0 >= P.n_keys) break;  // uniform across the wave
-    const int n = n0 + j;
-    float xs[SPLIT ? 1 : KS];  // this lane's dims 2 s + g of its key
-    sah_u4 xb[NB];             // SPLIT: dims 16 q + 8 g .. + 7 (sub-vectors of 8: both halves hold all)
-    sah_u4 x0;                 // key operand of the first instruction: with the norm in A, ones against its terms
-    if constexpr (SPLIT) {
-#pragma unroll
-      for (int q = 0; q < NB; ++q) xb[q] = nb[q];
-      request(n + 32 * PQM_NW);
-      x0 = xb[0];
-      if (KS == 4 && g) x0 = sah_u4{0x3f803f80u, 0x3f80u, 0u, 0u};
-    } else {
-      const int64_t off = key_offset(n);
-#pragma unroll
-      for (int s = 0; s < KS; ++s) xs[s] = (2 * s + g < d_sub) ? sah_load<DT>(P.k, off + 2 * s + g) : 0.f;
-    }
-    // accumulator of centre tile t: seeded with the norms, then the matrix instructions
-    auto product = [&](sah_f32x16& acc, int t) {
-      if constexpr (NORM_IN_A) {
-        acc = sah_f32x16{};
-      } else {
-        const float4* cn4 = (const float4*)(s_cn + (t * 2 + g) * 16);
-#pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4) {
-          const float4 c4 = cn4[q4];
-          acc[4 * q4] = c4.x; acc[4 * q4 + 1] = c4.y; acc[4 * q4 + 2] = c4.z; acc[4 * q4 + 3] = c4.w;
-        }
-      }
+    for (int kt = wave; kt < wg_tiles; kt += PQM_NW) {
+      const int n0 = (tg * wg_tiles + kt) * 32;
+      if (n0 >= P.n_keys) break;  // uniform across the wave
+      const int n = n0 + j;
+      float xs[SPLIT ? 1 : KS];  // this lane's dims 2 s + g of its key
+      sah_u4 xb[NB];             // SPLIT: dims 16 q + 8 g .. + 7 (sub-vectors of 8: both halves hold all)
+      sah_u4 x0;                 // key operand of the first instruction: with the norm in A, ones against its terms
       if constexpr (SPLIT) {
-        const uint4* ap = (const uint4*)s_a + (size_t)t * 64 * OPS + g * 32 + j;
-#pragma unroll
-        for (int op = 0; op < OPS; ++op) acc = sah_mfma_32x32x16<SAH_BF16>(ap[op * 64], __builtin_bit_cast(uint4, op ? xb[op % NB] : x0), acc);
-      } else if constexpr (KS >= 4) {
-        const float4* ap = (const float4*)(s_a + (size_t)(t * 2 + g) * 32 * KS) + j;
-#pragma unroll
-        for (int q = 0; q < KS / 4; ++q) {
-          const float4 a4 = ap[q * 32];
-          acc = sah_mfma_32x32x2_f32(a4.x, xs[4 * q], acc);
-          acc = sah_mfma_32x32x2_f32(a4.y, xs[4 * q + 1], acc);
-          acc = sah_mfma_32x32x2_f32(a4.z, xs[4 * q + 2], acc);
-          acc = sah_mfma_32x32x2_f32(a4.w, xs[4 * q + 3], acc);
+  #pragma unroll
+        for (int q = 0; q < NB; ++q) xb[q] = nb[q];
+        request(n + 32 * PQM_NW);
+        x0 = xb[0];
+        if (KS == 4 && g) x0 = sah_u4{0x3f803f80u, 0x3f80u, 0u, 0u};
+      } else {
+        const int64_t off = key_offset(n);
+  #pragma unroll
+        for (int s = 0; s < KS; ++s) xs[s] = (2 * s + g < d_sub) ? sah_load<DT>(P.k, off + 2 * s + g) : 0.f;
+      }
+      // accumulator of centre tile t: seeded with the norms, then the matrix instructions
+      auto product = [&](sah_f32x16& acc, int t) {
+        if constexpr (NORM_IN_A) {
+          acc = sah_f32x16{};
+        } else {
+          const float4* cn4 = (const float4*)(s_cn + (t * 2 + g) * 16);
+  #pragma unroll
+          for (int q4 = 0; q4 < 4; ++q4) {
+            const float4 c4 = cn4[q4];
+            acc[4 * q4] = c4.x; acc[4 * q4 + 1] = c4.y; acc[4 * q4 + 2] = c4.z; acc[4 * q4 + 3] = c4.w;
+          }
+        }
+        if constexpr (SPLIT) {
+          const uint4* ap = (const uint4*)s_a + (size_t)t * 64 * OPS + g * 32 + j;
+  #pragma unroll
+          for (int op = 0; op < OPS; ++op) acc = sah_mfma_32x32x16<SAH_BF16>(ap[op * 64], __builtin_bit_cast(uint4, op ? xb[op % NB] : x0), acc);
+        } else if constexpr (KS >= 4) {
+          const float4* ap = (const float4*)(s_a + (size_t)(t * 2 + g) * 32 * KS) + j;
+  #pragma unroll
+          for (int q = 0; q < KS / 4; ++q) {
+            const float4 a4 = ap[q * 32];
+            acc = sah_mfma_32x32x2_f32(a4.x, xs[4 * q], acc);
+            acc = sah_mfma_32x32x2_f32(a4.y, xs[4 * q + 1], acc);
+            acc = sah_mfma_32x32x2_f32(a4.z, xs[4 * q + 2], acc);
+            acc = sah_mfma_32x32x2_f32(a4.w, xs[4 * q + 3], acc);
+          }
+        } else {
+          const float* ap = s_a + ((t * 2 + g) * 32 + j) * KS;
+  #pragma unroll
+          for (int s = 0; s < KS; ++s) acc = sah_mfma_32x32x2_f32(ap[s], xs[s], acc);
+        }
+      };
+      // The smallest value and its tile; a value that is not a number makes its tile's minimum one, and such key tiles are
+      // evaluated again below. Without the split form also that tile's 16 values, from which the slot is found once at the end
+      // (27 vector instructions a tile; a search for the slot takes 48): strictly smaller in ascending tiles, lowest slot, so
+      // that the first minimum is kept. In the split form instead every slot's minimum over the tiles, two tiles to a three-way
+      // minimum, and the second smallest of the tiles' minima (20 instructions a tile): together they tell whether any other
+      // centre came near the smallest value, and with none near the smallest value's slot is the one whose minimum it is.
+      float best = INFINITY, second = INFINITY;
+      int bt = 0;
+      bool nan = false;
+      sah_f32x16 kept = {};
+      auto tile_min = [&](const sah_f32x16& acc, int t) -> bool {
+        float m = acc[0];
+  #pragma unroll
+        for (int v = 1; v < 16; ++v) m = PQM_MIN(m, acc[v]);
+        if (SPLIT) second = __builtin_amdgcn_fmed3f(best, second, m);
+        else nan |= m != m;
+        const bool less = m < best;
+        best = less ? m : best;
+        bt = less ? t : bt;
+        return less;
+      };
+      sah_f32x16 acc0, acc1;
+      if constexpr (SPLIT) {
+        product(acc0, 0);
+        tile_min(acc0, 0);
+        kept = acc0;
+        int t = 1;
+        for (; t + 1 < n_tiles; t += 2) {
+          product(acc0, t);
+          product(acc1, t + 1);
+  #pragma unroll
+          for (int v = 0; v < 16; ++v) kept[v] = PQM_MIN(PQM_MIN(kept[v], acc0[v]), acc1[v]);
+          tile_min(acc0, t);
+          tile_min(acc1, t + 1);
+        }
+        if (t < n_tiles) {
+          product(acc0, t);
+  #pragma unroll
+          for (int v = 0; v < 16; ++v) kept[v] = PQM_MIN(kept[v], acc0[v]);
+          tile_min(acc0, t);
         }
       } else {
-        const float* ap = s_a + ((t * 2 + g) * 32 + j) * KS;
-#pragma unroll
-        for (int s = 0; s < KS; ++s) acc = sah_mfma_32x32x2_f32(ap[s], xs[s], acc);
+        auto take_min = [&](const sah_f32x16& acc, int t) {
+          const bool less = tile_min(acc, t);
+  #pragma unroll
+          for (int v = 0; v < 16; ++v) kept[v] = less ? acc[v] : kept[v];
+        };
+        // two accumulators: a tile's products are issued before the minimum of the tile before is taken, which so never waits
+        // for a product just started
+        product(acc0, 0);
+        int t = 0;
+        for (; t + 2 < n_tiles; t += 2) {
+          product(acc1, t + 1);
+          take_min(acc0, t);
+          product(acc0, t + 2);
+          take_min(acc1, t + 1);
+        }
+        if (t + 1 < n_tiles) {
+          product(acc1, t + 1);
+          take_min(acc0, t);
+          take_min(acc1, t + 1);
+        } else {
+          take_min(acc0, t);
+        }
       }
-    };
-    // The smallest value and its tile; a value that is not a number makes its tile's minimum one, and such key tiles are
-    // evaluated again below. Without the split form also that tile's 16 values, from which the slot is found once at the end
-    // (27 vector instructions a tile; a search for the slot takes 48): strictly smaller in ascending tiles, lowest slot, so
-    // that the first minimum is kept. In the split form instead every slot's minimum over the tiles, two tiles to a three-way
-    // minimum, and the second smallest of the tiles' minima (20 instructions a tile): together they tell whether any other
-    // centre came near the smallest value, and with none near the smallest value's slot is the one whose minimum it is.
-    float best = INFINITY, second = INFINITY;
-    int bt = 0;
-    bool nan = false;
-    sah_f32x16 kept = {};
-    auto tile_min = [&](const sah_f32x16& acc, int t) -> bool {
-      float m = acc[0];
-#pragma unroll
-      for (int v = 1; v < 16; ++v) m = PQM_MIN(m, acc[v]);
-      if (SPLIT) second = __builtin_amdgcn_fmed3f(best, second, m);
-      else nan |= m != m;
-      const bool less = m < best;
-      best = less ? m : best;
-      bt = less ? t : bt;
-      return less;
-    };
-    sah_f32x16 acc0, acc1;
-    if constexpr (SPLIT) {
-      product(acc0, 0);
-      tile_min(acc0, 0);
-      kept = acc0;
-      int t = 1;
-      for (; t + 1 < n_tiles; t += 2) {
-        product(acc0, t);
-        product(acc1, t + 1);
-#pragma unroll
-        for (int v = 0; v < 16; ++v) kept[v] = PQM_MIN(PQM_MIN(kept[v], acc0[v]), acc1[v]);
-        tile_min(acc0, t);
-        tile_min(acc1, t + 1);
-      }
-      if (t < n_tiles) {
-        product(acc0, t);
-#pragma unroll
-        for (int v = 0; v < 16; ++v) kept[v] = PQM_MIN(kept[v], acc0[v]);
-        tile_min(acc0, t);
-      }
-    } else {
-      auto take_min = [&](const sah_f32x16& acc, int t) {
-        const bool less = tile_min(acc, t);
-#pragma unroll
-        for (int v = 0; v < 16; ++v) kept[v] = less ? acc[v] : kept[v];
-      };
-      // two accumulators: a tile's products are issued before the minimum of the tile before is taken, which so never waits
-      // for a product just started
-      product(acc0, 0);
-      int t = 0;
-      for (; t + 2 < n_tiles; t += 2) {
-        product(acc1, t + 1);
-        take_min(acc0, t);
-        product(acc0, t + 2);
-        take_min(acc1, t + 1);
-      }
-      if (t + 1 < n_tiles) {
-        product(acc1, t + 1);
-        take_min(acc0, t);
-        take_min(acc1, t + 1);
-      } else {
-        take_min(acc0, t);
-      }
+      conclude(kt, n, xb, xs, kept, best, second, bt, nan);
     }
-    conclude(kt, n, xb, xs, kept, best, second, bt, nan);
-  }
   }
   if (!SUMS) return;
   __syncthreads();
