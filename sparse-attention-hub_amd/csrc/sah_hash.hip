@@ -289,8 +289,9 @@ __global__ __launch_bounds__(SGM_NT, 4) void k_hash_sig_mfma(sig_params P, int n
 // instructions of a tile stand between the vector instructions of the epilogue of the tile before it: two elements to a matrix
 // instruction. Spaced like this they take 6 to 7 cycles of the SIMD's issue; eight in a row take 12 each at four waves a
 // SIMD (and 32 at one), since a wave that waits for the matrix unit keeps the issue port. Roundings are one instruction each
-// (sah_round1). What bounds it: vector issue, 1262 instructions per 32 vectors, 256 of them exponentials and reciprocals at half
-// rate: 88 % of the cycles of its steady state. 8 x 32 heads x 32768 keys: 1050 -> 900 us, 32 heads x 32801 keys 165 -> 137.
+// (sah_round1). What bounds it: vector issue, 1320 instructions per 32 vectors, 72 of them matrix ones and 256 exponentials and
+// reciprocals at half rate: by its counters the vector unit is active 94 % of the cycles, the matrix unit 34 %, inside them.
+// 8 x 32 heads x 32768 keys: 1059 -> 890 us, 32 heads x 32801 keys 179 -> 140 (one run, against k_hash_sig_mfma as it was).
 #define SGU_PITCH (128 + SGM_PAD)
 #define SGU_ROWS (128 + 128 + 32)
 template <int DT, int ACT>

@@ -103,6 +103,7 @@ class _AnswerWords(threading.local):
 
     def __init__(self) -> None:
         self.words = {}
+        self.blocks = {}  # the argument block of a question, and of its mask
         self.open = {}
 
 
@@ -136,8 +137,14 @@ class MaskQuestion:
         b, h, n_q, n = am.shape
         sb, sh, sq, _ = am.stride()
         self.one_query = n_q == 1
-        args = N.AmaskQuestion(N.AmaskReadArgs(N.AmaskClassifyArgs(
-            am.data_ptr(), sb, sh, sq, N.dtype_code(am.dtype), b, h, n_q, n, None, N.stream_ptr(dev)), scratch.data_ptr(), word.data_ptr()))
+        block = _ANSWERS.blocks.get(dev.index)
+        if block is None:
+            args = N.AmaskQuestion()
+            args.read.scratch, args.read.host_word = scratch.data_ptr(), word.data_ptr()
+            block = _ANSWERS.blocks[dev.index] = args, args.read.mask
+        args, m = block
+        m.amask, m.ms_b, m.ms_h, m.ms_l, m.dtype = am.data_ptr(), sb, sh, sq, N.dtype_code(am.dtype)
+        m.B, m.Hm, m.Lq, m.Lk, m.stream = b, h, n_q, n, N.stream_ptr(dev)
         N.call("sah_amask_ask", args)
         self._args = args
         _ANSWERS.open[dev.index] = self

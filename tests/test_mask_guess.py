@@ -74,6 +74,7 @@ def device(monkeypatch):
     monkeypatch.setattr(N, "work_floats", lambda *a: 64)
     monkeypatch.setattr(N, "members_work_floats", lambda *a: 64)
     monkeypatch.setattr(U, "_answer_words", answer_words)
+    monkeypatch.setattr(U, "_ANSWERS", U._AnswerWords())
     return r
 
 
