@@ -1105,3 +1105,40 @@ def test_one_kernel_masked_step_against_the_oracle(cuda, monkeypatch, form, dtyp
     # rounding of the output, and the order of the fp32 sums (values of about 1, at most 129 of them)
     unit = {torch.bfloat16: 2.0 ** -8, torch.float32: 2.0 ** -23}[dtype]
     assert bool(((got - want).abs() <= unit * want.abs() + 129 * 2.0 ** -23)[ok].all()), float(((got - want).abs())[ok].max())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_masked_steps_go_over_to_the_compact_codes(cuda, monkeypatch, dtype):
+    """A session whose rows grow past the length, and whose steps past the number, from which the compact form is built, with new
+    keys hashed in between: against the masker-by-masker path."""
+    import sparse_attention_hub_amd.sparse_attention as sa
+    from sparse_attention_hub_amd.sparse_attention.research_attention import decode_plan
+    from sparse_attention_hub_amd.sparse_attention.utils.hashattention_utils import random_hat_weights
+
+    monkeypatch.setattr(decode_plan, "_TWO_PLANE_KEYS", 600)
+    monkeypatch.setattr(decode_plan, "_TWO_PLANE_STEPS", 6)
+    B, Hq, Hkv, D, window = 2, 8, 2, 128, 70
+    cfgs = [sa.SinkMaskerConfig(sink_size=9), sa.LocalMaskerConfig(window_size=window), sa.HashAttentionTopKMaskerConfig(
+        heavy_size=50, hat_bits=32, hat_mlp_layers=3, hat_mlp_hidden_size=128, hat_mlp_activation="silu",
+        hat_weights=random_hat_weights(1, Hq, D, 32, 3, 128, dtype=dtype, seed=1))]
+    _, k, v = make_qkv(B, Hq, Hkv, 1, 800, D, dtype, seed=5, device=cuda)
+    outs = []
+    for planned in (True, False):
+        ra = sa.ResearchAttention.create_from_config(sa.ResearchAttentionConfig(masker_configs=cfgs))
+        ra.return_attention_weights = False
+        if not planned:
+            ra._plan_kind = None
+        meta, got, built = {}, [], []
+        for i in range(14):
+            n = 560 + 16 * i  # (every fourth step hashes 64 new keys)
+            q = make_qkv(B, Hq, Hkv, 1, 1, D, dtype, seed=100 + i, device=cuda)[0]
+            m = _hide(torch.zeros((B, 1, 1, n)), "padded", n, window, float(torch.finfo(dtype).min)).to(dtype).to(cuda)
+            got.append(ra.custom_attention(None, q, k[:, :, :n], v[:, :, :n], m, D ** -0.5, 0.0, sparse_meta_data=meta, layer_idx=0)[0].double())
+            built.append(meta["key"][0].pos is not None)
+        if planned:  # (the first call fills the cache)
+            assert built == [False] * 7 + [True] * 7
+            assert meta["key"][0].n_compact == meta["key"][0].n
+        outs.append(torch.stack(got))
+    a, b = outs
+    unit = {torch.bfloat16: 2.0 ** -7, torch.float32: 2.0 ** -18}[dtype]  # as of the steps under a mask that hides columns
+    assert bool(((a - b).abs() <= unit * b.abs() + (1e-6 if dtype == torch.float32 else 2.0 ** -18)).all())
