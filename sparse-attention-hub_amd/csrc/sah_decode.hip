@@ -198,7 +198,8 @@ __global__ __launch_bounds__(HSW_NT) void k_hash_decode(hdec_params P) {
 // same arithmetic, so the lists are identical and both write the same values to the row in memory), attends to its
 // share of the list, and the one that arrives last merges the partial results (att_merge_parts).
 // HID: under an additive mask that only hides columns (A.amask; hdec_row). Four layers of a padded batch of 4 at 12K keys, 1024
-// chosen: 193 us with the scores in memory (hashing 7, scores 5, selection and attention 29 a layer), 159 so (31 a layer).
+// chosen: 193 us with the scores in memory (hashing 7, scores 5, selection and attention 29 a layer), 159 so (31 a layer; 32 with
+// the codes in two planes, which nothing has to be built for).
 template <int DT, bool MF, bool CP, int D, bool SILU, bool HID>
 __global__ __launch_bounds__(HSW_NT) void k_hash_decode_attn(hdec_params P, att_params A, int cols_offset, int parts, float* work,
                                                              uint32_t* tickets) {
