@@ -20,7 +20,7 @@ from ...metric_logging import MicroMetricLogger
 from ..base import SparseAttention, SparseAttentionConfig
 from ..utils.mask import Mask
 from ..utils.mask_attention_utils import (
-    AdditiveMaskFacts, MaskQuestion, get_masked_attention_output, get_true_attention_output, mask_covers,
+    AdditiveMaskFacts, MaskQuestion, get_masked_attention_output, get_true_attention_output,
 )
 from ..utils.native_rows import NativeRows
 from .decode_plan import DecodePlan, plan_kind
@@ -187,15 +187,18 @@ class ResearchAttention(SparseAttention):
         am = attention_mask
         facts = self._mask_facts
         flags = facts.known(am)  # (of the layers behind the first, the usual call)
-        if (am.dim() != 4 or am.shape[-1] < keys.shape[2]
+        shape = am.shape
+        if (len(shape) != 4 or shape[3] < keys.shape[2]
                 or flags is None and am.dtype not in (torch.float32, torch.bfloat16, torch.float16)):
             return am, False, None, None
         same_type = am.dtype == queries.dtype  # (a lowest value of another type is none of the queries')
         if flags is None:
-            guess = facts.guess(am, sparse_meta_data)
+            guess = facts.guess(shape[2] == 1, sparse_meta_data)
             question = MaskQuestion(am)
-            covers = mask_covers(am, queries, keys.shape[2])  # (else it has to be zero, or is refused)
-            if plannable and covers and guess is not None and (guess == 0 or queries.shape[2] == 1):
+            q_shape = queries.shape
+            # (a mask that does not cover the call has to be zero, or is refused)
+            covers = shape[2] == q_shape[2] and shape[0] in (1, q_shape[0]) and shape[1] in (1, q_shape[1])
+            if plannable and covers and guess is not None and (guess == 0 or q_shape[2] == 1):
                 hides = not guess & _native.AMASK_GENERAL and same_type
                 out, error = None, None
                 try:
@@ -210,7 +213,7 @@ class ResearchAttention(SparseAttention):
                 error = None
                 if out is not None and (flags == guess or (guess and not (hides and flags & _native.AMASK_GENERAL))):
                     return am, hides, out, None
-            elif am.shape[2] > 1 and guess != 0 and covers:
+            elif shape[2] > 1 and guess != 0 and covers:
                 return am, False, None, question
             else:
                 flags = facts.take(question, sparse_meta_data)
@@ -229,12 +232,14 @@ class ResearchAttention(SparseAttention):
         # belong to the call: a step on another stream is not ordered with the ones that use them. So do those of a step whose
         # mask is guessed to be zero: it may turn out to be a masked one. A captured step's belong to its graph alone: what its
         # plan clears is clear when the graph runs, not now; and its mask is what the buffer holds then, which may be anything.
-        owner = (_native.stream_ptr(queries.device), threading.get_ident()) if masked or guessed else None
+        device = queries.device
+        stream = _native.stream_ptr(device)
+        owner = (stream, threading.get_ident()) if masked or guessed else None
         capturing = torch.cuda.is_current_stream_capturing() if masked else None
         if capturing:
             plan, only_hides = DecodePlan(self.maskers, self._plan_kind, queries, keys, True), False
         else:
-            key = (queries.device, queries.dtype, queries.shape, keys.shape[1], masked, None if masked else owner)
+            key = (device, queries.dtype, queries.shape, keys.shape[1], masked, None if masked else owner)
             plan = self._plans.get(key)
             if plan is None or plan.owner != owner:
                 if guessed and not masked:
@@ -242,7 +247,7 @@ class ResearchAttention(SparseAttention):
                     if len(guesses) >= _GUESSED_PLANS:
                         self._plans.pop(guesses[0], None)
                 plan = self._plans[key] = DecodePlan(self.maskers, self._plan_kind, queries, keys, masked, owner)
-        return plan.run(queries, keys, values, scaling, sparse_meta_data, layer_idx, attention_mask, only_hides, guessed, capturing)
+        return plan.run(queries, keys, values, scaling, sparse_meta_data, layer_idx, attention_mask, only_hides, guessed, capturing, stream)
 
     @classmethod
     def create_from_config(cls, config: SparseAttentionConfig) -> "ResearchAttention":

@@ -221,11 +221,11 @@ class DecodePlan:
     def run(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, scaling: float,
             sparse_meta_data: Dict[Any, Any], layer_idx: Optional[int],
             attention_mask: Optional[torch.Tensor] = None, only_hides: bool = False, guessed: bool = False,
-            capturing: Optional[bool] = None) -> Optional[torch.Tensor]:
+            capturing: Optional[bool] = None, stream: Optional[int] = None) -> Optional[torch.Tensor]:
         """One layer-step; returns the attention output (B, Lq, Hq, D) or None if not applicable. `only_hides`: the mask is known
         to hold nothing but zeros and entries at the lowest value of its type or -inf. `guessed`: the step's mask may be another
-        one, under which the step must not read or write what another stream has written. `capturing`: is the
-        stream, if the caller knows."""
+        one, under which the step must not read or write what another stream has written. `capturing`,
+        `stream`: is the stream being captured, and its handle, if the caller knows."""
         masked = self.masked
         if masked and (self.Lq != 1 or attention_mask.dim() != 4):
             return None
@@ -247,7 +247,8 @@ class DecodePlan:
             return None
         if masked:  # (the blocks of other plans keep their NULL masks)
             am_keep, am_ptr, am_b, am_h, am_l = additive_mask_args(attention_mask, q, Lk)
-        stream = N.stream_ptr(self.device)
+        if stream is None:
+            stream = N.stream_ptr(self.device)
         cap = sink + window + k_eff
         self._ensure_rows(cap, Lk)
         rows = self._rows_struct(Lk)

@@ -194,9 +194,9 @@ class AdditiveMaskFacts:
             return N.AMASK_NONZERO | N.AMASK_GENERAL  # nothing established: every consumer reads the mask itself
         return None
 
-    def guess(self, am: torch.Tensor, session: Any) -> Optional[int]:
-        """The flags of the session's last mask for as many queries (one, or several)."""
-        return session.get(self._one if am.shape[2] == 1 else self._several) if isinstance(session, dict) else None
+    def guess(self, one_query: bool, session: Any) -> Optional[int]:
+        """The flags of the session's last mask for one query, or for several."""
+        return session.get(self._one if one_query else self._several) if isinstance(session, dict) else None
 
     def take(self, question: MaskQuestion, session: Any = None) -> int:
         flags = question.settle()
