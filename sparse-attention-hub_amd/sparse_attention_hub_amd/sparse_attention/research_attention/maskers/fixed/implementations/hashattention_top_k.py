@@ -54,19 +54,21 @@ class PackedSignatureCache:
     `unpack()` rebuilds the +-1 float tensor for callers that want it.
     """
 
+    # (of the class, so that a cache pickled before they were there has them)
+    # the one stream on which the compact form's buffers were cleared and written, or a masked step will write them; None:
+    # there are none, SEVERAL_STREAMS: no one
+    compact_stream: Optional[int] = None
+    masked_steps = 0  # steps of one kernel under a mask that hides columns
+
     def __init__(self, batch: int, heads: int, bits: int, capacity: int, device: torch.device):
         self.bits = bits
         self.n = 0
         capacity = (capacity + 63) // 64 * 64  # rows of codes stay 16-byte aligned for the vector loads
         self.codes = torch.empty((batch, heads, capacity, 2), dtype=torch.int32, device=device)
-        # compact form for the decode kernel (built on demand by `compact_upto`): sign planes [B, Hq, pos_pitch],
+        # compact form for the decode kernel (built by decode steps that read it): sign planes [B, Hq, pos_pitch],
         # columns with a zero component [B, Hq, exc_cap, 4] and their number [B, Hq]; valid for `n_compact` keys
         self.pos = self.exc = self.exc_cnt = None
         self.n_compact = 0
-        # the one stream on which the compact form's buffers were cleared and written, or a masked step will write them; None:
-        # there are none, SEVERAL_STREAMS: no one
-        self.compact_stream: Optional[int] = None
-        self.masked_steps = 0  # steps of one kernel under a mask that hides columns
 
     @property
     def capacity(self) -> int:

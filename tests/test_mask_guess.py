@@ -316,3 +316,11 @@ def test_guesses_of_several_threads_make_one_plan_each(device):
     for stream in range(2 * base._GUESSED_PLANS):
         sessions[0].step("z", stream)
     assert len(ra._plans) == base._GUESSED_PLANS + 1
+
+
+def test_a_saved_session_may_be_of_an_earlier_version(device):
+    """A pickled signature cache holds the attributes its class had then."""
+    s = Session(device, attention("hash"), "hash")
+    for name in ("compact_stream", "masked_steps"):
+        s.cache.__dict__.pop(name, None)
+    assert one_kernel(s.step("h")) and len(s.step("-")) == 1
