@@ -184,7 +184,7 @@ class AdditiveMaskFacts:
     def __init__(self) -> None:
         self._seen: Tuple[Optional[torch.Tensor], int, int] = (None, -1, 0)  # tensor, its version, flags
         number = next(self._numbers)
-        self._one, self._several = f"additive_mask_{number}_one_query", f"additive_mask_{number}_several_queries"
+        self._one, self._several = f"{number} one query", f"{number} several queries"
 
     def known(self, am: torch.Tensor) -> Optional[int]:
         tensor, version, flags = self._seen
@@ -196,13 +196,14 @@ class AdditiveMaskFacts:
 
     def guess(self, one_query: bool, session: Any) -> Optional[int]:
         """The flags of the session's last mask for one query, or for several."""
-        return session.get(self._one if one_query else self._several) if isinstance(session, dict) else None
+        last = session.get("additive_mask_flags") if isinstance(session, dict) else None
+        return None if last is None else last.get(self._one if one_query else self._several)
 
     def take(self, question: MaskQuestion, session: Any = None) -> int:
         flags = question.settle()
         self._seen = (question.mask, question.version, flags)
-        if isinstance(session, dict):
-            session[self._one if question.one_query else self._several] = flags
+        if isinstance(session, dict):  # (a dictionary under a name, as the caches are)
+            session.setdefault("additive_mask_flags", {})[self._one if question.one_query else self._several] = flags
         return flags
 
     def flags(self, attention_mask: torch.Tensor) -> int:
